@@ -56,7 +56,7 @@ class AmrgpuSolverOps(C.Structure):
                 ("sweep_mixed", C.c_void_p), ("qad", C.c_void_p)]
 
 
-SOLVER_ABI = 1
+SOLVER_ABI = 2
 SOLVER_PLUGIN0 = 100
 
 

@@ -480,14 +480,21 @@ std::vector<int> march_cut(int mx) {
     return cut;
 }
 
-std::vector<MarchWave> plan_march(const Level& L) {
-    // (my, segment lanes) -> strips
+// the waves of a level whose grids are cut into row strips of at most `cap`
+// rows (near-equal pieces)
+std::vector<MarchWave> march_waves(const Level& L, int cap) {
+    // (rows, segment lanes) -> strips
     std::map<std::pair<int, int>, std::vector<MarchSeg>> groups;
     for (int p = 0; p < L.ngrids; p++) {
         const PatchDesc& pd = L.patches[p];
+        const int n = (pd.my + cap - 1) / cap;
         int x = 0;
         for (int w : march_cut(pd.mx)) {
-            groups[{pd.my, march_lanes(w)}].push_back(MarchSeg{p, (int16_t)x, (int16_t)w});
+            for (int i = 0; i < n; i++) {
+                const int y0 = (int)((int64_t)pd.my * i / n), y1 = (int)((int64_t)pd.my * (i + 1) / n);
+                groups[{y1 - y0, march_lanes(w)}].push_back(
+                    MarchSeg{p, (int16_t)x, (int16_t)w, (int16_t)y0, 0});
+            }
             x += w;
         }
     }
@@ -507,6 +514,40 @@ std::vector<MarchWave> plan_march(const Level& L) {
     std::stable_sort(waves.begin(), waves.end(),
                      [](const MarchWave& a, const MarchWave& b) { return a.my > b.my; });
     return waves;
+}
+
+// How tall to cut the strips.  A wave's march is a serial chain of rows (3.05
+// us a row with FP32 arithmetic, whatever else runs), so an uncut level takes
+// the tallest grid's march however few waves it has; every cut costs three
+// rows (the halo re-solved).  With the chip full the level's rows are bound by
+// vector issue instead, 1.37 times the single wave's rate per resident wave.
+// The two bounds are blended by their cubes, which follows the measured times
+// of 24 .. 4096 uneven grids within 15 % and picks a cap within 12 % of the
+// best measured one.  Mixed Euler level, mx, my even U[8,128], sweep uncut /
+// cut: 24 grids 404 / 29 us (4 rows), 256 430 / 85 us (12 .. 16 rows), 1024
+// 445 / 260 us (32 rows), 4096 843 / 849 us (96 rows).
+std::vector<MarchWave> plan_march(const Level& L) {
+    constexpr double SLOTS = 2048;   // 256 CUs x 4 SIMDs x 2 waves (the default register bound)
+    int tall = 1;
+    for (const auto& pd : L.patches) tall = std::max(tall, pd.my);
+    int best = tall;
+    double best_cost = 0;
+    for (int cap : {tall, 96, 64, 48, 32, 24, 16, 12, 8, 6, 4}) {
+        if (cap > tall) continue;
+        double rows = 0;             // of whole waves, were all their lanes used
+        int longest = 0;
+        for (const auto& pd : L.patches) {
+            const int n = (pd.my + cap - 1) / cap;
+            int lanes = 0;
+            for (int w : march_cut(pd.mx)) lanes += march_lanes(w);
+            rows += lanes / 64.0 * (pd.my + 3 * n);
+            longest = std::max(longest, (pd.my + n - 1) / n);
+        }
+        const double chain = longest + 3, issue = 1.37 * rows / SLOTS;
+        const double cost = std::cbrt(chain * chain * chain + issue * issue * issue);
+        if (best_cost == 0 || cost < best_cost) best = cap, best_cost = cost;
+    }
+    return march_waves(L, best);
 }
 
 constexpr size_t LDS_MAX = 160 * 1024;

@@ -2,8 +2,10 @@
 // every quantity in registers (no barriers; LDS only as per-lane storage).
 //
 // The work unit is one 64-lane wave holding up to four strips (segments of
-// 16, 32 or 64 lanes) of grids of the same height my.  A strip covers the
-// interior columns x0+1 .. x0+W of its grid (W <= segment width - 4); lane
+// 16, 32 or 64 lanes) of the same height my.  A strip covers the interior
+// columns x0+1 .. x0+W (W <= segment width - 4) and rows y0+1 .. y0+my of
+// its grid (rows below are counted from y0: a strip inside the grid re-solves
+// what its two halo rows on either side need, three steps of the march); lane
 // l of the segment owns strip cell k = l - 1 (k = -1 .. W+2, the strip plus
 // its two-cell halo on either side) and the x-interface between cells k-1
 // and k.  The wave marches J = -1 .. my+1 and at each step
@@ -146,7 +148,10 @@ __global__ __launch_bounds__(256, WGS) void sweep_march_kernel(SweepArgs a) {
     const bool seg_live = sidx < D->nseg;
     const MarchSeg sg = D->seg[seg_live ? sidx : 0];
     const PatchDesc pd = a.patches[sg.patch];
-    const int W = sg.w, x0 = sg.x0, my = D->my;
+    // rows of the strip: local row R is the grid's row y0 + R; the rows -1, 0
+    // and my+1, my+2 around them are ghost rows only at the grid's own edges
+    const int W = sg.w, x0 = sg.x0, y0 = sg.y0, my = D->my;
+    const bool at_bottom = y0 == 0, at_top = y0 + my == pd.my;
     const int k = min(l - 1, W + 2);                 // strip cell of this lane
     const bool live = seg_live && l <= W + 3;
     const int col = x0 + k;                          // patch-local 1-based column
@@ -156,8 +161,8 @@ __global__ __launch_bounds__(256, WGS) void sweep_march_kernel(SweepArgs a) {
     const bool ghost_cols = live && ((x0 == 0 && k <= 0) || (x0 + W == pd.mx && k >= W + 1));
     const int64_t plane = pd.plane;
     const int mitot = pd.mitot;
-    const S* qin = static_cast<const S*>(a.qin) + pd.off;
-    S* qout = static_cast<S*>(a.qout) + pd.off;
+    const S* qin = static_cast<const S*>(a.qin) + pd.off + (int64_t)y0 * mitot;
+    S* qout = static_cast<S*>(a.qout) + pd.off + (int64_t)y0 * mitot;
     const double dtdx_d = a.dt / a.dx, dtdy_d = a.dt / a.dy;
     const T dtdx = T(dtdx_d), dtdy = T(dtdy_d);
     const T hdy = T(0.5) * dtdy;
@@ -189,7 +194,8 @@ __global__ __launch_bounds__(256, WGS) void sweep_march_kernel(SweepArgs a) {
 #pragma unroll
             for (int m = 0; m < NV; m++) ring[slot(R)][m][tid] = p[m];
         }
-        if (ghost_cols || (x_cell && (R < 1 || R > my))) {
+        const bool own = R < 1 ? at_bottom : (R > my ? at_top : true);
+        if (own && (ghost_cols || (x_cell && (R < 1 || R > my)))) {
 #pragma unroll
             for (int m = 0; m < NV; m++) qout[m * plane + li] = MIXED ? p[m] : S(q[m]);
         }
@@ -339,17 +345,17 @@ __global__ __launch_bounds__(256, WGS) void sweep_march_kernel(SweepArgs a) {
                 if (live && x0 == 0 && k == 1) {
 #pragma unroll
                     for (int m = 0; m < NV; m++)
-                        per[(int64_t)(R - 1) * NV + m] = MIXED ? fxw[m] + double(fxm[m]) : double(fxm[m]);
+                        per[(int64_t)(y0 + R - 1) * NV + m] = MIXED ? fxw[m] + double(fxm[m]) : double(fxm[m]);
                 }
                 if (live && x0 + W == pd.mx && k == W + 1) {
 #pragma unroll
                     for (int m = 0; m < NV; m++)
-                        per[(int64_t)NV * (pd.my + pd.mx) + (int64_t)(R - 1) * NV + m] =
+                        per[(int64_t)NV * (pd.my + pd.mx) + (int64_t)(y0 + R - 1) * NV + m] =
                             MIXED ? fxw[m] + double(fxp[m]) : double(fxp[m]);
                 }
             }
         }
-        if (per && x_cell && (J == 1 || J == my + 1)) {
+        if (per && x_cell && ((J == 1 && at_bottom) || (J == my + 1 && at_top))) {
             // bottom y-edge 1 (gm) and top y-edge my+1 (gp): f_y of the row
             // below the edge plus G in the flux form
             const int64_t base = J == 1 ? (int64_t)NV * (2 * pd.my + pd.mx) : (int64_t)NV * pd.my;

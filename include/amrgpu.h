@@ -408,7 +408,7 @@ int amrgpu_get_gauge_records(int maxrec, int* nrec, int* gauge, int* level, doub
  * opaque pointers and return a hipError_t value (0 = success).  The table
  * records the sizes of those blocks as its translation unit saw them; the
  * library refuses a table built against other headers. */
-#define AMRGPU_SOLVER_ABI 1
+#define AMRGPU_SOLVER_ABI 2
 #define AMRGPU_SOLVER_PARAMS_MAX 16
 #define AMRGPU_SOLVER_PLUGIN0 100      /* id of the first registered solver */
 typedef struct amrgpu_solver_ops {

@@ -92,3 +92,28 @@ def test_march_fp32_arithmetic(gpu, solver, precision):
         assert rel_l1(new[k][2:-2, 2:-2], qo[2:-2, 2:-2]) <= 1e-5, k
         assert rel_l1(new[k][2:-2, 2:-2], tile[k][2:-2, 2:-2]) <= 1e-6, k
     assert abs(cfl - cfl_t) <= 1e-6 * cfl_t
+
+
+@pytest.mark.parametrize("ngrid", [1, 40, 300])
+def test_march_row_strips(gpu, ngrid):
+    """Row strips: the cap the planner picks grows with the level (a lone grid
+    is cut every 4 rows, 300 grids about every 16), so strips meet inside a
+    grid at different rows; heights on either side of the caps.  FP64 bit for
+    bit against the tile sweep."""
+    _, cfg = both_params(orc.EULER, precision=capi.FP64)
+    rng = np.random.default_rng(77 + ngrid)
+    heights = [97, 1, 4, 5, 16, 17, 33, 64, 65, 130]
+    boxes, qs, x0 = [], [], 0
+    for k in range(ngrid):
+        mx, my = int(rng.integers(1, 40)), heights[k % len(heights)]
+        boxes.append((x0, x0 + mx - 1, 0, my - 1))
+        qs.append(random_patch(rng, orc.EULER, mx, my))
+        x0 += mx
+    h = 1.0 / 256
+    print("march row strips", ngrid, flush=True)
+    new, old, cfl, dtn = _sweep(cfg, boxes, qs, capi.LAUNCH_MARCH, 0.1 * h, h)
+    tile, told, tcfl, tdtn = _sweep(cfg, boxes, qs, capi.LAUNCH_BATCHED, 0.1 * h, h)
+    for k in range(ngrid):
+        assert np.array_equal(new[k], tile[k]), (k, boxes[k])
+        assert np.array_equal(old[k], told[k]), k
+    assert cfl == tcfl and dtn == tdtn
