@@ -65,7 +65,8 @@ struct Level {
     // as an index on the next finer level; empty: planned here
     std::vector<std::vector<std::array<int, 5>>> listbc;
     std::vector<char> listbc_set;
-    // march sweep (launch mode AMRGPU_LAUNCH_MARCH): its wave table
+    // march sweep (launch mode AMRGPU_LAUNCH_MARCH, or the default mode where it
+    // is the faster FP64 sweep): its wave table
     std::vector<MarchWave> mwaves;
     MarchWave* d_mwaves = nullptr;
     // bulk transfer tables: patch element offsets, planes, first cell
@@ -516,38 +517,60 @@ std::vector<MarchWave> march_waves(const Level& L, int cap) {
     return waves;
 }
 
-// How tall to cut the strips.  A wave's march is a serial chain of rows (3.05
-// us a row with FP32 arithmetic, whatever else runs), so an uncut level takes
-// the tallest grid's march however few waves it has; every cut costs three
-// rows (the halo re-solved).  With the chip full the level's rows are bound by
-// vector issue instead, 1.37 times the single wave's rate per resident wave.
-// The two bounds are blended by their cubes, which follows the measured times
-// of 24 .. 4096 uneven grids within 15 % and picks a cap within 12 % of the
-// best measured one.  Mixed Euler level, mx, my even U[8,128], sweep uncut /
-// cut: 24 grids 404 / 29 us (4 rows), 256 430 / 85 us (12 .. 16 rows), 1024
-// 445 / 260 us (32 rows), 4096 843 / 849 us (96 rows).
-std::vector<MarchWave> plan_march(const Level& L) {
-    constexpr double SLOTS = 2048;   // 256 CUs x 4 SIMDs x 2 waves (the default register bound)
+// How tall to cut the strips, and what the march then costs (in rows of one
+// wave).  A wave's march is a serial chain of rows, so an uncut level takes the
+// tallest grid's march however few waves it has; every cut costs three rows
+// (the halo re-solved).  With the chip full the level's rows are bound by
+// vector issue instead.
+//   FP32 arithmetic, two waves per SIMD: 3.05 us a row alone, 1.37 times the
+//   lone wave's rate per resident wave when full; the two bounds blended by
+//   their cubes follow the measured times of 24 .. 4096 uneven grids within
+//   15 % and pick a cap within 12 % of the best.  Mixed Euler level, mx, my
+//   even U[8,128], sweep uncut / cut: 24 grids 404 / 29 us (4 rows), 256 430
+//   / 85 us (12 .. 16 rows), 1024 445 / 260 us (32 rows), 4096 843 / 849 us
+//   (96 rows).
+//   FP64, one wave per SIMD: 5.5 us a row, and waves beyond the SIMDs wait
+//   for a whole march: the rows of a full chip plus half a march (24 .. 2048
+//   grids within 20 %): 256 grids 811 uncut, 215 us cut, 2048 1316 / 1238.
+std::vector<MarchWave> plan_march(const Level& L, double* cost_out = nullptr) {
+    const bool f64 = run_precision() == 0;
+    constexpr double SIMDS = 1024;   // 256 CUs x 4
     int tall = 1;
     for (const auto& pd : L.patches) tall = std::max(tall, pd.my);
     int best = tall;
     double best_cost = 0;
     for (int cap : {tall, 96, 64, 48, 32, 24, 16, 12, 8, 6, 4}) {
         if (cap > tall) continue;
-        double rows = 0;             // of whole waves, were all their lanes used
+        double rows = 0, waves = 0;  // of whole waves, were all their lanes used
         int longest = 0;
         for (const auto& pd : L.patches) {
             const int n = (pd.my + cap - 1) / cap;
             int lanes = 0;
             for (int w : march_cut(pd.mx)) lanes += march_lanes(w);
             rows += lanes / 64.0 * (pd.my + 3 * n);
+            waves += lanes / 64.0 * n;
             longest = std::max(longest, (pd.my + n - 1) / n);
         }
-        const double chain = longest + 3, issue = 1.37 * rows / SLOTS;
-        const double cost = std::cbrt(chain * chain * chain + issue * issue * issue);
+        const double chain = longest + 3;
+        const double issue = f64 ? rows / SIMDS : 1.37 * rows / (2 * SIMDS);
+        const double cost = f64 ? (waves <= SIMDS ? chain : issue + 0.5 * chain)
+                                : std::cbrt(chain * chain * chain + issue * issue * issue);
         if (best_cost == 0 || cost < best_cost) best = cap, best_cost = cost;
     }
+    if (cost_out) *cost_out = best_cost;
     return march_waves(L, best);
+}
+
+// Whether the FP64 Euler sweep of a level is better off marching in the
+// default launch mode too (the two sweeps agree bit for bit): the march's
+// rows at 5.5 us against the tile sweep's 0.22 ns a cell over a floor of 38
+// us.  Measured march / tile: 24 grids 45 / 41 us, 100 99 / 118, 256 215 /
+// 261, 512 408 / 506, 1024 697 / 993, 2048 1238 / 1913.
+bool march_pays(const Level& L, double rows) {
+    double cells = 0;
+    for (const auto& pd : L.patches) cells += (double)pd.mx * pd.my;
+    const double tile = std::cbrt(38.0 * 38.0 * 38.0 + std::pow(2.2e-4 * cells, 3));
+    return 5.5 * rows + 10.0 < tile;
 }
 
 constexpr size_t LDS_MAX = 160 * 1024;
@@ -576,8 +599,14 @@ int plan_level(Level& L) {
     if (L.d_mwaves) hipFree(L.d_mwaves);
     L.d_mwaves = nullptr;
     L.mwaves.clear();
-    if (g.launch_mode == AMRGPU_LAUNCH_MARCH && L.ngrids > 0) {
-        L.mwaves = plan_march(L);
+    const bool pick = g.launch_mode == AMRGPU_LAUNCH_BATCHED && !g.plugin &&
+                      g.cfg.solver == SOLVER_EULER && run_precision() == 0 && g.auxk == 0;
+    if ((g.launch_mode == AMRGPU_LAUNCH_MARCH || pick) && L.ngrids > 0) {
+        double rows = 0;
+        L.mwaves = plan_march(L, &rows);
+        if (pick && !march_pays(L, rows)) L.mwaves.clear();
+    }
+    if (!L.mwaves.empty()) {
         HIPCHK(hipMalloc(&L.d_mwaves, L.mwaves.size() * sizeof(MarchWave)));
         HIPCHK(h2d(L.d_mwaves, L.mwaves.data(), L.mwaves.size() * sizeof(MarchWave)));
     }
@@ -1065,7 +1094,8 @@ int launch_sweep(Level& L, double dt, double* flux_out_dev, const int64_t* flux_
     auto launch = [&](const SweepArgs& x) { return run_sweep(run_precision(), x, L.lds, g.sweep_wgs); };
     hipError_t e = hipSuccess;
     tbegin(AMRGPU_KT_SWEEP);
-    if (g.launch_mode == AMRGPU_LAUNCH_MARCH && L.d_mwaves && !flux_out_dev && !rl.sv && !a.aux) {
+    if ((g.launch_mode == AMRGPU_LAUNCH_MARCH || g.launch_mode == AMRGPU_LAUNCH_BATCHED) &&
+        L.d_mwaves && !flux_out_dev && !rl.sv && !a.aux) {
         // the march sweep writes no per-edge flux arrays and no fluxsv
         // entries: a level with a finer level, or a call asking for the
         // flux arrays, takes the tile sweep

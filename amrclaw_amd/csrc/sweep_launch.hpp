@@ -85,7 +85,9 @@ static hipError_t sweep_layout(const SweepArgs& a, size_t lds, hipStream_t st) {
 // solver, whose tuned caps they match).
 // The march sweep (a.waves set): four independent waves per workgroup, no
 // LDS.  Its register bound: 2 waves per SIMD (256 VGPRs, the default), or 3
-// with FP32 arithmetic (wgs == 3: 168 VGPRs, part of the state spilled).
+// with FP32 arithmetic (wgs == 3: 168 VGPRs, part of the state spilled).  The
+// FP64 Euler march takes one wave per SIMD (396 registers, none spilled; at
+// two, 720 bytes a lane spilled: 1024 grids 1886 us against 697 us).
 // A level with aux arrays (a capacity or a solver that reads aux): the tile
 // sweep with the run-time layout, per-lane aux loads and the capacity
 // update (FP64 or FP32 storage; the mixed path has no aux variant).
@@ -140,6 +142,8 @@ static hipError_t sweep_solver(const SweepArgs& a, size_t lds, hipStream_t st, i
             }
             if (wgs == 3) return march_go<Sol, T, S, 3>(a, st);
         }
+        if constexpr (sizeof(T) == 8 && FIXED)
+            return std_method(a.meth) ? march_go<Sol, T, S, 1, true>(a, st) : march_go<Sol, T, S, 1>(a, st);
         return march_go<Sol, T, S, 2>(a, st);
     }
     if constexpr (sizeof(T) == 4 && sizeof(S) == 8) {

@@ -205,7 +205,9 @@ int amrgpu_flag_level(int level, int flag_gradient, double tolsp, int flag_richa
                       const int64_t* offsets, int64_t* nflagged);
 
 /* Sweep launch shape: AMRGPU_LAUNCH_BATCHED (default) puts all tiles of
- * all grids of a level into one launch, one workgroup per tile;
+ * all grids of a level into one launch, one workgroup per tile (an FP64
+ * Euler level without a finer level marches instead, as below, where that
+ * is faster: the same bits);
  * AMRGPU_LAUNCH_PERSISTENT launches as many workgroups as the device holds
  * and lets them take the level's tiles (largest first) from a device
  * counter; AMRGPU_LAUNCH_PER_PATCH issues one launch per grid, the plain
