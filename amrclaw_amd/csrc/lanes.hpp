@@ -12,10 +12,12 @@ namespace amrgpu {
 // sweep never uses: the limiter and the transverse terms read a neighbour
 // only from interfaces 1..n+1 of an n-cell slice, whose neighbours 0..n+2 sit
 // in the same segment (segment width >= n + 3).
+// The wave's own last (first) lane receives 0 (bound_ctrl), which lets the
+// compiler fold the move into the FP32 instruction that uses it.
 constexpr int DPP_WAVE_SHL1 = 0x130, DPP_WAVE_SHR1 = 0x138;
 template <int CTRL>
 __device__ __forceinline__ int dpp_move(int v) {
-    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, false);
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
 }
 template <int CTRL>
 __device__ __forceinline__ float dpp_move(float v) {
@@ -31,5 +33,13 @@ template <typename T>
 __device__ __forceinline__ T lane_down(T v, int) { return dpp_move<DPP_WAVE_SHL1>(v); }
 template <typename T>
 __device__ __forceinline__ T lane_up(T v, int) { return dpp_move<DPP_WAVE_SHR1>(v); }
+// lane i-1's a plus b, as one instruction with FP32 operands: left to
+// contract, b's last product and the sum become one fused operation and the
+// move an instruction of its own.
+template <typename T>
+__device__ __forceinline__ T lane_up_add(T a, T b) {
+#pragma clang fp contract(off)
+    return dpp_move<DPP_WAVE_SHR1>(a) + b;
+}
 
 }  // namespace amrgpu

@@ -71,6 +71,12 @@ template <typename T, class Mth = ExactMath<T>> struct Advection3 {
         bm[0] = dmin1(sp, T(0)) * asdq[0];
         bp[0] = dmax1(sp, T(0)) * asdq[0];
     }
+    __device__ static void split_times(const Physics3& ph, int ixyz, int icoor, const Cache& c,
+                                       T scale, const T asdq[NV], T bm[NV], T bp[NV]) {
+        split(ph, ixyz, icoor, nullptr, nullptr, c, asdq, bm, bp);
+        bm[0] = scale * bm[0];
+        bp[0] = scale * bp[0];
+    }
 };
 
 // ----------------------------------------------------------------------------
@@ -210,12 +216,50 @@ template <typename T, class Mth = ExactMath<T>> struct Euler3 {
         }
     }
 
+    // FP32: `scale` times the down- and up-going parts of d along md, by the
+    // strengths of the waves, without forming them (the eigenvectors share ud,
+    // u1, u2 and H): about 54 instructions against 70
+    __device__ static void split_scaled(const Cache& c, int md, int o1, int o2, const T* d,
+                                        T scale, T bm[NV], T bp[NV]) {
+        const T ud = c.u[md - 1], a = c.a, u1 = c.u[o1 - 1], u2 = c.u[o2 - 1];
+        const T a4 = c.g1a2 * (c.euv * d[0] + c.u[0] * d[1] + c.u[1] * d[2] + c.u[2] * d[3] - d[4]);
+        const T a2 = d[o1] - u1 * d[0];
+        const T a3 = d[o2] - u2 * d[0];
+        const T a5 = Mth::div(d[md] + (a - ud) * d[0] - a * a4, T(2) * a);
+        const T a1 = d[0] - a4 - a5;
+        const T uda = ud * a, hu2 = T(0.5) * c.u2;
+        auto side = [&](T s1, T s2, T s3, T out[NV]) {
+            const T e1 = s1 * a1, e4 = s2 * a4, e5 = s3 * a5, f2 = s2 * a2, f3 = s2 * a3;
+            const T sum = e1 + e5, dif = e5 - e1, all = sum + e4;
+            out[0] = all;
+            out[md] = ud * all + a * dif;
+            out[o1] = u1 * all + f2;
+            out[o2] = u2 * all + f3;
+            out[4] = c.enth * sum + uda * dif + hu2 * e4 + u1 * f2 + u2 * f3;
+        };
+        side(scale * dmin1(ud - a, T(0)), scale * dmin1(ud, T(0)), scale * dmin1(ud + a, T(0)), bm);
+        side(scale * dmax1(ud - a, T(0)), scale * dmax1(ud, T(0)), scale * dmax1(ud + a, T(0)), bp);
+    }
+
+    // scale times split (the fused step's double-transverse terms)
+    __device__ static void split_times(const Physics3&, int ixyz, int icoor, const Cache& c,
+                                       T scale, const T asdq[NV], T bm[NV], T bp[NV]) {
+        int mu, mv, mw;
+        triple3(ixyz, mu, mv, mw);
+        split_scaled(c, icoor == 2 ? mv : mw, icoor == 2 ? mw : mu, icoor == 2 ? mu : mv, asdq,
+                     scale, bm, bp);
+    }
+
     __device__ static void split(const Physics3&, int ixyz, int icoor, const T*, const T*,
                                  const Cache& c, const T asdq[NV], T bm[NV], T bp[NV]) {
         int mu, mv, mw;
         triple3(ixyz, mu, mv, mw);
         const int md = icoor == 2 ? mv : mw;
         const int o1 = icoor == 2 ? mw : mu, o2 = icoor == 2 ? mu : mv;
+        if constexpr (sizeof(T) == 4) {
+            split_scaled(c, md, o1, o2, asdq, T(1), bm, bp);
+            return;
+        }
         T wv[3][5], sp[3];
         waves(c, md, o1, o2, asdq, wv, sp);
 #pragma unroll

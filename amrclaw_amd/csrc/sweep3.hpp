@@ -65,6 +65,16 @@ struct Method3 {
     int32_t mthlim[NWMAX3];
 };
 
+// The standard method of the 3-D run configurations (method(2) = 2, method(3)
+// = 22, MC limiter on every wave, no f-waves): the fused step has an
+// instantiation with these switches fixed at compile time.
+template <class Sol> inline bool std_method3(const Method3& M) {
+    if (M.order != 2 || M.m3 != 2 || M.m4 != 2 || M.use_fwaves) return false;
+    for (int w = 0; w < Sol::NW; w++)
+        if (M.mthlim[w] != 4) return false;
+    return true;
+}
+
 struct Sweep3Args {
     void* q;                        // patch solutions (compute precision T)
     void* face;                     // flux blocks

@@ -31,6 +31,14 @@
 // from the reference, so the result agrees with it to FP32 rounding.  The
 // grid's ghost cells are read, never written: the step reads q from one
 // buffer and writes the updated interiors into another.
+//
+// Bound by vector issue (the SIMDs issue vector instructions in about 80 % of
+// their cycles at 4 cycles each), so what counts is instructions per
+// interface: the splits by wave strengths with the face weights in the speeds
+// (Euler3::split_scaled), the method's switches at compile time, a cell's
+// values together in LDS and scalar row bookkeeping took the Euler sweeps from
+// 2300 to 1830 vector instructions an interface and 256 uneven grids
+// (2,023,768 cells) from 984 to 700 us a step.
 #pragma once
 #include <cstdint>
 #include "lanes.hpp"
@@ -117,19 +125,26 @@ struct Digits3 {
 // increments to the nine cells (dQ, dP) around its own in nine ordered
 // steps, in each of which the wave's lanes touch distinct cells.  Rounds are
 // separated by barriers.
-template <class Sol, int D>
-__device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float* dq, int nbox,
-                                            int ncell, int tx, int ty, int tz, int bx, int by,
-                                            int wave, int wl, float& cfl) {
+//
+// STD: the method is known to be the standard one (std_method3: second order,
+// all transverse and double-transverse terms, MC limiter on every wave, no
+// f-waves), so its switches are compile-time constants.
+template <class Sol, int D, bool STD>
+__device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float* dq,
+                                            int tx, int ty, int tz, int bx, int by, int wave,
+                                            int wl, float& cfl) {
     using T = float;
     constexpr int NV = Sol::NV, NW = Sol::NW;
     constexpr int d = D;
     const Method3& M = a.meth;
-    const bool trans = M.m3 > 0, cq = M.m3 >= 2, tt = M.m4 > 0;
-    bool limit = false;
+    const bool trans = STD || M.m3 > 0, cq = STD || M.m3 >= 2, tt = STD || M.m4 > 0;
+    const bool tt2 = STD || M.m4 == 2, second = STD || M.order != 1;
+    bool limit = STD;
     for (int w = 0; w < NW; w++) limit = limit || M.mthlim[w] > 0;
-    // axes (r, Q, P): x (x, y, z), y (y, x, z), z (z, x, y); LDS strides
-    const int sx = 1, sy = bx, sz = bx * by;
+    // axes (r, Q, P): x (x, y, z), y (y, x, z), z (z, x, y); LDS strides (a
+    // cell's components lie together: NV is odd, so 64 cells in a row touch
+    // 64 banks, and a cell's values are one base and constant offsets)
+    const int sx = NV, sy = bx * NV, sz = bx * by * NV;
     const int tr = d == 1 ? tx : (d == 2 ? ty : tz);
     const int tq = d == 1 ? ty : tx;
     const int tp = d == 3 ? ty : tz;
@@ -137,9 +152,9 @@ __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float
     const int qsd = d == 1 ? sy : sx;
     const int psd = d == 3 ? sy : sz;
     // dq strides (tile cells, x fastest)
-    const int drs = d == 1 ? 1 : (d == 2 ? tx : tx * ty);
-    const int dqs = d == 1 ? tx : 1;
-    const int dps = d == 3 ? tx : tx * ty;
+    const int drs = NV * (d == 1 ? 1 : (d == 2 ? tx : tx * ty));
+    const int dqs = NV * (d == 1 ? tx : 1);
+    const int dps = NV * (d == 3 ? tx : tx * ty);
     const T dtdx = T(a.dtd[d - 1]);
     const T dtdy_p = T(a.dtd[d % 3]);
     const T dtdz_p = T(a.dtd[(d + 1) % 3]);
@@ -148,7 +163,7 @@ __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float
     const bool g_to_a = d != 2;
     const T half_t = T(0.5) * dtdx;
     const T sixth = T(1) / T(6);
-    const T g6 = sixth * dtdx * dtdz_p;
+    const T g6 = sixth * dtdx * dtdz_p;   // weights of the double-transverse terms
     const T h6 = sixth * dtdx * dtdy_p;
 
     // a line's lanes take its interfaces 0 .. tr; the limiter's outer
@@ -178,12 +193,12 @@ __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float
             const int Q = live ? Qr : -1;
             const int ec = live ? e : 0;
             // cells e-1 and e of the line (local -2 .. t+1)
-            const int b0 = 2 * (1 + sy + sz) + Q * qsd + P * psd + (ec - 1) * rs;
+            const int b0 = 2 * (sx + sy + sz) + P * psd + __mul24(Q, qsd) + __mul24(ec - 1, rs);
             T ql[NV], qrr[NV];
 #pragma unroll
             for (int m = 0; m < NV; m++) {
-                ql[m] = qs[m * nbox + b0];
-                qrr[m] = qs[m * nbox + b0 + rs];
+                ql[m] = qs[b0 + m];
+                qrr[m] = qs[b0 + rs + m];
             }
             const typename Sol::Cache cache = Sol::prep(M.ph, ql, qrr);
             T wave_[NW][NV], s[NW], amdq[NV], apdq[NV];
@@ -201,16 +216,19 @@ __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float
                 fadp[m] = T(0) - apdq[m];
                 cqxx[m] = T(0);
             }
-            if (M.order != 1) {
+            if (second) {
                 if (limit) {   // inlinelimiter.f on unlimited neighbour waves
-                    T wd[NW][NV], wu[NW][NV];
+                    // w(e) . w(e+1) at lane e; the product with the wave
+                    // before is the one of lane e-1
+                    T dotr[NW], dotl[NW];
 #pragma unroll
-                    for (int w = 0; w < NW; w++)
+                    for (int w = 0; w < NW; w++) {
+                        T x = T(0);
 #pragma unroll
-                        for (int m = 0; m < NV; m++) {
-                            wd[w][m] = lane_down(wave_[w][m], L);
-                            wu[w][m] = lane_up(wave_[w][m], L);
-                        }
+                        for (int m = 0; m < NV; m++) x = x + lane_down(wave_[w][m], L) * wave_[w][m];
+                        dotr[w] = x;
+                        dotl[w] = lane_up(x, L);
+                    }
                     if (live && (e == 0 || e == tr)) {
                         // the outer neighbour of the line's end: interface -1
                         // (cells -2, -1) for lane 0, tr+1 (cells tr, tr+1) for
@@ -219,35 +237,32 @@ __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float
                         T xl[NV], xr[NV];
 #pragma unroll
                         for (int m = 0; m < NV; m++) {
-                            xl[m] = qs[m * nbox + bx0];
-                            xr[m] = qs[m * nbox + bx0 + rs];
+                            xl[m] = qs[bx0 + m];
+                            xr[m] = qs[bx0 + rs + m];
                         }
                         const typename Sol::Cache cx = Sol::prep(M.ph, xl, xr);
                         T wx[NW][NV], sx_[NW], amx[NV], apx[NV];
                         Sol::rpn3(M.ph, d, xl, xr, cx, wx, sx_, amx, apx);
 #pragma unroll
-                        for (int w = 0; w < NW; w++)
+                        for (int w = 0; w < NW; w++) {
+                            T x = T(0);
 #pragma unroll
-                            for (int m = 0; m < NV; m++) {
-                                if (e == 0) wu[w][m] = wx[w][m];
-                                else wd[w][m] = wx[w][m];
-                            }
+                            for (int m = 0; m < NV; m++) x = x + wx[w][m] * wave_[w][m];
+                            if (e == 0) dotl[w] = x;
+                            else dotr[w] = x;
+                        }
                     }
                     if (live && e >= 0 && e <= tr) {
 #pragma unroll
                         for (int w = 0; w < NW; w++) {
-                            const int mth = M.mthlim[w];
+                            const int mth = STD ? 4 : M.mthlim[w];
                             if (mth == 0) continue;
-                            T wn2 = T(0), dotr = T(0), dotl = T(0);
+                            T wn2 = T(0);
 #pragma unroll
-                            for (int m = 0; m < NV; m++) {
-                                wn2 = wn2 + wave_[w][m] * wave_[w][m];
-                                dotr = dotr + wave_[w][m] * wd[w][m];
-                                dotl = dotl + wu[w][m] * wave_[w][m];
-                            }
+                            for (int m = 0; m < NV; m++) wn2 = wn2 + wave_[w][m] * wave_[w][m];
                             if (wn2 == T(0)) continue;
                             using Mth = typename Sol::Math;
-                            T rr = Mth::ratio(s[w] > T(0) ? dotl : dotr, wn2);
+                            T rr = Mth::ratio(s[w] > T(0) ? dotl[w] : dotr[w], wn2);
                             T wlim = phi_limiter3<Mth>(mth, rr);
 #pragma unroll
                             for (int m = 0; m < NV; m++) wave_[w][m] = wlim * wave_[w][m];
@@ -260,7 +275,7 @@ __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float
                     T c = T(0);
 #pragma unroll
                     for (int w = 0; w < NW; w++) {
-                        const T fac = M.use_fwaves ? (s[w] >= T(0) ? T(1) : T(-1)) : fabs(s[w]);
+                        const T fac = !STD && M.use_fwaves ? (s[w] >= T(0) ? T(1) : T(-1)) : fabs(s[w]);
                         c = c + T(0.5) * fac * (T(1) - fabs(s[w]) * dtdxave) * wave_[w][m];
                     }
                     cqxx[m] = c;
@@ -299,88 +314,51 @@ __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float
                     // fam 0 = gadd: primary split along icoor 2; fam 1 = hadd
                     const int ip = fam, is = 1 - fam;   // primary, secondary
                     const int icp = 2 + ip;
-                    const T w6 = fam == 0 ? g6 : h6;
-                    T tmp[NV], rm[NV], rp[NV], sm[NV], sp[NV];
-                    // right-cell partials of interface e (cell e): slot
-                    // k = (s-1)*3 + (o+1), flux3.f:450-505
-                    T v[6][NV];
-#pragma unroll
-                    for (int k = 0; k < 6; k++)
-#pragma unroll
-                        for (int m = 0; m < NV; m++) v[k][m] = T(0);
-#pragma unroll
-                    for (int m = 0; m < NV; m++) {
-                        v[1][m] = T(0) - half_t * As[ip][0][m];
-                        v[4][m] = T(0) - half_t * As[ip][1][m];
-                    }
-                    if (tt) {
-#pragma unroll
-                        for (int m = 0; m < NV; m++)
-                            tmp[m] = M.m4 == 2 ? As[is][1][m] - T(3) * Cs[is][1][m] : As[is][1][m];
-                        Sol::split(M.ph, d, icp, ql, qrr, cache, tmp, rm, rp);
-#pragma unroll
-                        for (int m = 0; m < NV; m++)
-                            tmp[m] = M.m4 == 2 ? As[is][0][m] - T(3) * Cs[is][0][m] : As[is][0][m];
-                        Sol::split(M.ph, d, icp, ql, qrr, cache, tmp, sm, sp);
-#pragma unroll
-                        for (int m = 0; m < NV; m++) {
-                            v[4][m] = v[4][m] + w6 * (rp[m] - sp[m]);
-                            v[1][m] = v[1][m] + w6 * (rm[m] - sm[m]);
-                            v[5][m] = T(0) - w6 * rp[m];
-                            v[2][m] = T(0) - w6 * rm[m];
-                            v[3][m] = T(0) + w6 * sp[m];
-                            v[0][m] = T(0) + w6 * sm[m];
-                        }
-                    }
-                    if (cq) {
-#pragma unroll
-                        for (int m = 0; m < NV; m++) {
-                            v[4][m] = v[4][m] + dtdx * Cs[ip][1][m];
-                            v[1][m] = v[1][m] + dtdx * Cs[ip][0][m];
-                        }
-                    }
-                    // cell e-1: the left neighbour's right-cell partials,
-                    // then this interface's left-cell increments (A-dq side)
-#pragma unroll
-                    for (int k = 0; k < 6; k++)
-#pragma unroll
-                        for (int m = 0; m < NV; m++) v[k][m] = lane_up(v[k][m], L);
-#pragma unroll
-                    for (int m = 0; m < NV; m++) {
-                        v[1][m] = v[1][m] - half_t * Ms[ip][0][m];
-                        v[4][m] = v[4][m] - half_t * Ms[ip][1][m];
-                    }
-                    if (tt) {
-#pragma unroll
-                        for (int m = 0; m < NV; m++)
-                            tmp[m] = M.m4 == 2 ? Ms[is][1][m] + T(3) * Cs[is][1][m] : Ms[is][1][m];
-                        Sol::split(M.ph, d, icp, ql, qrr, cache, tmp, rm, rp);
-#pragma unroll
-                        for (int m = 0; m < NV; m++)
-                            tmp[m] = M.m4 == 2 ? Ms[is][0][m] + T(3) * Cs[is][0][m] : Ms[is][0][m];
-                        Sol::split(M.ph, d, icp, ql, qrr, cache, tmp, sm, sp);
-#pragma unroll
-                        for (int m = 0; m < NV; m++) {
-                            v[4][m] = v[4][m] + w6 * (rp[m] - sp[m]);
-                            v[1][m] = v[1][m] + w6 * (rm[m] - sm[m]);
-                            v[5][m] = v[5][m] - w6 * rp[m];
-                            v[2][m] = v[2][m] - w6 * rm[m];
-                            v[3][m] = v[3][m] + w6 * sp[m];
-                            v[0][m] = v[0][m] + w6 * sm[m];
-                        }
-                    }
-                    if (cq) {
-#pragma unroll
-                        for (int m = 0; m < NV; m++) {
-                            v[4][m] = v[4][m] - dtdx * Cs[ip][1][m];
-                            v[1][m] = v[1][m] - dtdx * Cs[ip][0][m];
-                        }
-                    }
                     // slot (s, o) is the face Q+s-1 of cell row P+o (type
                     // A, across Q) or the face P+s-1 of cell row Q+o (type
                     // B, across P); a face enters the cells on its two sides
+                    // with weight h, which all its terms carry from here on
                     const bool to_a = (fam == 0) == g_to_a;
                     const T h = to_a ? dtQ : dtP;
+                    const T hw6 = h * (fam == 0 ? g6 : h6);
+                    const T hh = h * half_t, hc = h * dtdx;
+                    // The increments of cell e-1: right-cell partials of
+                    // interface e-1 (they move one lane up) and left-cell
+                    // increments of interface e, flux3.f:450-505.  Slot
+                    // k = (s-1)*3 + (o+1).  r: cell e (A+dq side), v: cell
+                    // e-1 (A-dq side); the correction enters them with
+                    // opposite signs.
+                    T v[6][NV], r[6][NV];
+                    auto half = [&](T (&x)[6][NV], const T (&S)[2][2][NV], const T sg) {
+#pragma unroll
+                        for (int m = 0; m < NV; m++) {
+                            x[1][m] = -hh * S[ip][0][m];
+                            x[4][m] = -hh * S[ip][1][m];
+                            if (cq) {
+                                x[1][m] = x[1][m] + sg * hc * Cs[ip][0][m];
+                                x[4][m] = x[4][m] + sg * hc * Cs[ip][1][m];
+                            }
+                        }
+                        if (tt) {
+                            // x[5], x[2] (o = +1) enter with a minus sign below
+                            T tmp[NV];
+#pragma unroll
+                            for (int m = 0; m < NV; m++)
+                                tmp[m] = tt2 ? S[is][1][m] - sg * T(3) * Cs[is][1][m] : S[is][1][m];
+                            Sol::split_times(M.ph, d, icp, cache, hw6, tmp, x[2], x[5]);
+#pragma unroll
+                            for (int m = 0; m < NV; m++)
+                                tmp[m] = tt2 ? S[is][0][m] - sg * T(3) * Cs[is][0][m] : S[is][0][m];
+                            Sol::split_times(M.ph, d, icp, cache, hw6, tmp, x[0], x[3]);
+#pragma unroll
+                            for (int m = 0; m < NV; m++) {
+                                x[4][m] = x[4][m] + (x[5][m] - x[3][m]);
+                                x[1][m] = x[1][m] + (x[2][m] - x[0][m]);
+                            }
+                        }
+                    };
+                    half(r, As, T(1));
+                    half(v, Ms, T(-1));
 #pragma unroll
                     for (int o = -1; o <= 1; o++) {
                         if (o != 0 && !tt) continue;
@@ -392,8 +370,9 @@ __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float
                             const int ku = to_a ? s2 + 3 * (o + 1) : (o + 1) + 3 * s2;
 #pragma unroll
                             for (int m = 0; m < NV; m++) {
-                                acc[kl][m] = acc[kl][m] - h * v[k][m];
-                                acc[ku][m] = acc[ku][m] + h * v[k][m];
+                                const T y = lane_up_add(r[k][m], v[k][m]);
+                                acc[kl][m] = o == 1 ? acc[kl][m] + y : acc[kl][m] - y;
+                                acc[ku][m] = o == 1 ? acc[ku][m] - y : acc[ku][m] + y;
                             }
                         }
                     }
@@ -403,7 +382,7 @@ __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float
             // cells (its lines share P and differ in Q)
             const int c = e - 1;
             const bool own = live && c >= 0 && c < tr;
-            const int dbase = Q * dqs + P * dps + c * drs;
+            const int dbase = P * dps + __mul24(Q, dqs) + __mul24(c, drs);
 #pragma unroll
             for (int k = 0; k < 9; k++) {
                 const int dQ = k % 3 - 1, dP = k / 3 - 1;
@@ -412,7 +391,7 @@ __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float
                     const int di = dbase + dQ * dqs + dP * dps;
 #pragma unroll
                     for (int m = 0; m < NV; m++) {
-                        T* x = &dq[m * ncell + di];
+                        T* x = &dq[di + m];
                         *x = *x + acc[k][m];
                     }
                 }
@@ -427,7 +406,7 @@ __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float
     }
 }
 
-template <class Sol>
+template <class Sol, bool STD>
 __global__ __launch_bounds__(TILE3_LANES, TILE3_WG_PER_CU) void sweep3_tile_kernel(Tile3Args a) {
     using T = float;
     constexpr int NV = Sol::NV;
@@ -439,8 +418,8 @@ __global__ __launch_bounds__(TILE3_LANES, TILE3_WG_PER_CU) void sweep3_tile_kern
     const int tx = td.tx, ty = td.ty, tz = td.tz;
     const int bx = tx + 4, by = ty + 4, bz = tz + 4;
     const int nbox = bx * by * bz, ncell = tx * ty * tz;
-    T* qs = reinterpret_cast<T*>(smem_raw);   // [NV][bz][by][bx], local -2 .. t+1
-    T* dq = qs + NV * nbox;                   // [NV][tz][ty][tx]
+    T* qs = reinterpret_cast<T*>(smem_raw);   // [bz][by][bx][NV], local -2 .. t+1
+    T* dq = qs + NV * nbox;                   // [tz][ty][tx][NV]
     const int tid = threadIdx.x;
 
     const int64_t mit = pt.mx + 4, mij = mit * (pt.my + 4);
@@ -452,24 +431,27 @@ __global__ __launch_bounds__(TILE3_LANES, TILE3_WG_PER_CU) void sweep3_tile_kern
     {
         Digits3 u(tid, bx, by, bz);
         for (int idx = tid; idx < NV * nbox; idx += TILE3_LANES, u.step())
-            qs[idx] = qin[u.m * plane + g0 + (int64_t)u.z * mij + (int64_t)u.y * mit + u.x];
+            qs[((u.z * by + u.y) * bx + u.x) * NV + u.m] = qin[u.m * plane + g0 + (int64_t)u.z * mij + (int64_t)u.y * mit + u.x];
     }
     for (int idx = tid; idx < NV * ncell; idx += TILE3_LANES) dq[idx] = T(0);
     __syncthreads();
 
-    const int wave = tid / 64, wl = tid - wave * 64;
+    // the wave's number in a scalar register, so that its rows and chunks are
+    // scalar work
+    const int wave = __builtin_amdgcn_readfirstlane(tid / 64), wl = tid - wave * 64;
     T cfl = T(0);
 
-    tile3_sweep<Sol, 1>(a, qs, dq, nbox, ncell, tx, ty, tz, bx, by, wave, wl, cfl);
-    tile3_sweep<Sol, 2>(a, qs, dq, nbox, ncell, tx, ty, tz, bx, by, wave, wl, cfl);
-    tile3_sweep<Sol, 3>(a, qs, dq, nbox, ncell, tx, ty, tz, bx, by, wave, wl, cfl);
+    tile3_sweep<Sol, 1, STD>(a, qs, dq, tx, ty, tz, bx, by, wave, wl, cfl);
+    tile3_sweep<Sol, 2, STD>(a, qs, dq, tx, ty, tz, bx, by, wave, wl, cfl);
+    tile3_sweep<Sol, 3, STD>(a, qs, dq, tx, ty, tz, bx, by, wave, wl, cfl);
 
     // q(t + dt) = q(t) + dq on the tile's cells
     T* qout = static_cast<T*>(a.qout) + pt.qoff;
     {
         Digits3 u(tid, tx, ty, tz);
         for (int idx = tid; idx < NV * ncell; idx += TILE3_LANES, u.step()) {
-            const T v = qs[u.m * nbox + (u.z + 2) * bx * by + (u.y + 2) * bx + (u.x + 2)] + dq[idx];
+            const T v = qs[((u.z + 2) * bx * by + (u.y + 2) * bx + (u.x + 2)) * NV + u.m] +
+                        dq[((u.z * ty + u.y) * tx + u.x) * NV + u.m];
             qout[u.m * plane + g0 + (int64_t)(u.z + 2) * mij + (int64_t)(u.y + 2) * mit + (u.x + 2)] = v;
         }
     }
