@@ -529,9 +529,12 @@ std::vector<MarchWave> march_waves(const Level& L, int cap) {
 //   even U[8,128], sweep uncut / cut: 24 grids 404 / 29 us (4 rows), 256 430
 //   / 85 us (12 .. 16 rows), 1024 445 / 260 us (32 rows), 4096 843 / 849 us
 //   (96 rows).
-//   FP64, one wave per SIMD: 5.5 us a row, and waves beyond the SIMDs wait
+//   FP64, one wave per SIMD: 4.9 us a row, and waves beyond the SIMDs wait
 //   for a whole march: the rows of a full chip plus half a march (24 .. 2048
-//   grids within 20 %): 256 grids 811 uncut, 215 us cut, 2048 1316 / 1238.
+//   grids within 20 %): 256 grids 811 us uncut, 215 cut, 2048 1316 / 1238.
+// (These were measured at one build; with the cells' shared quantities and the
+// sums by strength the cut marches take: mixed 24 grids 26 us, 256 81, 1024
+// 232, 4096 755; FP64 256 grids 207 us, 2048 1071.)
 std::vector<MarchWave> plan_march(const Level& L, double* cost_out = nullptr) {
     const bool f64 = run_precision() == 0;
     constexpr double SIMDS = 1024;   // 256 CUs x 4
@@ -563,14 +566,14 @@ std::vector<MarchWave> plan_march(const Level& L, double* cost_out = nullptr) {
 
 // Whether the FP64 Euler sweep of a level is better off marching in the
 // default launch mode too (the two sweeps agree bit for bit): the march's
-// rows at 5.5 us against the tile sweep's 0.22 ns a cell over a floor of 38
-// us.  Measured march / tile: 24 grids 45 / 41 us, 100 99 / 118, 256 215 /
-// 261, 512 408 / 506, 1024 697 / 993, 2048 1238 / 1913.
+// rows at 4.9 us against the tile sweep's 0.22 ns a cell over a floor of 38
+// us.  Measured march / tile: 24 grids 45 / 41 us, 100 99 / 118, 256 207 /
+// 261, 512 408 / 506, 1024 697 / 993, 2048 1071 / 1913.
 bool march_pays(const Level& L, double rows) {
     double cells = 0;
     for (const auto& pd : L.patches) cells += (double)pd.mx * pd.my;
     const double tile = std::cbrt(38.0 * 38.0 * 38.0 + std::pow(2.2e-4 * cells, 3));
-    return 5.5 * rows + 10.0 < tile;
+    return 4.9 * rows + 10.0 < tile;
 }
 
 constexpr size_t LDS_MAX = 160 * 1024;

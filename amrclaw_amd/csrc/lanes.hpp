@@ -33,13 +33,18 @@ template <typename T>
 __device__ __forceinline__ T lane_down(T v, int) { return dpp_move<DPP_WAVE_SHL1>(v); }
 template <typename T>
 __device__ __forceinline__ T lane_up(T v, int) { return dpp_move<DPP_WAVE_SHR1>(v); }
-// lane i-1's a plus b, as one instruction with FP32 operands: left to
+// lane i-1's (i+1's) a plus b, as one instruction with FP32 operands: left to
 // contract, b's last product and the sum become one fused operation and the
 // move an instruction of its own.
 template <typename T>
 __device__ __forceinline__ T lane_up_add(T a, T b) {
 #pragma clang fp contract(off)
     return dpp_move<DPP_WAVE_SHR1>(a) + b;
+}
+template <typename T>
+__device__ __forceinline__ T lane_down_add(T a, T b) {
+#pragma clang fp contract(off)
+    return dpp_move<DPP_WAVE_SHL1>(a) + b;
 }
 
 }  // namespace amrgpu

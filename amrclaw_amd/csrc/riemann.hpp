@@ -41,6 +41,22 @@ template <class S> struct sol_naux<S, decltype((void)S::NAUX, void())> {
     static constexpr int value = S::NAUX;
 };
 
+// whether a solver sums its waves by their strengths (wave_sum, rpt2_times;
+// taken with FP32 arithmetic only)
+template <class S, class = void> struct sol_by_strength { static constexpr bool value = false; };
+template <class S> struct sol_by_strength<S, decltype((void)S::BY_STRENGTH, void())> {
+    static constexpr bool value = S::BY_STRENGTH;
+};
+
+// whether a solver offers the quantities its solves derive from one state
+// alone (Cell, cell(), lane_up, and the Cell forms of prep and rpn2), which a
+// sweep that visits a cell several times computes once
+template <class S, class = void> struct sol_cells { static constexpr bool value = false; };
+template <class S> struct sol_cells<S, decltype((void)S::CELLS, void())> {
+    static constexpr bool value = S::CELLS;
+};
+struct NoCell {};
+
 // number of constants a plug-in solver may read (Physics::user)
 constexpr int SOLVER_PARAMS_MAX = 16;
 
@@ -219,6 +235,76 @@ template <typename T, class Mth = ExactMath<T>> struct EulerRoe {
     // (x + s*0); the FP64 instantiation keeps the reference's sequence
     static constexpr bool SKIPZ = sizeof(T) == 4;
 
+    // What the solves derive from one state.  FP64 (and exact arithmetic in
+    // general): every quotient and root as the solves below form it, so that
+    // sharing it between a cell's four interfaces changes no bit.  FP32: one
+    // reciprocal root gives sqrt(rho), 1/sqrt(rho) and 1/rho.
+    static constexpr bool CELLS = true;
+    struct Cell {
+        T sq;               // sqrt(rho)
+        T x[2], h;          // momenta and E + p over sq (FP32: x[0] = 1/sq, h = E + p)
+        T u[2], c;          // velocities (FP32: unused) and sound speed
+    };
+    __device__ static Cell cell(const Physics& ph, const T* q) {
+        const T gamma = T(ph.gamma), gamma1 = T(ph.gamma) - T(1);
+        Cell k;
+        if constexpr (SKIPZ) {
+            const T rs = __builtin_amdgcn_rsqf(q[0]);
+            k.sq = q[0] * rs;
+            k.x[0] = rs;
+            k.x[1] = k.u[0] = k.u[1] = T(0);
+            const T ri = rs * rs;
+            const T p = gamma1 * (q[3] - T(0.5) * (q[1] * q[1] + q[2] * q[2]) * ri);
+            k.h = q[3] + p;
+            k.c = Mth::sqrt(gamma * p * ri);
+        } else {
+            k.sq = Mth::sqrt(q[0]);
+            const T p = pressure(gamma1, q[0], q[1], q[2], q[3]);
+            k.x[0] = Mth::div(q[1], k.sq);
+            k.x[1] = Mth::div(q[2], k.sq);
+            k.h = Mth::div(q[3] + p, k.sq);
+            k.u[0] = Mth::div(q[1], q[0]);
+            k.u[1] = Mth::div(q[2], q[0]);
+            k.c = Mth::sqrt(Mth::div(gamma * p, q[0]));
+        }
+        return k;
+    }
+    // the cell of the lane before
+    template <class Move> __device__ static Cell moved(const Cell& k, Move up) {
+        Cell r;
+        r.sq = up(k.sq);
+        r.x[0] = up(k.x[0]);
+        r.x[1] = SKIPZ ? T(0) : up(k.x[1]);
+        r.h = up(k.h);
+        r.u[0] = SKIPZ ? T(0) : up(k.u[0]);
+        r.u[1] = SKIPZ ? T(0) : up(k.u[1]);
+        r.c = up(k.c);
+        return r;
+    }
+    __device__ static Cache prep(const Physics& ph, int ixy, const T* L, const T* R, const Cell& l,
+                                 const Cell& r) {
+        const int mu = (ixy == 1) ? 1 : 2, mv = (ixy == 1) ? 2 : 1;
+        const T gamma1 = T(ph.gamma) - T(1);
+        Cache c;
+        const T rhsq2 = l.sq + r.sq;
+        if constexpr (SKIPZ) {
+            const T i2 = __builtin_amdgcn_rcpf(rhsq2), wl = l.x[0] * i2, wr = r.x[0] * i2;
+            c.u = L[mu] * wl + R[mu] * wr;
+            c.v = L[mv] * wl + R[mv] * wr;
+            c.enth = l.h * wl + r.h * wr;
+        } else {
+            c.u = Mth::div(l.x[mu - 1] + r.x[mu - 1], rhsq2);
+            c.v = Mth::div(l.x[mv - 1] + r.x[mv - 1], rhsq2);
+            c.enth = Mth::div(l.h + r.h, rhsq2);
+        }
+        c.u2v2 = c.u * c.u + c.v * c.v;
+        const T a2 = gamma1 * (c.enth - T(0.5) * c.u2v2);
+        c.a = Mth::sqrt(a2);
+        c.g1a2 = Mth::div(gamma1, a2);
+        c.euv = c.enth - c.u2v2;
+        return c;
+    }
+
     __device__ static Cache prep(const Physics& ph, int ixy, const T* L, const T* R) {
         const int mu = (ixy == 1) ? 1 : 2, mv = (ixy == 1) ? 2 : 1;
         const T gamma1 = T(ph.gamma) - T(1);
@@ -243,6 +329,42 @@ template <typename T, class Mth = ExactMath<T>> struct EulerRoe {
         return gamma1 * (en - Mth::div(T(0.5) * (mx * mx + my * my), rho));
     }
 
+    // FP32 arithmetic: sums over the four waves by their strengths a1 (u-a),
+    // a2 (shear), a3 (entropy), a4 (u+a) times the coefficients c1 .. c4, along
+    // mu with the other momentum mv: the eigenvectors share u, v and H, so the
+    // waves need not be formed (13 operations against 14 per wave sum and as
+    // many to form or scale the waves)
+    static constexpr bool BY_STRENGTH = SKIPZ;
+    __device__ static void eigen_sum(int mu, int mv, T u, T v, T enth, T a, T hu2, T e1, T f, T e3,
+                                     T e4, T out[NV]) {
+        const T sum = e1 + e4, dif = e4 - e1, all = sum + e3;
+        out[0] = all;
+        out[mu] = u * all + a * dif;
+        out[mv] = v * all + f;
+        out[3] = enth * sum + u * a * dif + hu2 * e3 + v * f;
+    }
+    // sum of coef[k] * wave k of a normal solve (rpn2's waves)
+    __device__ static void wave_sum(int ixy, const Cache& c, const T wave[NW][NV],
+                                    const T coef[NW], T out[NV]) {
+        const int mu = (ixy == 1) ? 1 : 2, mv = (ixy == 1) ? 2 : 1;
+        eigen_sum(mu, mv, c.u, c.v, c.enth, c.a, T(0.5) * c.u2v2, coef[0] * wave[0][0],
+                  coef[1] * wave[1][mv], coef[2] * wave[2][0], coef[3] * wave[3][0], out);
+    }
+    // scale times rpt2
+    __device__ static void rpt2_times(int ixy, const Cache& c, T scale, const T d[NV], T bm[NV],
+                                      T bp[NV]) {
+        const int mu = (ixy == 1) ? 1 : 2, mv = (ixy == 1) ? 2 : 1;
+        const T u = c.u, v = c.v, a = c.a, hu2 = T(0.5) * c.u2v2;
+        const T a3 = c.g1a2 * (c.euv * d[0] + u * d[mu] + v * d[mv] - d[3]);
+        const T a2 = d[mu] - u * d[0];
+        const T a4 = Mth::div(d[mv] + (a - v) * d[0] - a * a3, T(2) * a);
+        const T a1 = d[0] - a3 - a4;
+        const T m1 = scale * dmin1(v - a, T(0)), m2 = scale * dmin1(v, T(0)), m4 = scale * dmin1(v + a, T(0));
+        const T p1 = scale * dmax1(v - a, T(0)), p2 = scale * dmax1(v, T(0)), p4 = scale * dmax1(v + a, T(0));
+        eigen_sum(mv, mu, v, u, c.enth, a, hu2, m1 * a1, m2 * a2, m2 * a3, m4 * a4, bm);
+        eigen_sum(mv, mu, v, u, c.enth, a, hu2, p1 * a1, p2 * a2, p2 * a3, p4 * a4, bp);
+    }
+
     // f(q) = (rho u, rho u^2 + p, rho u v, u (E + p)) along momentum mu (the
     // mixed path's FP64 fluxes): one division, by rho, shared by p and u
     __device__ static void flux(const Physics& ph, int ixy, const T* q, T f[NV]) {
@@ -259,6 +381,18 @@ template <typename T, class Mth = ExactMath<T>> struct EulerRoe {
     __device__ static void rpn2(const Physics& ph, int ixy, const T* L, const T* R,
                                 const T*, const T*, const Cache& c, T wave[NW][NV],
                                 T s[NW], T amdq[NV], T apdq[NV]) {
+        rpn2_from<false>(ph, ixy, L, R, Cell(), Cell(), c, wave, s, amdq, apdq);
+    }
+    __device__ static void rpn2(const Physics& ph, int ixy, const T* L, const T* R, const Cell& l,
+                                const Cell& r, const Cache& c, T wave[NW][NV], T s[NW],
+                                T amdq[NV], T apdq[NV]) {
+        rpn2_from<true>(ph, ixy, L, R, l, r, c, wave, s, amdq, apdq);
+    }
+    // KNOWN: the two states' cells are given
+    template <bool KNOWN>
+    __device__ static void rpn2_from(const Physics& ph, int ixy, const T* L, const T* R,
+                                     const Cell& cl, const Cell& cr, const Cache& c,
+                                     T wave[NW][NV], T s[NW], T amdq[NV], T apdq[NV]) {
         const int mu = (ixy == 1) ? 1 : 2, mv = (ixy == 1) ? 2 : 1;
         const T gamma = T(ph.gamma), gamma1 = T(ph.gamma) - T(1);
         const T u = c.u, v = c.v, enth = c.enth, a = c.a;
@@ -288,10 +422,15 @@ template <typename T, class Mth = ExactMath<T>> struct EulerRoe {
                     if (!(SKIPZ && wave_zero(ixy, mw, m)))
                         am[m] = am[m] + dmin1(s[mw], T(0)) * wave[mw][m];
         } else {
-            T rhoim1 = L[0];
-            T pim1 = pressure(gamma1, L[0], L[1], L[2], L[3]);
-            T cim1 = Mth::sqrt(Mth::div(gamma * pim1, rhoim1));
-            T s0 = Mth::div(L[mu], rhoim1) - cim1;
+            T s0;
+            if constexpr (KNOWN) {
+                s0 = (SKIPZ ? L[mu] * (cl.x[0] * cl.x[0]) : cl.u[mu - 1]) - cl.c;
+            } else {
+                T rhoim1 = L[0];
+                T pim1 = pressure(gamma1, L[0], L[1], L[2], L[3]);
+                T cim1 = Mth::sqrt(Mth::div(gamma * pim1, rhoim1));
+                s0 = Mth::div(L[mu], rhoim1) - cim1;
+            }
             if (!(s0 >= T(0) && s[0] > T(0))) {
                 T rho1 = L[0] + wave[0][0];
                 T rhou1 = L[mu] + wave[0][mu];
@@ -314,10 +453,15 @@ template <typename T, class Mth = ExactMath<T>> struct EulerRoe {
                     for (int m = 0; m < 4; m++)
                         am[m] = (SKIPZ && wave_zero(ixy, 1, m) ? am[m] : am[m] + s[1] * wave[1][m]) +
                                 s[2] * wave[2][m];
-                    T rhoi = R[0];
-                    T pi_ = pressure(gamma1, R[0], R[1], R[2], R[3]);
-                    T ci = Mth::sqrt(Mth::div(gamma * pi_, rhoi));
-                    T s3 = Mth::div(R[mu], rhoi) + ci;
+                    T s3;
+                    if constexpr (KNOWN) {
+                        s3 = (SKIPZ ? R[mu] * (cr.x[0] * cr.x[0]) : cr.u[mu - 1]) + cr.c;
+                    } else {
+                        T rhoi = R[0];
+                        T pi_ = pressure(gamma1, R[0], R[1], R[2], R[3]);
+                        T ci = Mth::sqrt(Mth::div(gamma * pi_, rhoi));
+                        s3 = Mth::div(R[mu], rhoi) + ci;
+                    }
                     T rho2 = R[0] - wave[3][0];
                     T rhou2 = R[mu] - wave[3][mu];
                     T rhov2 = R[mv] - wave[3][mv];
@@ -338,6 +482,18 @@ template <typename T, class Mth = ExactMath<T>> struct EulerRoe {
                         for (int m = 0; m < 4; m++) am[m] = am[m] + sf4 * wave[3][m];
                     }
                 }
+            }
+        }
+        if constexpr (SKIPZ) {
+            if (ph.efix) {
+                T df[NV];
+                wave_sum(ixy, c, wave, s, df);
+#pragma unroll
+                for (int m = 0; m < 4; m++) {
+                    amdq[m] = am[m];
+                    apdq[m] = df[m] - am[m];
+                }
+                return;
             }
         }
 #pragma unroll

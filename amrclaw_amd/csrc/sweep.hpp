@@ -22,6 +22,7 @@
 // barrier-separated steps, rows in ascending order, as the reference's
 // j (i) loop does.
 #pragma once
+#include <type_traits>
 #include "lanes.hpp"
 #include "level.hpp"
 
@@ -135,11 +136,15 @@ template <class Sol, typename T> struct LaneResult {
 //
 // AUX: the level has aux arrays; ax holds the lane's values (dtdx is then
 // unused: the two cells' dtdx1d replace it where flux2.f reads them).
-template <class Sol, typename T, bool FLUXFORM = false, bool STD = false, bool AUX = false>
+//
+// C: the solver's Cell when the caller has the two states' cells (cl, cr).
+template <class Sol, typename T, bool FLUXFORM = false, bool STD = false, bool AUX = false,
+          class C = NoCell>
 __device__ __forceinline__ void flux2_lane(const MethodArgs& M, int ixy, const T* ql,
                                            const T* qr, bool inner, int w, T dtdx,
                                            LaneResult<Sol, T>& o,
-                                           const LaneAux<T, lane_naux<Sol>()>* ax = nullptr) {
+                                           const LaneAux<T, lane_naux<Sol>()>* ax = nullptr,
+                                           const C& cl = C(), const C& cr = C()) {
     constexpr int NV = Sol::NV, NW = Sol::NW;
     constexpr bool SAUX = AUX && sol_naux<Sol>::value > 0;   // the solver reads aux
     const T dtl = AUX ? ax->dtl : dtdx, dtr = AUX ? ax->dtr : dtdx;
@@ -147,10 +152,16 @@ __device__ __forceinline__ void flux2_lane(const MethodArgs& M, int ixy, const T
     // the wave components that are zero by construction and the additions
     // of zero that the reference's sums start from
     constexpr bool SKIPZ = sizeof(T) == 4;
-    typename Sol::Cache cache = Sol::prep(M.ph, ixy, ql, qr);
+    typename Sol::Cache cache;
     T wave[NW][NV], s[NW], amdq[NV], apdq[NV];
-    Sol::rpn2(M.ph, ixy, ql, qr, SAUX ? ax->l : nullptr, SAUX ? ax->r : nullptr, cache, wave, s,
-              amdq, apdq);
+    if constexpr (std::is_same<C, NoCell>::value) {
+        cache = Sol::prep(M.ph, ixy, ql, qr);
+        Sol::rpn2(M.ph, ixy, ql, qr, SAUX ? ax->l : nullptr, SAUX ? ax->r : nullptr, cache, wave, s,
+                  amdq, apdq);
+    } else {
+        cache = Sol::prep(M.ph, ixy, ql, qr, cl, cr);
+        Sol::rpn2(M.ph, ixy, ql, qr, cl, cr, cache, wave, s, amdq, apdq);
+    }
 
     if (FLUXFORM) {
 #pragma unroll
@@ -172,12 +183,14 @@ __device__ __forceinline__ void flux2_lane(const MethodArgs& M, int ixy, const T
     }
     o.cfl = cfl;
 
-    T cqxx[NV];
+    constexpr bool BYS = SKIPZ && !AUX && sol_by_strength<Sol>::value;
+    T cqxx[NV], wlim[NW];   // by strength the limiter's factors stay apart from the waves
 #pragma unroll
     for (int m = 0; m < NV; m++) cqxx[m] = T(0);
     if (STD || M.order != 1) {
 #pragma unroll
         for (int mw = 0; mw < NW; mw++) {
+            wlim[mw] = T(1);
             T wn2 = T(0), dotr = T(0);
 #pragma unroll
             for (int m = 0; m < NV; m++) {
@@ -192,18 +205,28 @@ __device__ __forceinline__ void flux2_lane(const MethodArgs& M, int ixy, const T
                 using Mth = typename Sol::Math;
                 T r = Mth::ratio((s[mw] > T(0)) ? dotl : dotr, wn2);
                 T wl = phi_limiter<Mth>(mth, r);
+                wlim[mw] = wl;
 #pragma unroll
                 for (int m = 0; m < NV; m++)
-                    if (!(SKIPZ && Sol::wave_zero(ixy, mw, m))) wave[mw][m] = wl * wave[mw][m];
+                    if (!BYS && !(SKIPZ && Sol::wave_zero(ixy, mw, m))) wave[mw][m] = wl * wave[mw][m];
             }
         }
         const T dtdxave = T(0.5) * (dtl + dtr);
-#pragma unroll
-        for (int m = 0; m < NV; m++) {
-            T c = T(0);
+        if constexpr (BYS) {
+            T coef[NW];
 #pragma unroll
             for (int mw = 0; mw < NW; mw++) {
-                if (SKIPZ && Sol::wave_zero(ixy, mw, m)) continue;
+                T abs_sign = (!STD && M.use_fwaves) ? copysign(T(1), s[mw]) : fabs(s[mw]);
+                coef[mw] = wlim[mw] * (abs_sign * (T(1) - fabs(s[mw]) * dtdxave));
+            }
+            Sol::wave_sum(ixy, cache, wave, coef, cqxx);
+        }
+#pragma unroll
+        for (int m = 0; m < NV; m++) {
+            T c = BYS ? cqxx[m] : T(0);
+#pragma unroll
+            for (int mw = 0; mw < NW; mw++) {
+                if (BYS || (SKIPZ && Sol::wave_zero(ixy, mw, m))) continue;
                 T abs_sign = (!STD && M.use_fwaves) ? copysign(T(1), s[mw]) : fabs(s[mw]);
                 c = c + abs_sign * (T(1) - fabs(s[mw]) * dtdxave) * wave[mw][m];
             }
@@ -222,6 +245,18 @@ __device__ __forceinline__ void flux2_lane(const MethodArgs& M, int ixy, const T
             }
         }
         T bm1[NV], bp1[NV], bm2[NV], bp2[NV];
+        if constexpr (BYS) {
+            // 0.5 dtdx1d enters through the transverse speeds
+            const T hdt = T(0.5) * dtdx;
+            Sol::rpt2_times(ixy, cache, hdt, amdq, bm1, bp1);
+            Sol::rpt2_times(ixy, cache, hdt, apdq, bm2, bp2);
+#pragma unroll
+            for (int m = 0; m < NV; m++) {
+                o.g1[m] = -lane_down_add(bm1[m], bm2[m]);   // imp=1 result of interface k+1
+                o.g2[m] = -lane_down_add(bp1[m], bp2[m]);
+            }
+            return;
+        }
         Sol::rpt2(M.ph, ixy, 1, ql, qr, SAUX ? ax->lm : nullptr, SAUX ? ax->l : nullptr,
                   SAUX ? ax->lp : nullptr, cache, amdq, bm1, bp1);
         Sol::rpt2(M.ph, ixy, 2, ql, qr, SAUX ? ax->rm : nullptr, SAUX ? ax->r : nullptr,

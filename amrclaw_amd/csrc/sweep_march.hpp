@@ -32,6 +32,14 @@
 //   gadd(k,1) = (0 - 0.5 dtdx B(A-dq)(k+1)) - 0.5 dtdx B(A+dq)(k)
 // so an FP64 instantiation built without contraction reproduces the
 // reference bit for bit.
+//
+// Bound by vector issue: with FP32 arithmetic the SIMDs issue vector
+// instructions in 86 % of their cycles (4 cycles each) when the chip is full.
+// What a solve derives from one state alone (roots and quotients) is computed
+// once per cell and used by its four interfaces, with the same bits (Sol::Cell);
+// FP32 arithmetic sums the waves by their strengths.  4096 uneven mixed Euler
+// grids (18.9 M cells): 849 us a sweep before the two, 755 after; 2048 FP64
+// grids 1238 and 1071 us.
 #pragma once
 #include "sweep.hpp"
 
@@ -40,8 +48,9 @@ namespace amrgpu {
 // flux2.f after rpn2 for one interface whose neighbours' waves are known
 // through the dot products dotl (with the interface before) and dotr (with
 // the one after): CFL, limiter, second-order correction, transverse solves.
-// Returns the fluctuations fadm / fadp and the raw transverse results
-// B(A-dq) (bm1, bp1) and B(A+dq) (bm2, bp2); the caller assembles gadd from
+// Returns the fluctuations fadm / fadp and the transverse results
+// B(A-dq) (bm1, bp1) and B(A+dq) (bm2, bp2), raw or, where the solver sums by
+// strength, times 0.5 dtdx; the caller assembles gadd from
 // them and the neighbouring interfaces' results.  Same arithmetic as
 // flux2_lane.
 template <class Sol, typename T, bool FLUXFORM, bool STD = false>
@@ -64,12 +73,14 @@ __device__ __forceinline__ void flux2_finish(const MethodArgs& M, const int ixy,
 #pragma unroll
         for (int mw = 0; mw < NW; mw++) cfl = dmax1(dmax1(cfl, dtdx * s[mw]), -dtdx * s[mw]);
     }
-    T cqxx[NV];
+    constexpr bool BYS = SKIPZ && sol_by_strength<Sol>::value;
+    T cqxx[NV], wlim[NW];   // by strength the limiter's factors stay apart from the waves
 #pragma unroll
     for (int m = 0; m < NV; m++) cqxx[m] = T(0);
     if (STD || M.order != 1) {
 #pragma unroll
         for (int mw = 0; mw < NW; mw++) {
+            wlim[mw] = T(1);
             T wn2 = T(0);
 #pragma unroll
             for (int m = 0; m < NV; m++) {
@@ -81,18 +92,28 @@ __device__ __forceinline__ void flux2_finish(const MethodArgs& M, const int ixy,
                 using Mth = typename Sol::Math;
                 T r = Mth::ratio((s[mw] > T(0)) ? dotl[mw] : dotr[mw], wn2);
                 T wl = phi_limiter<Mth>(mth, r);
+                wlim[mw] = wl;
 #pragma unroll
                 for (int m = 0; m < NV; m++)
-                    if (!(SKIPZ && Sol::wave_zero(ixy, mw, m))) wave[mw][m] = wl * wave[mw][m];
+                    if (!BYS && !(SKIPZ && Sol::wave_zero(ixy, mw, m))) wave[mw][m] = wl * wave[mw][m];
             }
         }
         const T dtdxave = T(0.5) * (dtdx + dtdx);
-#pragma unroll
-        for (int m = 0; m < NV; m++) {
-            T c = T(0);
+        if constexpr (BYS) {
+            T coef[NW];
 #pragma unroll
             for (int mw = 0; mw < NW; mw++) {
-                if (SKIPZ && Sol::wave_zero(ixy, mw, m)) continue;
+                T abs_sign = (!STD && M.use_fwaves) ? copysign(T(1), s[mw]) : fabs(s[mw]);
+                coef[mw] = wlim[mw] * (abs_sign * (T(1) - fabs(s[mw]) * dtdxave));
+            }
+            Sol::wave_sum(ixy, cache, wave, coef, cqxx);
+        }
+#pragma unroll
+        for (int m = 0; m < NV; m++) {
+            T c = BYS ? cqxx[m] : T(0);
+#pragma unroll
+            for (int mw = 0; mw < NW; mw++) {
+                if (BYS || (SKIPZ && Sol::wave_zero(ixy, mw, m))) continue;
                 T abs_sign = (!STD && M.use_fwaves) ? copysign(T(1), s[mw]) : fabs(s[mw]);
                 c = c + abs_sign * (T(1) - fabs(s[mw]) * dtdxave) * wave[mw][m];
             }
@@ -109,8 +130,14 @@ __device__ __forceinline__ void flux2_finish(const MethodArgs& M, const int ixy,
                 apdq[m] = apdq[m] - cqxx[m];
             }
         }
-        Sol::rpt2(M.ph, ixy, 1, ql, qr, nullptr, nullptr, nullptr, cache, amdq, bm1, bp1);
-        Sol::rpt2(M.ph, ixy, 2, ql, qr, nullptr, nullptr, nullptr, cache, apdq, bm2, bp2);
+        if constexpr (BYS) {
+            // already times 0.5 dtdx1d, through the transverse speeds
+            Sol::rpt2_times(ixy, cache, T(0.5) * dtdx, amdq, bm1, bp1);
+            Sol::rpt2_times(ixy, cache, T(0.5) * dtdx, apdq, bm2, bp2);
+        } else {
+            Sol::rpt2(M.ph, ixy, 1, ql, qr, nullptr, nullptr, nullptr, cache, amdq, bm1, bp1);
+            Sol::rpt2(M.ph, ixy, 2, ql, qr, nullptr, nullptr, nullptr, cache, apdq, bm2, bp2);
+        }
     }
 }
 
@@ -132,12 +159,18 @@ __device__ __forceinline__ void wave_dots(const int ixy, const T a[Sol::NW][Sol:
     }
 }
 
+// the solver's Cell, or nothing
+template <class Sol, bool HAS> struct march_cell { using type = NoCell; };
+template <class Sol> struct march_cell<Sol, true> { using type = typename Sol::Cell; };
+
 template <class Sol, typename T, typename S, int WGS, bool STD = false>
 __global__ __launch_bounds__(256, WGS) void sweep_march_kernel(SweepArgs a) {
     constexpr int NV = Sol::NV, NW = Sol::NW;
     constexpr bool MIXED = sizeof(T) < sizeof(S);
     constexpr bool SKIPZ = sizeof(T) == 4;
+    constexpr bool CELLS = sol_cells<Sol>::value;
     using Cache = typename Sol::Cache;
+    using Cell = typename march_cell<Sol, CELLS>::type;
     const int wv = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (wv >= a.nwaves) return;   // the whole wave leaves
     // fields read from the table directly (a local copy of the wave's
@@ -176,18 +209,23 @@ __global__ __launch_bounds__(256, WGS) void sweep_march_kernel(SweepArgs a) {
     const int tid = threadIdx.x;
     auto slot = [](int R) { return (R + 3) % 3; };   // R >= -1
 
-    // row R of this lane's column in storage precision: issued a step
+    // this lane's column, row by row: the next row to load and the row the
+    // step accepts; a cell's components are a plane apart (each address is one
+    // 64-bit addition from the one before)
+    const S* pin = qin + (col + 1);
+    S* pout = qout + (col + 1);
+    // the next row in storage precision (from row -1 on): issued a step
     // before the row is needed, so the load's latency overlaps a step's work
-    auto fetch_row = [&](int R, S p[NV]) {
-        const int64_t li = (int64_t)(R + 1) * mitot + (col + 1);
+    auto fetch_row = [&](S p[NV]) {
+        const S* x = pin;
 #pragma unroll
-        for (int m = 0; m < NV; m++) p[m] = qin[m * plane + li];
+        for (int m = 0; m < NV; m++, x += plane) p[m] = *x;
+        pin += mitot;
     };
     // row R, fetched, in compute precision; the ghost cells of the output
     // keep their time-t values (stepgrid.f updates the interior only), each
-    // written by one lane
+    // written by one lane.  Afterwards pout is at row R + 1.
     auto accept_row = [&](int R, const S p[NV], T q[NV]) {
-        const int64_t li = (int64_t)(R + 1) * mitot + (col + 1);
 #pragma unroll
         for (int m = 0; m < NV; m++) q[m] = T(p[m]);
         if constexpr (MIXED) {
@@ -196,9 +234,11 @@ __global__ __launch_bounds__(256, WGS) void sweep_march_kernel(SweepArgs a) {
         }
         const bool own = R < 1 ? at_bottom : (R > my ? at_top : true);
         if (own && (ghost_cols || (x_cell && (R < 1 || R > my)))) {
+            S* x = pout;
 #pragma unroll
-            for (int m = 0; m < NV; m++) qout[m * plane + li] = MIXED ? p[m] : S(q[m]);
+            for (int m = 0; m < NV; m++, x += plane) *x = MIXED ? p[m] : S(q[m]);
         }
+        pout += mitot;
     };
     // row R (loaded at most two steps before) in storage precision
     auto stored_row = [&](int R, S p[NV]) {
@@ -234,12 +274,15 @@ __global__ __launch_bounds__(256, WGS) void sweep_march_kernel(SweepArgs a) {
     double* per = a.reg ? a.reg + perim_offset(pd, NV) : nullptr;
 
     S pn[NV];                   // the next row, in flight
-    fetch_row(-1, pn);
+    Cell kb, kc;                // what the solves derive from rows J, J+1 alone
+    fetch_row(pn);              // row -1
     accept_row(-1, pn, qb);
-    fetch_row(0, pn);
+    if constexpr (CELLS) kb = Sol::cell(a.meth.ph, qb);
+    fetch_row(pn);              // row 0
     for (int J = -1; J <= my + 1; J++) {
         accept_row(J + 1, pn, qc);
-        if (J + 2 <= my + 2) fetch_row(J + 2, pn);   // rows -1 .. my+2 exist
+        if constexpr (CELLS) kc = Sol::cell(a.meth.ph, qc);
+        if (J + 2 <= my + 2) fetch_row(pn);   // row J+2 (rows -1 .. my+2 exist)
 
         // 4. (first, while the y-sweep's values of this step are not yet
         // live) x-row J (J >= 0): the whole flux2 slice, neighbours by DPP
@@ -248,14 +291,23 @@ __global__ __launch_bounds__(256, WGS) void sweep_march_kernel(SweepArgs a) {
             T ql[NV];
 #pragma unroll
             for (int m = 0; m < NV; m++) ql[m] = lane_up(qb[m], 0);   // cell k-1
-            flux2_lane<Sol, T, MIXED, STD>(a.meth, 1, ql, qb, xs_inner, 0, dtdx, o);
+            Cell kl;
+            if constexpr (CELLS) kl = Sol::moved(kb, [](T v) { return lane_up(v, 0); });
+            flux2_lane<Sol, T, MIXED, STD, false, Cell>(a.meth, 1, ql, qb, xs_inner, 0, dtdx, o,
+                                                        nullptr, kl, kb);
             cfl = dmax1(cfl, o.cfl);
         }
 
         // 2. y-interface J+1 (rows J, J+1): Roe cache and rpn2
-        Cache cN = Sol::prep(a.meth.ph, 2, qb, qc);
+        Cache cN;
         T wN[NW][NV], sN[NW], amN[NV], apN[NV];
-        Sol::rpn2(a.meth.ph, 2, qb, qc, nullptr, nullptr, cN, wN, sN, amN, apN);
+        if constexpr (CELLS) {
+            cN = Sol::prep(a.meth.ph, 2, qb, qc, kb, kc);
+            Sol::rpn2(a.meth.ph, 2, qb, qc, kb, kc, cN, wN, sN, amN, apN);
+        } else {
+            cN = Sol::prep(a.meth.ph, 2, qb, qc);
+            Sol::rpn2(a.meth.ph, 2, qb, qc, nullptr, nullptr, cN, wN, sN, amN, apN);
+        }
         T dotr[NW];
         wave_dots<Sol, T>(2, wJ, wN, dotr);   // garbage at J = -1 (unused)
 
@@ -272,8 +324,13 @@ __global__ __launch_bounds__(256, WGS) void sweep_march_kernel(SweepArgs a) {
         if (trans && J >= 2) {
 #pragma unroll
             for (int m = 0; m < NV; m++) {
-                gy1[m] = (SKIPZ ? -(hdy * bm1[m]) : T(0) - hdy * bm1[m]) - hdy * bm2p[m];
-                gy2[m] = (SKIPZ ? -(hdy * bp1[m]) : T(0) - hdy * bp1[m]) - hdy * bp2p[m];
+                if constexpr (SKIPZ && sol_by_strength<Sol>::value) {
+                    gy1[m] = -(bm1[m] + bm2p[m]);
+                    gy2[m] = -(bp1[m] + bp2p[m]);
+                } else {
+                    gy1[m] = (SKIPZ ? -(hdy * bm1[m]) : T(0) - hdy * bm1[m]) - hdy * bm2p[m];
+                    gy2[m] = (SKIPZ ? -(hdy * bp1[m]) : T(0) - hdy * bp1[m]) - hdy * bp2p[m];
+                }
             }
         }
 
@@ -313,7 +370,6 @@ __global__ __launch_bounds__(256, WGS) void sweep_march_kernel(SweepArgs a) {
         }
         if (J >= 2) {
             const int R = J - 1;
-            const int64_t li = (int64_t)(R + 1) * mitot + (col + 1);
             T fxm_r[NV];
 #pragma unroll
             for (int m = 0; m < NV; m++) fxm_r[m] = lane_down(fxm[m], 0);   // x-edge i+1
@@ -324,18 +380,19 @@ __global__ __launch_bounds__(256, WGS) void sweep_march_kernel(SweepArgs a) {
                 for (int m = 0; m < NV; m++) fxw[m] = lane_up(fxc[m], 0);
             }
             if (x_cell) {
+                S* x = pout - 3 * (int64_t)mitot;   // row J-1 (pout: row J+2)
 #pragma unroll
-                for (int m = 0; m < NV; m++) {
+                for (int m = 0; m < NV; m++, x += plane) {
                     if constexpr (MIXED) {
                         const double q = pa[m];
                         const double dx_ = (fxc[m] - fxw[m]) + (double(fxm_r[m]) - double(fxp[m]));
                         const double dy_ = (fyc[m] - fy_p[m]) + (double(gym[m]) - double(gyp_p[m]));
-                        qout[m * plane + li] = q - dtdx_d * dx_ - dtdy_d * dy_;
+                        *x = q - dtdx_d * dx_ - dtdy_d * dy_;
                     } else {
                         const T q = qa[m];
                         const T dx_ = fxm_r[m] - fxp[m];
                         const T dy_ = gym[m] - gyp_p[m];
-                        qout[m * plane + li] = S(q - dtdx * dx_ - dtdy * dy_);
+                        *x = S(q - dtdx * dx_ - dtdy * dy_);
                     }
                 }
             }
@@ -394,6 +451,7 @@ __global__ __launch_bounds__(256, WGS) void sweep_march_kernel(SweepArgs a) {
             for (int m = 0; m < NV; m++) wJ[mw][m] = wN[mw][m];
         }
         cJ = cN;
+        kb = kc;
     }
     // Courant maximum of each strip's grid: reduce within the segment
     for (int off = segw >> 1; off >= 1; off >>= 1) cfl = dmax1(cfl, __shfl_xor(cfl, off, 64));
