@@ -47,11 +47,9 @@ struct Context3 {
     int step_mode = 0;                  // 0 phase kernels, 1 fused tiles
     bool fluxes_valid = false;          // the last step kept the flux arrays
     bool last_fused = false;            // the last step was the fused one
-    std::vector<Tile3> tiles;
+    Tile3Plan tiles;
     Tile3* d_tiles = nullptr;
     void* d_q2 = nullptr;
-    size_t tile_lds = 0;
-    int xcd_start[TILE3_XCDS] = {}, xcd_count[TILE3_XCDS] = {};
     unsigned long long* d_cfl = nullptr;
     std::vector<unsigned long long> h_cfl;
     // flagging (flag2refine) and conck state
@@ -120,8 +118,7 @@ void free_batch() {
     hipFree(g3.d_tiles);
     g3.d_q2 = nullptr;
     g3.d_tiles = nullptr;
-    g3.tiles.clear();
-    g3.tile_lds = 0;
+    g3.tiles = Tile3Plan();
     g3.fluxes_valid = false;
     g3.last_fused = false;
     hipFree(g3.d_cfl);
@@ -262,14 +259,24 @@ size_t tile3_bytes(int nv, int tx, int ty, int tz) {
 // the fused step's tiles, largest first, and the LDS the largest needs.  Each
 // grid is cut into kx x ky x kz near-equal tiles of at most TILE3_MAX cells
 // per direction whose LDS lets two workgroups
-// share a CU; of those cuts, the one with the fewest lane slots.
-void plan_tiles3(const std::vector<Patch3>& patches, int nv, std::vector<Tile3>& tiles,
-                 size_t& lds, int xcd_start[TILE3_XCDS], int xcd_count[TILE3_XCDS]) {
-    tiles.clear();
-    lds = 0;
+// share a CU; of those cuts, the one with the fewest lane slots.  With `faces`
+// (a level's marked faces per grid, each belonging to the tile of its cell, or
+// to the last tile beyond a grid's last cell) the tiles also hold the face map
+// and up to 16 KB of marks within that LDS; more marks cost occupancy only.
+void plan_tiles3(const std::vector<Patch3>& patches, int nv,
+                 const std::vector<std::vector<GridFace3>>* faces, Tile3Plan& plan) {
+    plan = Tile3Plan();
+    std::vector<Tile3>& tiles = plan.tiles;
+    size_t& lds = plan.lds;
+    int *xcd_start = plan.xcd_start, *xcd_count = plan.xcd_count;
     std::vector<std::vector<Tile3>> per(patches.size());
+    std::vector<std::vector<std::vector<Mark3>>> per_marks(patches.size());
     std::vector<int64_t> cost(patches.size(), 0);
-    const size_t cap = 160 * 1024 / TILE3_WG_PER_CU;
+    const size_t cap = 160 * 1024 / TILE3_WG_PER_CU - (faces ? 16 * 1024 : 0);
+    auto map_bytes = [&](int tx, int ty, int tz, int nmark) {
+        return !faces ? (size_t)0 : (nv == 5 ? mark3_lds_bytes<5>(tx, ty, tz, nmark)
+                                             : mark3_lds_bytes<1>(tx, ty, tz, nmark));
+    };
     std::vector<std::pair<int, int>> sx, sy, sz;
     for (int p = 0; p < (int)patches.size(); p++) {
         const Patch3& pt = patches[p];
@@ -296,7 +303,7 @@ void plan_tiles3(const std::vector<Patch3>& patches, int nv, std::vector<Tile3>&
                     const int mx_ = cnt[0][1] ? ext[0][1] : ext[0][0];
                     const int my_ = cnt[1][1] ? ext[1][1] : ext[1][0];
                     const int mz_ = cnt[2][1] ? ext[2][1] : ext[2][0];
-                    if (tile3_bytes(nv, mx_, my_, mz_) > cap) continue;
+                    if (tile3_bytes(nv, mx_, my_, mz_) + map_bytes(mx_, my_, mz_, 0) > cap) continue;
                     int64_t slots = 0;
                     for (int i = 0; i < 2; i++)
                         for (int j = 0; j < 2; j++)
@@ -329,8 +336,27 @@ void plan_tiles3(const std::vector<Patch3>& patches, int nv, std::vector<Tile3>&
                     t.tz = (int16_t)z.second;
                     per[p].push_back(t);
                     cost[p] += tile3_slots(t.tx, t.ty, t.tz);
-                    lds = std::max(lds, tile3_bytes(nv, t.tx, t.ty, t.tz));
                 }
+        per_marks[p].resize(per[p].size());
+        if (faces) {
+            // part of each axis that holds a cell (the last one past the end)
+            auto part = [](const std::vector<std::pair<int, int>>& s, int c) {
+                int i = 0;
+                while (i + 1 < (int)s.size() && c >= s[i + 1].first) i++;
+                return i;
+            };
+            for (const GridFace3& f : (*faces)[p]) {
+                const int i = part(sx, f.x), j = part(sy, f.y), l = part(sz, f.z);
+                per_marks[p][((size_t)l * sy.size() + j) * sx.size() + i].push_back(
+                    Mark3{(int16_t)(f.x - sx[i].first), (int16_t)(f.y - sy[j].first),
+                          (int16_t)(f.z - sz[l].first), (int16_t)f.dir});
+            }
+        }
+        for (size_t t = 0; t < per[p].size(); t++) {
+            const Tile3& d = per[p][t];
+            lds = std::max(lds, tile3_bytes(nv, d.tx, d.ty, d.tz) +
+                                    map_bytes(d.tx, d.ty, d.tz, (int)per_marks[p][t].size()));
+        }
     }
     // whole grids to one XCD each (workgroups go to the XCDs in turn), so
     // that neighbouring tiles share their halo rows in that XCD's L2: grids
@@ -350,7 +376,14 @@ void plan_tiles3(const std::vector<Patch3>& patches, int nv, std::vector<Tile3>&
     }
     for (int x = 0; x < TILE3_XCDS; x++) {
         xcd_start[x] = (int)tiles.size();
-        for (int p : bin[x]) tiles.insert(tiles.end(), per[p].begin(), per[p].end());
+        for (int p : bin[x])
+            for (size_t t = 0; t < per[p].size(); t++) {
+                Tile3 d = per[p][t];
+                d.mark0 = (int32_t)plan.marks.size();
+                d.nmark = (int32_t)per_marks[p][t].size();
+                plan.marks.insert(plan.marks.end(), per_marks[p][t].begin(), per_marks[p][t].end());
+                tiles.push_back(d);
+            }
         xcd_count[x] = (int)tiles.size() - xcd_start[x];
     }
 }
@@ -384,12 +417,12 @@ int define_batch(int npatch, const int* mx, const int* my, const int* mz) {
     HIPCHK3(hipMemsetAsync(g3.d_face, 0, std::max<int64_t>(1, fo) * g3.esize, g3.stream));
     if (g3.esize == 4) {
         // the fused step writes the second buffer
-        plan_tiles3(g3.patches, nv, g3.tiles, g3.tile_lds, g3.xcd_start, g3.xcd_count);
+        plan_tiles3(g3.patches, nv, nullptr, g3.tiles);
         HIPCHK3(hipMalloc(&g3.d_q2, std::max<int64_t>(1, qo) * g3.esize));
         HIPCHK3(hipMemsetAsync(g3.d_q2, 0, std::max<int64_t>(1, qo) * g3.esize, g3.stream));
-        HIPCHK3(hipMalloc(&g3.d_tiles, std::max<size_t>(1, g3.tiles.size()) * sizeof(Tile3)));
-        if (!g3.tiles.empty())
-            HIPCHK3(h2d3(g3.d_tiles, g3.tiles.data(), g3.tiles.size() * sizeof(Tile3)));
+        HIPCHK3(hipMalloc(&g3.d_tiles, std::max<size_t>(1, g3.tiles.tiles.size()) * sizeof(Tile3)));
+        if (!g3.tiles.tiles.empty())
+            HIPCHK3(h2d3(g3.d_tiles, g3.tiles.tiles.data(), g3.tiles.tiles.size() * sizeof(Tile3)));
     }
     HIPCHK3(hipMalloc(&g3.d_cfl, std::max(1, npatch) * sizeof(unsigned long long)));
     for (int k = 0; k < NKIND; k++) {
@@ -491,35 +524,50 @@ int step_io(const Step3IO& io, double dx, double dy, double dz, double dt, int e
     return AMRGPU_OK;
 }
 
-// the fused FP32 step of the batch: d_q -> d_q2 tile by tile, then swap
-int step_fused(double dx, double dy, double dz, double dt) {
+// the fused FP32 step, qin -> qout tile by tile
+int step_fused_io(const Fused3IO& io, double dx, double dy, double dz, double dt) {
     if (!(dx > 0) || !(dy > 0) || !(dz > 0) || !(dt >= 0))
         return fail3(AMRGPU_ERR_ARG, "bad mesh widths or time step");
-    if (g3.tile_lds > 160 * 1024)
-        return fail3(AMRGPU_ERR_UNSUPPORTED, "tile LDS %zu B exceeds a CU's", g3.tile_lds);
-    HIPCHK3(hipMemsetAsync(g3.d_cfl, 0, std::max(1, g3.npatch) * sizeof(unsigned long long),
+    if (io.plan->lds > 160 * 1024)
+        return fail3(AMRGPU_ERR_UNSUPPORTED, "tile LDS %zu B exceeds a CU's", io.plan->lds);
+    HIPCHK3(hipMemsetAsync(io.d_cfl, 0, std::max(1, io.npatch) * sizeof(unsigned long long),
                            g3.stream));
     Tile3Args a{};
-    a.qin = g3.d_q;
-    a.qout = g3.d_q2;
-    a.patches = g3.d_patches;
-    a.tiles = g3.d_tiles;
-    a.ntiles = (int)g3.tiles.size();
+    a.qin = io.qin;
+    a.qout = io.qout;
+    a.patches = io.d_patches;
+    a.tiles = io.d_tiles;
+    a.ntiles = (int)io.plan->tiles.size();
     for (int x = 0; x < TILE3_XCDS; x++) {
-        a.xcd_start[x] = g3.xcd_start[x];
-        a.xcd_count[x] = g3.xcd_count[x];
+        a.xcd_start[x] = io.plan->xcd_start[x];
+        a.xcd_count[x] = io.plan->xcd_count[x];
     }
     a.nv = g3.cfg.nvar;
     a.dtd[0] = dt / dx;
     a.dtd[1] = dt / dy;
     a.dtd[2] = dt / dz;
     a.meth = g3.meth;
-    a.cfl_patch = g3.d_cfl;
+    a.cfl_patch = io.d_cfl;
+    a.marks = io.d_marks;
+    a.face = static_cast<float*>(io.face);
     hipEvent_t stop;
     int rc = tbegin(0, &stop);
     if (rc) return rc;
-    HIPCHK3(launch_sweep3_tile_f32(g3.cfg.solver, a, g3.tile_lds, g3.stream));
-    rc = tend(stop);
+    HIPCHK3(launch_sweep3_tile_f32(g3.cfg.solver, a, io.plan->lds, g3.stream));
+    return tend(stop);
+}
+
+// of the batch: d_q -> d_q2, then swap
+int step_fused(double dx, double dy, double dz, double dt) {
+    Fused3IO io{};
+    io.qin = g3.d_q;
+    io.qout = g3.d_q2;
+    io.d_patches = g3.d_patches;
+    io.npatch = g3.npatch;
+    io.d_tiles = g3.d_tiles;
+    io.plan = &g3.tiles;
+    io.d_cfl = g3.d_cfl;
+    int rc = step_fused_io(io, dx, dy, dz, dt);
     if (rc) return rc;
     std::swap(g3.d_q, g3.d_q2);
     g3.fluxes_valid = false;
@@ -649,6 +697,14 @@ hipError_t ctx3_h2d(void* dst, const void* src, size_t n) { return h2d3(dst, src
 hipError_t ctx3_d2h(void* dst, const void* src, size_t n) { return d2h3(dst, src, n); }
 int ctx3_step(const Step3IO& io, double dx, double dy, double dz, double dt, int esize) {
     return step_io(io, dx, dy, dz, dt, esize);
+}
+bool ctx3_fused() { return g3.esize == 4 && g3.step_mode == 1; }
+int ctx3_step_fused(const Fused3IO& io, double dx, double dy, double dz, double dt) {
+    return step_fused_io(io, dx, dy, dz, dt);
+}
+void ctx3_plan_tiles(const std::vector<Patch3>& patches,
+                     const std::vector<std::vector<GridFace3>>& faces, Tile3Plan& plan) {
+    plan_tiles3(patches, g3.cfg.nvar, &faces, plan);
 }
 void ctx3_plan_blocks(const std::vector<Patch3>& patches, int plane_block,
                       std::vector<Block3> out[4]) {

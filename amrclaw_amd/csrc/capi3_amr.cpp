@@ -75,6 +75,14 @@ struct Lev3 {
     Upbnd3Cell* d_ucells = nullptr;
     Upbnd3Entry* d_uents = nullptr;
     Avg3Block* d_avg = nullptr;
+    // the fused FP32 step: its tiles with the faces the registers read, and
+    // the buffer it writes on the finest level (which keeps no old time; the
+    // others write their old buffer and swap roles)
+    Tile3Plan tiles;
+    Tile3* d_tiles = nullptr;
+    Mark3* d_marks = nullptr;
+    void* d_next = nullptr;
+    bool fused = false;           // planned, and its tiles fit
     // flagging (flag2refine, errf1) of the level's grids
     double* d_flags = nullptr;
     double* d_rflags = nullptr;
@@ -129,6 +137,10 @@ void free_plans(Lev3& L) {
     dfree(L.d_ucells);
     dfree(L.d_uents);
     dfree(L.d_avg);
+    dfree(L.d_tiles);
+    dfree(L.d_marks);
+    L.tiles = Tile3Plan();
+    L.fused = false;
     L.reg = Reg3Level();
 }
 
@@ -138,6 +150,7 @@ void free_level(Lev3& L) {
     for (auto& b : L.d_blocks) dfree(b);
     dfree(L.d_new);
     dfree(L.d_old);
+    dfree(L.d_next);
     dfree(L.d_cfl);
     dfree(L.d_partial);
     dfree(L.d_flags);
@@ -197,6 +210,60 @@ int ensure_fill_plans() {
     return AMRGPU_OK;
 }
 
+// The faces of a level's grids whose fluxes the registers read: fluxad.f's
+// grid perimeters (a fine level) and fluxsv.f's entries (a coarse one).
+std::vector<std::vector<GridFace3>> register_faces(const Lev3& L, bool fine) {
+    std::vector<std::vector<GridFace3>> out(L.patches.size());
+    std::vector<std::vector<bool>> seen(L.patches.size());
+    auto add = [&](int g, int dir, int x, int y, int z) {
+        const Patch3& p = L.patches[g];
+        auto& s = seen[g];
+        if (s.empty()) s.assign((size_t)3 * (p.mx + 1) * (p.my + 1) * (p.mz + 1), false);
+        const size_t at = (((size_t)dir * (p.mz + 1) + z) * (p.my + 1) + y) * (p.mx + 1) + x;
+        if (s[at]) return;
+        s[at] = true;
+        out[g].push_back(GridFace3{dir, x, y, z});
+    };
+    for (size_t g = 0; fine && g < L.patches.size(); g++) {
+        const Patch3& p = L.patches[g];
+        for (int z = 0; z < p.mz; z++)
+            for (int y = 0; y < p.my; y++) add(g, 0, 0, y, z), add(g, 0, p.mx, y, z);
+        for (int z = 0; z < p.mz; z++)
+            for (int x = 0; x < p.mx; x++) add(g, 1, x, 0, z), add(g, 1, x, p.my, z);
+        for (int y = 0; y < p.my; y++)
+            for (int x = 0; x < p.mx; x++) add(g, 2, x, y, 0), add(g, 2, x, y, p.mz);
+    }
+    for (const Sv3Entry& e : L.reg.sv) {
+        if (!e.write) continue;
+        // interior cell, 0-based; sides 1, 4, 5 its lower faces
+        const int x = e.I - 3, y = e.J - 3, z = e.K - 3;
+        switch (e.side) {
+        case 1: add(e.grid, 0, x, y, z); break;
+        case 2: add(e.grid, 1, x, y + 1, z); break;
+        case 3: add(e.grid, 0, x + 1, y, z); break;
+        case 4: add(e.grid, 1, x, y, z); break;
+        case 5: add(e.grid, 2, x, y, z); break;
+        default: add(e.grid, 2, x, y, z + 1); break;
+        }
+    }
+    return out;
+}
+
+int plan_fused(int level) {
+    Lev3& L = A.lev[level];
+    L.fused = false;
+    if (ctx3_esize() != 4 || L.patches.empty()) return AMRGPU_OK;
+    ctx3_plan_tiles(L.patches, register_faces(L, level >= 2), L.tiles);
+    if (L.tiles.lds > 160 * 1024) return AMRGPU_OK;   // too many marks in a tile
+    int rc = upload(L.d_tiles, L.tiles.tiles);
+    if (!rc) rc = upload(L.d_marks, L.tiles.marks);
+    if (rc) return rc;
+    if (level == A.H.nlev && !L.d_next)
+        HIPCHKA(hipMalloc(&L.d_next, std::max<int64_t>(1, L.q_elems) * sizeof(float)));
+    L.fused = true;
+    return AMRGPU_OK;
+}
+
 // saveqc programs and registers of every level: these need a properly
 // nested hierarchy (the ghost fill alone does not)
 int ensure_plans() {
@@ -237,6 +304,8 @@ int ensure_plans() {
             HIPCHKA(hipMalloc((void**)&L.d_reg, n * sizeof(double)));
             HIPCHKA(hipMemsetAsync(L.d_reg, 0, n * sizeof(double), ctx3_stream()));   // prepf.f
         }
+        rc = plan_fused(l);
+        if (rc) return rc;
         L.reg_gen = L.gen;
         L.reg_gen_coarse = l >= 2 ? A.lev[l - 1].gen : 0;
         L.reg_elems = L.reg.reg_elems;
@@ -634,25 +703,44 @@ int amrgpu3_advance_level(int level, double* dtlevnew, double* cfl_level) {
         if (cfl_level) *cfl_level = 0.0;
         return AMRGPU_OK;
     }
-    // old = new for levels below the finest (par_advanc)
-    if (level < A.H.nlev)
+    const bool fused = L.fused && ctx3_fused();
+    // old = new for levels below the finest (par_advanc); the fused step
+    // writes the other buffer and swaps the roles instead
+    if (level < A.H.nlev && !fused)
         HIPCHKA(hipMemcpyAsync(L.d_old, L.d_new, L.q_elems * ctx3_esize(), hipMemcpyDeviceToDevice, st));
     if (level > 1) {
         const Reg3Args ra = reg_args(level, 0);
         HIPCHKA(launch_qad3(ctx3_cfg().solver, ra, physics(), st));
     }
-    Step3IO io{};
-    io.q = L.d_new;
-    io.face = A.d_face;
-    io.d_patches = L.d_patches;
-    for (int k = 0; k < 4; k++) {
-        io.d_blocks[k] = L.d_blocks[k];
-        io.nblocks[k] = (int)L.blocks[k].size();
+    if (fused) {
+        void*& other = level < A.H.nlev ? L.d_old : L.d_next;
+        Fused3IO io{};
+        io.qin = L.d_new;
+        io.qout = other;
+        io.d_patches = L.d_patches;
+        io.npatch = (int)L.patches.size();
+        io.d_tiles = L.d_tiles;
+        io.d_marks = L.d_marks;
+        io.plan = &L.tiles;
+        io.face = A.d_face;
+        io.d_cfl = L.d_cfl;
+        rc = ctx3_step_fused(io, G.hx, G.hy, G.hz, L.possk);
+        if (rc) return rc;
+        std::swap(L.d_new, other);
+    } else {
+        Step3IO io{};
+        io.q = L.d_new;
+        io.face = A.d_face;
+        io.d_patches = L.d_patches;
+        for (int k = 0; k < 4; k++) {
+            io.d_blocks[k] = L.d_blocks[k];
+            io.nblocks[k] = (int)L.blocks[k].size();
+        }
+        io.npatch = (int)L.patches.size();
+        io.d_cfl = L.d_cfl;
+        rc = ctx3_step(io, G.hx, G.hy, G.hz, L.possk);
+        if (rc) return rc;
     }
-    io.npatch = (int)L.patches.size();
-    io.d_cfl = L.d_cfl;
-    rc = ctx3_step(io, G.hx, G.hy, G.hz, L.possk);
-    if (rc) return rc;
     if (has_fine(level)) {
         Reg3Args ra = reg_args(level + 1, level);
         HIPCHKA(launch_fluxsv3(ra, st));

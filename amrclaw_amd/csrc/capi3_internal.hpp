@@ -6,8 +6,33 @@
 
 #include "../../include/amrgpu3.h"
 #include "sweep3.hpp"
+#include "sweep3_tile.hpp"
 
 namespace amrgpu {
+
+// the fused step's tiles of a batch or level (sweep3_tile.hpp)
+struct Tile3Plan {
+    std::vector<Tile3> tiles;
+    std::vector<Mark3> marks;     // each tile's marked faces, tile by tile
+    size_t lds = 0;               // of the largest tile
+    int xcd_start[TILE3_XCDS] = {}, xcd_count[TILE3_XCDS] = {};
+};
+// a marked face of a grid: lower face, normal to dir, of its 0-based cell
+struct GridFace3 {
+    int dir, x, y, z;
+};
+// device arrays of one fused step of a level
+struct Fused3IO {
+    const void* qin;              // time t, ghost cells filled
+    void* qout;                   // time t + dt, with qin's ghost cells
+    const Patch3* d_patches;
+    int npatch;
+    const Tile3* d_tiles;
+    const Mark3* d_marks;
+    const Tile3Plan* plan;
+    void* face;                   // flux blocks: the marked faces are written
+    unsigned long long* d_cfl;
+};
 
 // device arrays of one step over a batch of grids
 struct Step3IO {
@@ -32,6 +57,11 @@ hipError_t ctx3_d2h(void* dst, const void* src, size_t n);
 // x-, y- and z-sweeps and the conservative update; esize 8 runs the FP64
 // kernels whatever the library's precision (0: the library's)
 int ctx3_step(const Step3IO& io, double dx, double dy, double dz, double dt, int esize = 0);
+// the same step by the fused FP32 kernel (ctx3_fused: FP32 and the fused mode)
+bool ctx3_fused();
+int ctx3_step_fused(const Fused3IO& io, double dx, double dy, double dz, double dt);
+void ctx3_plan_tiles(const std::vector<Patch3>& patches,
+                     const std::vector<std::vector<GridFace3>>& faces, Tile3Plan& plan);
 // the work lists of a batch: per sweep (grid, plane block), largest first;
 // update and totals (grid, 256 cells)
 void ctx3_plan_blocks(const std::vector<Patch3>& patches, int plane_block,

@@ -15,11 +15,11 @@ hipError_t launch_update3_f32(int nv, float* q, const float* face, const Patch3*
     return update3_launch<float>(nv, q, face, patches, blocks, nblocks, dtdx, dtdy, dtdz, st);
 }
 
-template <class Sol, bool STD>
-static hipError_t tile3_std_go(const Tile3Args& a, size_t lds, hipStream_t st) {
+template <class Sol, bool STD, bool MARK>
+static hipError_t tile3_one_go(const Tile3Args& a, size_t lds, hipStream_t st) {
     static size_t attr_lds = 0;
     if (lds > attr_lds) {
-        hipError_t e = hipFuncSetAttribute((const void*)sweep3_tile_kernel<Sol, STD>,
+        hipError_t e = hipFuncSetAttribute((const void*)sweep3_tile_kernel<Sol, STD, MARK>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
         attr_lds = lds;
@@ -27,15 +27,16 @@ static hipError_t tile3_std_go(const Tile3Args& a, size_t lds, hipStream_t st) {
     if (a.ntiles == 0) return hipSuccess;
     int most = 0;
     for (int x = 0; x < TILE3_XCDS; x++) most = a.xcd_count[x] > most ? a.xcd_count[x] : most;
-    hipLaunchKernelGGL((sweep3_tile_kernel<Sol, STD>), dim3(most * TILE3_XCDS), dim3(TILE3_LANES),
-                       lds, st, a);
+    hipLaunchKernelGGL((sweep3_tile_kernel<Sol, STD, MARK>), dim3(most * TILE3_XCDS),
+                       dim3(TILE3_LANES), lds, st, a);
     return hipGetLastError();
 }
 
 template <class Sol>
 static hipError_t tile3_go(const Tile3Args& a, size_t lds, hipStream_t st) {
-    return std_method3<Sol>(a.meth) ? tile3_std_go<Sol, true>(a, lds, st)
-                                    : tile3_std_go<Sol, false>(a, lds, st);
+    const bool sm = std_method3<Sol>(a.meth);
+    if (a.face) return sm ? tile3_one_go<Sol, true, true>(a, lds, st) : tile3_one_go<Sol, false, true>(a, lds, st);
+    return sm ? tile3_one_go<Sol, true, false>(a, lds, st) : tile3_one_go<Sol, false, false>(a, lds, st);
 }
 
 hipError_t launch_sweep3_tile_f32(int solver, const Tile3Args& a, size_t lds, hipStream_t st) {

@@ -51,10 +51,19 @@ constexpr int TILE3_LANES = 256;     // four waves
 constexpr int TILE3_XCDS = 8;        // workgroups go to the XCDs in turn
 constexpr int TILE3_WG_PER_CU = 2;   // workgroups a CU holds (LDS and registers sized for it)
 
-// a tile: grid `patch`, 0-based first interior cell (i0, j0, k0), extents
+// a tile: grid `patch`, 0-based first interior cell (i0, j0, k0), extents, and
+// its marked faces marks[mark0 ..+ nmark)
 struct Tile3 {
     int32_t patch;
     int16_t i0, j0, k0, tx, ty, tz, pad;
+    int32_t mark0, nmark;
+};
+
+// A face of a tile whose flux the coarse-fine registers read (fluxsv.f,
+// fluxad.f), in the tile's cells: the lower face, normal to dir (0 x, 1 y, 2
+// z), of cell (x, y, z); along dir the cell may be one past the tile.
+struct Mark3 {
+    int16_t x, y, z, dir;
 };
 
 struct Tile3Args {
@@ -70,7 +79,27 @@ struct Tile3Args {
     double dtd[3];                  // dt/dx, dt/dy, dt/dz
     Method3 meth;
     unsigned long long* cfl_patch;  // per-patch max Courant number (double bits)
+    // a level's step (null for a batch): the marked faces and the level's flux
+    // blocks, of which only those faces are written (merged form, as the phase
+    // kernels leave them); the ghost cells of qout receive qin's
+    const Mark3* marks;
+    float* face;
 };
+
+// Marked faces in LDS: for every face of the tile its mark's number + 1 (0:
+// none), the x-faces first; per mark the transverse increments and faddm
+// times dt/h, then faddp - faddm.
+struct Mark3Lds {
+    uint16_t* map;
+    float* acc;
+};
+__host__ __device__ constexpr int mark3_faces(int tx, int ty, int tz) {
+    return (tx + 1) * ty * tz + tx * (ty + 1) * tz + tx * ty * (tz + 1);
+}
+template <int NV>
+__host__ __device__ constexpr size_t mark3_lds_bytes(int tx, int ty, int tz, int nmark) {
+    return ((size_t)mark3_faces(tx, ty, tz) * 2 + 3) / 4 * 4 + (size_t)nmark * 2 * NV * sizeof(float);
+}
 
 // LDS of a tile workgroup: the staged box and the increments
 template <int NV>
@@ -112,6 +141,10 @@ struct Digits3 {
     }
 };
 
+__device__ __forceinline__ void lds_add(float* p, float v) {
+    __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
 // one sweep of a tile (D: 1 x, 2 y, 3 z, a template parameter so that every
 // component index of the solver is a compile-time constant).
 //
@@ -129,10 +162,15 @@ struct Digits3 {
 // STD: the method is known to be the standard one (std_method3: second order,
 // all transverse and double-transverse terms, MC limiter on every wave, no
 // f-waves), so its switches are compile-time constants.
-template <class Sol, int D, bool STD>
+//
+// MARK: increments to marked faces are also added to the faces' own sums.  A
+// wave's LDS additions happen in program order, each touching distinct faces;
+// waves of a round touch distinct faces as they touch distinct cells, so these
+// sums have a fixed order too.
+template <class Sol, int D, bool STD, bool MARK>
 __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float* dq,
                                             int tx, int ty, int tz, int bx, int by, int wave,
-                                            int wl, float& cfl) {
+                                            int wl, float& cfl, const Mark3Lds& mk) {
     using T = float;
     constexpr int NV = Sol::NV, NW = Sol::NW;
     constexpr int d = D;
@@ -161,6 +199,15 @@ __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float
     const T dtQ = T(a.dtd[d == 1 ? 1 : 0]);     // across Q (type A faces)
     const T dtP = T(a.dtd[d == 3 ? 1 : 2]);     // across P (type B faces)
     const bool g_to_a = d != 2;
+    // map indices of the faces across r, Q and P: base and strides of a cell's
+    // lower face in each of the three face arrays
+    const int nfx = (tx + 1) * ty * tz, nfy = tx * (ty + 1) * tz;
+    auto fbase = [&](int ax) { return ax == 0 ? 0 : (ax == 1 ? nfx : nfx + nfy); };
+    auto fstr = [&](int ax, int along) {
+        const int w = tx + (ax == 0), h = ty + (ax == 1);
+        return along == 0 ? 1 : (along == 1 ? w : w * h);
+    };
+    constexpr int AR = D - 1, AQ = D == 1 ? 1 : 0, AP = D == 3 ? 1 : 2;
     const T half_t = T(0.5) * dtdx;
     const T sixth = T(1) / T(6);
     const T g6 = sixth * dtdx * dtdz_p;   // weights of the double-transverse terms
@@ -299,6 +346,34 @@ __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float
                     acc[4][m] = T(0) - dtdx * (fadm[m] - fpl);
                 }
             }
+            const bool own = live && e >= 1;   // completes a cell of the tile's length
+            // adds v to the mark, if any, of the face at place i of the map
+            auto mark_add = [&](int i, bool ok, const T* v) {
+                const int id = ok ? mk.map[i] : 0;
+                if (id) {
+#pragma unroll
+                    for (int m = 0; m < NV; m++) lds_add(&mk.acc[(id - 1) * 2 * NV + m], v[m]);
+                }
+                return id;
+            };
+            if constexpr (MARK) {
+                T sc[NV];
+#pragma unroll
+                for (int m = 0; m < NV; m++) sc[m] = dtdx * fadm[m];
+                const int at = fbase(AR) + P * fstr(AR, AP) + __mul24(Q, fstr(AR, AQ)) + __mul24(e, fstr(AR, AR));
+                const int id = mark_add(at, live && Q >= 0 && Q < tq && P >= 0 && P < tp, sc);
+                if (id) {
+#pragma unroll
+                    for (int m = 0; m < NV; m++)
+                        mk.acc[((id - 1) * 2 + 1) * NV + m] = fadp[m] - fadm[m];
+                }
+            }
+            // the lower faces across Q and across P of this lane's cell
+            int atQ = 0, atP = 0;
+            if constexpr (MARK) {
+                atQ = fbase(AQ) + P * fstr(AQ, AP) + __mul24(Q, fstr(AQ, AQ)) + __mul24(e - 1, fstr(AQ, AR));
+                atP = fbase(AP) + P * fstr(AP, AP) + __mul24(Q, fstr(AP, AQ)) + __mul24(e - 1, fstr(AP, AR));
+            }
             if (trans) {
                 // the splits both families use, once: of cqxx, A+dq and A-dq
                 // along icoor 2 and 3 (index 0: 2, 1: 3; [0] down-, [1] up-going)
@@ -368,11 +443,21 @@ __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float
                             // lower cell (dQ, dP) and upper cell of the face
                             const int kl = to_a ? (s2 - 1) + 3 * (o + 1) : (o + 1) + 3 * (s2 - 1);
                             const int ku = to_a ? s2 + 3 * (o + 1) : (o + 1) + 3 * s2;
+                            T ys[NV];
 #pragma unroll
                             for (int m = 0; m < NV; m++) {
                                 const T y = lane_up_add(r[k][m], v[k][m]);
                                 acc[kl][m] = o == 1 ? acc[kl][m] + y : acc[kl][m] - y;
                                 acc[ku][m] = o == 1 ? acc[ku][m] - y : acc[ku][m] + y;
+                                ys[m] = o == 1 ? -y : y;
+                            }
+                            if constexpr (MARK) {
+                                const int fQ = to_a ? Q + s2 - 1 : Q + o, fP = to_a ? P + o : P + s2 - 1;
+                                const bool ok = own && fQ >= 0 && fQ < tq + (to_a ? 1 : 0) && fP >= 0 &&
+                                                fP < tp + (to_a ? 0 : 1);
+                                mark_add(to_a ? atQ + (s2 - 1) * fstr(AQ, AQ) + o * fstr(AQ, AP)
+                                              : atP + (s2 - 1) * fstr(AP, AP) + o * fstr(AP, AQ),
+                                         ok, ys);
                             }
                         }
                     }
@@ -381,7 +466,6 @@ __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float
             // nine ordered steps: in each, the wave's lanes add to distinct
             // cells (its lines share P and differ in Q)
             const int c = e - 1;
-            const bool own = live && c >= 0 && c < tr;
             const int dbase = P * dps + __mul24(Q, dqs) + __mul24(c, drs);
 #pragma unroll
             for (int k = 0; k < 9; k++) {
@@ -406,7 +490,7 @@ __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float
     }
 }
 
-template <class Sol, bool STD>
+template <class Sol, bool STD, bool MARK>
 __global__ __launch_bounds__(TILE3_LANES, TILE3_WG_PER_CU) void sweep3_tile_kernel(Tile3Args a) {
     using T = float;
     constexpr int NV = Sol::NV;
@@ -434,6 +518,24 @@ __global__ __launch_bounds__(TILE3_LANES, TILE3_WG_PER_CU) void sweep3_tile_kern
             qs[((u.z * by + u.y) * bx + u.x) * NV + u.m] = qin[u.m * plane + g0 + (int64_t)u.z * mij + (int64_t)u.y * mit + u.x];
     }
     for (int idx = tid; idx < NV * ncell; idx += TILE3_LANES) dq[idx] = T(0);
+    Mark3Lds mk{};
+    // a mark's place in the map: its face array, row by row
+    auto mark_at = [&](const Mark3& f) {
+        const int nfx = (tx + 1) * ty * tz, nfy = tx * (ty + 1) * tz;
+        const int w = tx + (f.dir == 0), h = ty + (f.dir == 1);
+        return (f.dir == 0 ? 0 : (f.dir == 1 ? nfx : nfx + nfy)) + (f.z * h + f.y) * w + f.x;
+    };
+    if constexpr (MARK) {
+        mk.map = reinterpret_cast<uint16_t*>(dq + NV * ncell);
+        const int words = (mark3_faces(tx, ty, tz) + 1) / 2;
+        mk.acc = dq + NV * ncell + words;
+        uint32_t* w = reinterpret_cast<uint32_t*>(mk.map);
+        for (int idx = tid; idx < words; idx += TILE3_LANES) w[idx] = 0;
+        for (int idx = tid; idx < td.nmark * 2 * NV; idx += TILE3_LANES) mk.acc[idx] = T(0);
+        __syncthreads();
+        for (int idx = tid; idx < td.nmark; idx += TILE3_LANES)
+            mk.map[mark_at(a.marks[td.mark0 + idx])] = (uint16_t)(idx + 1);
+    }
     __syncthreads();
 
     // the wave's number in a scalar register, so that its rows and chunks are
@@ -441,9 +543,9 @@ __global__ __launch_bounds__(TILE3_LANES, TILE3_WG_PER_CU) void sweep3_tile_kern
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64), wl = tid - wave * 64;
     T cfl = T(0);
 
-    tile3_sweep<Sol, 1, STD>(a, qs, dq, tx, ty, tz, bx, by, wave, wl, cfl);
-    tile3_sweep<Sol, 2, STD>(a, qs, dq, tx, ty, tz, bx, by, wave, wl, cfl);
-    tile3_sweep<Sol, 3, STD>(a, qs, dq, tx, ty, tz, bx, by, wave, wl, cfl);
+    tile3_sweep<Sol, 1, STD, MARK>(a, qs, dq, tx, ty, tz, bx, by, wave, wl, cfl, mk);
+    tile3_sweep<Sol, 2, STD, MARK>(a, qs, dq, tx, ty, tz, bx, by, wave, wl, cfl, mk);
+    tile3_sweep<Sol, 3, STD, MARK>(a, qs, dq, tx, ty, tz, bx, by, wave, wl, cfl, mk);
 
     // q(t + dt) = q(t) + dq on the tile's cells
     T* qout = static_cast<T*>(a.qout) + pt.qoff;
@@ -453,6 +555,40 @@ __global__ __launch_bounds__(TILE3_LANES, TILE3_WG_PER_CU) void sweep3_tile_kern
             const T v = qs[((u.z + 2) * bx * by + (u.y + 2) * bx + (u.x + 2)) * NV + u.m] +
                         dq[((u.z * ty + u.y) * tx + u.x) * NV + u.m];
             qout[u.m * plane + g0 + (int64_t)(u.z + 2) * mij + (int64_t)(u.y + 2) * mit + (u.x + 2)] = v;
+        }
+    }
+    if constexpr (MARK) {
+        // the grid's ghost cells keep their time-t values: of the staged box,
+        // what lies outside the grid, each cell written by the tile beside it
+        // (the tile's range extended by two cells at the grid's own sides)
+        const int xl = td.i0 == 0 ? 0 : 2, xh = td.i0 + tx == pt.mx ? bx : bx - 2;
+        const int yl = td.j0 == 0 ? 0 : 2, yh = td.j0 + ty == pt.my ? by : by - 2;
+        const int zl = td.k0 == 0 ? 0 : 2, zh = td.k0 + tz == pt.mz ? bz : bz - 2;
+        if (xl == 0 || xh == bx || yl == 0 || yh == by || zl == 0 || zh == bz) {
+            Digits3 u(tid, bx, by, bz);
+            for (int idx = tid; idx < NV * nbox; idx += TILE3_LANES, u.step()) {
+                const bool mine = u.x >= xl && u.x < xh && u.y >= yl && u.y < yh && u.z >= zl && u.z < zh;
+                const bool cell = u.x >= 2 && u.x < bx - 2 && u.y >= 2 && u.y < by - 2 && u.z >= 2 &&
+                                  u.z < bz - 2;
+                if (mine && !cell)
+                    qout[u.m * plane + g0 + (int64_t)u.z * mij + (int64_t)u.y * mit + u.x] =
+                        qs[((u.z * by + u.y) * bx + u.x) * NV + u.m];
+            }
+        }
+        // the marked faces into the grid's flux block: fm and fp - fm (gm, gp
+        // likewise), hm and hp
+        const Faces3 F = faces3(pt, NV);
+        for (int idx = tid; idx < td.nmark * NV; idx += TILE3_LANES) {
+            const int id = idx / NV, m = idx - id * NV;
+            const Mark3 f = a.marks[td.mark0 + id];
+            const T lo = T(double(mk.acc[id * 2 * NV + m]) / a.dtd[f.dir]);
+            const T df = mk.acc[(id * 2 + 1) * NV + m];
+            const int x = td.i0 + f.x, y = td.j0 + f.y, z = td.k0 + f.z;
+            const int w = pt.mx + (f.dir == 0), h = pt.my + (f.dir == 1);
+            const int64_t at = m * (f.dir == 0 ? F.sx : (f.dir == 1 ? F.sy : F.sz)) +
+                               ((int64_t)z * h + y) * w + x;
+            a.face[(f.dir == 0 ? F.fm : (f.dir == 1 ? F.gm : F.hm)) + at] = lo;
+            a.face[(f.dir == 0 ? F.fp : (f.dir == 1 ? F.gp : F.hp)) + at] = f.dir == 2 ? lo + df : df;
         }
     }
     double cd = double(cfl);
