@@ -22,13 +22,11 @@
 #include "kernels.hpp"
 #include "noalloc.hpp"
 #include "regs_plan.hpp"
+#include "xfer.hpp"
 
 namespace amrgpu {
 hipError_t launch_fill_u64(unsigned long long* p, unsigned long long v, int64_t n,
                            hipStream_t st);
-hipError_t launch_aos_soa(bool to_soa, int esize, double* stage, const int64_t* stage_off,
-                          const int64_t* off, const int32_t* plane, const int64_t* cell_start,
-                          int npatch, int nv, int64_t ncell, void* level, hipStream_t st);
 hipError_t launch_fill_stage(int esize, const FillArgs& a, hipStream_t st);
 hipError_t launch_gauges(int esize, const GaugeArgs& a, hipStream_t st);
 }
@@ -69,11 +67,7 @@ struct Level {
     // is the faster FP64 sweep): its wave table
     std::vector<MarchWave> mwaves;
     MarchWave* d_mwaves = nullptr;
-    // bulk transfer tables: patch element offsets, planes, first cell
-    int64_t* d_off = nullptr;
-    int32_t* d_plane = nullptr;
-    int64_t* d_cell_start = nullptr;
-    int64_t ncell_total = 0;       // cells incl. ghosts over all patches
+    XferGrid* d_xfer = nullptr;    // the patches for whole-level transfers
     // ghost-fill program (bound) of this level
     bool plan_valid = false;
     FillPlan plan;
@@ -173,6 +167,7 @@ struct Context {
     int mxnest = 0;
     int iregsz[MAXLV] = {}, jregsz[MAXLV] = {}, ratx[MAXLV] = {}, raty[MAXLV] = {};
     double hxposs[MAXLV] = {}, hyposs[MAXLV] = {};
+    XferRing xfer;                          // pinned ring of the grids' transfers
     unsigned long long* h_cfl = nullptr;   // pinned: the per-level-step Courant read-back
     int h_cfl_cap = 0;
     bool regs_valid = false;
@@ -355,9 +350,7 @@ void free_level(Level& L) {
         if (b) hipFree(b);
     if (L.d_cfl) hipFree(L.d_cfl);
     if (L.d_aux) hipFree(L.d_aux);
-    if (L.d_off) hipFree(L.d_off);
-    if (L.d_plane) hipFree(L.d_plane);
-    if (L.d_cell_start) hipFree(L.d_cell_start);
+    if (L.d_xfer) hipFree(L.d_xfer);
     double t = L.time, pk = L.possk;
     L = Level();
     L.time = t;
@@ -693,116 +686,59 @@ int define_level(int level, int ngrids, const int* ilo, const int* ihi, const in
             HIPCHK(dzero(L.d_aux, (size_t)L.nelem * g.auxk * sizeof(double)));
             L.aux_set = false;
         }
-        std::vector<int64_t> off(ngrids), cs(ngrids);
-        std::vector<int32_t> pl(ngrids);
+        std::vector<XferGrid> xg(ngrids);
         int64_t c = 0;
         for (int p = 0; p < ngrids; p++) {
-            off[p] = L.patches[p].off;
-            pl[p] = L.patches[p].plane;
-            cs[p] = c;
+            xg[p] = XferGrid{L.patches[p].off, L.patches[p].plane, c};
             c += L.patches[p].plane;
         }
-        L.ncell_total = c;
-        HIPCHK(hipMalloc(&L.d_off, ngrids * sizeof(int64_t)));
-        HIPCHK(hipMalloc(&L.d_plane, ngrids * sizeof(int32_t)));
-        HIPCHK(hipMalloc(&L.d_cell_start, ngrids * sizeof(int64_t)));
-        HIPCHK(h2d(L.d_off, off.data(), ngrids * sizeof(int64_t)));
-        HIPCHK(h2d(L.d_plane, pl.data(), ngrids * sizeof(int32_t)));
-        HIPCHK(h2d(L.d_cell_start, cs.data(), ngrids * sizeof(int64_t)));
+        HIPCHK(hipMalloc(&L.d_xfer, ngrids * sizeof(XferGrid)));
+        HIPCHK(h2d(L.d_xfer, xg.data(), ngrids * sizeof(XferGrid)));
     }
     int rc = plan_level(L);
     if (rc) free_level(L);   // refused tiling: leave the level without grids
     return rc;
 }
 
-// AoS FP64 host <-> SoA device (storage precision)
+// AoS FP64 host <-> SoA device (storage precision), one grid
+int xfer_grid(Level& L, bool to_dev, int grid, int which, double* q, bool both = false) {
+    const PatchDesc& pd = L.patches[grid];
+    XferArgs a{};
+    a.one = XferGrid{pd.off, pd.plane, 0};
+    a.ngrids = 1;
+    a.nv = g.cfg.nvar;
+    a.data = L.buf[which == 0 ? L.cur : 1 - L.cur];
+    a.data2 = both ? L.buf[which == 0 ? 1 - L.cur : L.cur] : nullptr;
+    HIPCHK(g.xfer.run(to_dev, (int)g.esize, a, (int64_t)a.nv * pd.plane, g.stream,
+                      [&](int64_t e0, int64_t e1, double* slot) {
+                          if (to_dev) std::memcpy(slot, q + e0, (e1 - e0) * sizeof(double));
+                          else std::memcpy(q + e0, slot, (e1 - e0) * sizeof(double));
+                      }));
+    return AMRGPU_OK;
+}
 int put_grid(Level& L, int grid, int which, const double* q) {
-    const PatchDesc& pd = L.patches[grid];
-    const int nv = g.cfg.nvar;
-    const int64_t n = (int64_t)nv * pd.plane;
-    void* dst = (char*)L.buf[which == 0 ? L.cur : 1 - L.cur] + pd.off * g.esize;
-    if (g.esize == 8) {
-        std::vector<double> h(n);
-        for (int64_t c = 0; c < pd.plane; c++)
-            for (int m = 0; m < nv; m++) h[m * pd.plane + c] = q[c * nv + m];
-        HIPCHK(h2d(dst, h.data(), n * 8));
-    } else {
-        std::vector<float> h(n);
-        for (int64_t c = 0; c < pd.plane; c++)
-            for (int m = 0; m < nv; m++) h[m * pd.plane + c] = (float)q[c * nv + m];
-        HIPCHK(h2d(dst, h.data(), n * 4));
-    }
-    return AMRGPU_OK;
+    return xfer_grid(L, true, grid, which, const_cast<double*>(q));
 }
+int get_grid(Level& L, int grid, int which, double* q) { return xfer_grid(L, false, grid, which, q); }
 
-int get_grid(Level& L, int grid, int which, double* q) {
-    const PatchDesc& pd = L.patches[grid];
-    const int nv = g.cfg.nvar;
-    const int64_t n = (int64_t)nv * pd.plane;
-    const void* src = (const char*)L.buf[which == 0 ? L.cur : 1 - L.cur] + pd.off * g.esize;
-    HIPCHK(hipStreamSynchronize(g.stream));
-    if (g.esize == 8) {
-        std::vector<double> h(n);
-        HIPCHK(d2h(h.data(), src, n * 8));
-        for (int64_t c = 0; c < pd.plane; c++)
-            for (int m = 0; m < nv; m++) q[c * nv + m] = h[m * pd.plane + c];
-    } else {
-        std::vector<float> h(n);
-        HIPCHK(d2h(h.data(), src, n * 4));
-        for (int64_t c = 0; c < pd.plane; c++)
-            for (int m = 0; m < nv; m++) q[c * nv + m] = (double)h[m * pd.plane + c];
-    }
-    return AMRGPU_OK;
-}
-
-// Bulk transfer of a whole level between the reference's heap layout
-// (alloc(loc + ...), one AoS FP64 block per grid at offsets[p]) and the
-// device.  Grids are gathered into one staging buffer, copied in one
-// transfer and transposed on the device.
+// A whole level between the reference's heap layout (alloc(loc + ...), one AoS
+// FP64 block per grid at offsets[p]) and the device.
 int xfer_level(Level& L, bool to_dev, int which, double* alloc_base, const int64_t* offsets) {
     if (L.ngrids == 0) return AMRGPU_OK;
     const int nv = g.cfg.nvar;
-    std::vector<int64_t> soff(L.ngrids);
-    int64_t tot = 0;
-    for (int p = 0; p < L.ngrids; p++) {
-        soff[p] = tot;
-        tot += (int64_t)nv * L.patches[p].plane;
-    }
-    double* h_stage = nullptr;
-    double* d_stage = nullptr;
-    int64_t* d_soff = nullptr;
-    HIPCHK(hipHostMalloc((void**)&h_stage, tot * sizeof(double), hipHostMallocDefault));
-    HIPCHK(hipMalloc(&d_stage, tot * sizeof(double)));
-    HIPCHK(hipMalloc(&d_soff, L.ngrids * sizeof(int64_t)));
-    HIPCHK(h2d(d_soff, soff.data(), L.ngrids * sizeof(int64_t)));
-    void* lvl = L.buf[which == 0 ? L.cur : 1 - L.cur];
-    int rc = AMRGPU_OK;
-    hipError_t e = hipSuccess;
-    if (to_dev) {
-        for (int p = 0; p < L.ngrids; p++)
-            std::memcpy(h_stage + soff[p], alloc_base + offsets[p],
-                        (size_t)nv * L.patches[p].plane * sizeof(double));
-        e = hipMemcpyAsync(d_stage, h_stage, tot * sizeof(double), hipMemcpyHostToDevice, g.stream);
-        if (e == hipSuccess)
-            e = launch_aos_soa(true, (int)g.esize, d_stage, d_soff, L.d_off, L.d_plane,
-                               L.d_cell_start, L.ngrids, nv, L.ncell_total, lvl, g.stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(g.stream);
-    } else {
-        e = launch_aos_soa(false, (int)g.esize, d_stage, d_soff, L.d_off, L.d_plane,
-                           L.d_cell_start, L.ngrids, nv, L.ncell_total, lvl, g.stream);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(h_stage, d_stage, tot * sizeof(double), hipMemcpyDeviceToHost, g.stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(g.stream);
-        if (e == hipSuccess)
-            for (int p = 0; p < L.ngrids; p++)
-                std::memcpy(alloc_base + offsets[p], h_stage + soff[p],
-                            (size_t)nv * L.patches[p].plane * sizeof(double));
-    }
-    if (e != hipSuccess) rc = fail(AMRGPU_ERR_HIP, "level transfer: %s", hipGetErrorString(e));
-    hipFree(d_soff);
-    hipFree(d_stage);
-    hipHostFree(h_stage);
-    return rc;
+    std::vector<int64_t> start(L.ngrids + 1, 0);
+    for (int p = 0; p < L.ngrids; p++) start[p + 1] = start[p] + (int64_t)nv * L.patches[p].plane;
+    XferArgs a{};
+    a.grids = L.d_xfer;
+    a.ngrids = L.ngrids;
+    a.nv = nv;
+    a.data = L.buf[which == 0 ? L.cur : 1 - L.cur];
+    HIPCHK(g.xfer.run(to_dev, (int)g.esize, a, start.back(), g.stream,
+                      [&](int64_t e0, int64_t e1, double* slot) {
+                          xfer_pieces(to_dev, start, [&](size_t p) { return alloc_base + offsets[p]; },
+                                      e0, e1, slot);
+                      }));
+    return AMRGPU_OK;
 }
 
 // hierarchy geometry for the planner
@@ -1798,6 +1734,7 @@ int amrgpu_finalize(void) {
         if (e) hipEventDestroy(e);
     hipFree(g.d_next);
     if (g.h_cfl) hipHostFree(g.h_cfl);
+    g.xfer.release();
     hipStreamDestroy(g.stream);
     g = Context();
     return AMRGPU_OK;
@@ -1855,7 +1792,8 @@ int amrgpu_stepgrid(int mx, int my, const double* q_in, double* q_out, double dx
     int rc = define_level(0, 1, &ilo, &ihi, &jlo, &jhi, dx, dy);
     if (rc) return rc;
     Level& L = g.levels[0];
-    rc = put_grid(L, 0, 0, q_in);
+    // ghost cells of the output keep the input values, as in stepgrid.f
+    rc = xfer_grid(L, true, 0, 0, const_cast<double*>(q_in), true);
     if (rc) return rc;
     const bool want_flux = fm && fp && gm && gp;
     const int nv = g.cfg.nvar;
@@ -1868,9 +1806,6 @@ int amrgpu_stepgrid(int mx, int my, const double* q_in, double* q_out, double dx
         HIPCHK(hipMalloc(&d_off, sizeof(int64_t)));
         HIPCHK(dzero(d_off, sizeof(int64_t)));
     }
-    // ghost cells of the output keep the input values, as in stepgrid.f
-    rc = put_grid(L, 0, 1, q_in);
-    if (rc) return rc;
     rc = sweep(L, dt, d_flux, d_off);
     if (rc) return rc;
     rc = get_grid(L, 0, 0, q_out);

@@ -26,6 +26,8 @@ namespace {
 const double RINFINITY3 = (double)10.e32f;   // amr_module's rinfinity
 constexpr int NKIND = 4;                      // x, y, z sweeps, update
 
+constexpr int PLANE_BLOCK3 = 4;   // planes per sweep workgroup of a batch (default)
+
 struct Context3 {
     bool inited = false;
     amrgpu3_config cfg{};
@@ -33,7 +35,7 @@ struct Context3 {
     size_t esize = 8;
     hipStream_t stream = nullptr;
     int npatch = 0;
-    int plane_block = 4;
+    int plane_block = PLANE_BLOCK3;
     std::vector<Patch3> patches;
     Patch3* d_patches = nullptr;
     std::vector<Block3> blocks[NKIND];
@@ -62,6 +64,7 @@ struct Context3 {
     std::vector<std::pair<hipEvent_t, hipEvent_t>> tev[NKIND];
     size_t tev_used[NKIND] = {};
     void* h_pin = nullptr;              // pinned staging of small read-backs
+    XferRing xfer;                      // pinned ring of the grids' transfers
 };
 constexpr size_t PIN3_BYTES = 1 << 16;
 
@@ -109,6 +112,20 @@ hipError_t d2h3(void* dst, const void* src, size_t n) {
     return e != hipSuccess ? e : hipStreamSynchronize(g3.stream);
 }
 
+// flag2refine's arrays of the batch
+void drop_flags() {
+    if (g3.stream && g3.d_flags) hipStreamSynchronize(g3.stream);
+    hipFree(g3.d_flags);
+    hipFree(g3.d_foff);
+    hipFree(g3.d_nflag);
+    hipFree(g3.d_partial);
+    g3.d_flags = nullptr;
+    g3.d_foff = nullptr;
+    g3.d_nflag = nullptr;
+    g3.d_partial = nullptr;
+    g3.foff.clear();
+}
+
 void free_batch() {
     if (g3.stream) hipStreamSynchronize(g3.stream);
     hipFree(g3.d_patches);
@@ -122,15 +139,7 @@ void free_batch() {
     g3.fluxes_valid = false;
     g3.last_fused = false;
     hipFree(g3.d_cfl);
-    hipFree(g3.d_flags);
-    hipFree(g3.d_foff);
-    hipFree(g3.d_nflag);
-    hipFree(g3.d_partial);
-    g3.d_flags = nullptr;
-    g3.d_foff = nullptr;
-    g3.d_nflag = nullptr;
-    g3.d_partial = nullptr;
-    g3.foff.clear();
+    drop_flags();
     for (int k = 0; k < NKIND; k++) {
         hipFree(g3.d_blocks[k]);
         g3.d_blocks[k] = nullptr;
@@ -435,44 +444,27 @@ int define_batch(int npatch, const int* mx, const int* my, const int* mz) {
     return AMRGPU_OK;
 }
 
-// host AoS q(nvar, mx+4, my+4, mz+4) <-> device SoA [m][k][j][i]
-int put_q(int p, const double* q) {
+// host AoS q(nvar, mx+4, my+4, mz+4) <-> device SoA [m][k][j][i].  To the
+// device both buffers of the fused step receive the grid (they keep the same
+// ghost cells).
+int xfer_q(bool to_dev, int p, double* q) {
     const Patch3& pt = g3.patches[p];
-    const int nv = g3.cfg.nvar;
     const int64_t cells = (int64_t)(pt.mx + 4) * (pt.my + 4) * (pt.mz + 4);
-    if (g3.esize == 8) {
-        std::vector<double> h(nv * cells);
-        for (int64_t c = 0; c < cells; c++)
-            for (int m = 0; m < nv; m++) h[m * cells + c] = q[c * nv + m];
-        HIPCHK3(h2d3(static_cast<double*>(g3.d_q) + pt.qoff, h.data(), h.size() * 8));
-    } else {
-        std::vector<float> h(nv * cells);
-        for (int64_t c = 0; c < cells; c++)
-            for (int m = 0; m < nv; m++) h[m * cells + c] = (float)q[c * nv + m];
-        HIPCHK3(h2d3(static_cast<float*>(g3.d_q) + pt.qoff, h.data(), h.size() * 4));
-        if (g3.d_q2)   // the fused step's output buffer keeps the same ghost cells
-            HIPCHK3(h2d3(static_cast<float*>(g3.d_q2) + pt.qoff, h.data(), h.size() * 4));
-    }
+    XferArgs a{};
+    a.one = XferGrid{pt.qoff, cells, 0};
+    a.ngrids = 1;
+    a.nv = g3.cfg.nvar;
+    a.data = g3.d_q;
+    a.data2 = to_dev ? g3.d_q2 : nullptr;
+    HIPCHK3(g3.xfer.run(to_dev, (int)g3.esize, a, a.nv * cells, g3.stream,
+                        [&](int64_t e0, int64_t e1, double* slot) {
+                            if (to_dev) std::memcpy(slot, q + e0, (e1 - e0) * sizeof(double));
+                            else std::memcpy(q + e0, slot, (e1 - e0) * sizeof(double));
+                        }));
     return AMRGPU_OK;
 }
-
-int get_q(int p, double* q) {
-    const Patch3& pt = g3.patches[p];
-    const int nv = g3.cfg.nvar;
-    const int64_t cells = (int64_t)(pt.mx + 4) * (pt.my + 4) * (pt.mz + 4);
-    if (g3.esize == 8) {
-        std::vector<double> h(nv * cells);
-        HIPCHK3(d2h3(h.data(), static_cast<double*>(g3.d_q) + pt.qoff, h.size() * 8));
-        for (int64_t c = 0; c < cells; c++)
-            for (int m = 0; m < nv; m++) q[c * nv + m] = h[m * cells + c];
-    } else {
-        std::vector<float> h(nv * cells);
-        HIPCHK3(d2h3(h.data(), static_cast<float*>(g3.d_q) + pt.qoff, h.size() * 4));
-        for (int64_t c = 0; c < cells; c++)
-            for (int m = 0; m < nv; m++) q[c * nv + m] = (double)h[m * cells + c];
-    }
-    return AMRGPU_OK;
-}
+int put_q(int p, const double* q) { return xfer_q(true, p, const_cast<double*>(q)); }
+int get_q(int p, double* q) { return xfer_q(false, p, q); }
 
 int step_io(const Step3IO& io, double dx, double dy, double dz, double dt, int es_override = 0) {
     const size_t es = es_override ? (size_t)es_override : g3.esize;
@@ -625,10 +617,38 @@ int get_fluxes(int p, double* const out[6]) {
     const int nv = g3.cfg.nvar;
     const Faces3 F = faces3(pt, nv);
     const int64_t n = faces3_elems(pt, nv);
-    std::vector<double> h(n);
+    const int mit = pt.mx + 4, mjt = pt.my + 4;
+    auto at = [&](int i, int j, int k) { return (((int64_t)(k + 1) * mjt + (j + 1)) * mit + (i + 1)) * nv; };
+    const int64_t base[6] = {F.fm, F.fp, F.gm, F.gp, F.hm, F.hp};
+    const int64_t cs[3] = {F.sx, F.sy, F.sz};
     if (g3.esize == 8) {
-        HIPCHK3(d2h3(h.data(), static_cast<double*>(g3.d_face) + pt.foff, n * 8));
-    } else {
+        // each array a grid of its interior faces; a row of faces is one
+        // contiguous piece of the caller's array
+        for (int k = 0; k < 6; k++) {
+            if (!out[k]) continue;
+            const int dir = k / 2;
+            const int ni = pt.mx + (dir == 0), nj = pt.my + (dir == 1);
+            XferArgs a{};
+            a.one = XferGrid{base[k], cs[dir], 0};
+            a.ngrids = 1;
+            a.nv = nv;
+            a.data = g3.d_face;
+            const int64_t row = (int64_t)ni * nv;
+            HIPCHK3(g3.xfer.run(false, 8, a, nv * cs[dir], g3.stream,
+                                [&](int64_t e0, int64_t e1, double* slot) {
+                                    for (int64_t e = e0; e < e1;) {
+                                        const int64_t r = e / row, end = std::min(e1, (r + 1) * row);
+                                        double* to = out[k] + at(1, (int)(r % nj) + 1, (int)(r / nj) + 1);
+                                        std::memcpy(to + (e - r * row), slot + (e - e0),
+                                                    (end - e) * sizeof(double));
+                                        e = end;
+                                    }
+                                }));
+        }
+        return AMRGPU_OK;
+    }
+    std::vector<double> h(n);
+    {
         std::vector<float> f(n);
         HIPCHK3(d2h3(f.data(), static_cast<float*>(g3.d_face) + pt.foff, n * 4));
         for (int64_t k = 0; k < n; k++) h[k] = f[k];
@@ -639,10 +659,6 @@ int get_fluxes(int p, double* const out[6]) {
         for (int64_t k = 0; k < nv * F.sy; k++)
             h[F.gp - pt.foff + k] = (double)(f[F.gm - pt.foff + k] + f[F.gp - pt.foff + k]);
     }
-    const int mit = pt.mx + 4, mjt = pt.my + 4;
-    auto at = [&](int i, int j, int k) { return (((int64_t)(k + 1) * mjt + (j + 1)) * mit + (i + 1)) * nv; };
-    const int64_t base[6] = {F.fm, F.fp, F.gm, F.gp, F.hm, F.hp};
-    const int64_t cs[3] = {F.sx, F.sy, F.sz};
     for (int a = 0; a < 6; a++) {
         if (!out[a]) continue;
         const int dir = a / 2;
@@ -693,6 +709,7 @@ int ctx3_fail(int code, const char* fmt, ...) {
     g3_err = buf;
     return code;
 }
+XferRing& ctx3_xfer() { return g3.xfer; }
 hipError_t ctx3_h2d(void* dst, const void* src, size_t n) { return h2d3(dst, src, n); }
 hipError_t ctx3_d2h(void* dst, const void* src, size_t n) { return d2h3(dst, src, n); }
 int ctx3_step(const Step3IO& io, double dx, double dy, double dz, double dt, int esize) {
@@ -824,6 +841,7 @@ int amrgpu3_finalize(void) {
     if (g3.stream) hipStreamDestroy(g3.stream);
     g3.stream = nullptr;
     if (g3.h_pin) hipHostFree(g3.h_pin);
+    g3.xfer.release();
     g3.h_pin = nullptr;
     g3.inited = false;
     g3.timing = false;
@@ -844,7 +862,7 @@ int amrgpu3_set_patches(int npatch, const int* mx, const int* my, const int* mz,
             return fail3(AMRGPU_ERR_UNSUPPORTED, "patch %d: a side exceeds %d cells", p,
                          SWEEP3_LANES - 3);
     }
-    g3.plane_block = plane_block ? plane_block : 4;
+    g3.plane_block = plane_block ? plane_block : PLANE_BLOCK3;
     return define_batch(npatch, mx, my, mz);
 }
 
@@ -893,8 +911,17 @@ int amrgpu3_stepgrid(int mx, int my, int mz, const double* q_in, double* q_out, 
     int rc = need_init();
     if (rc) return rc;
     if (!q_in || !q_out) return fail3(AMRGPU_ERR_ARG, "null q");
-    rc = amrgpu3_set_patches(1, &mx, &my, &mz, 0);
-    if (rc) return rc;
+    // the one-grid batch of the call before, when it has this shape: q and
+    // every flux array are written in full, and its flags are forgotten as a
+    // new batch's would be
+    if (g3.npatch == 1 && g3.patches[0].mx == mx && g3.patches[0].my == my &&
+        g3.patches[0].mz == mz && g3.plane_block == PLANE_BLOCK3) {
+        g3.fluxes_valid = g3.last_fused = false;
+        drop_flags();
+    } else {
+        rc = amrgpu3_set_patches(1, &mx, &my, &mz, 0);
+        if (rc) return rc;
+    }
     rc = put_q(0, q_in);
     if (rc) return rc;
     double cfl = 0.0;

@@ -56,6 +56,7 @@ struct Lev3 {
     Block3* d_blocks[4] = {};
     void* d_new = nullptr;
     void* d_old = nullptr;
+    XferGrid* d_xfer = nullptr;   // the grids for whole-level transfers
     int64_t q_elems = 0, face_elems = 0;
     double time = 0.0, possk = 0.0;
     unsigned long long* d_cfl = nullptr;
@@ -151,6 +152,7 @@ void free_level(Lev3& L) {
     dfree(L.d_new);
     dfree(L.d_old);
     dfree(L.d_next);
+    dfree(L.d_xfer);
     dfree(L.d_cfl);
     dfree(L.d_partial);
     dfree(L.d_flags);
@@ -191,6 +193,26 @@ int upload_fill(DevFill& f) {
         A.scratch_cap = f.plan.scratch_elems;
     }
     return rc;
+}
+
+// every grid of a level between the reference's heap and the device
+int xfer_level(Lev3& L, bool to_dev, int which, double* alloc_base, const int64_t* offsets) {
+    const int n = (int)L.patches.size();
+    if (n == 0) return AMRGPU_OK;
+    XferArgs a{};
+    a.grids = L.d_xfer;
+    a.ngrids = n;
+    a.nv = ctx3_cfg().nvar;
+    a.data = which == 0 ? L.d_new : L.d_old;
+    std::vector<int64_t> start(n + 1, 0);
+    for (int g = 0; g < n; g++) start[g + 1] = start[g] + q3_elems(L.patches[g], a.nv);
+    HIPCHKA(ctx3_xfer().run(to_dev, (int)ctx3_esize(), a, start.back(), ctx3_stream(),
+                            [&](int64_t e0, int64_t e1, double* slot) {
+                                xfer_pieces(to_dev, start,
+                                            [&](size_t g) { return alloc_base + offsets[g]; }, e0, e1,
+                                            slot);
+                            }));
+    return AMRGPU_OK;
 }
 
 // ghost-fill programs of every level (after a layout change)
@@ -575,7 +597,14 @@ int amrgpu3_set_level(int level, int ngrids, const int* boxes) {
     if (pb <= 0) pb = planes >= 4096 ? ctx3_plane_block() : (ctx3_esize() == 4 ? 1 : 2);
     ctx3_plan_blocks(L.patches, pb, L.blocks);
     const size_t es = ctx3_esize();
+    std::vector<XferGrid> xg;
+    int64_t cells = 0;
+    for (const auto& p : L.patches) {
+        xg.push_back(XferGrid{p.qoff, q3_elems(p, 1), cells});
+        cells += q3_elems(p, 1);
+    }
     rc = upload(L.d_patches, L.patches);
+    if (!rc) rc = upload(L.d_xfer, xg);
     for (int k = 0; k < 4 && !rc; k++) rc = upload(L.d_blocks[k], L.blocks[k]);
     if (rc) return rc;
     HIPCHKA(hipMalloc(&L.d_new, std::max<int64_t>(1, qo) * es));
@@ -627,46 +656,14 @@ int amrgpu3_put_level(int level, int which, const double* alloc_base, const int6
     int rc = check_level(level);
     if (rc) return rc;
     if (!alloc_base || !offsets) return ctx3_fail(AMRGPU_ERR_ARG, "null arrays");
-    Lev3& L = A.lev[level];
-    const int nv = ctx3_cfg().nvar;
-    const size_t es = ctx3_esize();
-    std::vector<char> h(std::max<int64_t>(1, L.q_elems) * es, 0);
-    for (size_t g = 0; g < L.patches.size(); g++) {
-        const Patch3& p = L.patches[g];
-        const int64_t cells = (int64_t)(p.mx + 4) * (p.my + 4) * (p.mz + 4);
-        const double* q = alloc_base + offsets[g];
-        for (int64_t c = 0; c < cells; c++)
-            for (int m = 0; m < nv; m++) {
-                const int64_t d = p.qoff + m * cells + c;
-                if (es == 8) reinterpret_cast<double*>(h.data())[d] = q[c * nv + m];
-                else reinterpret_cast<float*>(h.data())[d] = (float)q[c * nv + m];
-            }
-    }
-    HIPCHKA(ctx3_h2d(which == 0 ? L.d_new : L.d_old, h.data(), L.q_elems * es));
-    return AMRGPU_OK;
+    return xfer_level(A.lev[level], true, which, const_cast<double*>(alloc_base), offsets);
 }
 
 int amrgpu3_get_level(int level, int which, double* alloc_base, const int64_t* offsets) {
     int rc = check_level(level);
     if (rc) return rc;
     if (!alloc_base || !offsets) return ctx3_fail(AMRGPU_ERR_ARG, "null arrays");
-    Lev3& L = A.lev[level];
-    const int nv = ctx3_cfg().nvar;
-    const size_t es = ctx3_esize();
-    std::vector<char> h(std::max<int64_t>(1, L.q_elems) * es);
-    HIPCHKA(ctx3_d2h(h.data(), which == 0 ? L.d_new : L.d_old, L.q_elems * es));
-    for (size_t g = 0; g < L.patches.size(); g++) {
-        const Patch3& p = L.patches[g];
-        const int64_t cells = (int64_t)(p.mx + 4) * (p.my + 4) * (p.mz + 4);
-        double* q = alloc_base + offsets[g];
-        for (int64_t c = 0; c < cells; c++)
-            for (int m = 0; m < nv; m++) {
-                const int64_t d = p.qoff + m * cells + c;
-                q[c * nv + m] = es == 8 ? reinterpret_cast<const double*>(h.data())[d]
-                                        : (double)reinterpret_cast<const float*>(h.data())[d];
-            }
-    }
-    return AMRGPU_OK;
+    return xfer_level(A.lev[level], false, which, alloc_base, offsets);
 }
 
 int amrgpu3_bound_level(int level, double time) {

@@ -7,6 +7,7 @@
 #include "../../include/amrgpu3.h"
 #include "sweep3.hpp"
 #include "sweep3_tile.hpp"
+#include "xfer.hpp"
 
 namespace amrgpu {
 
@@ -50,6 +51,7 @@ const amrgpu3_config& ctx3_cfg();
 size_t ctx3_esize();
 hipStream_t ctx3_stream();
 int ctx3_plane_block();
+XferRing& ctx3_xfer();
 int ctx3_fail(int code, const char* fmt, ...);
 hipError_t ctx3_h2d(void* dst, const void* src, size_t n);
 hipError_t ctx3_d2h(void* dst, const void* src, size_t n);
