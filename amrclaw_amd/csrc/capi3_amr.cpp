@@ -76,6 +76,7 @@ struct Lev3 {
     Upbnd3Cell* d_ucells = nullptr;
     Upbnd3Entry* d_uents = nullptr;
     Avg3Block* d_avg = nullptr;
+    Pass3Plan pass;               // the level's two-pass FP64 step
     // the fused FP32 step: its tiles with the faces the registers read, and
     // the buffer it writes on the finest level (which keeps no old time; the
     // others write their old buffer and swap roles)
@@ -147,6 +148,7 @@ void free_plans(Lev3& L) {
 
 void free_level(Lev3& L) {
     free_plans(L);
+    L.pass.free();
     dfree(L.d_patches);
     for (auto& b : L.d_blocks) dfree(b);
     dfree(L.d_new);
@@ -735,6 +737,8 @@ int amrgpu3_advance_level(int level, double* dtlevnew, double* cfl_level) {
         }
         io.npatch = (int)L.patches.size();
         io.d_cfl = L.d_cfl;
+        io.patches = &L.patches;
+        io.pass = &L.pass;
         rc = ctx3_step(io, G.hx, G.hy, G.hz, L.possk);
         if (rc) return rc;
     }
@@ -845,8 +849,11 @@ int amrgpu3_flag_level(int level, double tolsp, int flag_richardson, double tol,
         Block3* d_bf[4] = {};
         Block3* d_bc[4] = {};
         int64_t* d_cstart = nullptr;
+        Pass3Plan pass_c, pass_f;
         auto cleanup = [&]() {
             hipStreamSynchronize(st);
+            pass_c.free();
+            pass_f.free();
             free_fill(D);
             hipFree(arena);
             hipFree(face);
@@ -905,6 +912,8 @@ int amrgpu3_flag_level(int level, double tolsp, int flag_richardson, double tol,
             }
             io.npatch = n;
             io.d_cfl = L.d_cfl;
+            io.patches = &R.crs;
+            io.pass = &pass_c;
             rc = ctx3_step(io, 2.0 * G.hx, 2.0 * G.hy, 2.0 * G.hz, 2. * L.possk, 8);
         }
         if (!rc) {
@@ -918,6 +927,8 @@ int amrgpu3_flag_level(int level, double tolsp, int flag_richardson, double tol,
             }
             io.npatch = n;
             io.d_cfl = L.d_cfl;
+            io.patches = &R.fine;
+            io.pass = &pass_f;
             rc = ctx3_step(io, G.hx, G.hy, G.hz, L.possk, 8);
         }
         if (!rc) {

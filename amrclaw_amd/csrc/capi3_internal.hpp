@@ -6,6 +6,7 @@
 
 #include "../../include/amrgpu3.h"
 #include "sweep3.hpp"
+#include "sweep3_pass.hpp"
 #include "sweep3_tile.hpp"
 #include "xfer.hpp"
 
@@ -35,6 +36,27 @@ struct Fused3IO {
     unsigned long long* d_cfl;
 };
 
+// The two-pass FP64 step of a batch (sweep3_pass.hpp): the waves of each sweep,
+// the face blocks, every grid's place in the work space, and the runs of grids
+// that share it.  Built on first use, on the device until freed.
+struct Pass3Run {
+    int w0[3], w1[3], f0, f1;
+};
+struct Pass3Plan {
+    bool built = false, ok = false;   // ok: every grid's work space is in bounds
+    std::vector<Pass3Run> runs;
+    int64_t ws_elems = 0;
+    Pass3Wave* d_waves[3] = {};
+    Block3* d_faces = nullptr;
+    Pass3Ws* d_off = nullptr;
+    void free() {
+        for (auto& w : d_waves) hipFree(w);
+        hipFree(d_faces);
+        hipFree(d_off);
+        *this = Pass3Plan();
+    }
+};
+
 // device arrays of one step over a batch of grids
 struct Step3IO {
     void* q;                      // solutions (compute precision)
@@ -44,6 +66,8 @@ struct Step3IO {
     int nblocks[4];
     int npatch;
     unsigned long long* d_cfl;    // per-grid Courant number (double bits)
+    const std::vector<Patch3>* patches;   // FP64: the host copy, and the batch's
+    Pass3Plan* pass;                      // two-pass plan (null: phase kernels)
 };
 
 bool ctx3_inited();

@@ -1,4 +1,7 @@
-// sweep3.hpp -- batched 3-D wave-propagation step over the patches of a level.
+// sweep3.hpp -- batched 3-D wave-propagation step over the patches of a level,
+// and what its other forms share (sweep3_tile.hpp: the fused FP32 step;
+// sweep3_pass.hpp: the FP64 step).  These phase kernels run the FP32 step whose
+// flux arrays are asked for, and FP64 grids too large for the two passes.
 //
 // step3.f:3-486 + flux3.f:4-633 + stepgrid.f (3-D):147-212 for every patch
 // of a batch, in four launches:

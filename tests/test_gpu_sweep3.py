@@ -254,3 +254,69 @@ def test_fused_step_is_deterministic(gpu):
     for a, b in zip(*out):
         assert np.array_equal(a, b)
     capi3.finalize3()
+
+
+# lines of one wave, of two pieces and of several (pieces of 61 cells), along
+# every axis; a one-cell grid
+PASS_SIZES = [(61, 5, 4), (62, 4, 5), (5, 123, 3), (3, 4, 124), (252, 2, 3), (2, 252, 1), (1, 3, 252),
+              (1, 1, 1), (64, 65, 2)]
+
+
+@pytest.mark.parametrize("case", [(orc.EULER, 2, 22, 4), (orc.EULER, 2, 11, 1),
+                                  (orc.ADVECTION, 2, 22, 4), (orc.EULER, 1, 0, 4)])
+def test_two_pass_fp64_long_lines(gpu, case):
+    """The FP64 step's two passes where lines are cut into pieces: solution,
+    six flux arrays and Courant number bit for bit with the oracle."""
+    p, c = params(case)
+    rng = np.random.default_rng(91)
+    capi3.init3(c)
+    try:
+        for mx, my, mz in PASS_SIZES:
+            print("two passes", case, (mx, my, mz), flush=True)
+            q = patch(rng, case[0], mx, my, mz)
+            dx, dy, dz, dt = mesh(mx, my, mz)
+            qo, fo, co, do = orc.stepgrid3(p, q, dx, dy, dz, dt)
+            qg, fg, cg, dg = capi3.stepgrid3(q, dx, dy, dz, dt, want_fluxes=True)
+            assert np.array_equal(qg, qo), (mx, my, mz)
+            assert cg == co and dg == do
+            for a, b in zip(interior_faces(fg, mx, my, mz), interior_faces(fo, mx, my, mz)):
+                assert np.array_equal(a, b), (mx, my, mz)
+    finally:
+        capi3.finalize3()
+
+
+def test_two_pass_fp64_runs(gpu):
+    """A batch whose work space takes two runs (14 grids of 60^3, 0.4 of 4 GB
+    each) steps every grid as a batch of its own does."""
+    rng = np.random.default_rng(92)
+    _, c = params((orc.EULER, 2, 22, 4))
+    base = patch(rng, orc.EULER, 60, 60, 60)
+    dx, dy, dz, dt = mesh(60, 60, 60)
+    scale = [1.0 + 0.01 * k for k in range(14)]
+    capi3.init3(c)
+    try:
+        capi3.set_patches3([(60, 60, 60)] * 14)
+        for k, s in enumerate(scale):
+            capi3.put_patch3(k, base * s)
+        cfl = capi3.step_patches3(dx, dy, dz, dt, npatch=14)
+        got = {k: capi3.get_patch3(k, base.shape) for k in (0, 9, 10, 13)}
+        for k, g in got.items():
+            one, _, c1, _ = capi3.stepgrid3(base * scale[k], dx, dy, dz, dt)
+            assert np.array_equal(one, g) and c1 == cfl[k], k
+    finally:
+        capi3.finalize3()
+
+
+def test_fp64_grid_beyond_the_work_space(gpu):
+    """A grid whose work space would pass 4 GB takes the phase kernels."""
+    p, c = params((orc.EULER, 1, 0, 4))
+    mx, my, mz = 150, 140, 130
+    q = patch(np.random.default_rng(93), orc.EULER, mx, my, mz)
+    dx, dy, dz, dt = mesh(mx, my, mz)
+    capi3.init3(c)
+    try:
+        qg, _, cg, dg = capi3.stepgrid3(q, dx, dy, dz, dt)
+    finally:
+        capi3.finalize3()
+    qo, _, co, do = orc.stepgrid3(p, q, dx, dy, dz, dt)
+    assert np.array_equal(qg, qo) and cg == co and dg == do
