@@ -27,7 +27,7 @@
 namespace amrgpu {
 hipError_t launch_fill_u64(unsigned long long* p, unsigned long long v, int64_t n,
                            hipStream_t st);
-hipError_t launch_fill_stage(int esize, const FillArgs& a, hipStream_t st);
+hipError_t launch_fill(int esize, const FillArgs& a, hipStream_t st);
 hipError_t launch_gauges(int esize, const GaugeArgs& a, hipStream_t st);
 }
 
@@ -39,6 +39,22 @@ constexpr int MAXLV = 12;          // reference maxlv = 10 (+ scratch slot 0)
 constexpr int NEVENTS = 16;
 // rinfinity = 10.e32 declared from a default-real literal (amr_module.f90)
 const double RINFINITY = (double)10.e32f;
+
+// a fill program's tables and scratch on the device
+struct FillDev {
+    FillItem* items = nullptr;
+    FillUnit* units = nullptr;
+    unsigned char* masks = nullptr;
+    double* scratch = nullptr;
+    int nunits = 0;
+    void free() {
+        void* ps[] = {items, units, masks, scratch};
+        for (void* p : ps)
+            if (p) hipFree(p);
+        *this = FillDev();
+    }
+    FillProg prog() const { return FillProg{items, units, scratch, masks, nunits, 0}; }
+};
 
 struct Level {
     int ngrids = 0;
@@ -71,10 +87,7 @@ struct Level {
     // ghost-fill program (bound) of this level
     bool plan_valid = false;
     FillPlan plan;
-    FillOp* d_ops = nullptr;
-    FillBuf* d_bufs = nullptr;
-    unsigned char* d_masks = nullptr;
-    double* d_scratch = nullptr;
+    FillDev dplan;
     // time of the level's grids (rnode(timemult)) and its step (possk)
     double time = 0.0, possk = 0.0;
     // coarse-fine registers: this level's arena (fine side) and the device
@@ -92,9 +105,7 @@ struct Level {
     int64_t navg_cells = 0;
     // saveqc program filling this level's qc1d from the next coarser level
     FillPlan sq;
-    FillOp* d_sq_ops = nullptr;
-    FillBuf* d_sq_bufs = nullptr;
-    double* d_sq_scratch = nullptr;
+    FillDev dsq;
     double* d_sq_aux = nullptr;          // the saveqc program's aux scratch (aux mode)
     // aux arrays of the grids (FP64, see Context::auxk), set by
     // amrgpu_put_level_aux
@@ -116,10 +127,7 @@ struct Level {
     // (inputs of the two stepgrid calls and their results) and the tiles
     bool rich_valid = false;
     RichPlan rich;
-    FillOp* d_rops = nullptr;
-    FillBuf* d_rbufs = nullptr;
-    unsigned char* d_rmasks = nullptr;
-    double* d_rscratch = nullptr;
+    FillDev drich;
     double* d_rin = nullptr;
     double* d_rout = nullptr;
     PatchDesc* d_rcrs = nullptr;
@@ -275,11 +283,10 @@ void tend(int kind) {
 
 void free_rich(Level& L) {
     quiesce();
-    void* ps[] = {L.d_rops, L.d_rbufs, L.d_rmasks, L.d_rscratch, L.d_rin, L.d_rout, L.d_rcrs,
-                  L.d_rfine, L.d_rtiles_c, L.d_rtiles_f, L.d_rcfl};
+    L.drich.free();
+    void* ps[] = {L.d_rin, L.d_rout, L.d_rcrs, L.d_rfine, L.d_rtiles_c, L.d_rtiles_f, L.d_rcfl};
     for (void* p : ps)
         if (p) hipFree(p);
-    L.d_rops = nullptr; L.d_rbufs = nullptr; L.d_rmasks = nullptr; L.d_rscratch = nullptr;
     L.d_rin = nullptr; L.d_rout = nullptr; L.d_rcrs = nullptr; L.d_rfine = nullptr;
     L.d_rtiles_c = nullptr; L.d_rtiles_f = nullptr; L.d_rcfl = nullptr;
     L.rich = RichPlan();
@@ -291,14 +298,7 @@ void free_rich(Level& L) {
 void free_plan(Level& L) {
     quiesce();
     free_rich(L);
-    if (L.d_ops) hipFree(L.d_ops);
-    if (L.d_bufs) hipFree(L.d_bufs);
-    if (L.d_masks) hipFree(L.d_masks);
-    if (L.d_scratch) hipFree(L.d_scratch);
-    L.d_ops = nullptr;
-    L.d_bufs = nullptr;
-    L.d_masks = nullptr;
-    L.d_scratch = nullptr;
+    L.dplan.free();
     L.plan = FillPlan();
     L.plan_valid = false;
 }
@@ -306,7 +306,8 @@ void free_plan(Level& L) {
 void free_regs(Level& L) {
     quiesce();
     void* ps[] = {L.d_reg, L.d_sv, L.d_qad, L.d_ucells, L.d_uents, L.d_avg, L.d_avg_start,
-                  L.d_sq_ops, L.d_sq_bufs, L.d_sq_scratch, L.d_sq_aux};
+                  L.d_sq_aux};
+    L.dsq.free();
     for (void* p : ps)
         if (p) hipFree(p);
     L.d_sq_aux = nullptr;
@@ -317,9 +318,6 @@ void free_regs(Level& L) {
     L.d_uents = nullptr;
     L.d_avg = nullptr;
     L.d_avg_start = nullptr;
-    L.d_sq_ops = nullptr;
-    L.d_sq_bufs = nullptr;
-    L.d_sq_scratch = nullptr;
     L.nqad = L.nucells = L.navg = 0;
     L.navg_cells = 0;
     L.sq = FillPlan();
@@ -773,6 +771,28 @@ HierGeom make_geom() {
     return H;
 }
 
+// a fill program onto the device, its buffers resolved with the grids of the
+// levels as they are now (a level's program is dropped when the layout of it
+// or of a coarser level changes); old: the grids of FILL_OLDSLOT
+int upload_fill(const FillPlan& P, FillDev& D, const std::vector<PatchDesc>* old = nullptr) {
+    const std::vector<FillItem> items =
+        fill_items(P, g.cfg.nvar, [&](int l) -> const std::vector<PatchDesc>& {
+            return old && l == FILL_OLDSLOT ? *old : g.levels[l].patches;
+        });
+    if (items.empty()) return AMRGPU_OK;
+    HIPCHK(hipMalloc(&D.items, items.size() * sizeof(FillItem)));
+    HIPCHK(h2d(D.items, items.data(), items.size() * sizeof(FillItem)));
+    HIPCHK(hipMalloc(&D.units, P.units.size() * sizeof(FillUnit)));
+    HIPCHK(h2d(D.units, P.units.data(), P.units.size() * sizeof(FillUnit)));
+    if (!P.masks.empty()) {
+        HIPCHK(hipMalloc(&D.masks, P.masks.size()));
+        HIPCHK(h2d(D.masks, P.masks.data(), P.masks.size()));
+    }
+    if (P.scratch_elems > 0) HIPCHK(hipMalloc(&D.scratch, P.scratch_elems * sizeof(double)));
+    D.nunits = (int)P.units.size();
+    return AMRGPU_OK;
+}
+
 int ensure_plan(int level) {
     Level& L = g.levels[level];
     if (L.plan_valid) return AMRGPU_OK;
@@ -782,20 +802,8 @@ int ensure_plan(int level) {
     std::string err;
     if (!plan_fill_level(H, level, g.cfg.nvar, L.plan, err))
         return fail(AMRGPU_ERR_ARG, "level %d ghost fill: %s", level, err.c_str());
-    const FillPlan& P = L.plan;
-    if (!P.ops.empty()) {
-        HIPCHK(hipMalloc(&L.d_ops, P.ops.size() * sizeof(FillOp)));
-        HIPCHK(h2d(L.d_ops, P.ops.data(), P.ops.size() * sizeof(FillOp)));
-    }
-    if (!P.bufs.empty()) {
-        HIPCHK(hipMalloc(&L.d_bufs, P.bufs.size() * sizeof(FillBuf)));
-        HIPCHK(h2d(L.d_bufs, P.bufs.data(), P.bufs.size() * sizeof(FillBuf)));
-    }
-    if (!P.masks.empty()) {
-        HIPCHK(hipMalloc(&L.d_masks, P.masks.size()));
-        HIPCHK(h2d(L.d_masks, P.masks.data(), P.masks.size()));
-    }
-    if (P.scratch_elems > 0) HIPCHK(hipMalloc(&L.d_scratch, P.scratch_elems * sizeof(double)));
+    int rc = upload_fill(L.plan, L.dplan);
+    if (rc) return rc;
     L.plan_valid = true;
     return AMRGPU_OK;
 }
@@ -824,24 +832,12 @@ int time_weights(double t, FillArgs& a, uint32_t mask) {
     return AMRGPU_OK;
 }
 
-// launch the stages of a fill program (ghost fill or saveqc) at time t
-// clear / nclear: an array the first stage's launch zeroes on the way (the
-// level's Courant maxima before its sweep); *cleared reports whether it ran
-int run_fill(const FillPlan& P, const FillOp* d_ops, const FillBuf* d_bufs,
-             const unsigned char* d_masks, double* d_scratch, double t,
-             unsigned long long* clear = nullptr, int64_t nclear = 0, bool* cleared = nullptr) {
-    if (cleared) *cleared = false;
-    FillArgs a{};
-    int rc = time_weights(t, a, P.src_levels_mask);
-    if (rc) return rc;
-    a.bufs = d_bufs;
-    a.scratch = d_scratch;
-    a.masks = d_masks;
+// the levels' storage and geometry for a fill program
+void fill_levels(FillArgs& a) {
     for (int l = 1; l < MAXLV && l < FILL_MAXLV; l++) {
         Level& S = g.levels[l];
         a.lvl_new[l] = S.buf[S.cur];
         a.lvl_old[l] = S.buf[1 - S.cur];
-        a.lvl_patches[l] = S.d_patches;
         a.lvl_reg[l] = S.d_reg;
         a.hx[l] = g.hxposs[l];
         a.hy[l] = g.hyposs[l];
@@ -850,19 +846,28 @@ int run_fill(const FillPlan& P, const FillOp* d_ops, const FillBuf* d_bufs,
     a.ylower = g.cfg.ylower;
     for (int k = 0; k < 4; k++) a.mthbc[k] = g.cfg.mthbc[k];
     a.nv = g.cfg.nvar;
+}
+
+// launch the ghost fill of a level at time t and, with `sq`, the saveqc
+// program of the next finer one beside it: saveqc copies the level's interior
+// (store1), the ghost fill writes its ghost cells.  clear / nclear: an array
+// zeroed on the way (the level's Courant maxima before its sweep); *cleared
+// reports whether a launch ran
+int run_fill(const FillPlan& P, const FillDev& D, const FillDev* sq, double t,
+             unsigned long long* clear = nullptr, int64_t nclear = 0, bool* cleared = nullptr) {
+    FillArgs a{};
+    int rc = time_weights(t, a, P.src_levels_mask);
+    if (rc) return rc;
+    fill_levels(a);
+    a.prog[0] = D.prog();
+    if (sq) a.prog[1] = sq->prog();
+    a.clear = clear;
+    a.nclear = nclear;
+    if (cleared) *cleared = a.prog[0].nunits + a.prog[1].nunits > 0 && nclear > 0;
     tbegin(AMRGPU_KT_FILL);
-    for (int s = 0; s < P.nstages; s++) {
-        a.ops = d_ops + P.stage_start[s];
-        a.nops = P.stage_start[s + 1] - P.stage_start[s];
-        const bool clr = clear && nclear > 0 && a.nops > 0 && (!cleared || !*cleared);
-        a.clear = clr ? clear : nullptr;
-        a.nclear = clr ? nclear : 0;
-        hipError_t e = launch_fill_stage((int)g.esize, a, g.stream);
-        if (e != hipSuccess) return fail(AMRGPU_ERR_HIP, "fill stage %d: %s", s, hipGetErrorString(e));
-        if (clr && cleared) *cleared = true;
-        if (clr && !cleared) clear = nullptr;
-    }
+    hipError_t e = launch_fill((int)g.esize, a, g.stream);
     tend(AMRGPU_KT_FILL);
+    if (e != hipSuccess) return fail(AMRGPU_ERR_HIP, "ghost fill: %s", hipGetErrorString(e));
     return AMRGPU_OK;
 }
 
@@ -871,7 +876,7 @@ int bound_level(int level, double t) {
     if (L.ngrids == 0) return AMRGPU_OK;
     int rc = ensure_plan(level);
     if (rc) return rc;
-    return run_fill(L.plan, L.d_ops, L.d_bufs, L.d_masks, L.d_scratch, t);
+    return run_fill(L.plan, L.dplan, nullptr, t);
 }
 
 template <typename T>
@@ -939,10 +944,7 @@ int ensure_regs() {
             L.nqad = (int)Rl.qad.size();
             if (!plan_saveqc(H, l, nv, L.sq, err))
                 return fail(AMRGPU_ERR_ARG, "level %d saveqc: %s", l, err.c_str());
-            if ((rc = upload(&L.d_sq_ops, L.sq.ops))) return rc;
-            if ((rc = upload(&L.d_sq_bufs, L.sq.bufs))) return rc;
-            if (L.sq.scratch_elems > 0)
-                HIPCHK(hipMalloc(&L.d_sq_scratch, L.sq.scratch_elems * sizeof(double)));
+            if ((rc = upload_fill(L.sq, L.dsq))) return rc;
             // the aux mode's scratch too, here and not in the level step (which
             // a hipGraph may capture)
             if (g.auxk > 0 && L.sq.scratch_elems > 0)
@@ -1118,11 +1120,10 @@ int run_saveqc_aux(int level) {
         HIPCHK(launch_fill_u64(reinterpret_cast<unsigned long long*>(F.d_sq_aux), bits, n, g.stream));
     }
     FillArgs a{};
-    a.bufs = F.d_sq_bufs;
-    a.scratch = F.d_sq_aux;
+    a.prog[0] = F.dsq.prog();
+    a.prog[0].scratch = F.d_sq_aux;
     for (int l = 1; l < MAXLV && l < FILL_MAXLV; l++) {
         Level& S = g.levels[l];
-        a.lvl_patches[l] = S.d_patches;
         a.lvl_reg[l] = S.d_reg;
         a.lvl_aux[l] = S.d_aux;
     }
@@ -1130,12 +1131,8 @@ int run_saveqc_aux(int level) {
     a.aux_mode = 1;
     a.naux = g.cfg.naux;
     a.auxk = g.auxk;
-    for (int s = 0; s < P.nstages; s++) {
-        a.ops = F.d_sq_ops + P.stage_start[s];
-        a.nops = P.stage_start[s + 1] - P.stage_start[s];
-        hipError_t e = launch_fill_stage((int)g.esize, a, g.stream);
-        if (e != hipSuccess) return fail(AMRGPU_ERR_HIP, "saveqc aux: %s", hipGetErrorString(e));
-    }
+    hipError_t e = launch_fill((int)g.esize, a, g.stream);
+    if (e != hipSuccess) return fail(AMRGPU_ERR_HIP, "saveqc aux: %s", hipGetErrorString(e));
     return AMRGPU_OK;
 }
 
@@ -1158,16 +1155,14 @@ int launch_level_step(int level) {
     Level& L = g.levels[level];
     int rc = ensure_plan(level);
     if (rc) return rc;
-    bool cfl_cleared = false;   // the fill's first launch zeroes the Courant maxima
-    rc = run_fill(L.plan, L.d_ops, L.d_bufs, L.d_masks, L.d_scratch, L.time, L.d_cfl,
+    const bool has_fine = level + 1 <= g.mxnest && level + 1 < MAXLV && g.levels[level + 1].ngrids > 0;
+    bool cfl_cleared = false;   // the fill zeroes the Courant maxima
+    rc = run_fill(L.plan, L.dplan, has_fine ? &g.levels[level + 1].dsq : nullptr, L.time, L.d_cfl,
                   L.ngrids, &cfl_cleared);
     if (rc) return rc;
-    const bool has_fine = level + 1 <= g.mxnest && level + 1 < MAXLV && g.levels[level + 1].ngrids > 0;
     RegLink rl;
     if (has_fine) {
         Level& F = g.levels[level + 1];
-        rc = run_fill(F.sq, F.d_sq_ops, F.d_sq_bufs, nullptr, F.d_sq_scratch, L.time);
-        if (rc) return rc;
         if (g.auxk > 0) {
             rc = run_saveqc_aux(level + 1);
             if (rc) return rc;
@@ -1389,13 +1384,8 @@ int ensure_rich(int level) {
     std::string err;
     if (!plan_richardson(H, level, g.cfg.nvar, L.rich, err))
         return fail(AMRGPU_ERR_ARG, "level %d Richardson estimate: %s", level, err.c_str());
-    const FillPlan& P = L.rich.fill;
-    int rc;
-    std::vector<FillOp> ops = P.ops;
-    if ((rc = upload(&L.d_rops, ops))) return rc;
-    if ((rc = upload(&L.d_rbufs, P.bufs))) return rc;
-    if ((rc = upload(&L.d_rmasks, P.masks))) return rc;
-    if (P.scratch_elems > 0) HIPCHK(hipMalloc(&L.d_rscratch, P.scratch_elems * sizeof(double)));
+    int rc = upload_fill(L.rich.fill, L.drich);
+    if (rc) return rc;
     HIPCHK(hipMalloc(&L.d_rin, std::max<int64_t>(L.rich.arena_elems, 1) * sizeof(double)));
     HIPCHK(hipMalloc(&L.d_rout, std::max<int64_t>(L.rich.arena_elems, 1) * sizeof(double)));
     if ((rc = upload(&L.d_rcrs, L.rich.crs))) return rc;
@@ -1420,31 +1410,13 @@ int richardson(int level, bool big_old, int mbuff, double tol, int iorder) {
     FillArgs a{};
     rc = time_weights(tpre, a, L.rich.fill.src_levels_mask);
     if (rc) return rc;
-    a.bufs = L.d_rbufs;
-    a.scratch = L.d_rscratch;
-    a.masks = L.d_rmasks;
+    fill_levels(a);
+    a.prog[0] = L.drich.prog();
     a.arena = L.d_rin;
     a.big_old = big_old ? 1 : 0;
-    for (int l = 1; l < MAXLV && l < FILL_MAXLV; l++) {
-        Level& S = g.levels[l];
-        a.lvl_new[l] = S.buf[S.cur];
-        a.lvl_old[l] = S.buf[1 - S.cur];
-        a.lvl_patches[l] = S.d_patches;
-        a.lvl_reg[l] = S.d_reg;
-        a.hx[l] = g.hxposs[l];
-        a.hy[l] = g.hyposs[l];
-    }
-    a.xlower = g.cfg.xlower;
-    a.ylower = g.cfg.ylower;
-    for (int k = 0; k < 4; k++) a.mthbc[k] = g.cfg.mthbc[k];
-    a.nv = g.cfg.nvar;
     tbegin(AMRGPU_KT_FLAG);
-    for (int s = 0; s < L.rich.fill.nstages; s++) {
-        a.ops = L.d_rops + L.rich.fill.stage_start[s];
-        a.nops = L.rich.fill.stage_start[s + 1] - L.rich.fill.stage_start[s];
-        hipError_t e = launch_fill_stage((int)g.esize, a, g.stream);
-        if (e != hipSuccess) return fail(AMRGPU_ERR_HIP, "Richardson fill stage %d: %s", s, hipGetErrorString(e));
-    }
+    hipError_t ef = launch_fill((int)g.esize, a, g.stream);
+    if (ef != hipSuccess) return fail(AMRGPU_ERR_HIP, "Richardson fill: %s", hipGetErrorString(ef));
     // the 2 dt step on 2 h (prepbigstep.f:61-64) and the dt step
     // (prepregstep.f:24-27), FP64, into the output arena
     SweepArgs sa{};
@@ -2280,17 +2252,14 @@ int amrgpu_regrid_level(int level, int ngrids, const int* ilo, const int* ihi, c
     Level& L = g.levels[level];
     // keep the old grids' new-time values and descriptors: define_level
     // frees the rest of the old level
+    const std::vector<PatchDesc> old_patches = L.patches;
     std::vector<std::array<int, 4>> old_boxes;
-    for (const auto& pd : L.patches) old_boxes.push_back({pd.ilo, pd.ihi, pd.jlo, pd.jhi});
+    for (const auto& pd : old_patches) old_boxes.push_back({pd.ilo, pd.ihi, pd.jlo, pd.jhi});
     void* old_buf = L.buf[L.cur];
-    PatchDesc* old_d = L.d_patches;
     L.buf[L.cur] = nullptr;
-    L.d_patches = nullptr;
     auto drop_old = [&]() {
         if (old_buf) hipFree(old_buf);
-        if (old_d) hipFree(old_d);
         old_buf = nullptr;
-        old_d = nullptr;
     };
     rc = define_level(level, ngrids, ilo, ihi, jlo, jhi, g.hxposs[level], g.hyposs[level]);
     if (rc) {
@@ -2313,54 +2282,26 @@ int amrgpu_regrid_level(int level, int ngrids, const int* ilo, const int* ihi, c
         drop_old();
         return fail(AMRGPU_ERR_ARG, "level %d regrid: %s", level, err.c_str());
     }
-    FillOp* d_ops = nullptr;
-    FillBuf* d_bufs = nullptr;
-    unsigned char* d_masks = nullptr;
-    double* d_scratch = nullptr;
-    auto drop_plan = [&]() {
-        void* ps[] = {d_ops, d_bufs, d_masks, d_scratch};
-        for (void* p : ps)
-            if (p) hipFree(p);
-    };
-    hipError_t e = hipSuccess;
-    if (!P.ops.empty()) e = hipMalloc(&d_ops, P.ops.size() * sizeof(FillOp));
-    if (e == hipSuccess && !P.ops.empty()) e = h2d(d_ops, P.ops.data(), P.ops.size() * sizeof(FillOp));
-    if (e == hipSuccess && !P.bufs.empty()) e = hipMalloc(&d_bufs, P.bufs.size() * sizeof(FillBuf));
-    if (e == hipSuccess && !P.bufs.empty()) e = h2d(d_bufs, P.bufs.data(), P.bufs.size() * sizeof(FillBuf));
-    if (e == hipSuccess && !P.masks.empty()) e = hipMalloc(&d_masks, P.masks.size());
-    if (e == hipSuccess && !P.masks.empty()) e = h2d(d_masks, P.masks.data(), P.masks.size());
-    if (e == hipSuccess && P.scratch_elems > 0)
-        e = hipMalloc(&d_scratch, (size_t)P.scratch_elems * sizeof(double));
+    FillDev D;
+    rc = upload_fill(P, D, &old_patches);
+    if (rc) {
+        D.free();
+        drop_old();
+        return rc;
+    }
     FillArgs a{};
-    a.bufs = d_bufs;
-    a.scratch = d_scratch;
-    a.masks = d_masks;
+    fill_levels(a);
     for (int l = 1; l < MAXLV && l < FILL_MAXLV; l++) {
-        Level& S = g.levels[l];
-        a.lvl_new[l] = S.buf[S.cur];
-        a.lvl_old[l] = S.buf[1 - S.cur];
-        a.lvl_patches[l] = S.d_patches;
-        a.lvl_reg[l] = S.d_reg;
-        a.hx[l] = g.hxposs[l];
-        a.hy[l] = g.hyposs[l];
         a.tmode[l] = TIME_NEW;
         a.alphai[l] = 1.0;
         a.alphac[l] = 0.0;
     }
     a.lvl_new[FILL_OLDSLOT] = old_buf;
     a.lvl_old[FILL_OLDSLOT] = old_buf;
-    a.lvl_patches[FILL_OLDSLOT] = old_d;
-    a.xlower = g.cfg.xlower;
-    a.ylower = g.cfg.ylower;
-    for (int k = 0; k < 4; k++) a.mthbc[k] = g.cfg.mthbc[k];
-    a.nv = g.cfg.nvar;
-    for (int s = 0; e == hipSuccess && s < P.nstages; s++) {
-        a.ops = d_ops + P.stage_start[s];
-        a.nops = P.stage_start[s + 1] - P.stage_start[s];
-        e = launch_fill_stage((int)g.esize, a, g.stream);
-    }
+    a.prog[0] = D.prog();
+    hipError_t e = launch_fill((int)g.esize, a, g.stream);
     if (e == hipSuccess) e = hipStreamSynchronize(g.stream);
-    drop_plan();
+    D.free();
     drop_old();
     if (e != hipSuccess) return fail(AMRGPU_ERR_HIP, "level %d regrid: %s", level, hipGetErrorString(e));
     return AMRGPU_OK;

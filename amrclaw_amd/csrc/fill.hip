@@ -1,4 +1,4 @@
-// fill.hip -- executes one stage of a ghost-cell fill program.
+// fill.hip -- executes ghost-cell fill programs.
 // Built with -ffp-contract=off: the time blend and the coarse-fine
 // interpolation are evaluated exactly as the reference's FP64 code.
 #include <hip/hip_runtime.h>
@@ -9,85 +9,78 @@ namespace amrgpu {
 
 template <typename S>
 struct BufRef {
-    S* lvl;          // kind 0
-    double* scr;     // kind 1
-    int64_t off;
+    S* lvl;          // a level's storage
+    double* scr;     // FP64 scratch or arena
     int32_t nrow, plane;
-    __device__ double load(int m, int i, int j) const {
-        int64_t k = off + (int64_t)m * plane + (int64_t)j * nrow + i;
-        return lvl ? (double)lvl[k] : scr[k];
-    }
-    __device__ void store(int m, int i, int j, double v) const {
-        int64_t k = off + (int64_t)m * plane + (int64_t)j * nrow + i;
+    __device__ double load(int m, int i, int j) const { return at((int64_t)m * plane + (int64_t)j * nrow + i); }
+    __device__ double at(int64_t k) const { return lvl ? (double)lvl[k] : scr[k]; }
+    __device__ void store(int m, int i, int j, double v) const { put((int64_t)m * plane + (int64_t)j * nrow + i, v); }
+    __device__ void put(int64_t k, double v) const {
         if (lvl) lvl[k] = (S)v; else scr[k] = v;
     }
 };
 
 template <typename S>
-__device__ BufRef<S> bufref(const FillArgs& a, int b) {
-    const FillBuf fb = a.bufs[b];
+__device__ BufRef<S> bufref(const FillArgs& a, const FillProg& pr, int space, int64_t off, int nrow,
+                            int plane) {
     BufRef<S> r;
-    if (fb.kind == 0) {
-        r.lvl = static_cast<S*>(a.lvl_new[fb.level]);
-        r.scr = nullptr;
-        r.off = a.lvl_patches[fb.level][fb.patch].off;
-    } else {
-        r.lvl = nullptr;
-        r.scr = fb.kind == 1 ? a.scratch : a.arena;
-        r.off = fb.off;
-    }
-    r.nrow = fb.nrow;
-    r.plane = fb.plane;
+    r.lvl = space >= 0 ? static_cast<S*>(a.lvl_new[space]) + off : nullptr;
+    r.scr = space >= 0 ? nullptr : (space == FSP_SCRATCH ? pr.scratch : a.arena) + off;
+    r.nrow = nrow;
+    r.plane = plane;
     return r;
+}
+
+// cell idx of the ring cstore.f walks: sides 1 (left column), 2 (top row), 3
+// (right column), 4 (bottom row) of the coarsened patch, corners excluded
+__device__ __forceinline__ int64_t ring_cell(int idx, int nrow, int ncol) {
+    const int n1 = ncol - 2, n2 = nrow - 2;
+    int i, j;
+    if (idx < n1) { i = 0; j = 1 + idx; }
+    else if (idx < n1 + n2) { i = 1 + idx - n1; j = ncol - 1; }
+    else if (idx < 2 * n1 + n2) { i = nrow - 1; j = 1 + idx - n1 - n2; }
+    else { i = 1 + idx - 2 * n1 - n2; j = 0; }
+    return (int64_t)j * nrow + i;
 }
 
 // the aux-mode copy of a saveqc program: aux values of the coarse grids
 // into the coarse patch (icall.f's aux part) and the patch's ring into
 // auxc1d (cstore.f); NEEDS_TO_BE_SET stays where no coarse grid reached
-__device__ void fill_aux_op(const FillArgs& a, const FillOp& op, int tid) {
+template <int NT>
+__device__ void fill_aux_op(const FillArgs& a, const FillProg& pr, const FillItem& op, int tid) {
     const int na = a.naux;
     if (op.type == FOP_COPY) {
-        const PatchDesc sp = a.lvl_patches[op.src_level][op.src];
-        const double* sa = a.lvl_aux[op.src_level] + sp.off * a.auxk;
-        const FillBuf fb = a.bufs[op.dst];
-        double* da = a.scratch + fb.off * a.auxk;
+        const double* sa = a.lvl_aux[op.src_space] + op.src_off * a.auxk + op.src_shift;
+        double* da = pr.scratch + op.dst_off * a.auxk + op.dst_shift;
         const int ncell = op.ni * op.nj;
-        for (int t = tid; t < ncell * na; t += 256) {
+        for (int t = tid; t < ncell * na; t += NT) {
             const int c = t / ncell, r = t - c * ncell;
             const int dj = r / op.ni, di = r - dj * op.ni;
-            da[(int64_t)c * fb.plane + (int64_t)(op.dj0 + dj) * fb.nrow + (op.di0 + di)] =
-                sa[(int64_t)c * sp.plane + (int64_t)(op.sj0 + dj) * sp.mitot + (op.si0 + di)];
+            da[(int64_t)c * op.dst_plane + (int64_t)dj * op.dst_nrow + di] =
+                sa[(int64_t)c * op.src_plane + (int64_t)dj * op.src_nrow + di];
         }
     } else if (op.type == FOP_RING) {
-        const FillBuf fb = a.bufs[op.src];
-        const double* sa = a.scratch + fb.off * a.auxk;
-        const PatchDesc pf = a.lvl_patches[op.level][op.si0];
-        double* ac1d = a.lvl_reg[op.level] + aux_ring_offset(pf, a.nv);
-        const int nrow = op.ni, ncol = op.nj;
-        const int n1 = ncol - 2, n2 = nrow - 2;
-        const int len = 2 * (n1 + n2);
-        for (int t = tid; t < len * na; t += 256) {
+        const double* sa = pr.scratch + op.src_off * a.auxk;
+        double* ac1d = a.lvl_reg[op.level] + op.aux_off;
+        const int len = 2 * (op.ni - 2 + op.nj - 2);
+        for (int t = tid; t < len * na; t += NT) {
             const int idx = t / na, c = t - idx * na;
-            int i, j;
-            if (idx < n1) { i = 0; j = 1 + idx; }
-            else if (idx < n1 + n2) { i = 1 + idx - n1; j = ncol - 1; }
-            else if (idx < 2 * n1 + n2) { i = nrow - 1; j = 1 + idx - n1 - n2; }
-            else { i = 1 + idx - 2 * n1 - n2; j = 0; }
-            ac1d[(int64_t)idx * na + c] = sa[(int64_t)c * fb.plane + (int64_t)j * nrow + i];
+            ac1d[(int64_t)idx * na + c] = sa[(int64_t)c * op.src_plane + ring_cell(idx, op.ni, op.nj)];
         }
     }
 }
 
-// t = tid + 256 k written as digits (i, j, m) of the radices (ni, nj):
-// stepped by 256 with one carry per digit instead of two integer divisions
+// t = tid + NT k written as digits (i, j, m) of the radices (ni, nj):
+// stepped by NT with one carry per digit instead of two integer divisions
 // per element (a digit plus its step plus a carry stays below twice its
 // radix, so one subtraction brings it back)
+template <int NT>
 struct Digits2 {
     int i, j, m, si, sj, sm, ni, nj;
     __device__ __forceinline__ Digits2(int t, int ni_, int nj_)
         : ni(ni_ > 0 ? ni_ : 1), nj(nj_ > 0 ? nj_ : 1) {   // (an empty op runs no element)
         i = t % ni; t /= ni; j = t % nj; m = t / nj;
-        int r = 256;
+        int r = NT;
         si = r % ni; r /= ni; sj = r % nj; sm = r / nj;
     }
     __device__ __forceinline__ void step() {
@@ -101,48 +94,127 @@ struct Digits2 {
     }
 };
 
-template <typename S>
-__global__ __launch_bounds__(256) void fill_stage_kernel(FillArgs a) {
-    const FillOp op = a.ops[blockIdx.x];
-    const int tid = threadIdx.x, nv = a.nv;
-    if (a.clear && blockIdx.x == 0)
-        for (int64_t t = tid; t < a.nclear; t += 256) a.clear[t] = 0ull;
-    if (a.aux_mode) {
-        fill_aux_op(a, op, tid);
-        return;
+// every element (cell x component) of a rectangle from `load` into `dst`,
+// four elements a thread in flight
+template <int NT, typename S, class Load>
+__device__ __forceinline__ void copy_rect(const FillItem& op, const BufRef<S>& dst, int tid, int nv,
+                                          const Load& load) {
+    const int n = op.ni * op.nj * nv;
+    Digits2<NT> u(tid, op.ni, op.nj);
+    for (int t = tid; t < n; t += 4 * NT) {
+        double v[4];
+        int64_t d[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++, u.step()) {
+            d[k] = t + NT * k < n ? (int64_t)u.m * dst.plane + (int64_t)u.j * dst.nrow + u.i : -1;
+            if (d[k] >= 0) v[k] = load((int64_t)u.m * op.src_plane + (int64_t)u.j * op.src_nrow + u.i);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            if (d[k] >= 0) dst.put(op.dst_shift + d[k], v[k]);
     }
-    const BufRef<S> dst = bufref<S>(a, op.dst);
+}
+
+// components n .. n + C - 1 of the interpolation at one fine cell: all the
+// coarse values are loaded before the first store (to an array the compiler
+// cannot tell apart from theirs)
+template <int C, typename S>
+__device__ __forceinline__ void interp_cell(const BufRef<S>& crs, const BufRef<S>& dst, int n, int64_t s,
+                                            int64_t d, double eta1, double eta2) {
+    double p10[C], m10[C], c0[C], p01[C], m01[C];
+#pragma unroll
+    for (int k = 0; k < C; k++) {
+        const int64_t b = s + (int64_t)(n + k) * crs.plane;
+        p10[k] = crs.at(b + 1);
+        m10[k] = crs.at(b - 1);
+        c0[k] = crs.at(b);
+        p01[k] = crs.at(b + crs.nrow);
+        m01[k] = crs.at(b - crs.nrow);
+    }
+#pragma unroll
+    for (int k = 0; k < C; k++) {
+        const double dupc = p10[k] - c0[k], dumc = c0[k] - m10[k], ducc = p10[k] - m10[k];
+        double du = fmin(fabs(dupc), fabs(dumc));
+        du = fmin(2.0 * du, 0.5 * fabs(ducc));
+        const double fu = fmax(0.0, copysign(1.0, dupc * dumc));
+        const double uslope = du * copysign(1.0, ducc) * fu;
+        const double dvpc = p01[k] - c0[k], dvmc = c0[k] - m01[k], dvcc = p01[k] - m01[k];
+        double dv = fmin(fabs(dvpc), fabs(dvmc));
+        dv = fmin(2.0 * dv, 0.5 * fabs(dvcc));
+        const double fv = fmax(0.0, copysign(1.0, dvpc * dvmc));
+        const double vslope = dv * copysign(1.0, dvcc) * fv;
+        dst.put(d + (int64_t)(n + k) * dst.plane, c0[k] + eta1 * uslope + eta2 * vslope);
+    }
+}
+
+// one side of bc2amr: the cells [i0, i0 + ni) x [j0, j0 + nj) from the cells
+// `from` maps them to (none of them on this side), component `flip` negated
+template <int NT, typename S, class From>
+__device__ __forceinline__ void bc_side(const BufRef<S>& b, int tid, int nv, int ni, int nj, int i0,
+                                        int j0, int flip, const From& from) {
+    constexpr int B = 8;
+    const int n = ni * nj * nv;
+    Digits2<NT> u(tid, ni, nj);
+    for (int t = tid; t < n; t += B * NT) {
+        double v[B];
+        int64_t d[B];
+#pragma unroll
+        for (int k = 0; k < B; k++, u.step()) {
+            int i = i0 + u.i, j = j0 + u.j;
+            d[k] = t + NT * k < n ? (int64_t)u.m * b.plane + (int64_t)j * b.nrow + i : -1;
+            if (d[k] >= 0) {
+                from(i, j);
+                v[k] = b.load(u.m, i, j);
+                if (u.m == flip) v[k] = -v[k];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < B; k++)
+            if (d[k] >= 0) b.put(d[k], v[k]);
+    }
+}
+
+constexpr int FILL_CHUNK = 8;   // items read at a time
+constexpr int FILL_WORDS = sizeof(FillItem) / 4;
+
+// an item out of LDS into scalar registers
+__device__ __forceinline__ FillItem uniform_item(const int32_t* sh) {
+    union { FillItem it; int32_t w[FILL_WORDS]; } u;
+#pragma unroll
+    for (int k = 0; k < FILL_WORDS; k++) u.w[k] = __builtin_amdgcn_readfirstlane(sh[k]);
+    return u.it;
+}
+
+// one operation, over the threads of the workgroup
+template <typename S, int NT>
+__device__ __forceinline__ void fill_op(const FillArgs& a, const FillProg& pr, const FillItem& op, int tid) {
+    const int nv = a.nv;
+    const BufRef<S> dst = bufref<S>(a, pr, op.dst_space, op.dst_off, op.dst_nrow, op.dst_plane);
     const int ncell = op.ni * op.nj;
 
     if (op.type == FOP_COPY) {
-        const PatchDesc sp = a.lvl_patches[op.src_level][op.src];
-        const S* qn = static_cast<const S*>(a.lvl_new[op.src_level]) + sp.off;
-        const S* qo = static_cast<const S*>(a.lvl_old[op.src_level]) + sp.off;
-        int mode = a.tmode[op.src_level];
+        const S* qn = static_cast<const S*>(a.lvl_new[op.src_space]) + op.src_off + op.src_shift;
+        const S* qo = static_cast<const S*>(a.lvl_old[op.src_space]) + op.src_off + op.src_shift;
+        int mode = a.tmode[op.src_space];
         if (op.flags & FOPF_FORCE_NEW) mode = TIME_NEW;
         else if (op.flags & FOPF_FORCE_OLD) mode = TIME_OLD;
         else if (op.flags & FOPF_BIG) mode = a.big_old ? TIME_OLD : TIME_NEW;
-        const double ai = a.alphai[op.src_level], ac = a.alphac[op.src_level];
-        Digits2 u(tid, op.ni, op.nj);
-        for (int t = tid; t < ncell * nv; t += 256, u.step()) {
-            const int m = u.m, dj = u.j, di = u.i;
-            const int64_t s = (int64_t)m * sp.plane + (int64_t)(op.sj0 + dj) * sp.mitot + (op.si0 + di);
-            double v;
-            if (mode == TIME_NEW) v = (double)qn[s];
-            else if (mode == TIME_OLD) v = (double)qo[s];
-            else v = (double)qn[s] * ai + (double)qo[s] * ac;
-            dst.store(m, op.di0 + di, op.dj0 + dj, v);
-        }
+        const double ai = a.alphai[op.src_space], ac = a.alphac[op.src_space];
+        const S* q1 = mode == TIME_OLD ? qo : qn;
+        if (mode != TIME_BLEND)
+            copy_rect<NT, S>(op, dst, tid, nv, [&](int64_t k) { return (double)q1[k]; });
+        else
+            copy_rect<NT, S>(op, dst, tid, nv, [&](int64_t k) { return (double)qn[k] * ai + (double)qo[k] * ac; });
     } else if (op.type == FOP_INTERP) {
-        const BufRef<S> crs = bufref<S>(a, op.src);
+        const BufRef<S> crs = bufref<S>(a, pr, op.src_space, op.src_off, op.src_nrow, op.src_plane);
         const double dxf = a.hx[op.level], dyf = a.hy[op.level];
         const double dxc = a.hx[op.level - 1], dyc = a.hy[op.level - 1];
         const double xlow_coarse = a.xlower + op.iplo * dxc;
         const double ylow_coarse = a.ylower + op.jplo * dyc;
         const double ratiox = (double)op.ratx, ratioy = (double)op.raty;
-        const unsigned char* mask = a.masks + op.mask_off;
-        Digits2 u(tid, op.ni, 1 << 30);   // (i, j) of cell c; j does not wrap
-        for (int c = tid; c < ncell; c += 256, u.step()) {
+        const unsigned char* mask = pr.masks + op.mask_off;
+        Digits2<NT> u(tid, op.ni, 1 << 30);   // (i, j) of cell c; j does not wrap
+        for (int c = tid; c < ncell; c += NT, u.step()) {
             if (mask[c]) continue;
             const int jf = u.j + 1, if_ = u.i + 1;   // 1-based
             const int j_coarse = (int)floor((double)(jf + op.jlo - 1) / ratioy) - op.jplo + 1;
@@ -153,36 +225,23 @@ __global__ __launch_bounds__(256) void fill_stage_kernel(FillArgs a) {
             const double xcent_coarse = xlow_coarse + ((double)i_coarse - .5) * dxc;
             const double xcent_fine = a.xlower + ((double)(if_ - 1 + op.ilo) + .5) * dxf;
             const double eta1 = (xcent_fine - xcent_coarse) / dxc;
-            const int ic = i_coarse - 1, jc = j_coarse - 1;                  // 0-based
-            for (int n = 0; n < nv; n++) {
-                const double valp10 = crs.load(n, ic + 1, jc);
-                const double valm10 = crs.load(n, ic - 1, jc);
-                const double valc = crs.load(n, ic, jc);
-                const double valp01 = crs.load(n, ic, jc + 1);
-                const double valm01 = crs.load(n, ic, jc - 1);
-                const double dupc = valp10 - valc, dumc = valc - valm10, ducc = valp10 - valm10;
-                double du = fmin(fabs(dupc), fabs(dumc));
-                du = fmin(2.0 * du, 0.5 * fabs(ducc));
-                const double fu = fmax(0.0, copysign(1.0, dupc * dumc));
-                const double uslope = du * copysign(1.0, ducc) * fu;
-                const double dvpc = valp01 - valc, dvmc = valc - valm01, dvcc = valp01 - valm01;
-                double dv = fmin(fabs(dvpc), fabs(dvmc));
-                dv = fmin(2.0 * dv, 0.5 * fabs(dvcc));
-                const double fv = fmax(0.0, copysign(1.0, dvpc * dvmc));
-                const double vslope = dv * copysign(1.0, dvcc) * fv;
-                const double valint = valc + eta1 * uslope + eta2 * vslope;
-                dst.store(n, op.di0 + if_ - 1, op.dj0 + jf - 1, valint);
-            }
+            const int64_t s = (int64_t)(j_coarse - 1) * crs.nrow + i_coarse - 1;
+            const int64_t d = op.dst_shift + (int64_t)u.j * dst.nrow + u.i;
+            int n = 0;
+            for (; n + 4 <= nv; n += 4) interp_cell<4, S>(crs, dst, n, s, d, eta1, eta2);
+            if (nv - n == 3) interp_cell<3, S>(crs, dst, n, s, d, eta1, eta2);
+            else if (nv - n == 2) interp_cell<2, S>(crs, dst, n, s, d, eta1, eta2);
+            else if (nv - n == 1) interp_cell<1, S>(crs, dst, n, s, d, eta1, eta2);
         }
     } else if (op.type == FOP_FILVAL) {
         // src: the coarse patch grown by one coarse cell (ni x nj); dst: the
         // new grid; mask: its interior cells, row by row, 1 where an old
         // grid supplied the value (the reference's setflags test)
-        const BufRef<S> crs = bufref<S>(a, op.src);
+        const BufRef<S> crs = bufref<S>(a, pr, op.src_space, op.src_off, op.src_nrow, op.src_plane);
         const int rx = op.ratx, ry = op.raty, mic = op.ni, mjc = op.nj;
         const int ncx = mic - 2, ncc = ncx * (mjc - 2), nx = ncx * rx;
-        const unsigned char* mask = a.masks + op.mask_off;
-        for (int t = tid; t < ncc * nv; t += 256) {
+        const unsigned char* mask = pr.masks + op.mask_off;
+        for (int t = tid; t < ncc * nv; t += NT) {
             const int m = t / ncc, c = t - m * ncc;
             const int jc = c / ncx + 1, ic = c - (jc - 1) * ncx + 1;   // 0-based, 1..mic-2
             const double vc = crs.load(m, ic, jc);
@@ -207,34 +266,20 @@ __global__ __launch_bounds__(256) void fill_stage_kernel(FillArgs a) {
             }
         }
     } else if (op.type == FOP_COPYBACK) {
-        const BufRef<S> src = bufref<S>(a, op.src);
-        for (int t = tid; t < ncell * nv; t += 256) {
-            const int m = t / ncell, c = t - m * ncell;
-            const int dj = c / op.ni, di = c - dj * op.ni;
-            dst.store(m, op.di0 + di, op.dj0 + dj, src.load(m, di, dj));
-        }
+        const BufRef<S> src = bufref<S>(a, pr, op.src_space, op.src_off, op.src_nrow, op.src_plane);
+        copy_rect<NT, S>(op, dst, tid, nv, [&](int64_t k) { return src.at(k); });
     } else if (op.type == FOP_RING) {
-        // cstore.f: sides 1 (left column), 2 (top row), 3 (right column),
-        // 4 (bottom row) of the coarsened patch, corners excluded
-        const BufRef<S> src = bufref<S>(a, op.src);
-        const PatchDesc pf = a.lvl_patches[op.level][op.si0];
-        double* qc1d = a.lvl_reg[op.level] + pf.reg_off + (int64_t)nv * pf.lenbc;
-        const int nrow = op.ni, ncol = op.nj;
-        const int n1 = ncol - 2, n2 = nrow - 2;
-        const int len = 2 * (n1 + n2);
-        for (int t = tid; t < len * nv; t += 256) {
+        const BufRef<S> src = bufref<S>(a, pr, op.src_space, op.src_off, op.src_nrow, op.src_plane);
+        double* qc1d = a.lvl_reg[op.level] + op.dst_off;
+        const int len = 2 * (op.ni - 2 + op.nj - 2);
+        for (int t = tid; t < len * nv; t += NT) {
             const int idx = t / nv, m = t - idx * nv;
-            int i, j;
-            if (idx < n1) { i = 0; j = 1 + idx; }
-            else if (idx < n1 + n2) { i = 1 + idx - n1; j = ncol - 1; }
-            else if (idx < 2 * n1 + n2) { i = nrow - 1; j = 1 + idx - n1 - n2; }
-            else { i = 1 + idx - 2 * n1 - n2; j = 0; }
-            qc1d[(int64_t)idx * nv + m] = src.load(m, i, j);
+            qc1d[(int64_t)idx * nv + m] = src.at((int64_t)m * src.plane + ring_cell(idx, op.ni, op.nj));
         }
     } else if (op.type == FOP_COARSEN) {
         // coarsen.f:15-30: dst(i, j) = mean of src(2i..2i+1, 2j..2j+1)
-        const BufRef<S> src = bufref<S>(a, op.src);
-        for (int t = tid; t < ncell * nv; t += 256) {
+        const BufRef<S> src = bufref<S>(a, pr, op.src_space, op.src_off, op.src_nrow, op.src_plane);
+        for (int t = tid; t < ncell * nv; t += NT) {
             const int m = t / ncell, c = t - m * ncell;
             const int j = c / op.ni, i = c - j * op.ni;
             const double v = (src.load(m, 2 * i, 2 * j) + src.load(m, 2 * i + 1, 2 * j) +
@@ -242,71 +287,90 @@ __global__ __launch_bounds__(256) void fill_stage_kernel(FillArgs a) {
             dst.store(m, i, j, v);
         }
     } else if (op.type == FOP_BC) {
-        // sides in the reference's order, each complete before the next
+        // sides in the reference's order, each complete before the next:
+        // extrapolation (1) or mirrored (wall, 3)
         const int nrow = op.ni, ncol = op.nj;
-        // left: columns 0..nxl-1 from column nxl (extrapolation) or mirrored (wall)
-        const int nxl = op.bc[0];
+        const int nxl = op.bc[0], nyb = op.bc[2];
+        const int ibeg = op.bc[1], jbeg = op.bc[3];   // 1-based first column / row set
         if (nxl > 0 && (a.mthbc[0] == 1 || a.mthbc[0] == 3)) {
-            for (int t = tid; t < nxl * ncol; t += 256) {
-                const int j = t / nxl, i = t - j * nxl;
-                const int isrc = a.mthbc[0] == 1 ? nxl : 2 * nxl - 1 - i;
-                for (int m = 0; m < nv; m++) {
-                    double v = dst.load(m, isrc, j);
-                    if (a.mthbc[0] == 3 && m == 1) v = -v;
-                    dst.store(m, i, j, v);
-                }
-            }
+            const bool wall = a.mthbc[0] == 3;
+            bc_side<NT>(dst, tid, nv, nxl, ncol, 0, 0, wall ? 1 : -1,
+                        [=](int& i, int&) { i = wall ? 2 * nxl - 1 - i : nxl; });
         }
         __syncthreads();
-        const int ibeg = op.bc[1];              // 1-based first column set
         if (ibeg > 0 && (a.mthbc[1] == 1 || a.mthbc[1] == 3)) {
-            const int nr = nrow - ibeg + 1;
-            for (int t = tid; t < nr * ncol; t += 256) {
-                const int j = t / nr, i = ibeg - 1 + (t - j * nr);
-                const int isrc = a.mthbc[1] == 1 ? ibeg - 2 : 2 * ibeg - 1 - (i + 1) - 1;
-                for (int m = 0; m < nv; m++) {
-                    double v = dst.load(m, isrc, j);
-                    if (a.mthbc[1] == 3 && m == 1) v = -v;
-                    dst.store(m, i, j, v);
-                }
-            }
+            const bool wall = a.mthbc[1] == 3;
+            bc_side<NT>(dst, tid, nv, nrow - ibeg + 1, ncol, ibeg - 1, 0, wall ? 1 : -1,
+                        [=](int& i, int&) { i = wall ? 2 * ibeg - 3 - i : ibeg - 2; });
         }
         __syncthreads();
-        const int nyb = op.bc[2];
         if (nyb > 0 && (a.mthbc[2] == 1 || a.mthbc[2] == 3)) {
-            for (int t = tid; t < nyb * nrow; t += 256) {
-                const int j = t / nrow, i = t - j * nrow;
-                const int jsrc = a.mthbc[2] == 1 ? nyb : 2 * nyb - 1 - j;
-                for (int m = 0; m < nv; m++) {
-                    double v = dst.load(m, i, jsrc);
-                    if (a.mthbc[2] == 3 && m == 2) v = -v;
-                    dst.store(m, i, j, v);
-                }
-            }
+            const bool wall = a.mthbc[2] == 3;
+            bc_side<NT>(dst, tid, nv, nrow, nyb, 0, 0, wall ? 2 : -1,
+                        [=](int&, int& j) { j = wall ? 2 * nyb - 1 - j : nyb; });
         }
         __syncthreads();
-        const int jbeg = op.bc[3];
         if (jbeg > 0 && (a.mthbc[3] == 1 || a.mthbc[3] == 3)) {
-            const int nc = ncol - jbeg + 1;
-            for (int t = tid; t < nc * nrow; t += 256) {
-                const int j = jbeg - 1 + t / nrow, i = t - (t / nrow) * nrow;
-                const int jsrc = a.mthbc[3] == 1 ? jbeg - 2 : 2 * jbeg - 1 - (j + 1) - 1;
-                for (int m = 0; m < nv; m++) {
-                    double v = dst.load(m, i, jsrc);
-                    if (a.mthbc[3] == 3 && m == 2) v = -v;
-                    dst.store(m, i, j, v);
-                }
-            }
+            const bool wall = a.mthbc[3] == 3;
+            bc_side<NT>(dst, tid, nv, nrow, ncol - jbeg + 1, 0, jbeg - 1, wall ? 2 : -1,
+                        [=](int&, int& j) { j = wall ? 2 * jbeg - 3 - j : jbeg - 2; });
         }
     }
 }
 
-hipError_t launch_fill_stage(int esize, const FillArgs& a, hipStream_t st) {
-    if (a.nops <= 0) return hipSuccess;
-    if (esize == 8)
-        hipLaunchKernelGGL(fill_stage_kernel<double>, dim3(a.nops), dim3(256), 0, st, a);
+// One workgroup per unit.  The unit's items are read into LDS FILL_CHUNK at a
+// time.  Items of one stage do not wait for each other: each starts with the
+// wave after the one that the item before it ended with, so that several small
+// ones (a coarse patch out of four grids) run on different waves.
+//
+// Bound by latency, a unit's chain of dependent loads.  A level step of 28
+// periodic advection grids took 4 launches of 3.6 us and now one of 7.9 us for
+// the ghost fill and the finer level's saveqc together, a Euler one of 39 grids
+// 17.6 -> 10.8 us, the three of a coarse step of 2,048 grids 271 -> 215 us.
+template <typename S, int NT>
+__global__ __launch_bounds__(NT) void fill_kernel(FillArgs a) {
+    __shared__ int32_t sh[FILL_CHUNK * FILL_WORDS];
+    const int tid = threadIdx.x;
+    if (a.clear && blockIdx.x == 0)
+        for (int64_t t = tid; t < a.nclear; t += NT) a.clear[t] = 0ull;
+    const int first = a.prog[0].nunits;
+    const bool second = (int)blockIdx.x >= first;
+    const FillProg& pr = a.prog[second ? 1 : 0];
+    const FillUnit un = pr.units[blockIdx.x - (second ? first : 0)];
+    int rot = 0;
+    for (int k0 = 0; k0 < un.n; k0 += FILL_CHUNK) {
+        const int nk = un.n - k0 < FILL_CHUNK ? un.n - k0 : FILL_CHUNK;
+        const int32_t* src = reinterpret_cast<const int32_t*>(pr.items + un.item0 + k0);
+        if (k0 > 0) __syncthreads();
+        for (int w = tid; w < nk * FILL_WORDS; w += NT) sh[w] = src[w];
+        __syncthreads();
+        for (int k = 0; k < nk; k++) {
+            const FillItem op = uniform_item(sh + k * FILL_WORDS);
+            if (op.sync) __syncthreads();
+            const int t = (tid - rot) & (NT - 1);
+            if (a.aux_mode) fill_aux_op<NT>(a, pr, op, t);
+            else fill_op<S, NT>(a, pr, op, t);
+            const int n = op.type == FOP_COPY ? op.ni * op.nj * a.nv : op.ni * op.nj;
+            rot = (rot + ((n + 63) & ~63)) & (NT - 1);
+        }
+    }
+}
+
+hipError_t launch_fill(int esize, const FillArgs& a, hipStream_t st) {
+    const int n = a.prog[0].nunits + a.prog[1].nunits;
+    if (n <= 0) return hipSuccess;
+    // many units: two waves each, so that more of them are resident (level 2 of
+    // 2,048 grids, 11,845 units: 92 us at four waves, 82 at two, 108 at one);
+    // few: the longest one decides (24 grids, 111 units: 21.6, 28.6, 39.8 us)
+    const bool narrow = n >= 4096;
+    if (esize == 8 && narrow)
+        hipLaunchKernelGGL((fill_kernel<double, 128>), dim3(n), dim3(128), 0, st, a);
+    else if (esize == 8)
+        hipLaunchKernelGGL((fill_kernel<double, 256>), dim3(n), dim3(256), 0, st, a);
+    else if (narrow)
+        hipLaunchKernelGGL((fill_kernel<float, 128>), dim3(n), dim3(128), 0, st, a);
     else
-        hipLaunchKernelGGL(fill_stage_kernel<float>, dim3(a.nops), dim3(256), 0, st, a);
+        hipLaunchKernelGGL((fill_kernel<float, 256>), dim3(n), dim3(256), 0, st, a);
     return hipGetLastError();
 }
 

@@ -5,9 +5,11 @@
 // periodic split, on the index boxes of the hierarchy once per regrid.  It
 // emits a list of operations on "buffers" (the level's patches and FP64
 // scratch arrays for the coarse patches valcrse and periodic pieces
-// valPatch), each tagged with a dependency stage.  At every level step one
-// launch per stage executes all operations of that stage, one workgroup per
-// operation.  Values are computed in FP64 in the reference's order.
+// valPatch), each tagged with a dependency stage.  Operations that depend on
+// each other (a coarse patch, its boundary conditions and the interpolation
+// out of it) form a unit; at every level step one launch executes all units,
+// one workgroup per unit with a barrier between its stages.  Values are
+// computed in FP64 in the reference's order.
 #pragma once
 #include <cstdint>
 #include "types.hpp"
@@ -66,16 +68,42 @@ struct FillOp {
     int32_t pad;
 };
 
+// An operation as the device reads it (32 words): the buffers resolved to an
+// address space, an offset, and the shift of the rectangle's first cell.
+constexpr int32_t FSP_SCRATCH = -1, FSP_ARENA = -2;   // spaces; >= 0: that level's storage
+struct FillItem {
+    int32_t type, flags;
+    int32_t sync;             // a barrier before it: a stage of the unit ends
+    int32_t dst_space, src_space;
+    int32_t dst_nrow, dst_plane, src_nrow, src_plane;
+    int32_t dst_shift, src_shift;
+    int32_t ni, nj;
+    int32_t mask_off;
+    int64_t dst_off, src_off;
+    int64_t aux_off;          // RING: the grid's auxc1d in the register arena (dst_off: qc1d)
+    int32_t ilo, jlo, iplo, jplo, ratx, raty;
+    int32_t level;            // INTERP, FILVAL: fine level; RING: level of the register arena
+    int32_t pad;
+    int32_t bc[4];
+};
+// the items [item0, item0 + n) one workgroup executes
+struct FillUnit { int32_t item0, n; };
+
 enum TimeMode : int32_t { TIME_NEW = 0, TIME_OLD = 1, TIME_BLEND = 2 };
 
-struct FillArgs {
-    const FillOp* ops;
-    const FillBuf* bufs;
+// a program on the device
+struct FillProg {
+    const FillItem* items;
+    const FillUnit* units;
     double* scratch;
     const unsigned char* masks;
+    int32_t nunits, pad;
+};
+
+struct FillArgs {
+    FillProg prog[2];                    // run side by side: neither reads what the other writes
     void* lvl_new[FILL_MAXLV];           // level storage, new time (store1)
     void* lvl_old[FILL_MAXLV];           // old time (store2)
-    const PatchDesc* lvl_patches[FILL_MAXLV];
     double* lvl_reg[FILL_MAXLV];          // register arenas (FOP_RING)
     double alphai[FILL_MAXLV], alphac[FILL_MAXLV];
     int32_t tmode[FILL_MAXLV];
@@ -83,7 +111,7 @@ struct FillArgs {
     double xlower, ylower;
     int32_t mthbc[4];
     int32_t nv;
-    int32_t nops;
+    int32_t pad1;
     double* arena;                        // kind-2 buffers
     int32_t big_old;                      // FOPF_BIG copies read store2
     int32_t pad;
@@ -93,9 +121,8 @@ struct FillArgs {
     int64_t nclear;
     // aux mode (a saveqc program run a second time for the aux values,
     // saveqc.f:60-90 and cstore.f): copies read the levels' aux arrays
-    // (FP64, naux components, patch p at off * auxk), scratch buffer b's
-    // component c starts at scratch + bufs[b].off * auxk + c * plane, rings
-    // write auxc1d; boundary conditions leave aux alone
+    // (FP64, naux components): both sides' buffers start at auxk times their
+    // offset, rings write auxc1d; boundary conditions leave aux alone
     const double* lvl_aux[FILL_MAXLV];
     int32_t aux_mode, naux, auxk, pad2;
 };

@@ -433,6 +433,45 @@ struct Planner {
         }
     }
 
+    // cstore reads the outermost cells of the coarse patch only, and its
+    // boundary conditions cells near their side: of the copies
+    // [copies0, nops0) into it keep the cells within that depth of an edge
+    void keep_rim(size_t copies0, size_t nops0, int nrow, int ncol) {
+        int d = 1;
+        if (P.ops.size() > nops0) {
+            const FillOp& bc = P.ops.back();
+            const int width[4] = {bc.bc[0], bc.bc[1] ? nrow - bc.bc[1] + 1 : 0, bc.bc[2],
+                                  bc.bc[3] ? ncol - bc.bc[3] + 1 : 0};
+            for (int s = 0; s < 4; s++)   // mirrored: as deep again; extrapolated: one cell
+                d = std::max(d, H.mthbc[s] == 3 ? 2 * width[s] : width[s] + 1);
+        }
+        if (2 * d >= nrow || 2 * d >= ncol) return;
+        const std::vector<FillOp> all(P.ops.begin() + copies0, P.ops.end());
+        P.ops.resize(copies0);
+        for (size_t k = 0; k < all.size(); k++) {
+            const FillOp& op = all[k];
+            if (copies0 + k >= nops0) {
+                push(op);
+                continue;
+            }
+            const int rim[4][4] = {{0, nrow, 0, d}, {0, nrow, ncol - d, ncol},
+                                   {0, d, d, ncol - d}, {nrow - d, nrow, d, ncol - d}};
+            for (const auto& r : rim) {
+                const int i0 = std::max(op.di0, r[0]), i1 = std::min(op.di0 + op.ni, r[1]);
+                const int j0 = std::max(op.dj0, r[2]), j1 = std::min(op.dj0 + op.nj, r[3]);
+                if (i0 >= i1 || j0 >= j1) continue;
+                FillOp part = op;
+                part.si0 += i0 - op.di0;
+                part.sj0 += j0 - op.dj0;
+                part.di0 = i0;
+                part.dj0 = j0;
+                part.ni = i1 - i0;
+                part.nj = j1 - j0;
+                push(part);
+            }
+        }
+    }
+
     // saveqc.f:13-109 for grid k of fine level `level`: coarsened patch
     // grown by one coarse cell, copied from the coarse grids (preicall.f for
     // periodic domains), bc2amr, then cstore's ring into the register
@@ -446,6 +485,7 @@ struct Planner {
         const int ichi = (b[1] + 1) / rx, jchi = (b[3] + 1) / ry;
         const int nrow = ichi - iclo + 1, ncol = jchi - jclo + 1;
         const int S = scratch(nrow, ncol);
+        const size_t copies0 = P.ops.size();
         std::vector<unsigned char> covered((size_t)nrow * ncol, 0);
         bool sticks = iclo < 0 || ichi == C.iregsz || jclo < 0 || jchi == C.jregsz;
         if (sticks && (H.xperdom || H.yperdom || H.spheredom)) {
@@ -508,6 +548,7 @@ struct Planner {
         for (int j = 0; j < ncol; j++)
             for (int i = 0; i < nrow; i++)
                 if (!set[(size_t)j * nrow + i]) return fail("saveqc: fine grid not properly nested in the coarse level");
+        keep_rim(copies0, nops0, nrow, ncol);
         FillOp ring{};
         ring.type = FOP_RING;
         ring.dst = S;
@@ -675,13 +716,128 @@ struct Planner {
 
 }  // namespace
 
+// whether `late`, of a later stage, touches a cell of the buffer that `early`
+// wrote: interpolation leaves out the cells its mask marks
+static bool meets(const FillPlan& P, const FillOp& early, const FillOp& late) {
+    const int i0 = std::max(early.di0, late.di0), i1 = std::min(early.di0 + early.ni, late.di0 + late.ni);
+    const int j0 = std::max(early.dj0, late.dj0), j1 = std::min(early.dj0 + early.nj, late.dj0 + late.nj);
+    if (i0 >= i1 || j0 >= j1) return false;
+    if (late.type != FOP_INTERP) return true;
+    const unsigned char* m = P.masks.data() + late.mask_off;
+    for (int j = j0; j < j1; j++)
+        for (int i = i0; i < i1; i++)
+            if (!m[(size_t)(j - late.dj0) * late.ni + (i - late.di0)]) return true;
+    return false;
+}
+
+// Order the operations into units: those that must run one after the other
+// end up in the same unit, sorted by stage.  A scratch or arena buffer ties
+// all its operations together; so does a grid whose boundary conditions (or
+// another operation) read it, as these read what the others wrote.  In other
+// grids the ghost strips are written by operations that meet no cell of each
+// other, and a same-level copy reads interiors, which a fill does not write.
 static void finish_plan(FillPlan& P) {
     std::stable_sort(P.ops.begin(), P.ops.end(),
                      [](const FillOp& a, const FillOp& b) { return a.stage < b.stage; });
-    P.nstages = P.ops.empty() ? 0 : P.ops.back().stage + 1;
-    P.stage_start.assign(P.nstages + 1, 0);
-    for (const auto& op : P.ops) P.stage_start[op.stage + 1]++;
-    for (int s = 0; s < P.nstages; s++) P.stage_start[s + 1] += P.stage_start[s];
+    const int n = (int)P.ops.size();
+    std::vector<int> up(n);
+    for (int k = 0; k < n; k++) up[k] = k;
+    auto root = [&](int k) {
+        while (up[k] != k) k = up[k] = up[up[k]];
+        return k;
+    };
+    auto tie = [&](int a, int b) {
+        a = root(a);
+        b = root(b);
+        up[std::max(a, b)] = std::min(a, b);
+    };
+    std::vector<std::vector<int>> uses(P.bufs.size());
+    std::vector<char> read(P.bufs.size(), 0);
+    for (int k = 0; k < n; k++) {
+        const FillOp& op = P.ops[k];
+        uses[op.dst].push_back(k);
+        if (op.type == FOP_BC || op.type == FOP_FILVAL) read[op.dst] = 1;
+        if (op.type != FOP_COPY && op.type != FOP_BC) {
+            if (op.src != op.dst) uses[op.src].push_back(k);
+            read[op.src] = 1;
+        }
+    }
+    for (size_t b = 0; b < P.bufs.size(); b++) {
+        const std::vector<int>& u = uses[b];
+        if (P.bufs[b].kind != 0 || read[b]) {
+            for (size_t k = 1; k < u.size(); k++) tie(u[0], u[k]);
+            continue;
+        }
+        for (size_t x = 0; x < u.size(); x++)
+            for (size_t y = 0; y < u.size(); y++)
+                if (P.ops[u[x]].stage < P.ops[u[y]].stage && meets(P, P.ops[u[x]], P.ops[u[y]]))
+                    tie(u[x], u[y]);
+    }
+    // large units first: the last ones to start should be short
+    std::vector<int64_t> cost(n, 0);
+    for (int k = 0; k < n; k++) cost[root(k)] += 256 + (int64_t)P.ops[k].ni * P.ops[k].nj;
+    P.order.resize(n);
+    for (int k = 0; k < n; k++) P.order[k] = k;
+    std::stable_sort(P.order.begin(), P.order.end(), [&](int a, int b) {
+        const int ra = root(a), rb = root(b);
+        return ra != rb && cost[ra] != cost[rb] ? cost[ra] > cost[rb] : ra < rb;
+    });
+    P.units.clear();
+    for (int k = 0; k < n; k++) {
+        if (k == 0 || root(P.order[k]) != root(P.order[k - 1])) P.units.push_back(FillUnit{k, 0});
+        P.units.back().n++;
+    }
+}
+
+std::vector<FillItem> fill_items(const FillPlan& P, int nvar,
+                                 const std::function<const std::vector<PatchDesc>&(int)>& patches) {
+    std::vector<FillItem> items;
+    items.reserve(P.ops.size());
+    auto place = [&](int b, int32_t& space, int64_t& off, int32_t& nrow, int32_t& plane) {
+        const FillBuf& fb = P.bufs[b];
+        space = fb.kind == 0 ? fb.level : (fb.kind == 1 ? FSP_SCRATCH : FSP_ARENA);
+        off = fb.kind == 0 ? patches(fb.level)[fb.patch].off : fb.off;
+        nrow = fb.nrow;
+        plane = fb.plane;
+    };
+    for (const FillUnit& un : P.units)
+        for (int k = un.item0; k < un.item0 + un.n; k++) {
+            const FillOp& op = P.ops[P.order[k]];
+            FillItem it{};
+            it.type = op.type;
+            it.flags = op.flags;
+            it.sync = k > un.item0 && op.stage != P.ops[P.order[k - 1]].stage;
+            it.ni = op.ni;
+            it.nj = op.nj;
+            it.mask_off = op.mask_off;
+            it.ilo = op.ilo;
+            it.jlo = op.jlo;
+            it.iplo = op.iplo;
+            it.jplo = op.jplo;
+            it.ratx = op.ratx;
+            it.raty = op.raty;
+            it.level = op.level;
+            for (int c = 0; c < 4; c++) it.bc[c] = op.bc[c];
+            place(op.dst, it.dst_space, it.dst_off, it.dst_nrow, it.dst_plane);
+            it.dst_shift = op.dj0 * it.dst_nrow + op.di0;
+            if (op.type == FOP_COPY) {
+                const PatchDesc& sp = patches(op.src_level)[op.src];
+                it.src_space = op.src_level;
+                it.src_off = sp.off;
+                it.src_nrow = sp.mitot;
+                it.src_plane = sp.plane;
+                it.src_shift = op.sj0 * sp.mitot + op.si0;
+            } else if (op.type != FOP_BC) {
+                place(op.src, it.src_space, it.src_off, it.src_nrow, it.src_plane);
+            }
+            if (op.type == FOP_RING) {
+                const PatchDesc& pf = patches(op.level)[op.si0];
+                it.dst_off = pf.reg_off + (int64_t)nvar * pf.lenbc;
+                it.aux_off = aux_ring_offset(pf, nvar);
+            }
+            items.push_back(it);
+        }
+    return items;
 }
 
 bool plan_filval(const HierGeom& H, int level, int nvar, FillPlan& P, std::string& err) {

@@ -2,6 +2,7 @@
 #pragma once
 #include <array>
 #include <cstdint>
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -50,11 +51,16 @@ struct FillPlan {
     std::vector<FillBuf> bufs;
     std::vector<FillOp> ops;                 // sorted by stage
     std::vector<unsigned char> masks;
-    std::vector<int> stage_start;            // ops of stage s: [stage_start[s], stage_start[s+1])
-    int nstages = 0;
+    std::vector<int> order;                  // the operations unit by unit, each by stage
+    std::vector<FillUnit> units;             // what one workgroup executes, in that order
     int64_t scratch_elems = 0;
     uint32_t src_levels_mask = 0;            // levels read as time sources
 };
+
+// the operations as the device reads them; patches(level): the descriptors of
+// the grids of that level (or slot)
+std::vector<FillItem> fill_items(const FillPlan& P, int nvar,
+                                 const std::function<const std::vector<PatchDesc>&(int)>& patches);
 
 bool plan_fill_level(const HierGeom& H, int level, int nvar, FillPlan& P, std::string& err);
 

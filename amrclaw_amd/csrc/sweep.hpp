@@ -64,20 +64,6 @@ struct SweepArgs {
     int32_t naux, auxk, mcapa, pad2;
 };
 
-// Perimeter flux block of a fine grid (FP64, after svdflx and qc1d):
-// side 0 left fm at x-edge 1 (rows 1..my), side 1 top gp at y-edge my+1
-// (columns 1..mx), side 2 right fp at x-edge mx+1, side 3 bottom gm at
-// y-edge 1; component fastest.  These are the fluxes fluxad.f:36-92 adds.
-__host__ __device__ inline int64_t perim_offset(const PatchDesc& pd, int nv) {
-    return pd.reg_off + 2 * (int64_t)nv * pd.lenbc;
-}
-// auxc1d(naux, lenbc) of a fine grid when its level has aux arrays: the
-// coarse ring's aux values cstore.f saves, after the perimeter block
-__host__ __device__ inline int64_t aux_ring_offset(const PatchDesc& pd, int nv) {
-    return perim_offset(pd, nv) + 2 * (int64_t)nv * (pd.mx + pd.my);
-}
-
-
 // limiter function of inlinelimiter.f:58-94
 template <class Mth, typename T>
 __device__ __forceinline__ T phi_limiter(int mth, T r) {

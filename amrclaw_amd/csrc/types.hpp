@@ -25,6 +25,19 @@ struct PatchDesc {
     int32_t pad;
 };
 
+// Perimeter flux block of a fine grid (FP64, after svdflx and qc1d):
+// side 0 left fm at x-edge 1 (rows 1..my), side 1 top gp at y-edge my+1
+// (columns 1..mx), side 2 right fp at x-edge mx+1, side 3 bottom gm at
+// y-edge 1; component fastest.  These are the fluxes fluxad.f:36-92 adds.
+constexpr int64_t perim_offset(const PatchDesc& pd, int nv) {
+    return pd.reg_off + 2 * (int64_t)nv * pd.lenbc;
+}
+// auxc1d(naux, lenbc) of a fine grid when its level has aux arrays: the
+// coarse ring's aux values cstore.f saves, after the perimeter block
+constexpr int64_t aux_ring_offset(const PatchDesc& pd, int nv) {
+    return perim_offset(pd, nv) + 2 * (int64_t)nv * (pd.mx + pd.my);
+}
+
 // fluxsv.f entry of a coarse grid: its interior cell (I, J) (1-based),
 // side 1..4 of that cell, fine grid `kid` of the next level and the slot
 // `lkid` (1-based) of the kid's register (setuse.f:61-213)

@@ -6,7 +6,7 @@ import pytest
 
 from amrclaw_amd import capi
 from oracle import orc
-from tests.common import random_hierarchy
+from tests.common import Hier, random_hierarchy
 
 pytestmark = pytest.mark.gpu
 
@@ -69,4 +69,39 @@ def test_bound_level_rejects_unavailable_time(gpu):
     capi.load_hierarchy(H)
     with pytest.raises(capi.AmrgpuError, match="not available"):
         capi.bound_level(H.nlev, 5.0)
+    capi.finalize()
+
+
+@pytest.mark.parametrize("nvar,cells,step,bc", [(3, 6, 8, (1, 3, 3, 1)), (1, 4, 6, (2, 2, 1, 1)),
+                                                (3, 46, 50, (3, 1, 1, 3))])
+def test_bound_level_many_units(gpu, nvar, cells, step, bc):
+    """A level of many little grids (thousands of units, two-wave workgroups),
+    grids apart from each other or side by side on a periodic domain (units of
+    more items than are read at a time), and larger ones that touch the
+    boundary: as the oracle's bound."""
+    rng = np.random.default_rng(cells)
+    n = 192
+    xper = bc[0] == 2
+    H = Hier(nvar, mthbc=bc, xper=xper, yper=False)
+    cut = np.linspace(0, n, 7).astype(int)
+    H.add_level([(cut[a], cut[a + 1] - 1, cut[b], cut[b + 1] - 1) for b in range(6) for a in range(6)],
+                1.0 / n, 1.0 / n, 0.08, 1.0, n, n, 2, 2)
+    H.add_level([(i, i + cells - 1, j, j + cells - 1) for j in range(0, 2 * n - cells + 1, step)
+                 for i in range((j // step % 2) * 2, 2 * n - cells + 1, step)],
+                0.5 / n, 0.5 / n, 0.04, 0.96, 2 * n, 2 * n, 2, 2)
+    for L in H.levels:
+        L["qnew"][:] = rng.normal(size=L["qnew"].shape)
+        L["qold"][:] = rng.normal(size=L["qold"].shape)
+    solver = orc.ACOUSTICS if nvar == 3 else orc.ADVECTION
+    p = orc.make_params(solver)
+    capi.init(capi.make_config(solver, mthbc=bc))
+    capi.load_hierarchy(H)
+    for l in (1, 2):
+        t = H.levels[l - 1]["time"]
+        print("bound many", nvar, cells, l, len(H.levels[l - 1]["boxes"]), flush=True)
+        Ho = H.copy()
+        for k in range(len(H.levels[l - 1]["boxes"])):
+            orc.bound(p, Ho, l, k, t)
+        capi.bound_level(l, t)
+        assert np.array_equal(capi.read_level(H, l), Ho.levels[l - 1]["qnew"]), l
     capi.finalize()
