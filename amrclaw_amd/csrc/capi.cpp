@@ -100,9 +100,8 @@ struct Level {
     UpbndEntry* d_uents = nullptr;
     int nucells = 0;
     AvgBlock* d_avg = nullptr;
-    int64_t* d_avg_start = nullptr;
-    int navg = 0;
-    int64_t navg_cells = 0;
+    AvgTile* d_avg_tiles = nullptr;
+    int navg_tiles = 0;
     // saveqc program filling this level's qc1d from the next coarser level
     FillPlan sq;
     FillDev dsq;
@@ -305,7 +304,7 @@ void free_plan(Level& L) {
 
 void free_regs(Level& L) {
     quiesce();
-    void* ps[] = {L.d_reg, L.d_sv, L.d_qad, L.d_ucells, L.d_uents, L.d_avg, L.d_avg_start,
+    void* ps[] = {L.d_reg, L.d_sv, L.d_qad, L.d_ucells, L.d_uents, L.d_avg, L.d_avg_tiles,
                   L.d_sq_aux};
     L.dsq.free();
     for (void* p : ps)
@@ -317,9 +316,8 @@ void free_regs(Level& L) {
     L.d_ucells = nullptr;
     L.d_uents = nullptr;
     L.d_avg = nullptr;
-    L.d_avg_start = nullptr;
-    L.nqad = L.nucells = L.navg = 0;
-    L.navg_cells = 0;
+    L.d_avg_tiles = nullptr;
+    L.nqad = L.nucells = L.navg_tiles = 0;
     L.sq = FillPlan();
     for (auto& t : L.tiles) t.reg_lo = t.reg_hi = 0;
     for (auto& p : L.patches) p.reg_off = 0, p.lenbc = 0;
@@ -984,9 +982,8 @@ int ensure_regs() {
             if ((rc = upload(&L.d_uents, Rl.uents))) return rc;
             L.nucells = (int)Rl.ucells.size();
             if ((rc = upload(&L.d_avg, Rl.avg))) return rc;
-            if ((rc = upload(&L.d_avg_start, Rl.avg_start))) return rc;
-            L.navg = (int)Rl.avg.size();
-            L.navg_cells = Rl.avg_start.empty() ? 0 : Rl.avg_start.back();
+            if ((rc = upload(&L.d_avg_tiles, Rl.avg_tiles))) return rc;
+            L.navg_tiles = (int)Rl.avg_tiles.size();
         }
         HIPCHK(h2d(L.d_patches, L.patches.data(), L.ngrids * sizeof(PatchDesc)));
         HIPCHK(h2d(L.d_tiles, L.tiles.data(), L.tiles.size() * sizeof(TileDesc)));
@@ -1332,7 +1329,8 @@ int update_level(int level) {
     a.nv = g.cfg.nvar;
     a.entries = C.d_uents;
     a.blocks = C.d_avg;
-    a.nblocks = C.navg;
+    a.tiles = C.d_avg_tiles;
+    a.ntiles = C.navg_tiles;
     a.ratx = g.ratx[level];
     a.raty = g.raty[level];
     a.patches = C.d_patches;
@@ -1348,7 +1346,7 @@ int update_level(int level) {
         a.auxk = g.auxk;
     }
     tbegin(AMRGPU_KT_UPDATE);
-    hipError_t e = launch_update((int)g.esize, a, C.d_avg_start, C.navg_cells, g.stream);
+    hipError_t e = launch_update((int)g.esize, a, g.stream);
     tend(AMRGPU_KT_UPDATE);
     if (e != hipSuccess) return fail(AMRGPU_ERR_HIP, "update: %s", hipGetErrorString(e));
     return AMRGPU_OK;

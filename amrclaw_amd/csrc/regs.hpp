@@ -25,6 +25,12 @@ struct AvgBlock {
     int32_t fi0, fj0;
 };
 
+// 256 coarse cells of a block, from its cell c0 on (row by row), averaged by
+// one workgroup
+struct AvgTile {
+    int32_t block, c0;
+};
+
 // qad.f: one coarse segment (register slot) of one side of a fine grid
 struct QadItem {
     int32_t grid;
@@ -61,7 +67,8 @@ struct UpdateArgs {
     int32_t nv;
     const UpbndEntry* entries;
     const AvgBlock* blocks;
-    int32_t nblocks;
+    const AvgTile* tiles;
+    int32_t ntiles;
     int32_t ratx, raty;
     const PatchDesc* patches;       // coarse level
     const PatchDesc* fine_patches;  // fine level

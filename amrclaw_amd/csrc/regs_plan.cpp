@@ -137,9 +137,40 @@ bool plan_registers(const HierGeom& H, int nvar, RegLevel* R, std::string& err) 
             if (it != last.end()) Rl.sv_write[it->second] = 0;
             last[key] = e;
         }
+        // averaging blocks
+        for (size_t m = 0; m < C.boxes.size(); m++) {
+            const auto& cb = C.boxes[m];
+            for (size_t kid = 0; kid < F.boxes.size(); kid++) {
+                const auto& fb = F.boxes[kid];
+                int iclo = fb[0] / rx, jclo = fb[2] / ry, ichi = fb[1] / rx, jchi = fb[3] / ry;
+                int iplo = std::max(cb[0], iclo), jplo = std::max(cb[2], jclo);
+                int iphi = std::min(cb[1], ichi), jphi = std::min(cb[3], jchi);
+                if (iplo > iphi || jplo > jphi) continue;
+                AvgBlock a;
+                a.grid = (int)m;
+                a.kid = (int)kid;
+                a.ci0 = iplo - cb[0] + NGHOST;
+                a.cj0 = jplo - cb[2] + NGHOST;
+                a.ni = iphi - iplo + 1;
+                a.nj = jphi - jplo + 1;
+                a.fi0 = iplo * rx - fb[0] + NGHOST;
+                a.fj0 = jplo * ry - fb[2] + NGHOST;
+                Rl.avg.push_back(a);
+                for (int64_t c = 0; c < (int64_t)a.ni * a.nj; c += 256)
+                    Rl.avg_tiles.push_back(AvgTile{(int32_t)Rl.avg.size() - 1, (int32_t)c});
+            }
+        }
         // upbnd programs: per coarse cell, its entries in list order
+        size_t blk = 0;   // the blocks stand in the order of their coarse grids
         for (size_t m = 0; m < C.boxes.size(); m++) {
             const int mitot = C.boxes[m][1] - C.boxes[m][0] + 1 + 2 * NGHOST;
+            const int mjtot = C.boxes[m][3] - C.boxes[m][2] + 1 + 2 * NGHOST;
+            std::vector<char> covered((size_t)mitot * mjtot, 0);
+            for (; blk < Rl.avg.size() && Rl.avg[blk].grid == (int)m; blk++) {
+                const AvgBlock& a = Rl.avg[blk];
+                for (int j = a.cj0; j < a.cj0 + a.nj; j++)
+                    std::fill_n(covered.begin() + (size_t)j * mitot + a.ci0, a.ni, 1);
+            }
             std::map<int, std::vector<UpbndEntry>> cells;   // key: cell index
             std::map<int, int> iused;
             std::vector<int> order;
@@ -160,33 +191,11 @@ bool plan_registers(const HierGeom& H, int nvar, RegLevel* R, std::string& err) 
                 c.grid = (int)m;
                 c.i = key % mitot;
                 c.j = key / mitot;
+                if (covered[key]) continue;
                 c.e0 = (int32_t)Rl.uents.size();
                 for (const auto& en : cells[key]) Rl.uents.push_back(en);
                 c.e1 = (int32_t)Rl.uents.size();
                 Rl.ucells.push_back(c);
-            }
-        }
-        // averaging blocks
-        Rl.avg_start.push_back(0);
-        for (size_t m = 0; m < C.boxes.size(); m++) {
-            const auto& cb = C.boxes[m];
-            for (size_t kid = 0; kid < F.boxes.size(); kid++) {
-                const auto& fb = F.boxes[kid];
-                int iclo = fb[0] / rx, jclo = fb[2] / ry, ichi = fb[1] / rx, jchi = fb[3] / ry;
-                int iplo = std::max(cb[0], iclo), jplo = std::max(cb[2], jclo);
-                int iphi = std::min(cb[1], ichi), jphi = std::min(cb[3], jchi);
-                if (iplo > iphi || jplo > jphi) continue;
-                AvgBlock a;
-                a.grid = (int)m;
-                a.kid = (int)kid;
-                a.ci0 = iplo - cb[0] + NGHOST;
-                a.cj0 = jplo - cb[2] + NGHOST;
-                a.ni = iphi - iplo + 1;
-                a.nj = jphi - jplo + 1;
-                a.fi0 = iplo * rx - fb[0] + NGHOST;
-                a.fj0 = jplo * ry - fb[2] + NGHOST;
-                Rl.avg.push_back(a);
-                Rl.avg_start.push_back(Rl.avg_start.back() + (int64_t)a.ni * a.nj);
             }
         }
     }

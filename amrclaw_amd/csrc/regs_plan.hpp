@@ -19,10 +19,10 @@ struct RegLevel {
     std::vector<SvEntry> sv;
     std::vector<int32_t> sv_grid_start;   // ngrids + 1
     std::vector<unsigned char> sv_write;  // 1: this entry writes its slot in fluxsv
-    std::vector<UpbndCell> ucells;
+    std::vector<UpbndCell> ucells;        // but those a finer grid covers: averaging sets them
     std::vector<UpbndEntry> uents;
     std::vector<AvgBlock> avg;
-    std::vector<int64_t> avg_start;       // nblocks + 1 cell offsets
+    std::vector<AvgTile> avg_tiles;
     // fine side: qad work items
     std::vector<QadItem> qad;
 };

@@ -124,6 +124,33 @@ def test_level_update_launch_variants(gpu, mode, graphs):
         capi.finalize()
 
 
+@pytest.mark.parametrize("ratio,seed", [(3, 0), (4, 1), (5, 2)])
+def test_level_update_other_ratios_bit_exact(gpu, ratio, seed):
+    """Refinement by 3, 4 and 5: register slots of fewer, as many and more
+    fine faces than the lanes that share a slot; averages of r x r cells."""
+    solver, nvar, states, dt1 = PHYS["euler"]
+    bc, xper, yper = BCS[3]
+    rng = np.random.default_rng(40 + seed)
+    H = nested_hierarchy(rng, states, nvar, nlev=2, ratio=ratio, mthbc=bc, xper=xper, yper=yper,
+                         dt1=dt1, nfine=4)
+    p, cfg = both_params(solver, precision=capi.FP64)
+    for k in range(4):
+        cfg.mthbc[k] = bc[k]
+    O = orc.OracleAMR(p, H.copy())
+    capi.init(cfg)
+    try:
+        D = DeviceAMR(H)
+        lo, ld = [], []
+        for _ in range(2):
+            berger_oliger(O, 1, H.nlev, ratio, lo)
+            berger_oliger(D, 1, H.nlev, ratio, ld)
+        assert lo == ld
+        for l in (1, 2):
+            assert np.array_equal(capi.read_level(H, l, 0), O.H.levels[l - 1]["qnew"]), l
+    finally:
+        capi.finalize()
+
+
 @pytest.mark.parametrize("precision", [capi.FP32, capi.MIXED])
 @pytest.mark.parametrize("phys", ["acoustics", "euler"])
 @pytest.mark.parametrize("case", BCS[:3])
