@@ -25,6 +25,7 @@
 #include "xfer.hpp"
 
 namespace amrgpu {
+hipError_t launch_sv_map(int32_t* map, const MarchSvCell* c, int n, hipStream_t st);
 hipError_t launch_fill_u64(unsigned long long* p, unsigned long long v, int64_t n,
                            hipStream_t st);
 hipError_t launch_fill(int esize, const FillArgs& a, hipStream_t st);
@@ -94,6 +95,8 @@ struct Level {
     // programs of fluxsv / upbnd / averaging (coarse side) and qad (fine side)
     double* d_reg = nullptr;
     SvEntry* d_sv = nullptr;
+    int32_t* d_svmap = nullptr;    // the march sweep's fluxsv entries (null: no march here)
+    MarchSv* d_msv = nullptr;
     QadItem* d_qad = nullptr;
     int nqad = 0;
     UpbndCell* d_ucells = nullptr;
@@ -304,7 +307,7 @@ void free_plan(Level& L) {
 
 void free_regs(Level& L) {
     quiesce();
-    void* ps[] = {L.d_reg, L.d_sv, L.d_qad, L.d_ucells, L.d_uents, L.d_avg, L.d_avg_tiles,
+    void* ps[] = {L.d_reg, L.d_sv, L.d_svmap, L.d_msv, L.d_qad, L.d_ucells, L.d_uents, L.d_avg, L.d_avg_tiles,
                   L.d_sq_aux};
     L.dsq.free();
     for (void* p : ps)
@@ -312,6 +315,8 @@ void free_regs(Level& L) {
     L.d_sq_aux = nullptr;
     L.d_reg = nullptr;
     L.d_sv = nullptr;
+    L.d_svmap = nullptr;
+    L.d_msv = nullptr;
     L.d_qad = nullptr;
     L.d_ucells = nullptr;
     L.d_uents = nullptr;
@@ -888,6 +893,47 @@ int upload(T** dst, const std::vector<T>& v) {
     return AMRGPU_OK;
 }
 
+// The march sweep's fluxsv entries of a level: the map of its cells and the
+// entries of each marked cell one after the other.  No room for the map on the
+// card: none, and the tile sweep steps the level.
+int march_entries(Level& L, const RegLevel& fine, const RegLevel& R) {
+    const int nv = g.cfg.nvar;
+    std::vector<MarchSv> ents;
+    std::vector<MarchSvCell> cells;
+    for (int m = 0; m < L.ngrids; m++) {
+        const PatchDesc& pd = L.patches[m];
+        std::vector<std::pair<int64_t, int>> at;   // (cell, entry)
+        for (int e = R.sv_grid_start[m]; e < R.sv_grid_start[m + 1]; e++)
+            if (R.sv_write[e])
+                at.push_back({(int64_t)(R.sv[e].J + NGHOST - 1) * pd.mitot + R.sv[e].I + NGHOST - 1, e});
+        std::stable_sort(at.begin(), at.end(),
+                         [](const auto& a, const auto& b) { return a.first < b.first; });
+        for (size_t k = 0; k < at.size(); k++) {
+            const SvEntry& s = R.sv[at[k].second];
+            if (k == 0 || at[k].first != at[k - 1].first)
+                cells.push_back(MarchSvCell{pd.off / nv + at[k].first, (int32_t)ents.size(), 0});
+            ents.push_back(MarchSv{fine.reg_off[s.kid] + (int64_t)nv * (s.lkid - 1), s.side,
+                                   k + 1 < at.size() && at[k + 1].first == at[k].first});
+        }
+    }
+    const int64_t n = (L.nelem / nv + 2) / 2 * 2;
+    const hipError_t e = hipMalloc(&L.d_svmap, n * sizeof(int32_t));
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        L.d_svmap = nullptr;
+        return AMRGPU_OK;
+    }
+    MarchSvCell* d_cells = nullptr;
+    int rc = upload(&L.d_msv, ents);
+    if (!rc) rc = upload(&d_cells, cells);
+    if (rc) return rc;
+    HIPCHK(launch_fill_u64(reinterpret_cast<unsigned long long*>(L.d_svmap), 0ull, n / 2, g.stream));
+    HIPCHK(launch_sv_map(L.d_svmap, d_cells, (int)cells.size(), g.stream));
+    quiesce();
+    if (d_cells) hipFree(d_cells);
+    return AMRGPU_OK;
+}
+
 // Register layout and programs of the whole hierarchy (prepf.f / prepc.f
 // at every regrid).  Arenas start at zero, as prepf.f:44-48 leaves them.
 int ensure_regs() {
@@ -978,6 +1024,7 @@ int ensure_regs() {
                 L.tiles[t].reg_hi = (int32_t)flat.size();
             }
             if ((rc = upload(&L.d_sv, flat))) return rc;
+            if (!L.mwaves.empty() && (rc = march_entries(L, R[l + 1], Rl))) return rc;
             if ((rc = upload(&L.d_ucells, Rl.ucells))) return rc;
             if ((rc = upload(&L.d_uents, Rl.uents))) return rc;
             L.nucells = (int)Rl.ucells.size();
@@ -1033,11 +1080,14 @@ int launch_sweep(Level& L, double dt, double* flux_out_dev, const int64_t* flux_
     hipError_t e = hipSuccess;
     tbegin(AMRGPU_KT_SWEEP);
     if ((g.launch_mode == AMRGPU_LAUNCH_MARCH || g.launch_mode == AMRGPU_LAUNCH_BATCHED) &&
-        L.d_mwaves && !flux_out_dev && !rl.sv && !a.aux) {
-        // the march sweep writes no per-edge flux arrays and no fluxsv
-        // entries: a level with a finer level, or a call asking for the
-        // flux arrays, takes the tile sweep
+        L.d_mwaves && !flux_out_dev && (!rl.sv || L.d_svmap) && !a.aux) {
+        // the march sweep writes no per-edge flux arrays: a call asking for
+        // them takes the tile sweep
         SweepArgs x = a;
+        if (rl.sv) {
+            x.svmap = L.d_svmap;
+            x.msv = L.d_msv;
+        }
         x.waves = L.d_mwaves;
         x.nwaves = (int)L.mwaves.size();
         e = run_sweep(run_precision(), x, 0, g.march_wgs);

@@ -57,6 +57,9 @@ struct SweepArgs {
     // fields are then unused
     const MarchWave* waves;
     int32_t nwaves;
+    // its fluxsv entries when a finer level exists (else null; sv is then unused)
+    const int32_t* svmap;
+    const MarchSv* msv;
     // aux arrays of the level (FP64, naux components per cell; patch p's
     // component a of cell li at aux[patches[p].off * auxk + a * plane + li])
     // and the capacity component (1-based, 0: none, step2.f90:91-95)

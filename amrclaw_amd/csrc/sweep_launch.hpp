@@ -113,8 +113,11 @@ static hipError_t sweep_aux_go(const SweepArgs& a, size_t lds, hipStream_t st) {
 template <class Sol, typename T, typename S, int MWGS, bool STD = false>
 static hipError_t march_go(const SweepArgs& a, hipStream_t st) {
     if (a.nwaves == 0) return hipSuccess;
-    hipLaunchKernelGGL((sweep_march_kernel<Sol, T, S, MWGS, STD>), dim3((a.nwaves + 3) / 4),
-                       dim3(256), 0, st, a);
+    const dim3 grid((a.nwaves + 3) / 4);
+    if (a.svmap)
+        hipLaunchKernelGGL((sweep_march_kernel<Sol, T, S, MWGS, STD, true>), grid, dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL((sweep_march_kernel<Sol, T, S, MWGS, STD, false>), grid, dim3(256), 0, st, a);
     return hipGetLastError();
 }
 

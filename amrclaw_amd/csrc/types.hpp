@@ -45,6 +45,15 @@ struct SvEntry {
     int32_t I, J, side, kid, lkid, pad;
 };
 
+// The march sweep's form of the entries: those of one cell in a row (all but
+// the last with `more`), found through a map of the level's cells
+// (patch p's cell li at off / nv + li): 0, or the first entry's number + 1.
+struct MarchSv {
+    int64_t slot;       // element of the finer level's register arena
+    int32_t side, more;
+};
+struct MarchSvCell { int64_t cell; int32_t first, pad; };
+
 // One workgroup's piece of a patch for the sweep.  Interior cells
 // i0+1..i0+tx, j0+1..j0+ty of patch `patch`.  wx/wy: lanes per x-row /
 // y-column segment (16, 32 or 64, >= tx+3 / ty+3).

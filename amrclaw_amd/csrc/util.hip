@@ -1,6 +1,7 @@
 // util.hip -- small device helpers used by the host library.
 #include <hip/hip_runtime.h>
 #include <cstdint>
+#include "types.hpp"
 #include "xfer.hpp"
 
 namespace amrgpu {
@@ -17,6 +18,18 @@ hipError_t launch_fill_u64(unsigned long long* p, unsigned long long v, int64_t 
     if (n <= 0) return hipSuccess;
     int blocks = (int)((n + 255) / 256);
     hipLaunchKernelGGL(fill_u64_kernel, dim3(blocks), dim3(256), 0, st, p, v, n);
+    return hipGetLastError();
+}
+
+// map[cell] = first + 1 of every record (MarchSvCell), on a cleared map
+__global__ void sv_map_kernel(int32_t* map, const MarchSvCell* c, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) map[c[i].cell] = c[i].first + 1;
+}
+
+hipError_t launch_sv_map(int32_t* map, const MarchSvCell* c, int n, hipStream_t st) {
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(sv_map_kernel, dim3((n + 255) / 256), dim3(256), 0, st, map, c, n);
     return hipGetLastError();
 }
 

@@ -206,16 +206,15 @@ int amrgpu_flag_level(int level, int flag_gradient, double tolsp, int flag_richa
 
 /* Sweep launch shape: AMRGPU_LAUNCH_BATCHED (default) puts all tiles of
  * all grids of a level into one launch, one workgroup per tile (an FP64
- * Euler level without a finer level marches instead, as below, where that
- * is faster: the same bits);
+ * Euler level marches instead, as below, where that is faster: the same
+ * bits);
  * AMRGPU_LAUNCH_PERSISTENT launches as many workgroups as the device holds
  * and lets them take the level's tiles (largest first) from a device
  * counter; AMRGPU_LAUNCH_PER_PATCH issues one launch per grid, the plain
  * per-patch GPU path, kept as the comparison baseline;
- * AMRGPU_LAUNCH_MARCH runs the sweep of a level that has no finer level as
- * column strips marching up the rows with every quantity in registers (one
- * Riemann solve per interface instead of the tiles' halo re-solves; levels
- * with a finer level keep the tile sweep).  Results are identical (FP64) or
+ * AMRGPU_LAUNCH_MARCH runs the sweep of a level as column strips marching
+ * up the rows with every quantity in registers (one Riemann solve per
+ * interface instead of the tiles' halo re-solves).  Results are identical (FP64) or
  * agree to FP32 rounding.  No reference counterpart. */
 enum { AMRGPU_LAUNCH_BATCHED = 0, AMRGPU_LAUNCH_PER_PATCH = 1, AMRGPU_LAUNCH_PERSISTENT = 2,
        AMRGPU_LAUNCH_MARCH = 3 };

@@ -10,7 +10,7 @@ import pytest
 
 from amrclaw_amd import capi
 from oracle import orc
-from tests.common import (acoustic_states, berger_oliger, both_params, nested_hierarchy,
+from tests.common import (Hier, acoustic_states, berger_oliger, both_params, nested_hierarchy,
                           rel_l1, smooth_euler)
 
 pytestmark = pytest.mark.gpu
@@ -124,15 +124,25 @@ def test_level_update_launch_variants(gpu, mode, graphs):
         capi.finalize()
 
 
-@pytest.mark.parametrize("ratio,seed", [(3, 0), (4, 1), (5, 2)])
-def test_level_update_other_ratios_bit_exact(gpu, ratio, seed):
+@pytest.mark.parametrize("ratio", [3, 4, 5])
+def test_level_update_other_ratios_bit_exact(gpu, ratio):
     """Refinement by 3, 4 and 5: register slots of fewer, as many and more
     fine faces than the lanes that share a slot; averages of r x r cells."""
     solver, nvar, states, dt1 = PHYS["euler"]
     bc, xper, yper = BCS[3]
-    rng = np.random.default_rng(40 + seed)
-    H = nested_hierarchy(rng, states, nvar, nlev=2, ratio=ratio, mthbc=bc, xper=xper, yper=yper,
-                         dt1=dt1, nfine=4)
+    rng = np.random.default_rng(40 + ratio)
+    H = Hier(nvar, mthbc=bc, xper=xper, yper=yper)
+    H.add_level([(0, 12, 0, 19), (13, 23, 0, 19)], 1 / 24, 1 / 20, dt1, 0.0, 24, 20, ratio, ratio)
+    # side by side, across the coarse grids' edge, at the domain's edge
+    coarse = [(3, 8, 3, 7), (9, 15, 3, 9), (17, 22, 12, 19)]
+    H.add_level([(a * ratio, (b + 1) * ratio - 1, c * ratio, (d + 1) * ratio - 1)
+                 for a, b, c, d in coarse], 1 / 24 / ratio, 1 / 20 / ratio, dt1 / ratio, 0.0,
+                24 * ratio, 20 * ratio, ratio, ratio)
+    for l, L in enumerate(H.levels, start=1):
+        for k in range(len(L["boxes"])):
+            grid = H.grid(l, k, 0)
+            grid[:] = states(rng, grid.shape[:2])
+            H.grid(l, k, 1)[:] = grid
     p, cfg = both_params(solver, precision=capi.FP64)
     for k in range(4):
         cfg.mthbc[k] = bc[k]
@@ -146,6 +156,36 @@ def test_level_update_other_ratios_bit_exact(gpu, ratio, seed):
             berger_oliger(D, 1, H.nlev, ratio, ld)
         assert lo == ld
         for l in (1, 2):
+            assert np.array_equal(capi.read_level(H, l, 0), O.H.levels[l - 1]["qnew"]), l
+    finally:
+        capi.finalize()
+
+
+@pytest.mark.parametrize("phys", ["acoustics", "euler"])
+@pytest.mark.parametrize("split,case", [((1, 1), BCS[2]), ((2, 3), BCS[1])])
+def test_march_writes_fluxsv_bit_exact(gpu, phys, split, case):
+    """A coarse level that marches (grids of several column and row strips,
+    fine grids on strip edges and side by side) saves the fluxes its finer
+    level's registers need: the refluxed solution is the oracle's, FP64."""
+    solver, nvar, states, dt1 = PHYS[phys]
+    bc, xper, yper = case
+    rng = np.random.default_rng(17)
+    H = nested_hierarchy(rng, states, nvar, nx=150, ny=93, mthbc=bc, xper=xper, yper=yper,
+                         dt1=dt1 * 24 / 150, nfine=14, level1_split=split)
+    p, cfg = both_params(solver, precision=capi.FP64)
+    for k in range(4):
+        cfg.mthbc[k] = bc[k]
+    O = orc.OracleAMR(p, H.copy())
+    capi.init(cfg)
+    try:
+        capi.set_launch_mode(capi.LAUNCH_MARCH)
+        D = DeviceAMR(H)
+        lo, ld = [], []
+        for _ in range(2):
+            berger_oliger(O, 1, H.nlev, 2, lo)
+            berger_oliger(D, 1, H.nlev, 2, ld)
+        assert lo == ld
+        for l in range(1, H.nlev + 1):
             assert np.array_equal(capi.read_level(H, l, 0), O.H.levels[l - 1]["qnew"]), l
     finally:
         capi.finalize()
