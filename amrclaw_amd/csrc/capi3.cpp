@@ -248,21 +248,10 @@ void split_tile3(int n, int k, std::vector<std::pair<int, int>>& out) {
     }
 }
 
-// lane slots the fused kernel spends on a tile (its schedule: per sweep,
-// rows of lines in three classes, four waves of chunks of 64 / (tr + 1)
-// lines per round, 256 lanes per round)
+// lane slots the fused kernel spends on a tile: 256 a round of its schedule
 int64_t tile3_slots(int tx, int ty, int tz) {
-    const int t3[3][3] = {{tx, ty, tz}, {ty, tx, tz}, {tz, tx, ty}};
-    int64_t slots = 0;
-    for (const auto& t : t3) {
-        const int tr = t[0], tq = t[1], tp = t[2];
-        const int lpw = 64 / (tr + 1), K = (tq + 2 + lpw - 1) / lpw;
-        for (int c3 = 0; c3 < 3; c3++) {
-            const int nrows = (tp + 4 - c3) / 3, wpr = std::min(nrows, 4);
-            slots += (int64_t)((nrows * K + wpr - 1) / wpr) * 256;
-        }
-    }
-    return slots;
+    return 256ll * (tile3_rounds(tx, ty, tz).rounds + tile3_rounds(ty, tx, tz).rounds +
+                    tile3_rounds(tz, tx, ty).rounds);
 }
 size_t tile3_bytes(int nv, int tx, int ty, int tz) {
     return (size_t)nv * ((size_t)(tx + 4) * (ty + 4) * (tz + 4) + (size_t)tx * ty * tz) *

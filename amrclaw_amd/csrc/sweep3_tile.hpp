@@ -21,10 +21,10 @@
 //     (3-D):150-173 with fm = fp = F for the transverse increments of
 //     step3.f:221-250, 279-310), the normal fluxes as
 //     q(c) -= dt/h (faddm(c+1) - faddp(c));
-//   * the lines are scheduled so that no two waves of a round touch the same
-//     cell and the lanes of a wave add in ordered steps (tile3_sweep): no
-//     atomics, the sums are formed in a fixed order and the result is
-//     deterministic.
+//   * four waves solve at once, any lines, and add in two phases whose waves
+//     touch no cell of each other, the lanes of a wave in ordered steps
+//     (tile3_rounds, tile3_sweep): no atomics on dq, the sums are formed in a
+//     fixed order and the result is deterministic.
 // The per-interface arithmetic (rpn3, limiter, cqxx, the rpt3 / rptt3
 // splits and their 1/2, 1/6 weights, flux3.f:220-628) is that of the phase
 // kernel; only the order in which each cell's increments are summed differs
@@ -38,7 +38,10 @@
 // (Euler3::split_scaled), the method's switches at compile time, a cell's
 // values together in LDS and scalar row bookkeeping took the Euler sweeps from
 // 2300 to 1830 vector instructions an interface and 256 uneven grids
-// (2,023,768 cells) from 984 to 700 us a step.
+// (2,023,768 cells) from 984 to 700 us a step.  Full chunks from any rows, added
+// in two phases, instead of waves of one row each in three classes of rows: 700
+// -> 680 us, 6 grids 141 -> 134, the levels of a 64^3 run (tiles of 8 .. 11
+// cells) 11.7 -> 10.2 ms.
 #pragma once
 #include <cstdint>
 #include "lanes.hpp"
@@ -88,7 +91,7 @@ struct Tile3Args {
 
 // Marked faces in LDS: for every face of the tile its mark's number + 1 (0:
 // none), the x-faces first; per mark the transverse increments and faddm
-// times dt/h, then faddp - faddm.
+// times dt/h, a sum for the waves of either phase, then faddp - faddm.
 struct Mark3Lds {
     uint16_t* map;
     float* acc;
@@ -98,13 +101,31 @@ __host__ __device__ constexpr int mark3_faces(int tx, int ty, int tz) {
 }
 template <int NV>
 __host__ __device__ constexpr size_t mark3_lds_bytes(int tx, int ty, int tz, int nmark) {
-    return ((size_t)mark3_faces(tx, ty, tz) * 2 + 3) / 4 * 4 + (size_t)nmark * 2 * NV * sizeof(float);
+    return ((size_t)mark3_faces(tx, ty, tz) * 2 + 3) / 4 * 4 + (size_t)nmark * 3 * NV * sizeof(float);
 }
 
 // LDS of a tile workgroup: the staged box and the increments
 template <int NV>
 __host__ __device__ constexpr size_t tile3_lds_bytes(int bx, int by, int bz, int cells) {
     return ((size_t)NV * bx * by * bz + (size_t)NV * cells) * sizeof(float);
+}
+
+// The schedule of a sweep over the (tq + 2) (tp + 2) lines through a tile and
+// around it: chunks of 64 / (tr + 1) lines, dealt to the waves in blocks, one
+// chunk a wave and round.  A line's increments reach the cells within one line
+// of it, so two lines at least 2 n + 3 apart in the order (n: the length of the
+// fast axis) touch no cell of each other.  Four waves work in two phases,
+// waves 0 and 2 before 1 and 3, if that holds between the chunks of waves two
+// apart; else (tiles of 4 cells and less) two waves do.
+struct Tile3Rounds {
+    int rounds, waves;
+};
+__host__ __device__ inline Tile3Rounds tile3_rounds(int tr, int tq, int tp) {
+    const int lpw = 64 / (tr + 1), n = (tq < tp ? tq : tp) + 2;
+    const int chunks = ((tq + 2) * (tp + 2) + lpw - 1) / lpw;
+    const int four = (chunks + 3) / 4;
+    if ((2 * four - 1) * lpw + 1 >= 2 * n + 3) return {four, 4};
+    return {(chunks + 1) / 2, 2};
 }
 
 // Wave-synchronous ordering: the LDS accesses of one wave before this point
@@ -220,27 +241,31 @@ __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float
     const int lpw = 64 / L;                    // lines of a chunk
     const int li = wl / L;                     // this lane's line in the chunk
     const int e = wl - li * L;                 // interface e: between cells e-1, e
-    const int K = (tq + 2 + lpw - 1) / lpw;    // chunks per row
+    // the lines in order, the shorter of the two axes across them running
+    // fastest; wave w takes chunks w R .. w R + R - 1, one a round
+    const Tile3Rounds sch = tile3_rounds(tr, tq, tp);
+    const bool qfast = tq <= tp;
+    const int nfast = (qfast ? tq : tp) + 2, nlines = (tq + 2) * (tp + 2);
+    const int inv = 65536 / nfast + 1;         // line / nfast = line * inv >> 16 (line < 300)
+    const int phase = wave & 1;
 #pragma unroll 1
-    for (int c3 = 0; c3 < 3; c3++) {
-        const int nrows = (tp + 4 - c3) / 3;   // rows P = -1 + c3 + 3 i
-        const int wpr = nrows < 4 ? nrows : 4;
-        const int npairs = nrows * K;
-        const int nrounds = (npairs + wpr - 1) / wpr;
-        // pair = rd * wpr + wave as (row, chunk) = (pair % nrows, pair / nrows),
-        // stepped by wpr <= nrows a round (one carry)
-        int prow = wave < wpr ? wave : 0, pchunk = 0;
-#pragma unroll 1
-        for (int rd = 0; rd < nrounds; rd++) {
-            const int pair = rd * wpr + wave;
-            const bool wlive = wave < wpr && pair < npairs;
-            const int P = -1 + c3 + 3 * (wlive ? prow : 0);
-            const int Qr = -1 + (wlive ? pchunk : 0) * lpw + li;
-            const bool live = wlive && li < lpw && Qr <= tq;
-            const int Q = live ? Qr : -1;
-            const int ec = live ? e : 0;
+    for (int rd = 0; rd < sch.rounds; rd++) {
+        const int chunk = wave * sch.rounds + rd;
+        const bool wlive = wave < sch.waves && chunk * lpw < nlines;   // (the whole wave)
+        const int line0 = chunk * lpw + li;
+        const bool live = wlive && li < lpw && line0 < nlines;
+        const int line = live ? line0 : 0;
+        const int slow = __mul24(line, inv) >> 16, fast = line - __mul24(slow, nfast);
+        const int Q = (qfast ? fast : slow) - 1, P = (qfast ? slow : fast) - 1;
+        const int ec = live ? e : 0;
+        const bool own = live && e >= 1;   // completes a cell of the tile's length
+        // lane e completes cell c = e-1 of the line (tile cells 0 .. t-1):
+        // acc[(dQ+1) + 3 (dP+1)] collects its increments to cell
+        // (c, Q+dQ, P+dP)
+        T acc[9][NV];
+        if (wlive) {
             // cells e-1 and e of the line (local -2 .. t+1)
-            const int b0 = 2 * (sx + sy + sz) + P * psd + __mul24(Q, qsd) + __mul24(ec - 1, rs);
+            const int b0 = 2 * (sx + sy + sz) + __mul24(P, psd) + __mul24(Q, qsd) + __mul24(ec - 1, rs);
             T ql[NV], qrr[NV];
 #pragma unroll
             for (int m = 0; m < NV; m++) {
@@ -330,10 +355,6 @@ __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float
                     fadp[m] = fadp[m] + c;
                 }
             }
-            // lane e completes cell c = e-1 of the line (tile cells 0 .. t-1):
-            // acc[(dQ+1) + 3 (dP+1)] collects its increments to cell
-            // (c, Q+dQ, P+dP)
-            T acc[9][NV];
 #pragma unroll
             for (int k = 0; k < 9; k++)
 #pragma unroll
@@ -346,13 +367,12 @@ __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float
                     acc[4][m] = T(0) - dtdx * (fadm[m] - fpl);
                 }
             }
-            const bool own = live && e >= 1;   // completes a cell of the tile's length
             // adds v to the mark, if any, of the face at place i of the map
             auto mark_add = [&](int i, bool ok, const T* v) {
                 const int id = ok ? mk.map[i] : 0;
                 if (id) {
 #pragma unroll
-                    for (int m = 0; m < NV; m++) lds_add(&mk.acc[(id - 1) * 2 * NV + m], v[m]);
+                    for (int m = 0; m < NV; m++) lds_add(&mk.acc[((id - 1) * 3 + phase) * NV + m], v[m]);
                 }
                 return id;
             };
@@ -360,19 +380,19 @@ __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float
                 T sc[NV];
 #pragma unroll
                 for (int m = 0; m < NV; m++) sc[m] = dtdx * fadm[m];
-                const int at = fbase(AR) + P * fstr(AR, AP) + __mul24(Q, fstr(AR, AQ)) + __mul24(e, fstr(AR, AR));
+                const int at = fbase(AR) + __mul24(P, fstr(AR, AP)) + __mul24(Q, fstr(AR, AQ)) + __mul24(e, fstr(AR, AR));
                 const int id = mark_add(at, live && Q >= 0 && Q < tq && P >= 0 && P < tp, sc);
                 if (id) {
 #pragma unroll
                     for (int m = 0; m < NV; m++)
-                        mk.acc[((id - 1) * 2 + 1) * NV + m] = fadp[m] - fadm[m];
+                        mk.acc[((id - 1) * 3 + 2) * NV + m] = fadp[m] - fadm[m];
                 }
             }
             // the lower faces across Q and across P of this lane's cell
             int atQ = 0, atP = 0;
             if constexpr (MARK) {
-                atQ = fbase(AQ) + P * fstr(AQ, AP) + __mul24(Q, fstr(AQ, AQ)) + __mul24(e - 1, fstr(AQ, AR));
-                atP = fbase(AP) + P * fstr(AP, AP) + __mul24(Q, fstr(AP, AQ)) + __mul24(e - 1, fstr(AP, AR));
+                atQ = fbase(AQ) + __mul24(P, fstr(AQ, AP)) + __mul24(Q, fstr(AQ, AQ)) + __mul24(e - 1, fstr(AQ, AR));
+                atP = fbase(AP) + __mul24(P, fstr(AP, AP)) + __mul24(Q, fstr(AP, AQ)) + __mul24(e - 1, fstr(AP, AR));
             }
             if (trans) {
                 // the splits both families use, once: of cqxx, A+dq and A-dq
@@ -463,10 +483,14 @@ __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float
                     }
                 }
             }
-            // nine ordered steps: in each, the wave's lanes add to distinct
-            // cells (its lines share P and differ in Q)
+        }
+        // nine ordered steps: in each, the wave's lanes add to distinct cells
+        // (its lines differ).  First the waves of phase 0 add, then those of
+        // phase 1; the waves of a phase touch no cell of each other
+        // (tile3_rounds).
+        auto add = [&] {
             const int c = e - 1;
-            const int dbase = P * dps + __mul24(Q, dqs) + __mul24(c, drs);
+            const int dbase = __mul24(P, dps) + __mul24(Q, dqs) + __mul24(c, drs);
 #pragma unroll
             for (int k = 0; k < 9; k++) {
                 const int dQ = k % 3 - 1, dP = k / 3 - 1;
@@ -481,12 +505,11 @@ __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float
                 }
                 wave_sync();
             }
-            __syncthreads();   // the next round's waves may touch these cells
-            prow += wpr;
-            const int carry = prow >= nrows;
-            prow -= carry ? nrows : 0;
-            pchunk += carry;
-        }
+        };
+        __syncthreads();   // phase 1 of the round before has added
+        if (wlive && phase == 0) add();
+        __syncthreads();
+        if (wlive && phase == 1) add();
     }
 }
 
@@ -531,7 +554,7 @@ __global__ __launch_bounds__(TILE3_LANES, TILE3_WG_PER_CU) void sweep3_tile_kern
         mk.acc = dq + NV * ncell + words;
         uint32_t* w = reinterpret_cast<uint32_t*>(mk.map);
         for (int idx = tid; idx < words; idx += TILE3_LANES) w[idx] = 0;
-        for (int idx = tid; idx < td.nmark * 2 * NV; idx += TILE3_LANES) mk.acc[idx] = T(0);
+        for (int idx = tid; idx < td.nmark * 3 * NV; idx += TILE3_LANES) mk.acc[idx] = T(0);
         __syncthreads();
         for (int idx = tid; idx < td.nmark; idx += TILE3_LANES)
             mk.map[mark_at(a.marks[td.mark0 + idx])] = (uint16_t)(idx + 1);
@@ -546,6 +569,7 @@ __global__ __launch_bounds__(TILE3_LANES, TILE3_WG_PER_CU) void sweep3_tile_kern
     tile3_sweep<Sol, 1, STD, MARK>(a, qs, dq, tx, ty, tz, bx, by, wave, wl, cfl, mk);
     tile3_sweep<Sol, 2, STD, MARK>(a, qs, dq, tx, ty, tz, bx, by, wave, wl, cfl, mk);
     tile3_sweep<Sol, 3, STD, MARK>(a, qs, dq, tx, ty, tz, bx, by, wave, wl, cfl, mk);
+    __syncthreads();
 
     // q(t + dt) = q(t) + dq on the tile's cells
     T* qout = static_cast<T*>(a.qout) + pt.qoff;
@@ -581,8 +605,8 @@ __global__ __launch_bounds__(TILE3_LANES, TILE3_WG_PER_CU) void sweep3_tile_kern
         for (int idx = tid; idx < td.nmark * NV; idx += TILE3_LANES) {
             const int id = idx / NV, m = idx - id * NV;
             const Mark3 f = a.marks[td.mark0 + id];
-            const T lo = T(double(mk.acc[id * 2 * NV + m]) / a.dtd[f.dir]);
-            const T df = mk.acc[(id * 2 + 1) * NV + m];
+            const T lo = T(double(mk.acc[id * 3 * NV + m] + mk.acc[(id * 3 + 1) * NV + m]) / a.dtd[f.dir]);
+            const T df = mk.acc[(id * 3 + 2) * NV + m];
             const int x = td.i0 + f.x, y = td.j0 + f.y, z = td.k0 + f.z;
             const int w = pt.mx + (f.dir == 0), h = pt.my + (f.dir == 1);
             const int64_t at = m * (f.dir == 0 ? F.sx : (f.dir == 1 ? F.sy : F.sz)) +
