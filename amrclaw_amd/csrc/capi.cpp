@@ -25,6 +25,7 @@
 #include "xfer.hpp"
 
 namespace amrgpu {
+hipError_t launch_copy_u64(unsigned long long* dst, const unsigned long long* src, int n, hipStream_t st);
 hipError_t launch_sv_map(int32_t* map, const MarchSvCell* c, int n, hipStream_t st);
 hipError_t launch_fill_u64(unsigned long long* p, unsigned long long v, int64_t n,
                            hipStream_t st);
@@ -629,6 +630,19 @@ int check_level(int level) {
     return AMRGPU_OK;
 }
 
+// pinned room for the Courant maxima of n grids (here, not in a level step: a
+// captured step holds the address, and a layout change drops captured steps)
+int grow_h_cfl(int n) {
+    if (n <= g.h_cfl_cap) return AMRGPU_OK;
+    quiesce();
+    if (g.h_cfl) hipHostFree(g.h_cfl);
+    g.h_cfl = nullptr;
+    g.h_cfl_cap = 0;
+    HIPCHK(hipHostMalloc((void**)&g.h_cfl, (size_t)n * sizeof(unsigned long long), hipHostMallocDefault));
+    g.h_cfl_cap = n;
+    return AMRGPU_OK;
+}
+
 int define_level(int level, int ngrids, const int* ilo, const int* ihi, const int* jlo,
                  const int* jhi, double hx, double hy) {
     Level& L = g.levels[level];
@@ -674,6 +688,7 @@ int define_level(int level, int ngrids, const int* ilo, const int* ihi, const in
         L.cylo.push_back(L.patches[p].jlo * hy + g.cfg.ylower);
     }
     if (ngrids > 0) {
+        if (int rc = grow_h_cfl(ngrids)) return rc;
         HIPCHK(hipMalloc(&L.d_patches, ngrids * sizeof(PatchDesc)));
         HIPCHK(h2d(L.d_patches, L.patches.data(), ngrids * sizeof(PatchDesc)));
         for (auto& b : L.buf) {
@@ -1121,18 +1136,10 @@ int sweep(Level& L, double dt, double* flux_out_dev, const int64_t* flux_off_dev
     return rc;
 }
 
-int level_cfl(Level& L, double dt, double* cfl_level, double* dtlevnew) {
-    if (L.ngrids > g.h_cfl_cap) {
-        if (g.h_cfl) hipHostFree(g.h_cfl);
-        g.h_cfl = nullptr;
-        g.h_cfl_cap = 0;
-        HIPCHK(hipHostMalloc((void**)&g.h_cfl, (size_t)L.ngrids * sizeof(unsigned long long),
-                             hipHostMallocDefault));
-        g.h_cfl_cap = L.ngrids;
-    }
-    if (L.ngrids > 0)
-        HIPCHK(hipMemcpyAsync(g.h_cfl, L.d_cfl, L.ngrids * sizeof(unsigned long long),
-                              hipMemcpyDeviceToHost, g.stream));
+// sent: the level step's last kernel has written the grids' Courant maxima to
+// g.h_cfl
+int level_cfl(Level& L, double dt, double* cfl_level, double* dtlevnew, bool sent = false) {
+    if (!sent) HIPCHK(launch_copy_u64(g.h_cfl, L.d_cfl, L.ngrids, g.stream));
     HIPCHK(hipStreamSynchronize(g.stream));
     double cmax = 0.0, dmin = RINFINITY;
     for (int p = 0; p < L.ngrids; p++) {
@@ -1196,6 +1203,11 @@ int aux_ready(int lo, int hi) {
 
 // advanc.f:16-305 for one level: ghost fill, saveqc of the finer level,
 // the sweep with fluxsv / fluxad's perimeter fluxes, qad + fluxad, time
+// Whether a level step ends with the register fix-up kernel, which then also
+// writes the Courant maxima to the host: one launch fewer (28 periodic
+// advection grids, a level step with its read-back 34 -> 32 us).
+bool sends_cfl(int level) { return level > 1 && g.levels[level].nqad > 0; }
+
 // the launches of one level step (bound, saveqc of the finer level, sweep,
 // qad + fluxad), issued on the stream with the current state; no host sync
 int launch_level_step(int level) {
@@ -1221,8 +1233,11 @@ int launch_level_step(int level) {
     if (level > 1) rl.reg = L.d_reg;
     rc = launch_sweep(L, L.possk, nullptr, nullptr, rl, cfl_cleared);
     if (rc) return rc;
-    if (level > 1 && L.nqad > 0) {
+    if (sends_cfl(level)) {
         QadArgs a{};
+        a.cfl = L.d_cfl;
+        a.cfl_host = g.h_cfl;
+        a.ncfl = L.ngrids;
         a.items = L.d_qad;
         a.nitems = L.nqad;
         a.nv = g.cfg.nvar;
@@ -1360,7 +1375,7 @@ int advance_level(int level, double* dtlevnew, double* cfl_level) {
     }
     L.cur = 1 - L.cur;                                           // new <-> old roles
     L.time = L.time + L.possk;                                   // advanc.f:289
-    if (cfl_level || dtlevnew) return level_cfl(L, L.possk, cfl_level, dtlevnew);
+    if (cfl_level || dtlevnew) return level_cfl(L, L.possk, cfl_level, dtlevnew, sends_cfl(level));
     return AMRGPU_OK;
 }
 
@@ -1702,6 +1717,7 @@ int amrgpu_init(const amrgpu_config* cfg) {
     // the device address of amrgpu_stepgrid_noalloc's static work space on
     // this GPU
     HIPCHK(noalloc_init());
+    if (int rc = grow_h_cfl(1)) return rc;
     g.txmax = 28;
     g.tymax = (g.esize == 8 && !g.mixed) ? 12 : 28;
     g.inited = true;
@@ -1882,10 +1898,8 @@ int amrgpu_stepgrid_noalloc(int mx, int my, const double* q_in, double* q_out, d
         return fail(AMRGPU_ERR_ARG, "tile caps %dx%d need %zu bytes of LDS", g.txmax, g.tymax, lds);
     unsigned char* qa = base + NOALLOC_DATA_OFF;
     unsigned char* qb = qa + bytes;
-    HIPCHK(noalloc_setup(base, mx, my, tw, th, ntx, nty, g.stream));
-    HIPCHK(noalloc_transpose(true, (int)g.esize, q_in, nullptr, qa, nv, (int)plane, g.stream));
-    // ghost cells of the output keep the input values, as in stepgrid.f
-    HIPCHK(noalloc_transpose(true, (int)g.esize, q_in, nullptr, qb, nv, (int)plane, g.stream));
+    HIPCHK(noalloc_begin(base, mx, my, tw, th, ntx, nty, (int)g.esize, q_in, qa, qb, nv, (int)plane,
+                         g.stream));
     SweepArgs a{};
     a.qin = qa;
     a.qout = qb;
@@ -1900,12 +1914,10 @@ int amrgpu_stepgrid_noalloc(int mx, int my, const double* q_in, double* q_out, d
     a.cfl_patch = reinterpret_cast<unsigned long long*>(base + NOALLOC_CFL_OFF);
     hipError_t e = run_sweep(run_precision(), a, lds, g.sweep_wgs);
     if (e != hipSuccess) return fail(AMRGPU_ERR_HIP, "sweep launch: %s", hipGetErrorString(e));
-    HIPCHK(noalloc_transpose(false, (int)g.esize, nullptr, q_out, qb, nv, (int)plane, g.stream));
-    unsigned long long cb = 0;
-    HIPCHK(hipMemcpyAsync(&cb, base + NOALLOC_CFL_OFF, sizeof cb, hipMemcpyDeviceToHost, g.stream));
+    HIPCHK(noalloc_end(base, (int)g.esize, qb, q_out, nv, (int)plane, g.h_cfl, g.stream));
     HIPCHK(hipStreamSynchronize(g.stream));
     double c;
-    std::memcpy(&c, &cb, 8);
+    std::memcpy(&c, g.h_cfl, 8);
     if (cflgrid) *cflgrid = c;
     if (dtnew) *dtnew = c > 0.0 ? dt * g.cfg.cfl / c : RINFINITY;   // stepgrid.f:206-212
     return AMRGPU_OK;

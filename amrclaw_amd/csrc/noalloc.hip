@@ -39,12 +39,20 @@ unsigned char* noalloc_scratch() {
     return static_cast<unsigned char*>(g_scratch[dev]);
 }
 
-// The descriptor of the one grid and its tiles: tile t covers x-tile
-// t % ntx and y-tile t / ntx, tw x th cells except at the grid's upper
-// edges (the tiling split_axis gives the host-planned levels); the Courant
-// maximum starts at zero.
-__global__ void noalloc_setup_kernel(unsigned char* base, int mx, int my, int tw, int th, int ntx,
-                                     int nty) {
+// Before the sweep, one launch: the descriptor of the one grid and its tiles
+// (tile t covers x-tile t % ntx and y-tile t / ntx, tw x th cells except at the
+// grid's upper edges, the tiling split_axis gives the host-planned levels), the
+// Courant maximum at zero, and the grid from the reference's AoS FP64
+// q(nv, mitot, mjtot) to SoA (S), into the array the sweep reads and the one it
+// writes (whose ghost cells keep the input values, as in stepgrid.f).
+//
+// A call is bound by its launches and the wait: 16x12 acoustics took 42 us with
+// setup, two transposes, sweep, transpose and a copy of the Courant number, and
+// takes 28 with this, the sweep and the kernel below.
+template <typename S>
+__global__ void noalloc_begin_kernel(unsigned char* base, int mx, int my, int tw, int th, int ntx,
+                                     int nty, const double* __restrict__ aos, S* __restrict__ qa,
+                                     S* __restrict__ qb, int nv, int plane) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t == 0) {
         PatchDesc pd{};
@@ -72,51 +80,49 @@ __global__ void noalloc_setup_kernel(unsigned char* base, int mx, int my, int tw
         d.wy = (int16_t)(d.ty + 3 <= 16 ? 16 : (d.ty + 3 <= 32 ? 32 : 64));
         reinterpret_cast<TileDesc*>(base + NOALLOC_TILES_OFF)[t] = d;
     }
+    if (t >= plane) return;
+    for (int m = 0; m < nv; m++) {
+        const S v = (S)aos[(int64_t)t * nv + m];
+        qa[(int64_t)m * plane + t] = v;
+        qb[(int64_t)m * plane + t] = v;
+    }
 }
 
-// one grid, the reference's AoS FP64 q(nv, mitot, mjtot) <-> SoA (S)
+// After the sweep: the grid back to AoS FP64 and the Courant maximum into
+// pinned host memory.
 template <typename S>
-__global__ void noalloc_to_soa_kernel(const double* __restrict__ aos, S* __restrict__ soa, int nv,
-                                      int plane) {
+__global__ void noalloc_end_kernel(const S* __restrict__ soa, double* __restrict__ aos, int nv,
+                                   int plane, const unsigned long long* cfl,
+                                   unsigned long long* cfl_host) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= plane) return;
-    for (int m = 0; m < nv; m++) soa[(int64_t)m * plane + c] = (S)aos[(int64_t)c * nv + m];
-}
-
-template <typename S>
-__global__ void noalloc_to_aos_kernel(const S* __restrict__ soa, double* __restrict__ aos, int nv,
-                                      int plane) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c == 0) *cfl_host = *cfl;
     if (c >= plane) return;
     for (int m = 0; m < nv; m++) aos[(int64_t)c * nv + m] = (double)soa[(int64_t)m * plane + c];
 }
 
-hipError_t noalloc_setup(unsigned char* base, int mx, int my, int tw, int th, int ntx, int nty,
+hipError_t noalloc_begin(unsigned char* base, int mx, int my, int tw, int th, int ntx, int nty,
+                         int esize, const double* aos, void* qa, void* qb, int nv, int plane,
                          hipStream_t st) {
-    const int n = ntx * nty;
-    hipLaunchKernelGGL(noalloc_setup_kernel, dim3((n + 255) / 256), dim3(256), 0, st, base, mx, my,
-                       tw, th, ntx, nty);
+    const dim3 grid((plane + 255) / 256), block(256);   // (a grid has more cells than tiles)
+    if (esize == 8)
+        hipLaunchKernelGGL(noalloc_begin_kernel<double>, grid, block, 0, st, base, mx, my, tw, th,
+                           ntx, nty, aos, (double*)qa, (double*)qb, nv, plane);
+    else
+        hipLaunchKernelGGL(noalloc_begin_kernel<float>, grid, block, 0, st, base, mx, my, tw, th,
+                           ntx, nty, aos, (float*)qa, (float*)qb, nv, plane);
     return hipGetLastError();
 }
 
-hipError_t noalloc_transpose(bool to_soa, int esize, const double* aos_in, double* aos_out,
-                             void* soa, int nv, int plane, hipStream_t st) {
+hipError_t noalloc_end(const unsigned char* base, int esize, const void* soa, double* aos, int nv,
+                       int plane, unsigned long long* cfl_host, hipStream_t st) {
     const dim3 grid((plane + 255) / 256), block(256);
-    if (to_soa) {
-        if (esize == 8)
-            hipLaunchKernelGGL(noalloc_to_soa_kernel<double>, grid, block, 0, st, aos_in,
-                               (double*)soa, nv, plane);
-        else
-            hipLaunchKernelGGL(noalloc_to_soa_kernel<float>, grid, block, 0, st, aos_in,
-                               (float*)soa, nv, plane);
-    } else {
-        if (esize == 8)
-            hipLaunchKernelGGL(noalloc_to_aos_kernel<double>, grid, block, 0, st,
-                               (const double*)soa, aos_out, nv, plane);
-        else
-            hipLaunchKernelGGL(noalloc_to_aos_kernel<float>, grid, block, 0, st,
-                               (const float*)soa, aos_out, nv, plane);
-    }
+    const auto* cfl = reinterpret_cast<const unsigned long long*>(base + NOALLOC_CFL_OFF);
+    if (esize == 8)
+        hipLaunchKernelGGL(noalloc_end_kernel<double>, grid, block, 0, st, (const double*)soa, aos,
+                           nv, plane, cfl, cfl_host);
+    else
+        hipLaunchKernelGGL(noalloc_end_kernel<float>, grid, block, 0, st, (const float*)soa, aos, nv,
+                           plane, cfl, cfl_host);
     return hipGetLastError();
 }
 

@@ -22,12 +22,14 @@ constexpr size_t NOALLOC_DATA_BYTES = NOALLOC_SCRATCH_BYTES - NOALLOC_DATA_OFF;
 hipError_t noalloc_init();
 // The current GPU's address of the array, or nullptr before noalloc_init.
 unsigned char* noalloc_scratch();
-// Write the grid's descriptor and tile table and clear its Courant maximum.
-hipError_t noalloc_setup(unsigned char* base, int mx, int my, int tw, int th, int ntx, int nty,
+// Write the grid's descriptor and tile table, clear its Courant maximum, and
+// take the grid from AoS FP64 (the reference's layout) to SoA of the storage
+// precision, twice.
+hipError_t noalloc_begin(unsigned char* base, int mx, int my, int tw, int th, int ntx, int nty,
+                         int esize, const double* aos, void* qa, void* qb, int nv, int plane,
                          hipStream_t st);
-// AoS FP64 (the reference's layout) -> SoA of the storage precision
-// (to_soa, from aos_in) or back (into aos_out).
-hipError_t noalloc_transpose(bool to_soa, int esize, const double* aos_in, double* aos_out,
-                             void* soa, int nv, int plane, hipStream_t st);
+// The stepped grid back to AoS, its Courant maximum into pinned host memory.
+hipError_t noalloc_end(const unsigned char* base, int esize, const void* soa, double* aos, int nv,
+                       int plane, unsigned long long* cfl_host, hipStream_t st);
 
 }  // namespace amrgpu

@@ -42,6 +42,7 @@ template <class Sol, typename S, int G>
 __global__ __launch_bounds__(64) void finereg_kernel(QadArgs a, Physics ph) {
     constexpr int NV = Sol::NV, NW = Sol::NW;
     const int t = (blockIdx.x * 64 + threadIdx.x) / G, g = threadIdx.x % G;
+    for (int i = blockIdx.x * 64 + threadIdx.x; i < a.ncfl; i += gridDim.x * 64) a.cfl_host[i] = a.cfl[i];
     if (t >= a.nitems) return;
     const QadItem it = a.items[t];
     const PatchDesc pd = a.patches[it.grid];

@@ -58,7 +58,10 @@ struct QadArgs {
     const double* aux;
     int32_t auxk;
     int32_t auxtype[8];
-    int32_t pad;
+    // the grids' Courant maxima, final here, to pinned host memory
+    int32_t ncfl;
+    const unsigned long long* cfl;
+    unsigned long long* cfl_host;
 };
 
 struct UpdateArgs {

@@ -21,6 +21,19 @@ hipError_t launch_fill_u64(unsigned long long* p, unsigned long long v, int64_t 
     return hipGetLastError();
 }
 
+// a few words from the device to pinned host memory
+__global__ void copy_u64_kernel(unsigned long long* dst, const unsigned long long* src, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) dst[i] = src[i];
+}
+
+hipError_t launch_copy_u64(unsigned long long* dst, const unsigned long long* src, int n,
+                           hipStream_t st) {
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(copy_u64_kernel, dim3((n + 255) / 256), dim3(256), 0, st, dst, src, n);
+    return hipGetLastError();
+}
+
 // map[cell] = first + 1 of every record (MarchSvCell), on a cleared map
 __global__ void sv_map_kernel(int32_t* map, const MarchSvCell* c, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
