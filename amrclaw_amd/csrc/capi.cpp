@@ -395,12 +395,42 @@ struct Tiling {
     std::vector<TileDesc> tiles;
     std::vector<int> patch_tile_start;
     size_t lds = 0;
+    size_t lds_caps = 0;   // of the largest tile the caps as set would give
     int layout = 0;
 };
+
+// LDS of the largest tile that caps give a grid
+size_t caps_lds(int mx, int my, int txmax, int tymax) {
+    const int tx = std::min(split_axis(mx, txmax)[0].second, mx);
+    const int ty = std::min(split_axis(my, tymax)[0].second, my);
+    return (g.esize == 8 && !g.mixed) ? sweep_lds_bytes<double>(g.cfg.nvar, tx, ty)
+                                      : sweep_lds_bytes<float>(g.cfg.nvar, tx, ty, g.mixed);
+}
+
+// The caps a sweep of few grids is cut with: a tile of 12x12 cells is one pass
+// of the workgroup's 256 lanes in either direction (14 rows of 15 interfaces),
+// a larger one two or more, so while there are few the smaller tiles are done
+// sooner: up to one a CU, with the Euler solver's longer solves three.  Level
+// sweeps with the wait, tuned caps / 12x12: mixed Euler 236 tiles 36.7 / 20.1
+// us, 802 37.5 / 30.3, 2262 40.9 / 46.8; FP64 Euler 124 tiles 27.5 / 19.4, 830
+// 41.3 / 36.3, 1925 57.2 / 57.5; FP64 acoustics 84 tiles 15.1 / 12.6, 374 19.1 /
+// 21.5, 993 24.8 / 34.1.
+constexpr int SMALL_CAP = 12, SMALL_TILES = 256, SMALL_TILES_EULER = 768;
+void small_caps(const std::vector<PatchDesc>& grids, int& txmax, int& tymax) {
+    const int cx = std::min(txmax, SMALL_CAP), cy = std::min(tymax, SMALL_CAP);
+    int64_t n = 0;
+    for (const auto& pd : grids) n += (int64_t)((pd.mx + cx - 1) / cx) * ((pd.my + cy - 1) / cy);
+    if (n > (g.cfg.solver == SOLVER_EULER && !g.plugin ? SMALL_TILES_EULER : SMALL_TILES)) return;
+    txmax = cx;
+    tymax = cy;
+}
 
 Tiling make_tiling(const Level& L, int txmax, int tymax, int launch_mode) {
     Tiling T;
     const int nv = g.cfg.nvar;
+    for (const auto& pd : L.patches) T.lds_caps = std::max(T.lds_caps, caps_lds(pd.mx, pd.my, txmax, tymax));
+    if (launch_mode == AMRGPU_LAUNCH_BATCHED || launch_mode == AMRGPU_LAUNCH_MARCH)
+        small_caps(L.patches, txmax, tymax);
     for (int p = 0; p < L.ngrids; p++) {
         const PatchDesc& pd = L.patches[p];
         auto xs = split_axis(pd.mx, txmax), ys = split_axis(pd.my, tymax);
@@ -578,8 +608,9 @@ constexpr size_t LDS_MAX = 160 * 1024;
 // the level changes.
 int plan_level(Level& L) {
     Tiling T = make_tiling(L, g.txmax, g.tymax, g.launch_mode);
-    if (T.lds > LDS_MAX)
-        return fail(AMRGPU_ERR_ARG, "tile caps %dx%d need %zu bytes of LDS", g.txmax, g.tymax, T.lds);
+    if (T.lds_caps > LDS_MAX)
+        return fail(AMRGPU_ERR_ARG, "tile caps %dx%d need %zu bytes of LDS", g.txmax, g.tymax,
+                    T.lds_caps);
     g.layout_version++;
     free_graphs(L);
     g.regs_valid = false;
@@ -617,9 +648,9 @@ int check_tiling(int txmax, int tymax, int launch_mode) {
     for (const auto& L : g.levels)
         if (L.ngrids) {
             Tiling T = make_tiling(L, txmax, tymax, launch_mode);
-            if (T.lds > LDS_MAX)
+            if (T.lds_caps > LDS_MAX)
                 return fail(AMRGPU_ERR_ARG, "tile caps %dx%d need %zu bytes of LDS", txmax, tymax,
-                            T.lds);
+                            T.lds_caps);
         }
     return AMRGPU_OK;
 }
@@ -1880,11 +1911,19 @@ int amrgpu_stepgrid_noalloc(int mx, int my, const double* q_in, double* q_out, d
                     "grid %dx%d needs %lld bytes of work space; amrgpu_stepgrid_noalloc holds %lld",
                     mx, my, (long long)(2 * bytes), (long long)NOALLOC_DATA_BYTES);
     // the tiling amrgpu_stepgrid's level planner gives one grid
-    const auto xs = split_axis(mx, g.txmax), ys = split_axis(my, g.tymax);
+    int txmax = g.txmax, tymax = g.tymax;
+    const size_t asked = caps_lds(mx, my, txmax, tymax);
+    if (asked > LDS_MAX)
+        return fail(AMRGPU_ERR_ARG, "tile caps %dx%d need %zu bytes of LDS", g.txmax, g.tymax, asked);
+    PatchDesc one{};
+    one.mx = mx;
+    one.my = my;
+    small_caps({one}, txmax, tymax);
+    const auto xs = split_axis(mx, txmax), ys = split_axis(my, tymax);
     const int ntx = (int)xs.size(), nty = (int)ys.size(), tw = xs[0].second, th = ys[0].second;
     if ((int64_t)ntx * nty > NOALLOC_MAX_TILES)
         return fail(AMRGPU_ERR_ARG, "grid %dx%d has %d tiles at caps %dx%d; at most %d", mx, my,
-                    ntx * nty, g.txmax, g.tymax, NOALLOC_MAX_TILES);
+                    ntx * nty, txmax, tymax, NOALLOC_MAX_TILES);
     const bool f32 = g.mixed || g.esize == 4;
     size_t lds = f32 ? sweep_lds_bytes<float>(nv, tw, th, g.mixed) : sweep_lds_bytes<double>(nv, tw, th);
     const int lx = f32 ? 28 : 12, ly = 12;
@@ -1894,8 +1933,6 @@ int amrgpu_stepgrid_noalloc(int mx, int my, const double* q_in, double* q_out, d
         lds = std::max(lds, f32 ? sweep_lds_bytes<float>(nv, lx, ly, g.mixed)
                                 : sweep_lds_bytes<double>(nv, lx, ly));
     }
-    if (lds > LDS_MAX)
-        return fail(AMRGPU_ERR_ARG, "tile caps %dx%d need %zu bytes of LDS", g.txmax, g.tymax, lds);
     unsigned char* qa = base + NOALLOC_DATA_OFF;
     unsigned char* qb = qa + bytes;
     HIPCHK(noalloc_begin(base, mx, my, tw, th, ntx, nty, (int)g.esize, q_in, qa, qb, nv, (int)plane,

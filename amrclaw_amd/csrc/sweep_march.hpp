@@ -40,7 +40,8 @@
 // parameter: as a run-time check it cost the levels without it 6 %.
 //
 // Bound by vector issue: with FP32 arithmetic the SIMDs issue vector
-// instructions in 86 % of their cycles (4 cycles each) when the chip is full.
+// instructions in 80 to 90 % of their cycles (3.5 to 4 cycles each) when the
+// chip is full.
 // What a solve derives from one state alone (roots and quotients) is computed
 // once per cell and used by its four interfaces, with the same bits (Sol::Cell);
 // FP32 arithmetic sums the waves by their strengths.  4096 uneven mixed Euler

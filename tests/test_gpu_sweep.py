@@ -10,7 +10,7 @@ import pytest
 
 from amrclaw_amd import capi
 from oracle import orc
-from tests.common import both_params, random_patch, rel_l1
+from tests.common import SOLVERS, both_params, random_patch, rel_l1
 
 pytestmark = pytest.mark.gpu
 
@@ -234,3 +234,37 @@ def test_mixed_occupancy_bounds_agree(gpu):
                 capi.set_occupancy(bad)
     finally:
         capi.finalize()
+
+
+@pytest.mark.parametrize("solver", ["acoustics", "euler"])
+@pytest.mark.parametrize("ngrids", [9, 120])
+def test_small_tiles_bit_exact(gpu, solver, ngrids):
+    """Levels of few grids are cut into smaller tiles in the batched launch (9
+    grids) and as the caps say beyond that (120); the persistent launch always
+    takes the caps: the same FP64 bits and Courant number."""
+    sid = SOLVERS[solver]
+    rng = np.random.default_rng(ngrids)
+    sizes = [(12, 12), (13, 13), (28, 12), (29, 25), (1, 40), (40, 1), (11, 30), (61, 37), (16, 12)]
+    sizes = [sizes[k % len(sizes)] for k in range(ngrids)]
+    boxes, x = [], 0
+    for mx, my in sizes:
+        boxes.append((x, x + mx - 1, 0, my - 1))
+        x += mx
+    qs = [random_patch(rng, sid, mx, my) for mx, my in sizes]
+    _, cfg = both_params(sid, precision=capi.FP64)
+    got = {}
+    for mode in (capi.LAUNCH_BATCHED, capi.LAUNCH_PERSISTENT):
+        capi.init(cfg)
+        try:
+            capi.set_launch_mode(mode)
+            capi.set_level(1, np.array(boxes), 1 / 64, 1 / 48)
+            for k, q in enumerate(qs):
+                capi.put_grid(1, k, q)
+            cfl = capi.sweep_level(1, 0.002)
+            got[mode] = [capi.get_grid(1, k, q.shape) for k, q in enumerate(qs)], cfl
+        finally:
+            capi.finalize()
+    a, b = got[capi.LAUNCH_BATCHED], got[capi.LAUNCH_PERSISTENT]
+    assert a[1] == b[1]
+    for k, (x, y) in enumerate(zip(a[0], b[0])):
+        assert np.array_equal(x, y), sizes[k]
