@@ -40,7 +40,7 @@
 // parameter: as a run-time check it cost the levels without it 6 %.
 //
 // Bound by vector issue: with FP32 arithmetic the SIMDs issue vector
-// instructions in 80 to 90 % of their cycles (3.5 to 4 cycles each) when the
+// instructions in 73 to 91 % of their cycles (3.2 to 4 cycles each) when the
 // chip is full.
 // What a solve derives from one state alone (roots and quotients) is computed
 // once per cell and used by its four interfaces, with the same bits (Sol::Cell);

@@ -49,13 +49,13 @@ HBM_PEAK_GBS = 8000.0
 # plain-copy calibration: FETCH_SIZE x 2 KiB, WRITE_SIZE x 1 KiB); the
 # summaries and commands are the files named here.
 MEASURED_TRAFFIC = {
-    ("euler2d", "mixed", 4096, "batched"): (1200800 * 2048 + 783700 * 1024,
+    ("euler2d", "mixed", 4096, "batched"): (1201199 * 2048 + 806229 * 1024,
                                             "profiles/level_update_euler_mixed_4096.md"),
     ("euler2d", "fp32", 4096, "batched"): (459126 * 2048 + 450853 * 1024,
                                            "profiles/level_update_euler_fp32_4096.md"),
-    ("euler2d", "mixed", 4096, "march"): (397129 * 2048 + 782660 * 1024,
+    ("euler2d", "mixed", 4096, "march"): (413374 * 2048 + 782991 * 1024,
                                           "profiles/level_update_euler_mixed_4096_march.md"),
-    ("euler3d", "fp32", 512, "fused"): (69557 * 2048 + 96870 * 1024,
+    ("euler3d", "fp32", 512, "fused"): (69493 * 2048 + 96823 * 1024,
                                         "profiles/step3_euler_fp32_512_fused.md"),
     ("euler3d", "fp32", 512, "phases"): (
         (271400 + 875200 + 1415000 + 330700) * 2048 + (801800 + 1136000 + 1143000 + 98580) * 1024,
@@ -64,15 +64,18 @@ MEASURED_TRAFFIC = {
 # Vector-ALU wave instructions per launch of the same kernels (rocprofv3
 # --pmc SQ_INSTS_VALU of the default workloads; the summaries named here).
 MEASURED_VALU = {
-    ("euler2d", "mixed", 4096, "march"): (423823602,
+    ("euler2d", "mixed", 4096, "march"): (370749671,
                                           "profiles/level_update_euler_mixed_4096_march.md"),
-    ("euler2d", "mixed", 4096, "batched"): (757577540,
+    ("euler2d", "mixed", 4096, "batched"): (684756659,
                                             "profiles/level_update_euler_mixed_4096.md"),
-    ("euler3d", "fp32", 512, "fused"): (967839559, "profiles/step3_euler_fp32_512_fused.md"),
+    ("euler3d", "fp32", 512, "fused"): (575255843, "profiles/step3_euler_fp32_512_fused.md"),
 }
 SIMD_COUNT = 1024                 # 256 CUs x 4 SIMDs
 CLOCK_HZ = 2.4e9                  # peak engine clock
-VALU_ISSUE_CYCLES = 2             # a SIMD issues one wave64 VALU instruction per 2 cycles
+# cycles of a SIMD per wave64 vector instruction: 4 for FP32 arithmetic (16
+# lanes a cycle, the packed forms not used), less for some moves; the densest
+# rate measured here is one per 3.2 (the mixed tile sweep)
+VALU_ISSUE_CYCLES = 3.2
 METRIC = "cell-updates/s, FP32-batched vs FP64 per-patch at fixed L1 err; % HBM peak"
 
 
