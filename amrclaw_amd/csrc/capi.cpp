@@ -1232,12 +1232,11 @@ int aux_ready(int lo, int hi) {
     return AMRGPU_OK;
 }
 
-// advanc.f:16-305 for one level: ghost fill, saveqc of the finer level,
-// the sweep with fluxsv / fluxad's perimeter fluxes, qad + fluxad, time
-// Whether a level step ends with the register fix-up kernel, which then also
-// writes the Courant maxima to the host: one launch fewer (28 periodic
-// advection grids, a level step with its read-back 34 -> 32 us).
-bool sends_cfl(int level) { return level > 1 && g.levels[level].nqad > 0; }
+// Whether a level step ends with the library's own register fix-up kernel,
+// which then also writes the Courant maxima to the host: one launch fewer (28
+// periodic advection grids, a level step with its read-back 34 -> 32 us).  A
+// plug-in's launcher is the application's and owes the registers only.
+bool sends_cfl(int level) { return level > 1 && g.levels[level].nqad > 0 && !g.plugin; }
 
 // the launches of one level step (bound, saveqc of the finer level, sweep,
 // qad + fluxad), issued on the stream with the current state; no host sync
@@ -1264,11 +1263,13 @@ int launch_level_step(int level) {
     if (level > 1) rl.reg = L.d_reg;
     rc = launch_sweep(L, L.possk, nullptr, nullptr, rl, cfl_cleared);
     if (rc) return rc;
-    if (sends_cfl(level)) {
+    if (level > 1 && L.nqad > 0) {
         QadArgs a{};
-        a.cfl = L.d_cfl;
-        a.cfl_host = g.h_cfl;
-        a.ncfl = L.ngrids;
+        if (sends_cfl(level)) {
+            a.cfl = L.d_cfl;
+            a.cfl_host = g.h_cfl;
+            a.ncfl = L.ngrids;
+        }
         a.items = L.d_qad;
         a.nitems = L.nqad;
         a.nv = g.cfg.nvar;

@@ -58,7 +58,8 @@ struct QadArgs {
     const double* aux;
     int32_t auxk;
     int32_t auxtype[8];
-    // the grids' Courant maxima, final here, to pinned host memory
+    // the grids' Courant maxima, final here, to pinned host memory (ncfl 0: left
+    // to a launch of the library's, as after a plug-in's kernel)
     int32_t ncfl;
     const unsigned long long* cfl;
     unsigned long long* cfl_host;
