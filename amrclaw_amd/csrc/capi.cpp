@@ -665,12 +665,40 @@ int check_level(int level) {
 // captured step holds the address, and a layout change drops captured steps)
 int grow_h_cfl(int n) {
     if (n <= g.h_cfl_cap) return AMRGPU_OK;
+    unsigned long long* p = nullptr;   // the array at hand stays until this one is there
+    HIPCHK(hipHostMalloc((void**)&p, (size_t)n * sizeof(unsigned long long), hipHostMallocDefault));
     quiesce();
     if (g.h_cfl) hipHostFree(g.h_cfl);
-    g.h_cfl = nullptr;
-    g.h_cfl_cap = 0;
-    HIPCHK(hipHostMalloc((void**)&g.h_cfl, (size_t)n * sizeof(unsigned long long), hipHostMallocDefault));
+    g.h_cfl = p;
     g.h_cfl_cap = n;
+    return AMRGPU_OK;
+}
+
+// the device arrays of a level whose grids are defined
+int alloc_level(Level& L) {
+    const int ngrids = L.ngrids;
+    if (int rc = grow_h_cfl(ngrids)) return rc;
+    HIPCHK(hipMalloc(&L.d_patches, ngrids * sizeof(PatchDesc)));
+    HIPCHK(h2d(L.d_patches, L.patches.data(), ngrids * sizeof(PatchDesc)));
+    for (auto& b : L.buf) {
+        HIPCHK(hipMalloc(&b, (size_t)L.nelem * g.esize));
+        HIPCHK(dzero(b, (size_t)L.nelem * g.esize));
+    }
+    HIPCHK(hipMalloc(&L.d_cfl, ngrids * sizeof(unsigned long long)));
+    HIPCHK(hipMalloc(&L.d_partial, ngrids * sizeof(double)));
+    if (g.auxk > 0) {
+        HIPCHK(hipMalloc(&L.d_aux, (size_t)L.nelem * g.auxk * sizeof(double)));
+        HIPCHK(dzero(L.d_aux, (size_t)L.nelem * g.auxk * sizeof(double)));
+        L.aux_set = false;
+    }
+    std::vector<XferGrid> xg(ngrids);
+    int64_t c = 0;
+    for (int p = 0; p < ngrids; p++) {
+        xg[p] = XferGrid{L.patches[p].off, L.patches[p].plane, c};
+        c += L.patches[p].plane;
+    }
+    HIPCHK(hipMalloc(&L.d_xfer, ngrids * sizeof(XferGrid)));
+    HIPCHK(h2d(L.d_xfer, xg.data(), ngrids * sizeof(XferGrid)));
     return AMRGPU_OK;
 }
 
@@ -702,10 +730,11 @@ int define_level(int level, int ngrids, const int* ilo, const int* ihi, const in
         pd.ilo = ilo[p]; pd.ihi = ihi[p]; pd.jlo = jlo[p]; pd.jhi = jhi[p];
         pd.mx = ihi[p] - ilo[p] + 1;
         pd.my = jhi[p] - jlo[p] + 1;
-        if (pd.mx < 1 || pd.my < 1)
-            return fail(AMRGPU_ERR_ARG, "grid %d of level %d is empty", p, level);
-        if (pd.mx > 30000 || pd.my > 30000)
-            return fail(AMRGPU_ERR_ARG, "grid %d of level %d too large", p, level);
+        if (pd.mx < 1 || pd.my < 1 || pd.mx > 30000 || pd.my > 30000) {
+            const bool empty = pd.mx < 1 || pd.my < 1;
+            free_level(L);
+            return fail(AMRGPU_ERR_ARG, "grid %d of level %d %s", p, level, empty ? "is empty" : "too large");
+        }
         pd.mitot = pd.mx + 2 * ng;
         pd.plane = pd.mitot * (pd.my + 2 * ng);
         pd.off = off;
@@ -718,32 +747,9 @@ int define_level(int level, int ngrids, const int* ilo, const int* ihi, const in
         L.cxlo.push_back(L.patches[p].ilo * hx + g.cfg.xlower);    // grdfit2.f:98-101
         L.cylo.push_back(L.patches[p].jlo * hy + g.cfg.ylower);
     }
-    if (ngrids > 0) {
-        if (int rc = grow_h_cfl(ngrids)) return rc;
-        HIPCHK(hipMalloc(&L.d_patches, ngrids * sizeof(PatchDesc)));
-        HIPCHK(h2d(L.d_patches, L.patches.data(), ngrids * sizeof(PatchDesc)));
-        for (auto& b : L.buf) {
-            HIPCHK(hipMalloc(&b, (size_t)L.nelem * g.esize));
-            HIPCHK(dzero(b, (size_t)L.nelem * g.esize));
-        }
-        HIPCHK(hipMalloc(&L.d_cfl, ngrids * sizeof(unsigned long long)));
-        HIPCHK(hipMalloc(&L.d_partial, ngrids * sizeof(double)));
-        if (g.auxk > 0) {
-            HIPCHK(hipMalloc(&L.d_aux, (size_t)L.nelem * g.auxk * sizeof(double)));
-            HIPCHK(dzero(L.d_aux, (size_t)L.nelem * g.auxk * sizeof(double)));
-            L.aux_set = false;
-        }
-        std::vector<XferGrid> xg(ngrids);
-        int64_t c = 0;
-        for (int p = 0; p < ngrids; p++) {
-            xg[p] = XferGrid{L.patches[p].off, L.patches[p].plane, c};
-            c += L.patches[p].plane;
-        }
-        HIPCHK(hipMalloc(&L.d_xfer, ngrids * sizeof(XferGrid)));
-        HIPCHK(h2d(L.d_xfer, xg.data(), ngrids * sizeof(XferGrid)));
-    }
-    int rc = plan_level(L);
-    if (rc) free_level(L);   // refused tiling: leave the level without grids
+    int rc = ngrids > 0 ? alloc_level(L) : AMRGPU_OK;
+    if (!rc) rc = plan_level(L);
+    if (rc) free_level(L);   // no memory or a refused tiling: leave the level without grids
     return rc;
 }
 

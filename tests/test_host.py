@@ -46,3 +46,43 @@ def child_plugin_courant(fake):
         assert len(fake.launches("copy_u64")) == 1, level
     assert calls == [8]
     capi.finalize()
+
+
+def test_refused_allocation_leaves_levels_whole():
+    """A level whose arrays cannot be allocated is left without grids, and the
+    pinned Courant array that the other levels' steps write stays theirs."""
+    run("child_refused_level")
+
+
+def child_refused_level(fake):
+    from amrclaw_amd import capi
+    H = nested_hierarchy(np.random.default_rng(1), flat_states(4), 4, nlev=2, dt1=0.004)
+    many = [(8 * i, 8 * i + 3, 0, 3) for i in range(200)]
+    capi.init(capi.make_config(capi.EULER))
+    for kind in (fake_hip.PINNED, fake_hip.DEVICE):
+        capi.load_hierarchy(H)
+        capi.set_level(2, [], 0.01, 0.01)
+        live = fake.live(fake_hip.DEVICE)
+        for n in range(1, 100):
+            fake.refuse(kind, n)
+            try:
+                capi.set_level(2, many, 0.01, 0.01)
+            except capi.AmrgpuError:
+                pass
+            else:
+                break
+            assert fake.live(fake_hip.DEVICE) == live, (kind, n)
+            fake.clear()
+            dt, cfl = capi.sweep_level(2, 1e-3)[::-1]
+            assert cfl == 0.0 and not fake.launches("sweep"), (kind, n)
+            capi.sweep_level(1, 1e-3)
+            assert [x[2] != 0 for x in fake.launches("copy_u64")] == [True], (kind, n)
+        assert n > 1, kind
+        fake.refuse(kind, 0)
+        for bad in ((0, 3, 4, 3), (0, 30000, 0, 3)):     # an empty grid, too large a one
+            with pytest.raises(capi.AmrgpuError):
+                capi.set_level(2, many + [bad], 0.01, 0.01)
+            with pytest.raises(capi.AmrgpuError):
+                capi.put_grid(2, 0, np.ones((8, 8, 4)))
+    capi.finalize()
+    assert fake.live(fake_hip.DEVICE) == fake.live(fake_hip.PINNED) == 0
