@@ -390,8 +390,7 @@ void plan_tiles3(const std::vector<Patch3>& patches, int nv,
     }
 }
 
-int define_batch(int npatch, const int* mx, const int* my, const int* mz) {
-    free_batch();
+int alloc_batch(int npatch, const int* mx, const int* my, const int* mz) {
     const int nv = g3.cfg.nvar;
     g3.patches.resize(npatch);
     int64_t qo = 0, fo = 0;
@@ -435,6 +434,13 @@ int define_batch(int npatch, const int* mx, const int* my, const int* mz) {
     g3.h_cfl.assign(npatch, 0);
     HIPCHK3(hipStreamSynchronize(g3.stream));
     return AMRGPU_OK;
+}
+
+int define_batch(int npatch, const int* mx, const int* my, const int* mz) {
+    free_batch();
+    const int rc = alloc_batch(npatch, mx, my, mz);
+    if (rc) free_batch();   // a batch is there whole or not at all
+    return rc;
 }
 
 // host AoS q(nvar, mx+4, my+4, mz+4) <-> device SoA [m][k][j][i].  To the

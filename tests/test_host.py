@@ -86,3 +86,39 @@ def child_refused_level(fake):
                 capi.put_grid(2, 0, np.ones((8, 8, 4)))
     capi.finalize()
     assert fake.live(fake_hip.DEVICE) == fake.live(fake_hip.PINNED) == 0
+
+
+def test_refused_batch_is_not_kept():
+    """amrgpu3_stepgrid keeps its one-grid batch for the next call of the same
+    shape, but not one whose arrays could not all be allocated."""
+    run("child_refused_batch")
+
+
+def child_refused_batch(fake):
+    from amrclaw_amd import capi, capi3
+    q = np.ones((9, 8, 10, 5))
+    for precision in (capi.FP64, capi.FP32):
+        capi3.init3(capi3.make_config3(capi.EULER, precision=precision))
+        refused = 0
+        for n in range(1, 100):
+            capi3.set_patches3([(3, 3, 3)])
+            fake.refuse(fake_hip.DEVICE, n)
+            try:
+                capi3.set_patches3([(6, 4, 5)])
+            except capi.AmrgpuError:
+                refused += 1
+                with pytest.raises(capi.AmrgpuError):
+                    capi3.get_patch3(0, q.shape)
+                with pytest.raises(capi.AmrgpuError):
+                    fake.refuse(fake_hip.DEVICE, 1)
+                    capi3.stepgrid3(q, 0.1, 0.1, 0.1, 0.01)
+            else:
+                break
+        fake.refuse(fake_hip.DEVICE, 0)
+        assert refused >= 8
+        capi3.stepgrid3(q, 0.1, 0.1, 0.1, 0.01)
+        allocs = fake.allocs(fake_hip.DEVICE)
+        capi3.stepgrid3(q, 0.1, 0.1, 0.1, 0.01)     # the batch at hand
+        assert fake.allocs(fake_hip.DEVICE) == allocs
+        capi3.finalize3()
+        assert fake.live(fake_hip.DEVICE) == fake.live(fake_hip.PINNED) == 0
