@@ -468,13 +468,11 @@ int get_q(int p, double* q) { return xfer_q(false, p, q); }
 // The two-pass plan of a batch.  Runs of grids share a work space of at most
 // PASS3_BYTES: fuller runs fill the chip better (512 grids of 8 .. 32 cells a
 // side, 4.1 M cells: 9.6 ms in runs of 256 MB, 8.2 of 1 GB, 7.6 of 4 GB), and
-// 4 GB of 288 are cheap.  A batch with a grid that alone needs more (beyond
-// 134^3 cells) takes the phase kernels.
+// 4 GB of 288 are cheap.  A batch with a grid that alone needs more (Euler:
+// beyond 135^3 cells) takes the phase kernels.
 constexpr int64_t PASS3_BYTES = 4ll << 30;
 
-int build_pass3(const std::vector<Patch3>& patches, Pass3Plan& pp) {
-    pp.free();
-    pp.built = true;
+hipError_t build_pass3(const std::vector<Patch3>& patches, Pass3Plan& pp) {
     const int nv = g3.cfg.nvar;
     std::vector<Pass3Wave> waves[3];
     std::vector<Block3> faces;
@@ -494,7 +492,7 @@ int build_pass3(const std::vector<Patch3>& patches, Pass3Plan& pp) {
         const Patch3& pt = patches[p];
         int64_t need = 0;
         for (int d = 1; d <= 3; d++) need += (pass3_elems(pt, d, nv) + 15) / 16 * 16;
-        if (need > cap) return AMRGPU_OK;   // not ok: the phase kernels
+        if (need > cap) return hipSuccess;   // not ok: the phase kernels
         if (used > 0 && used + need > cap) close();
         for (int d = 1; d <= 3; d++) {
             off[p].off[d - 1] = used;
@@ -512,29 +510,45 @@ int build_pass3(const std::vector<Patch3>& patches, Pass3Plan& pp) {
         hipError_t e = hipMalloc((void**)&d, std::max<size_t>(1, h.size()) * sizeof(h[0]));
         return e != hipSuccess || h.empty() ? e : h2d3(d, h.data(), h.size() * sizeof(h[0]));
     };
-    for (int d = 0; d < 3; d++) HIPCHK3(up(pp.d_waves[d], waves[d]));
-    HIPCHK3(up(pp.d_faces, faces));
-    HIPCHK3(up(pp.d_off, off));
-    pp.ok = true;
-    return AMRGPU_OK;
+    hipError_t e = hipSuccess;
+    for (int d = 0; d < 3 && e == hipSuccess; d++) e = up(pp.d_waves[d], waves[d]);
+    if (e == hipSuccess) e = up(pp.d_faces, faces);
+    if (e == hipSuccess) e = up(pp.d_off, off);
+    pp.ok = e == hipSuccess;
+    return e;
 }
 
-// The work space of a plan; where the card has no room for it, the batch takes
-// the phase kernels.
-int pass3_ws(Pass3Plan& pp) {
-    if (!pp.ok || pp.ws_elems <= g3.ws_cap) return AMRGPU_OK;
-    HIPCHK3(hipStreamSynchronize(g3.stream));
+// the work space of a plan
+hipError_t pass3_ws(const Pass3Plan& pp) {
+    if (!pp.ok || pp.ws_elems <= g3.ws_cap) return hipSuccess;
+    hipError_t e = hipStreamSynchronize(g3.stream);
+    if (e != hipSuccess) return e;
     hipFree(g3.d_ws);
     g3.d_ws = nullptr;
     g3.ws_cap = 0;
-    const hipError_t e = hipMalloc(&g3.d_ws, pp.ws_elems * sizeof(double));
+    e = hipMalloc(&g3.d_ws, pp.ws_elems * sizeof(double));
+    if (e == hipSuccess) g3.ws_cap = pp.ws_elems;
+    return e;
+}
+
+// The plan and its work space, made on the first step of a layout.  Where the
+// card has no room for either, the batch takes the phase kernels, until its
+// layout changes.
+int ready_pass3(const std::vector<Patch3>& patches, Pass3Plan& pp) {
+    hipError_t e = hipSuccess;
+    if (!pp.built) {
+        pp.free();
+        e = build_pass3(patches, pp);
+        pp.built = e == hipSuccess;
+    }
+    if (e == hipSuccess) e = pass3_ws(pp);
     if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();
-        pp.ok = false;
+        pp.free();
+        pp.built = true;   // and not ok
         return AMRGPU_OK;
     }
     HIPCHK3(e);
-    g3.ws_cap = pp.ws_elems;
     return AMRGPU_OK;
 }
 
@@ -588,11 +602,7 @@ int step_io(const Step3IO& io, double dx, double dy, double dz, double dt, int e
     const int solver = g3.cfg.solver;
     bool passes = false;
     if (es == 8 && io.pass) {
-        if (!io.pass->built) {
-            int rc = build_pass3(*io.patches, *io.pass);
-            if (rc) return rc;
-        }
-        int rc = pass3_ws(*io.pass);
+        int rc = ready_pass3(*io.patches, *io.pass);
         if (rc) return rc;
         passes = io.pass->ok;
         if (passes) {

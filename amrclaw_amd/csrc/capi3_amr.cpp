@@ -273,17 +273,31 @@ std::vector<std::vector<GridFace3>> register_faces(const Lev3& L, bool fine) {
     return out;
 }
 
+// The fused step of a level; where a tile's marks or the card have no room for
+// it, the level takes the phase kernels.
 int plan_fused(int level) {
     Lev3& L = A.lev[level];
     L.fused = false;
     if (ctx3_esize() != 4 || L.patches.empty()) return AMRGPU_OK;
     ctx3_plan_tiles(L.patches, register_faces(L, level >= 2), L.tiles);
     if (L.tiles.lds > 160 * 1024) return AMRGPU_OK;   // too many marks in a tile
-    int rc = upload(L.d_tiles, L.tiles.tiles);
-    if (!rc) rc = upload(L.d_marks, L.tiles.marks);
-    if (rc) return rc;
-    if (level == A.H.nlev && !L.d_next)
-        HIPCHKA(hipMalloc(&L.d_next, std::max<int64_t>(1, L.q_elems) * sizeof(float)));
+    dfree(L.d_tiles);
+    dfree(L.d_marks);
+    auto up = [](auto*& d, const auto& h) {
+        hipError_t e = hipMalloc((void**)&d, std::max<size_t>(1, h.size()) * sizeof(h[0]));
+        return e != hipSuccess || h.empty() ? e : ctx3_h2d(d, h.data(), h.size() * sizeof(h[0]));
+    };
+    hipError_t e = up(L.d_tiles, L.tiles.tiles);
+    if (e == hipSuccess) e = up(L.d_marks, L.tiles.marks);
+    if (e == hipSuccess && level == A.H.nlev && !L.d_next)
+        e = hipMalloc(&L.d_next, std::max<int64_t>(1, L.q_elems) * sizeof(float));
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        dfree(L.d_tiles);
+        dfree(L.d_marks);
+        return AMRGPU_OK;
+    }
+    HIPCHKA(e);
     L.fused = true;
     return AMRGPU_OK;
 }

@@ -43,7 +43,7 @@ struct Pass3Run {
     int w0[3], w1[3], f0, f1;
 };
 struct Pass3Plan {
-    bool built = false, ok = false;   // ok: every grid's work space is in bounds
+    bool built = false, ok = false;   // built and not ok: the phase kernels
     std::vector<Pass3Run> runs;
     int64_t ws_elems = 0;
     Pass3Wave* d_waves[3] = {};

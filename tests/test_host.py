@@ -122,3 +122,64 @@ def child_refused_batch(fake):
         assert fake.allocs(fake_hip.DEVICE) == allocs
         capi3.finalize3()
         assert fake.live(fake_hip.DEVICE) == fake.live(fake_hip.PINNED) == 0
+
+
+def test_steps3_without_memory_take_the_phase_kernels():
+    """The 3-D steps that need memory of their own (the two-pass FP64 step, the
+    fused FP32 step of a level) give way to the phase kernels where any part of it
+    is refused."""
+    run("child_steps3_without_memory")
+
+
+def child_steps3_without_memory(fake):
+    from amrclaw_amd import capi, capi3
+    from tests.common3 import nested_hierarchy3, smooth_euler3
+    phases, passes, tiles = "sweep3_phase", "pass3_solve", "sweep3_tile"
+
+    def step():
+        fake.clear()
+        capi3.step_patches3(0.1, 0.1, 0.1, 0.01)
+        return bool(fake.launches(phases)), bool(fake.launches(passes))
+
+    capi3.init3(capi3.make_config3(capi.EULER))
+    sizes = [(6, 5, 4), (8, 3, 7)]
+    capi3.set_patches3(sizes)
+    n0 = fake.allocs(fake_hip.DEVICE)
+    assert step() == (False, True)
+    nstep = fake.allocs(fake_hip.DEVICE) - n0
+    for n in range(1, nstep + 1):
+        capi3.finalize3()
+        capi3.init3(capi3.make_config3(capi.EULER))
+        capi3.set_patches3(sizes)
+        before = fake.live(fake_hip.DEVICE)
+        fake.refuse(fake_hip.DEVICE, n)
+        assert step() == (True, False) == step(), n       # and the steps after it
+        assert fake.live(fake_hip.DEVICE) == before, n
+        capi3.set_patches3(sizes)
+        assert step() == (False, True), n                 # a new layout asks again
+    capi3.finalize3()
+
+    H = nested_hierarchy3(np.random.default_rng(3), smooth_euler3, 5, nlev=2)
+    survived = 0
+    for n in range(1, 200):
+        capi3.init3(capi3.make_config3(capi.EULER, precision=capi.FP32))
+        capi3.load_hierarchy3(H)
+        n0 = fake.allocs(fake_hip.DEVICE)
+        fake.refuse(fake_hip.DEVICE, n)
+        fake.clear()
+        try:
+            for level in (1, 2):
+                capi3.advance_level3(level)
+        except capi.AmrgpuError:
+            pass
+        else:
+            used = fake.allocs(fake_hip.DEVICE) - n0
+            survived += used >= n
+            assert len(fake.launches(tiles)) == (1 if used >= n else 2), n
+            assert bool(fake.launches(phases)) == (used >= n), n
+        fake.refuse(fake_hip.DEVICE, 0)
+        capi3.finalize3()
+        if n > fake.allocs(fake_hip.DEVICE) - n0:
+            break
+    assert survived == 5      # tiles and marks of either level, the finest's second buffer
+    assert fake.live(fake_hip.DEVICE) == fake.live(fake_hip.PINNED) == 0
