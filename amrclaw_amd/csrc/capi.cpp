@@ -636,7 +636,14 @@ int plan_level(Level& L) {
         if (pick && !march_pays(L, rows)) L.mwaves.clear();
     }
     if (!L.mwaves.empty()) {
-        HIPCHK(hipMalloc(&L.d_mwaves, L.mwaves.size() * sizeof(MarchWave)));
+        const hipError_t e = hipMalloc(&L.d_mwaves, L.mwaves.size() * sizeof(MarchWave));
+        if (e == hipErrorOutOfMemory && pick) {   // the tile sweep needs no table
+            (void)hipGetLastError();
+            L.d_mwaves = nullptr;
+            L.mwaves.clear();
+            return AMRGPU_OK;
+        }
+        HIPCHK(e);
         HIPCHK(h2d(L.d_mwaves, L.mwaves.data(), L.mwaves.size() * sizeof(MarchWave)));
     }
     return AMRGPU_OK;
@@ -946,7 +953,7 @@ int upload(T** dst, const std::vector<T>& v) {
 }
 
 // The march sweep's fluxsv entries of a level: the map of its cells and the
-// entries of each marked cell one after the other.  No room for the map on the
+// entries of each marked cell one after the other.  No room for them on the
 // card: none, and the tile sweep steps the level.
 int march_entries(Level& L, const RegLevel& fine, const RegLevel& R) {
     const int nv = g.cfg.nvar;
@@ -969,20 +976,28 @@ int march_entries(Level& L, const RegLevel& fine, const RegLevel& R) {
         }
     }
     const int64_t n = (L.nelem / nv + 2) / 2 * 2;
-    const hipError_t e = hipMalloc(&L.d_svmap, n * sizeof(int32_t));
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        L.d_svmap = nullptr;
-        return AMRGPU_OK;
-    }
     MarchSvCell* d_cells = nullptr;
-    int rc = upload(&L.d_msv, ents);
-    if (!rc) rc = upload(&d_cells, cells);
-    if (rc) return rc;
-    HIPCHK(launch_fill_u64(reinterpret_cast<unsigned long long*>(L.d_svmap), 0ull, n / 2, g.stream));
-    HIPCHK(launch_sv_map(L.d_svmap, d_cells, (int)cells.size(), g.stream));
+    auto up = [](auto*& d, const auto& h) {
+        hipError_t e = hipMalloc((void**)&d, std::max<size_t>(1, h.size()) * sizeof(h[0]));
+        return e != hipSuccess || h.empty() ? e : h2d(d, h.data(), h.size() * sizeof(h[0]));
+    };
+    hipError_t e = hipMalloc(&L.d_svmap, n * sizeof(int32_t));
+    if (e == hipSuccess) e = up(L.d_msv, ents);
+    if (e == hipSuccess) e = up(d_cells, cells);
+    if (e == hipSuccess)
+        e = launch_fill_u64(reinterpret_cast<unsigned long long*>(L.d_svmap), 0ull, n / 2, g.stream);
+    if (e == hipSuccess) e = launch_sv_map(L.d_svmap, d_cells, (int)cells.size(), g.stream);
     quiesce();
     if (d_cells) hipFree(d_cells);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        if (L.d_svmap) hipFree(L.d_svmap);
+        if (L.d_msv) hipFree(L.d_msv);
+        L.d_svmap = nullptr;
+        L.d_msv = nullptr;
+        return AMRGPU_OK;
+    }
+    HIPCHK(e);
     return AMRGPU_OK;
 }
 

@@ -183,3 +183,49 @@ def child_steps3_without_memory(fake):
             break
     assert survived == 5      # tiles and marks of either level, the finest's second buffer
     assert fake.live(fake_hip.DEVICE) == fake.live(fake_hip.PINNED) == 0
+
+
+def test_march_tables_without_memory():
+    """A level that marches because it is faster does without where the march's
+    tables (its waves; with a finer level the map and entries of fluxsv) are
+    refused: the tile sweep steps it."""
+    run("child_march_tables")
+
+
+def child_march_tables(fake):
+    from amrclaw_amd import capi
+    boxes = [(100 * i, 100 * i + 99, 100 * j, 100 * j + 99) for j in range(8) for i in range(8)]
+    fine = [(220, 259, 220, 259), (300, 339, 300, 349)]
+
+    def load():
+        capi.set_geometry([800, 1600], [800, 1600], [2, 2], [2, 2], [1 / 800, 1 / 1600],
+                          [1 / 800, 1 / 1600])
+        capi.set_level(1, boxes, 1 / 800, 1 / 800)
+        capi.set_level(2, fine, 1 / 1600, 1 / 1600)
+        for level in (1, 2):
+            capi.set_time(level, 0.0, 1e-4 / level)
+
+    survived = 0
+    for n in range(0, 200):
+        capi.init(capi.make_config(capi.EULER))
+        n0 = fake.allocs(fake_hip.DEVICE)
+        fake.refuse(fake_hip.DEVICE, n)
+        fake.clear()
+        try:
+            load()
+            capi.advance_level(1)
+        except capi.AmrgpuError:
+            pass
+        else:
+            used = fake.allocs(fake_hip.DEVICE) - n0
+            marched = bool(fake.launches("sweep_march"))
+            assert marched == (n == 0 or used < n), n
+            assert marched or fake.launches("sweep_kernel"), n
+            survived += not marched
+        fake.refuse(fake_hip.DEVICE, 0)
+        total = fake.allocs(fake_hip.DEVICE) - n0
+        capi.finalize()
+        assert fake.live(fake_hip.DEVICE) == 0, n
+        if n > total:
+            break
+    assert survived == 4      # the waves, the map, its cells, the entries
