@@ -172,6 +172,7 @@ struct Context {
     hipStream_t stream = nullptr;
     hipEvent_t ev[NEVENTS] = {};
     int txmax = 28, tymax = 28;
+    bool caps_asked = false;               // by amrgpu_set_tiling
     int sweep_wgs = 0;   // occupancy bound of the mixed sweep (0: its default)
     int march_wgs = 0;   // occupancy bound of the march sweep (0: its default)
     Level levels[MAXLV];
@@ -407,16 +408,17 @@ size_t caps_lds(int mx, int my, int txmax, int tymax) {
                                       : sweep_lds_bytes<float>(g.cfg.nvar, tx, ty, g.mixed);
 }
 
-// The caps a sweep of few grids is cut with: a tile of 12x12 cells is one pass
-// of the workgroup's 256 lanes in either direction (14 rows of 15 interfaces),
-// a larger one two or more, so while there are few the smaller tiles are done
-// sooner: up to one a CU, with the Euler solver's longer solves three.  Level
-// sweeps with the wait, tuned caps / 12x12: mixed Euler 236 tiles 36.7 / 20.1
+// The caps a sweep of few grids is cut with where the caller has asked for none
+// (amrgpu_set_tiling): a tile of 12x12 cells is one pass of the workgroup's 256
+// lanes in either direction (14 rows of 15 interfaces), a larger one two or
+// more, so while there are few the smaller tiles are done sooner: up to one a
+// CU, with the Euler solver's longer solves three.  Level sweeps with the wait, tuned caps / 12x12: mixed Euler 236 tiles 36.7 / 20.1
 // us, 802 37.5 / 30.3, 2262 40.9 / 46.8; FP64 Euler 124 tiles 27.5 / 19.4, 830
 // 41.3 / 36.3, 1925 57.2 / 57.5; FP64 acoustics 84 tiles 15.1 / 12.6, 374 19.1 /
 // 21.5, 993 24.8 / 34.1.
 constexpr int SMALL_CAP = 12, SMALL_TILES = 256, SMALL_TILES_EULER = 768;
 void small_caps(const std::vector<PatchDesc>& grids, int& txmax, int& tymax) {
+    if (g.caps_asked) return;
     const int cx = std::min(txmax, SMALL_CAP), cy = std::min(tymax, SMALL_CAP);
     int64_t n = 0;
     for (const auto& pd : grids) n += (int64_t)((pd.mx + cx - 1) / cx) * ((pd.my + cy - 1) / cy);
@@ -1862,6 +1864,7 @@ int amrgpu_set_tiling(int txmax, int tymax) {
     if (rc0) return rc0;
     g.txmax = tx;
     g.tymax = ty;
+    g.caps_asked = g.caps_asked || txmax || tymax;
     for (auto& L : g.levels)
         if (L.ngrids) {
             int rc = plan_level(L);

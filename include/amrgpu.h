@@ -89,8 +89,9 @@ int amrgpu_finalize(void);
 /* Copy the last error message (NUL-terminated, truncated to len). */
 int amrgpu_last_error(char* buf, int len);
 
-/* Tile-size caps of the sweep (autotuner knob); 0 keeps the current value.  A
- * level of few grids may be cut into smaller tiles than the caps allow. */
+/* Tile-size caps of the sweep (autotuner knob); 0 keeps the current value.
+ * Until caps are asked for, a level of few grids is cut into smaller tiles than
+ * the library's own caps allow. */
 int amrgpu_set_tiling(int txmax, int tymax);
 /* Occupancy bounds (autotuner knobs, no counterpart in the reference):
  * 5, 6 or 7 set the workgroups per CU the register allocation of the

@@ -229,3 +229,43 @@ def child_march_tables(fake):
         if n > total:
             break
     assert survived == 4      # the waves, the map, its cells, the entries
+
+
+def test_tile_caps_bind():
+    """The caps of amrgpu_set_tiling are the caller's also on levels of few grids;
+    only the library's own are narrowed there."""
+    run("child_tile_caps")
+
+
+def child_tile_caps(fake):
+    from amrclaw_amd import capi
+    boxes = [(28 * i, 28 * i + 27, 0, 27) for i in range(4)]
+
+    def tiles(call):
+        fake.clear()
+        call()
+        return [x[1] for x in fake.launches("sweep_kernel")]
+
+    one = lambda: capi.stepgrid_noalloc(28, 28, 1, 1, 0.01, 0.01, 1e-3)
+    level = lambda: capi.sweep_level(1, 1e-3)
+    for solver in (capi.EULER, capi.ACOUSTICS):
+        for mode in (capi.LAUNCH_BATCHED, capi.LAUNCH_PER_PATCH):
+            capi.init(capi.make_config(solver, precision=capi.MIXED))
+            capi.set_launch_mode(mode)
+            capi.set_level(1, boxes, 0.01, 0.01)
+            batched = mode == capi.LAUNCH_BATCHED
+            assert tiles(level) == ([4 * 9] if batched else [1] * 4)
+            assert tiles(one) == [9]
+            capi.set_tiling(0, 0)                     # nothing asked for
+            assert sum(tiles(level)) == (4 * 9 if batched else 4) and tiles(one) == [9]
+            capi.set_tiling(28, 28)
+            assert sum(tiles(level)) == 4 and tiles(one) == [1]
+            capi.set_tiling(0, 16)
+            assert sum(tiles(level)) == 8 and tiles(one) == [2]
+            capi.set_level(1, boxes[:3], 0.01, 0.01)
+            assert sum(tiles(level)) == 6
+            capi.finalize()
+    capi.init(capi.make_config(capi.EULER, precision=capi.MIXED))
+    capi.set_level(1, boxes, 0.01, 0.01)
+    assert tiles(level) == [4 * 9]                    # a new context's caps are its own again
+    capi.finalize()
