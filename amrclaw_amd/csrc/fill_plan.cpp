@@ -702,8 +702,10 @@ struct Planner {
         op.stage = 2;
         if (P.masks.size() + (size_t)nx * ny > (size_t)INT32_MAX) return fail("filval: masks too large");
         op.mask_off = (int32_t)P.masks.size();
+        P.masks.resize(P.masks.size() + (size_t)nx * ny);
         for (int j = 0; j < ny; j++)
-            for (int i = 0; i < nx; i++) P.masks.push_back(cov[(size_t)(j + ng) * mitot + (i + ng)]);
+            std::copy_n(cov.begin() + (size_t)(j + ng) * mitot + ng, nx,
+                        P.masks.begin() + op.mask_off + (size_t)j * nx);
         push(op);
         return true;
     }
@@ -736,10 +738,19 @@ static bool meets(const FillPlan& P, const FillOp& early, const FillOp& late) {
 // another operation) read it, as these read what the others wrote.  In other
 // grids the ghost strips are written by operations that meet no cell of each
 // other, and a same-level copy reads interiors, which a fill does not write.
+// In a new grid the interpolation (FILVAL) leaves out the cells its mask marks,
+// those that the copies of old grids write, so these go side by side.
 static void finish_plan(FillPlan& P) {
-    std::stable_sort(P.ops.begin(), P.ops.end(),
-                     [](const FillOp& a, const FillOp& b) { return a.stage < b.stage; });
     const int n = (int)P.ops.size();
+    std::vector<int> at_stage;   // by stage, as planned within one
+    for (const FillOp& op : P.ops) {
+        if ((int)at_stage.size() < op.stage + 2) at_stage.resize(op.stage + 2, 0);
+        at_stage[op.stage + 1]++;
+    }
+    for (size_t s = 1; s < at_stage.size(); s++) at_stage[s] += at_stage[s - 1];
+    std::vector<FillOp> sorted(n);
+    for (const FillOp& op : P.ops) sorted[at_stage[op.stage]++] = op;
+    P.ops.swap(sorted);
     std::vector<int> up(n);
     for (int k = 0; k < n; k++) up[k] = k;
     auto root = [&](int k) {
@@ -751,42 +762,52 @@ static void finish_plan(FillPlan& P) {
         b = root(b);
         up[std::max(a, b)] = std::min(a, b);
     };
-    std::vector<std::vector<int>> uses(P.bufs.size());
-    std::vector<char> read(P.bufs.size(), 0);
+    const int nb = (int)P.bufs.size();
+    std::vector<char> tied(nb);   // buffers that tie all their operations
+    for (int b = 0; b < nb; b++) tied[b] = P.bufs[b].kind != 0;
+    for (const FillOp& op : P.ops) {
+        if (op.type == FOP_BC) tied[op.dst] = 1;
+        if (op.type != FOP_COPY && op.type != FOP_BC) tied[op.src] = 1;
+    }
+    // the operation before on a tied buffer; on the others the list of those
+    // that write it (first, then next)
+    std::vector<int> before(nb, -1), next(n, -1);
     for (int k = 0; k < n; k++) {
         const FillOp& op = P.ops[k];
-        uses[op.dst].push_back(k);
-        if (op.type == FOP_BC || op.type == FOP_FILVAL) read[op.dst] = 1;
-        if (op.type != FOP_COPY && op.type != FOP_BC) {
-            if (op.src != op.dst) uses[op.src].push_back(k);
-            read[op.src] = 1;
+        auto use = [&](int b) {
+            if (before[b] >= 0) tie(before[b], k);
+            before[b] = k;
+        };
+        if (tied[op.dst]) {
+            use(op.dst);
+        } else {
+            next[k] = before[op.dst];
+            before[op.dst] = k;
+            if (op.type != FOP_FILVAL)
+                for (int x = next[k]; x >= 0; x = next[x])
+                    if (P.ops[x].stage < op.stage && meets(P, P.ops[x], op)) tie(x, k);
         }
-    }
-    for (size_t b = 0; b < P.bufs.size(); b++) {
-        const std::vector<int>& u = uses[b];
-        if (P.bufs[b].kind != 0 || read[b]) {
-            for (size_t k = 1; k < u.size(); k++) tie(u[0], u[k]);
-            continue;
-        }
-        for (size_t x = 0; x < u.size(); x++)
-            for (size_t y = 0; y < u.size(); y++)
-                if (P.ops[u[x]].stage < P.ops[u[y]].stage && meets(P, P.ops[u[x]], P.ops[u[y]]))
-                    tie(u[x], u[y]);
+        if (op.type != FOP_COPY && op.type != FOP_BC && op.src != op.dst) use(op.src);
     }
     // large units first: the last ones to start should be short
     std::vector<int64_t> cost(n, 0);
-    for (int k = 0; k < n; k++) cost[root(k)] += 256 + (int64_t)P.ops[k].ni * P.ops[k].nj;
-    P.order.resize(n);
-    for (int k = 0; k < n; k++) P.order[k] = k;
-    std::stable_sort(P.order.begin(), P.order.end(), [&](int a, int b) {
-        const int ra = root(a), rb = root(b);
-        return ra != rb && cost[ra] != cost[rb] ? cost[ra] > cost[rb] : ra < rb;
-    });
-    P.units.clear();
+    std::vector<int> count(n, 0), roots;
     for (int k = 0; k < n; k++) {
-        if (k == 0 || root(P.order[k]) != root(P.order[k - 1])) P.units.push_back(FillUnit{k, 0});
-        P.units.back().n++;
+        up[k] = root(k);
+        cost[up[k]] += 256 + (int64_t)P.ops[k].ni * P.ops[k].nj;
+        if (count[up[k]]++ == 0) roots.push_back(up[k]);
     }
+    std::sort(roots.begin(), roots.end(),
+              [&](int a, int b) { return cost[a] != cost[b] ? cost[a] > cost[b] : a < b; });
+    P.units.clear();
+    int at = 0;
+    for (int r : roots) {
+        P.units.push_back(FillUnit{at, count[r]});
+        at += count[r];
+        count[r] = P.units.back().item0;   // from here on: where its next operation goes
+    }
+    P.order.resize(n);
+    for (int k = 0; k < n; k++) P.order[count[up[k]]++] = k;
 }
 
 std::vector<FillItem> fill_items(const FillPlan& P, int nvar,

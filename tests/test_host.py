@@ -269,3 +269,24 @@ def child_tile_caps(fake):
     capi.set_level(1, boxes, 0.01, 0.01)
     assert tiles(level) == [4 * 9]                    # a new context's caps are its own again
     capi.finalize()
+
+
+def test_regrid_copies_run_side_by_side():
+    """The copies of old grids into a new one touch no cell of each other or of the
+    interpolation: each has a workgroup of its own."""
+    run("child_regrid_units")
+
+
+def child_regrid_units(fake):
+    from amrclaw_amd import capi
+    old = [(32 + 16 * i, 47 + 16 * i, 32 + 16 * j, 47 + 16 * j) for j in range(4) for i in range(4)]
+    new = [(34, 97, 34, 97)]
+    capi.init(capi.make_config(capi.EULER))
+    capi.set_geometry([64, 128], [64, 128], [2, 2], [2, 2], [1 / 64, 1 / 128], [1 / 64, 1 / 128])
+    capi.set_level(1, [(0, 63, 0, 63)], 1 / 64, 1 / 64)
+    capi.set_level(2, old, 1 / 128, 1 / 128)
+    fake.clear()
+    capi.regrid_level(2, new, 0.0)
+    # 16 copies; the coarse patch and the interpolation out of it together
+    assert [x[1] for x in fake.launches("fill_kernel")] == [17]
+    capi.finalize()
