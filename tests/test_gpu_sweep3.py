@@ -350,3 +350,26 @@ def test_fused_fp32_small_tiles_and_order(gpu):
             assert np.array_equal(runs[0][k], runs[1][k]), sizes[k]
     finally:
         capi3.finalize3()
+
+
+@pytest.mark.parametrize("solver", [orc.EULER, orc.ADVECTION])
+def test_two_pass_courant_of_shared_workgroups(gpu, solver):
+    """Grids of 1 .. 9 waves a sweep, four waves to a workgroup wherever grids
+    begin: each keeps its own Courant number, bit for bit the oracle's."""
+    p, c = params((solver, 2, 22, 4))
+    rng = np.random.default_rng(95)
+    sizes = [tuple(int(v) for v in rng.integers(1, 9, 3)) for _ in range(60)]
+    qs = [patch(rng, solver, *s) * (1.0 + 0.02 * k) for k, s in enumerate(sizes)]
+    dx, dy, dz, dt = 1.0 / 40, 1.0 / 36, 1.0 / 44, 0.05 / 44
+    capi3.init3(c)
+    try:
+        capi3.set_patches3(sizes)
+        for k, q in enumerate(qs):
+            capi3.put_patch3(k, q)
+        cfl = capi3.step_patches3(dx, dy, dz, dt, npatch=len(qs))
+        for k, q in enumerate(qs):
+            want, _, co, _ = orc.stepgrid3(p, q, dx, dy, dz, dt)
+            assert np.array_equal(capi3.get_patch3(k, q.shape), want), sizes[k]
+            assert cfl[k] == co, sizes[k]
+    finally:
+        capi3.finalize3()
