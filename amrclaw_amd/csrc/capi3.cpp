@@ -531,14 +531,44 @@ hipError_t pass3_ws(const Pass3Plan& pp) {
     return e;
 }
 
+// Whether a batch is better off in two passes (both give the same bits).  The
+// Euler solver is: its phase kernels solve each interface several times.  The
+// advection solver's phase kernels take little more than a chain of rounds (256
+// lanes of a plane) per workgroup, the longest or the sum over some 640
+// workgroups at work, and the passes their traffic, by the cell.  us a step,
+// phases / passes: method(3) = 22, 8 grids of 40^3 824 / 213, 512 of 6x7x5 115 /
+// 72, 64 of 40^3 1,272 / 1,281, 512 of 16^3 520 / 804; method(3) = 0, 8 of 40^3
+// 225 / 173, 2 of 60^3 357 / 118, 64 of 40^3 322 / 755, 512 of 16^3 208 / 222.
+bool pass3_pays(const Step3IO& io) {
+    if (g3.cfg.solver != SOLVER_ADVECTION) return true;
+    int64_t chain = 0, work = 0;
+    for (int d = 0; d < 3; d++) {
+        int64_t longest = 0;
+        for (const Block3& b : io.blocks[d]) {
+            const int64_t c = block_cost((*io.patches)[b.patch], d, b);
+            longest = std::max(longest, c);
+            work += c;
+        }
+        chain += longest;
+    }
+    int64_t cells = 0;
+    for (const Patch3& p : *io.patches) cells += (int64_t)p.mx * p.my * p.mz;
+    const Method3& M = g3.meth;
+    const double round = M.m4 > 0 ? 4.9 : (M.m3 > 0 ? 3.7 : (M.order > 1 ? 1.25 : 0.85));
+    const double phases = 30.0 + round * std::max((double)chain, work / 640.0);
+    const double passes = 40.0 + (M.m3 > 0 ? 3.3e-4 : 1.7e-4) * cells;
+    return passes < phases;
+}
+
 // The plan and its work space, made on the first step of a layout.  Where the
-// card has no room for either, the batch takes the phase kernels, until its
-// layout changes.
-int ready_pass3(const std::vector<Patch3>& patches, Pass3Plan& pp) {
+// card has no room for either, or they do not pay, the batch takes the phase
+// kernels, until its layout changes.
+int ready_pass3(const Step3IO& io) {
+    Pass3Plan& pp = *io.pass;
     hipError_t e = hipSuccess;
     if (!pp.built) {
         pp.free();
-        e = build_pass3(patches, pp);
+        if (pass3_pays(io)) e = build_pass3(*io.patches, pp);
         pp.built = e == hipSuccess;
     }
     if (e == hipSuccess) e = pass3_ws(pp);
@@ -602,7 +632,7 @@ int step_io(const Step3IO& io, double dx, double dy, double dz, double dt, int e
     const int solver = g3.cfg.solver;
     bool passes = false;
     if (es == 8 && io.pass) {
-        int rc = ready_pass3(*io.patches, *io.pass);
+        int rc = ready_pass3(io);
         if (rc) return rc;
         passes = io.pass->ok;
         if (passes) {
@@ -720,6 +750,7 @@ int step_batch(double dx, double dy, double dz, double dt, double* cflgrid, bool
     io.npatch = g3.npatch;
     io.d_cfl = g3.d_cfl;
     io.patches = &g3.patches;
+    io.blocks = g3.blocks;
     io.pass = &g3.pass;
     int rc = step_io(io, dx, dy, dz, dt);
     if (rc) return rc;

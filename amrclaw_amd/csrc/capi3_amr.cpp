@@ -752,6 +752,7 @@ int amrgpu3_advance_level(int level, double* dtlevnew, double* cfl_level) {
         io.npatch = (int)L.patches.size();
         io.d_cfl = L.d_cfl;
         io.patches = &L.patches;
+        io.blocks = L.blocks;
         io.pass = &L.pass;
         rc = ctx3_step(io, G.hx, G.hy, G.hz, L.possk);
         if (rc) return rc;
@@ -927,6 +928,7 @@ int amrgpu3_flag_level(int level, double tolsp, int flag_richardson, double tol,
             io.npatch = n;
             io.d_cfl = L.d_cfl;
             io.patches = &R.crs;
+            io.blocks = bc;
             io.pass = &pass_c;
             rc = ctx3_step(io, 2.0 * G.hx, 2.0 * G.hy, 2.0 * G.hz, 2. * L.possk, 8);
         }
@@ -942,6 +944,7 @@ int amrgpu3_flag_level(int level, double tolsp, int flag_richardson, double tol,
             io.npatch = n;
             io.d_cfl = L.d_cfl;
             io.patches = &R.fine;
+            io.blocks = bf;
             io.pass = &pass_f;
             rc = ctx3_step(io, G.hx, G.hy, G.hz, L.possk, 8);
         }

@@ -66,7 +66,8 @@ struct Step3IO {
     int nblocks[4];
     int npatch;
     unsigned long long* d_cfl;    // per-grid Courant number (double bits)
-    const std::vector<Patch3>* patches;   // FP64: the host copy, and the batch's
+    const std::vector<Patch3>* patches;   // FP64: the host copies, and the batch's
+    const std::vector<Block3>* blocks;
     Pass3Plan* pass;                      // two-pass plan (null: phase kernels)
 };
 

@@ -290,3 +290,26 @@ def child_regrid_units(fake):
     # 16 copies; the coarse patch and the interpolation out of it together
     assert [x[1] for x in fake.launches("fill_kernel")] == [17]
     capi.finalize()
+
+
+@pytest.mark.parametrize("sizes,transverse,passes", [
+    ([(40, 40, 40)] * 8, 22, True), ([(40, 40, 40)] * 8, 0, True),
+    ([(40, 40, 40)] * 64, 0, False), ([(16, 16, 16)] * 512, 22, False),
+    ([(16, 16, 16)] * 512, 0, False), ([(6, 7, 5)] * 512, 22, True), ([(1, 1, 1)], 22, True)])
+def test_route_of_fp64_advection_steps(sizes, transverse, passes):
+    """Batches that fill the chip keep the phase kernels where these are the
+    faster ones: the advection solver's (Euler always takes the passes)."""
+    run("child_advection_route", sizes, transverse, passes)
+
+
+def child_advection_route(fake, sizes, transverse, passes):
+    from amrclaw_amd import capi, capi3
+    for solver, want in ((capi.ADVECTION, passes), (capi.EULER, True)):
+        capi3.init3(capi3.make_config3(solver, transverse=transverse))
+        capi3.set_patches3(sizes[:200])
+        capi3.set_patches3(sizes)                      # the route is the layout's
+        fake.clear()
+        capi3.step_patches3(0.1, 0.1, 0.1, 0.01)
+        assert bool(fake.launches("pass3_solve")) == want, solver
+        assert bool(fake.launches("sweep3_phase")) == (not want), solver
+        capi3.finalize3()
