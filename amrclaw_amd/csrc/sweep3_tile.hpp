@@ -46,6 +46,7 @@
 #include <cstdint>
 #include "lanes.hpp"
 #include "sweep3.hpp"
+#include "tile3_rounds.hpp"
 
 namespace amrgpu {
 
@@ -110,24 +111,6 @@ __host__ __device__ constexpr size_t tile3_lds_bytes(int bx, int by, int bz, int
     return ((size_t)NV * bx * by * bz + (size_t)NV * cells) * sizeof(float);
 }
 
-// The schedule of a sweep over the (tq + 2) (tp + 2) lines through a tile and
-// around it: chunks of 64 / (tr + 1) lines, dealt to the waves in blocks, one
-// chunk a wave and round.  A line's increments reach the cells within one line
-// of it, so two lines at least 2 n + 3 apart in the order (n: the length of the
-// fast axis) touch no cell of each other.  Four waves work in two phases,
-// waves 0 and 2 before 1 and 3, if that holds between the chunks of waves two
-// apart; else (tiles of 4 cells and less) two waves do.
-struct Tile3Rounds {
-    int rounds, waves;
-};
-__host__ __device__ inline Tile3Rounds tile3_rounds(int tr, int tq, int tp) {
-    const int lpw = 64 / (tr + 1), n = (tq < tp ? tq : tp) + 2;
-    const int chunks = ((tq + 2) * (tp + 2) + lpw - 1) / lpw;
-    const int four = (chunks + 3) / 4;
-    if ((2 * four - 1) * lpw + 1 >= 2 * n + 3) return {four, 4};
-    return {(chunks + 1) / 2, 2};
-}
-
 // Wave-synchronous ordering: the LDS accesses of one wave before this point
 // are complete and visible to its other lanes after it (as __syncwarp).
 __device__ __forceinline__ void wave_sync() {
@@ -169,25 +152,24 @@ __device__ __forceinline__ void lds_add(float* p, float v) {
 // one sweep of a tile (D: 1 x, 2 y, 3 z, a template parameter so that every
 // component index of the solver is a compile-time constant).
 //
-// Schedule: the lines of the sweep form rows of constant P (P = -1 .. tp),
-// each of tq + 2 lines Q = -1 .. tq.  A wave takes a chunk of up to
-// lpw = 64 / (tr + 1) consecutive lines of one row, tr + 1 lanes per line.
-// The rows are taken in three classes ((P + 1) mod 3); in a round the four
-// waves take chunks of distinct rows of one class, which lie three or more
-// rows apart, so the cells their lines touch (P - 1 .. P + 1) are disjoint.
-// Within a wave the lines of a chunk touch common cells; each lane adds its
-// increments to the nine cells (dQ, dP) around its own in nine ordered
-// steps, in each of which the wave's lanes touch distinct cells.  Rounds are
-// separated by barriers.
+// Schedule (tile3_rounds): the lines Q = -1 .. tq, P = -1 .. tp in one order, in
+// which a wave takes chunks of up to lpw = 64 / (tr + 1) consecutive lines, from
+// any rows, tr + 1 lanes per line.  The waves that add at the same time hold
+// lines at least 2 n + 3 apart, so the cells these touch are disjoint: all waves
+// of a round where the tile has lines enough, else those of a phase.  Within a
+// wave the lines of a chunk touch common cells; each lane adds its increments to
+// the nine cells (dQ, dP) around its own in ordered steps, in each of which the
+// wave's lanes touch distinct cells.
 //
 // STD: the method is known to be the standard one (std_method3: second order,
 // all transverse and double-transverse terms, MC limiter on every wave, no
 // f-waves), so its switches are compile-time constants.
 //
-// MARK: increments to marked faces are also added to the faces' own sums.  A
-// wave's LDS additions happen in program order, each touching distinct faces;
-// waves of a round touch distinct faces as they touch distinct cells, so these
-// sums have a fixed order too.
+// MARK: increments to marked faces are also added to the faces' own sums, one
+// for either phase, while the waves solve.  A wave's LDS additions happen in
+// program order, each touching distinct faces; the waves of a phase touch
+// distinct faces as they touch distinct cells, so these sums have a fixed order
+// too.
 template <class Sol, int D, bool STD, bool MARK>
 __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float* dq,
                                             int tx, int ty, int tz, int bx, int by, int wave,
@@ -484,15 +466,13 @@ __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float
                 }
             }
         }
-        // nine ordered steps: in each, the wave's lanes add to distinct cells
-        // (its lines differ).  First the waves of phase 0 add, then those of
-        // phase 1; the waves of a phase touch no cell of each other
-        // (tile3_rounds).
+        // ordered steps: in each, the wave's lanes add to distinct cells (its lines
+        // differ).  All waves add at once where they touch no cell of each other
+        // (tile3_rounds), else first those of phase 0, then those of phase 1.
         auto add = [&] {
             const int c = e - 1;
             const int dbase = __mul24(P, dps) + __mul24(Q, dqs) + __mul24(c, drs);
-#pragma unroll
-            for (int k = 0; k < 9; k++) {
+            auto step = [&](const int k) {
                 const int dQ = k % 3 - 1, dP = k / 3 - 1;
                 const bool in = own && Q + dQ >= 0 && Q + dQ < tq && P + dP >= 0 && P + dP < tp;
                 if (in) {
@@ -504,12 +484,20 @@ __device__ __forceinline__ void tile3_sweep(const Tile3Args& a, float* qs, float
                     }
                 }
                 wave_sync();
+            };
+            if (!trans) {
+                step(4);   // nothing goes past the line's own cells
+                return;
             }
+#pragma unroll
+            for (int k = 0; k < 9; k++) step(k);
         };
-        __syncthreads();   // phase 1 of the round before has added
-        if (wlive && phase == 0) add();
-        __syncthreads();
-        if (wlive && phase == 1) add();
+        __syncthreads();   // the waves of the round before have added
+        if (wlive && (phase == 0 || sch.phases == 1)) add();
+        if (sch.phases == 2) {
+            __syncthreads();
+            if (wlive && phase == 1) add();
+        }
     }
 }
 
