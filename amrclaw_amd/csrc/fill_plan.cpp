@@ -719,10 +719,19 @@ struct Planner {
 }  // namespace
 
 // whether `late`, of a later stage, touches a cell of the buffer that `early`
-// wrote: interpolation leaves out the cells its mask marks
-static bool meets(const FillPlan& P, const FillOp& early, const FillOp& late) {
-    const int i0 = std::max(early.di0, late.di0), i1 = std::min(early.di0 + early.ni, late.di0 + late.ni);
-    const int j0 = std::max(early.dj0, late.dj0), j1 = std::min(early.dj0 + early.nj, late.dj0 + late.nj);
+// wrote: interpolation leaves out the cells its mask marks, boundary conditions
+// touch the cells they set and, beside these, those they set them from
+static bool meets(const FillPlan& P, const FillOp& early, const FillOp& late, const int mthbc[4]) {
+    const int e0 = early.di0, e1 = early.di0 + early.ni, f0 = early.dj0, f1 = early.dj0 + early.nj;
+    if (late.type == FOP_BC) {
+        const int nxl = late.bc[0], ibeg = late.bc[1], nyb = late.bc[2], jbeg = late.bc[3];
+        auto low = [](int n, int m) { return m == 3 ? 2 * n : n + 1; };
+        auto high = [](int beg, int n, int m) { return m == 3 ? 2 * beg - 2 - n : beg - 2; };
+        return (nxl > 0 && e0 < low(nxl, mthbc[0])) || (ibeg > 0 && e1 > high(ibeg, late.ni, mthbc[1])) ||
+               (nyb > 0 && f0 < low(nyb, mthbc[2])) || (jbeg > 0 && f1 > high(jbeg, late.nj, mthbc[3]));
+    }
+    const int i0 = std::max(e0, late.di0), i1 = std::min(e1, late.di0 + late.ni);
+    const int j0 = std::max(f0, late.dj0), j1 = std::min(f1, late.dj0 + late.nj);
     if (i0 >= i1 || j0 >= j1) return false;
     if (late.type != FOP_INTERP) return true;
     const unsigned char* m = P.masks.data() + late.mask_off;
@@ -734,13 +743,13 @@ static bool meets(const FillPlan& P, const FillOp& early, const FillOp& late) {
 
 // Order the operations into units: those that must run one after the other
 // end up in the same unit, sorted by stage.  A scratch or arena buffer ties
-// all its operations together; so does a grid whose boundary conditions (or
-// another operation) read it, as these read what the others wrote.  In other
-// grids the ghost strips are written by operations that meet no cell of each
-// other, and a same-level copy reads interiors, which a fill does not write.
+// all its operations together; so does a grid that an operation reads as its
+// source.  In other grids the ghost strips are written by operations that mostly
+// meet no cell of each other or of the boundary conditions, and a same-level copy
+// reads interiors, which a fill does not write.
 // In a new grid the interpolation (FILVAL) leaves out the cells its mask marks,
 // those that the copies of old grids write, so these go side by side.
-static void finish_plan(FillPlan& P) {
+static void finish_plan(FillPlan& P, const int mthbc[4]) {
     const int n = (int)P.ops.size();
     std::vector<int> at_stage;   // by stage, as planned within one
     for (const FillOp& op : P.ops) {
@@ -766,7 +775,6 @@ static void finish_plan(FillPlan& P) {
     std::vector<char> tied(nb);   // buffers that tie all their operations
     for (int b = 0; b < nb; b++) tied[b] = P.bufs[b].kind != 0;
     for (const FillOp& op : P.ops) {
-        if (op.type == FOP_BC) tied[op.dst] = 1;
         if (op.type != FOP_COPY && op.type != FOP_BC) tied[op.src] = 1;
     }
     // the operation before on a tied buffer; on the others the list of those
@@ -785,7 +793,8 @@ static void finish_plan(FillPlan& P) {
             before[op.dst] = k;
             if (op.type != FOP_FILVAL)
                 for (int x = next[k]; x >= 0; x = next[x])
-                    if (P.ops[x].stage < op.stage && meets(P, P.ops[x], op)) tie(x, k);
+                    if (P.ops[x].stage < op.stage && meets(P, P.ops[x], op, mthbc))
+                        tie(x, k);
         }
         if (op.type != FOP_COPY && op.type != FOP_BC && op.src != op.dst) use(op.src);
     }
@@ -874,7 +883,7 @@ bool plan_filval(const HierGeom& H, int level, int nvar, FillPlan& P, std::strin
             err = pl.err.empty() ? "filval planning failed" : pl.err;
             return false;
         }
-    finish_plan(P);
+    finish_plan(P, H.mthbc);
     return true;
 }
 
@@ -886,7 +895,7 @@ bool plan_saveqc(const HierGeom& H, int level, int nvar, FillPlan& P, std::strin
             err = pl.err.empty() ? "saveqc planning failed" : pl.err;
             return false;
         }
-    finish_plan(P);
+    finish_plan(P, H.mthbc);
     return true;
 }
 
@@ -971,7 +980,7 @@ bool plan_richardson(const HierGeom& H, int level, int nvar, RichPlan& R, std::s
         R.crs.push_back(pc);
         R.fine.push_back(pf);
     }
-    finish_plan(P);
+    finish_plan(P, H.mthbc);
     return true;
 }
 
@@ -983,7 +992,7 @@ bool plan_fill_level(const HierGeom& H, int level, int nvar, FillPlan& P, std::s
             err = pl.err.empty() ? "ghost-fill planning failed" : pl.err;
             return false;
         }
-    finish_plan(P);
+    finish_plan(P, H.mthbc);
     return true;
 }
 
