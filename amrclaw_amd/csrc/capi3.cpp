@@ -248,10 +248,21 @@ void split_tile3(int n, int k, std::vector<std::pair<int, int>>& out) {
     }
 }
 
-// lane slots the fused kernel spends on a tile: 256 a round of its schedule
+// lane slots the fused kernel spends on a tile: 256 a round of its schedule (a
+// table: a cut of a grid is one of hundreds that are compared)
 int64_t tile3_slots(int tx, int ty, int tz) {
-    return 256ll * (tile3_rounds(tx, ty, tz).rounds + tile3_rounds(ty, tx, tz).rounds +
-                    tile3_rounds(tz, tx, ty).rounds);
+    constexpr int N = TILE3_MAX + 1;
+    static const std::vector<int32_t> table = [] {
+        std::vector<int32_t> t((size_t)N * N * N, 0);
+        for (int x = 1; x < N; x++)
+            for (int y = 1; y < N; y++)
+                for (int z = 1; z < N; z++)
+                    t[((size_t)x * N + y) * N + z] =
+                        256 * (tile3_rounds(x, y, z).rounds + tile3_rounds(y, x, z).rounds +
+                               tile3_rounds(z, x, y).rounds);
+        return t;
+    }();
+    return table[((size_t)tx * N + ty) * N + tz];
 }
 size_t tile3_bytes(int nv, int tx, int ty, int tz) {
     return (size_t)nv * ((size_t)(tx + 4) * (ty + 4) * (tz + 4) + (size_t)tx * ty * tz) *
@@ -262,11 +273,11 @@ size_t tile3_bytes(int nv, int tx, int ty, int tz) {
 // grid is cut into kx x ky x kz near-equal tiles of at most TILE3_MAX cells
 // per direction whose LDS lets two workgroups
 // share a CU; of those cuts, the one with the fewest lane slots.  With `faces`
-// (a level's marked faces per grid, each belonging to the tile of its cell, or
-// to the last tile beyond a grid's last cell) the tiles also hold the face map
-// and up to 16 KB of marks within that LDS; more marks cost occupancy only.
-void plan_tiles3(const std::vector<Patch3>& patches, int nv,
-                 const std::vector<std::vector<GridFace3>>* faces, Tile3Plan& plan) {
+// (a level's marked faces, each belonging to the tile of its cell, or to the last
+// tile beyond a grid's last cell) the tiles also hold the face map and up to 16
+// KB of marks within that LDS; more marks cost occupancy only.
+void plan_tiles3(const std::vector<Patch3>& patches, int nv, const LevelFaces3* faces,
+                 Tile3Plan& plan) {
     plan = Tile3Plan();
     std::vector<Tile3>& tiles = plan.tiles;
     size_t& lds = plan.lds;
@@ -347,7 +358,24 @@ void plan_tiles3(const std::vector<Patch3>& patches, int nv,
                 while (i + 1 < (int)s.size() && c >= s[i + 1].first) i++;
                 return i;
             };
-            for (const GridFace3& f : (*faces)[p]) {
+            for (size_t k = 0; faces->perimeter && k < per[p].size(); k++) {
+                const Tile3& t = per[p][k];
+                std::vector<Mark3>& m = per_marks[p][k];
+                const int16_t tx = t.tx, ty = t.ty, tz = t.tz;
+                for (int16_t x : {int16_t(0), tx})   // the tile's sides that are the grid's
+                    if (x == 0 ? t.i0 == 0 : t.i0 + tx == pt.mx)
+                        for (int16_t z = 0; z < tz; z++)
+                            for (int16_t y = 0; y < ty; y++) m.push_back(Mark3{x, y, z, 0});
+                for (int16_t y : {int16_t(0), ty})
+                    if (y == 0 ? t.j0 == 0 : t.j0 + ty == pt.my)
+                        for (int16_t z = 0; z < tz; z++)
+                            for (int16_t x = 0; x < tx; x++) m.push_back(Mark3{x, y, z, 1});
+                for (int16_t z : {int16_t(0), tz})
+                    if (z == 0 ? t.k0 == 0 : t.k0 + tz == pt.mz)
+                        for (int16_t y = 0; y < ty; y++)
+                            for (int16_t x = 0; x < tx; x++) m.push_back(Mark3{x, y, z, 2});
+            }
+            for (const GridFace3& f : faces->others[p]) {
                 const int i = part(sx, f.x), j = part(sy, f.y), l = part(sz, f.z);
                 per_marks[p][((size_t)l * sy.size() + j) * sx.size() + i].push_back(
                     Mark3{(int16_t)(f.x - sx[i].first), (int16_t)(f.y - sy[j].first),
@@ -506,14 +534,23 @@ hipError_t build_pass3(const std::vector<Patch3>& patches, Pass3Plan& pp) {
         for (int64_t b = 0; b < nf; b++) faces.push_back(Block3{p, (int)b, 0, 0});
     }
     close();
-    auto up = [&](auto*& d, const auto& h) {
-        hipError_t e = hipMalloc((void**)&d, std::max<size_t>(1, h.size()) * sizeof(h[0]));
-        return e != hipSuccess || h.empty() ? e : h2d3(d, h.data(), h.size() * sizeof(h[0]));
+    // the tables in one array and one copy: a Richardson estimate makes two plans
+    // for a step each
+    std::vector<char> host;
+    auto put = [&](const auto& v) {
+        const size_t at = (host.size() + 255) / 256 * 256, n = v.size() * sizeof(v[0]);
+        host.resize(at + n);
+        if (n) std::memcpy(host.data() + at, v.data(), n);
+        return at;
     };
-    hipError_t e = hipSuccess;
-    for (int d = 0; d < 3 && e == hipSuccess; d++) e = up(pp.d_waves[d], waves[d]);
-    if (e == hipSuccess) e = up(pp.d_faces, faces);
-    if (e == hipSuccess) e = up(pp.d_off, off);
+    const size_t at_wave[3] = {put(waves[0]), put(waves[1]), put(waves[2])};
+    const size_t at_face = put(faces), at_off = put(off);
+    hipError_t e = hipMalloc(&pp.d_tables, std::max<size_t>(1, host.size()));
+    if (e == hipSuccess && !host.empty()) e = h2d3(pp.d_tables, host.data(), host.size());
+    char* base = static_cast<char*>(pp.d_tables);
+    for (int d = 0; d < 3; d++) pp.d_waves[d] = reinterpret_cast<Pass3Wave*>(base + at_wave[d]);
+    pp.d_faces = reinterpret_cast<Block3*>(base + at_face);
+    pp.d_off = reinterpret_cast<Pass3Ws*>(base + at_off);
     pp.ok = e == hipSuccess;
     return e;
 }
@@ -880,8 +917,7 @@ bool ctx3_fused() { return g3.esize == 4 && g3.step_mode == 1; }
 int ctx3_step_fused(const Fused3IO& io, double dx, double dy, double dz, double dt) {
     return step_fused_io(io, dx, dy, dz, dt);
 }
-void ctx3_plan_tiles(const std::vector<Patch3>& patches,
-                     const std::vector<std::vector<GridFace3>>& faces, Tile3Plan& plan) {
+void ctx3_plan_tiles(const std::vector<Patch3>& patches, const LevelFaces3& faces, Tile3Plan& plan) {
     plan_tiles3(patches, g3.cfg.nvar, &faces, plan);
 }
 void ctx3_plan_blocks(const std::vector<Patch3>& patches, int plane_block,

@@ -236,27 +236,22 @@ int ensure_fill_plans() {
 
 // The faces of a level's grids whose fluxes the registers read: fluxad.f's
 // grid perimeters (a fine level) and fluxsv.f's entries (a coarse one).
-std::vector<std::vector<GridFace3>> register_faces(const Lev3& L, bool fine) {
-    std::vector<std::vector<GridFace3>> out(L.patches.size());
+LevelFaces3 register_faces(const Lev3& L, bool fine) {
+    LevelFaces3 out;
+    out.perimeter = fine;
+    out.others.resize(L.patches.size());
     std::vector<std::vector<bool>> seen(L.patches.size());
     auto add = [&](int g, int dir, int x, int y, int z) {
         const Patch3& p = L.patches[g];
+        const int c = dir == 0 ? x : (dir == 1 ? y : z), n = dir == 0 ? p.mx : (dir == 1 ? p.my : p.mz);
+        if (fine && (c == 0 || c == n)) return;   // on the perimeter
         auto& s = seen[g];
         if (s.empty()) s.assign((size_t)3 * (p.mx + 1) * (p.my + 1) * (p.mz + 1), false);
         const size_t at = (((size_t)dir * (p.mz + 1) + z) * (p.my + 1) + y) * (p.mx + 1) + x;
         if (s[at]) return;
         s[at] = true;
-        out[g].push_back(GridFace3{dir, x, y, z});
+        out.others[g].push_back(GridFace3{dir, x, y, z});
     };
-    for (size_t g = 0; fine && g < L.patches.size(); g++) {
-        const Patch3& p = L.patches[g];
-        for (int z = 0; z < p.mz; z++)
-            for (int y = 0; y < p.my; y++) add(g, 0, 0, y, z), add(g, 0, p.mx, y, z);
-        for (int z = 0; z < p.mz; z++)
-            for (int x = 0; x < p.mx; x++) add(g, 1, x, 0, z), add(g, 1, x, p.my, z);
-        for (int y = 0; y < p.my; y++)
-            for (int x = 0; x < p.mx; x++) add(g, 2, x, y, 0), add(g, 2, x, y, p.mz);
-    }
     for (const Sv3Entry& e : L.reg.sv) {
         if (!e.write) continue;
         // interior cell, 0-based; sides 1, 4, 5 its lower faces

@@ -23,6 +23,12 @@ struct Tile3Plan {
 struct GridFace3 {
     int dir, x, y, z;
 };
+// the marked faces of a level's grids: their perimeters, if so, and others, each
+// once
+struct LevelFaces3 {
+    bool perimeter = false;
+    std::vector<std::vector<GridFace3>> others;
+};
 // device arrays of one fused step of a level
 struct Fused3IO {
     const void* qin;              // time t, ghost cells filled
@@ -46,13 +52,12 @@ struct Pass3Plan {
     bool built = false, ok = false;   // built and not ok: the phase kernels
     std::vector<Pass3Run> runs;
     int64_t ws_elems = 0;
+    void* d_tables = nullptr;         // one allocation, these in it
     Pass3Wave* d_waves[3] = {};
     Block3* d_faces = nullptr;
     Pass3Ws* d_off = nullptr;
     void free() {
-        for (auto& w : d_waves) hipFree(w);
-        hipFree(d_faces);
-        hipFree(d_off);
+        hipFree(d_tables);
         *this = Pass3Plan();
     }
 };
@@ -87,8 +92,7 @@ int ctx3_step(const Step3IO& io, double dx, double dy, double dz, double dt, int
 // the same step by the fused FP32 kernel (ctx3_fused: FP32 and the fused mode)
 bool ctx3_fused();
 int ctx3_step_fused(const Fused3IO& io, double dx, double dy, double dz, double dt);
-void ctx3_plan_tiles(const std::vector<Patch3>& patches,
-                     const std::vector<std::vector<GridFace3>>& faces, Tile3Plan& plan);
+void ctx3_plan_tiles(const std::vector<Patch3>& patches, const LevelFaces3& faces, Tile3Plan& plan);
 // the work lists of a batch: per sweep (grid, plane block), largest first;
 // update and totals (grid, 256 cells)
 void ctx3_plan_blocks(const std::vector<Patch3>& patches, int plane_block,
