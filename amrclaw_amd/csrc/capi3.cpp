@@ -212,6 +212,25 @@ int64_t block_cost(const Patch3& pt, int d, const Block3& b) {
     return (int64_t)(b.pe - b.pb + 2) * rounds;
 }
 
+// the rounds of the three sweeps' longest workgroups, one after the other, and
+// of all of them
+struct PhaseRounds3 {
+    double chain, work;
+};
+PhaseRounds3 phase_rounds(const std::vector<Patch3>& patches, const std::vector<Block3>* blocks) {
+    PhaseRounds3 r{0, 0};
+    for (int d = 0; d < 3; d++) {
+        int64_t longest = 0;
+        for (const Block3& b : blocks[d]) {
+            const int64_t c = block_cost(patches[b.patch], d, b);
+            longest = std::max(longest, c);
+            r.work += c;
+        }
+        r.chain += longest;
+    }
+    return r;
+}
+
 // the batch's work lists: per sweep, (patch, plane block) in decreasing
 // cost, so that the longest workgroups start first; update, (patch, 256
 // cells)
@@ -418,6 +437,28 @@ void plan_tiles3(const std::vector<Patch3>& patches, int nv, const LevelFaces3* 
     }
 }
 
+// Whether a level's FP32 step is better off fused.  The Euler solver's is (its
+// phase kernels solve each interface several times).  The advection solver's
+// takes the rounds of its largest tile, two tiles at work on a CU, and its phase
+// kernels theirs: us a level step, phases / fused, method(3) = 22, one grid of 12^3
+// 81 / 137 (one tile), of 14^3 86 / 139, of 8^3 76 / 77, of 16^3 118 / 89 (tiles
+// of 8^3), of 22^3 125 / 105, of 46^3 396 / 197, 27 of 12^3 105 / 146; method(3) =
+// 0, 12^3 63 / 84, 8^3 65 / 56, 30^3 96 / 103, 46^3 152 / 118.
+bool fused_pays(const std::vector<Patch3>& patches, const std::vector<Block3>* blocks,
+                const Tile3Plan& plan) {
+    if (g3.cfg.solver != SOLVER_ADVECTION) return true;
+    int64_t slots = 0;
+    for (const Tile3& t : plan.tiles) slots = std::max(slots, tile3_slots(t.tx, t.ty, t.tz));
+    const PhaseRounds3 r = phase_rounds(patches, blocks);
+    const Method3& M = g3.meth;
+    const double full = std::max(1.0, plan.tiles.size() / (256.0 * TILE3_WG_PER_CU));
+    const bool standard = std_method3<Advection3<float, FastMathF32>>(M);
+    const double fused = M.m3 > 0 ? 42.0 + (standard ? 2.35 : 2.75) * full * (slots / 256)
+                                  : 32.0 + 1.3 * full * (slots / 256);
+    const double phases = 60.0 + (M.m3 > 0 ? 2.9 : 0.85) * std::max(r.chain, r.work / 768.0);
+    return fused < phases;
+}
+
 int alloc_batch(int npatch, const int* mx, const int* my, const int* mz) {
     const int nv = g3.cfg.nvar;
     g3.patches.resize(npatch);
@@ -578,21 +619,12 @@ hipError_t pass3_ws(const Pass3Plan& pp) {
 // 225 / 173, 2 of 60^3 357 / 118, 64 of 40^3 322 / 755, 512 of 16^3 208 / 222.
 bool pass3_pays(const Step3IO& io) {
     if (g3.cfg.solver != SOLVER_ADVECTION) return true;
-    int64_t chain = 0, work = 0;
-    for (int d = 0; d < 3; d++) {
-        int64_t longest = 0;
-        for (const Block3& b : io.blocks[d]) {
-            const int64_t c = block_cost((*io.patches)[b.patch], d, b);
-            longest = std::max(longest, c);
-            work += c;
-        }
-        chain += longest;
-    }
+    const PhaseRounds3 r = phase_rounds(*io.patches, io.blocks);
     int64_t cells = 0;
     for (const Patch3& p : *io.patches) cells += (int64_t)p.mx * p.my * p.mz;
     const Method3& M = g3.meth;
     const double round = M.m4 > 0 ? 4.9 : (M.m3 > 0 ? 3.7 : (M.order > 1 ? 1.25 : 0.85));
-    const double phases = 30.0 + round * std::max((double)chain, work / 640.0);
+    const double phases = 30.0 + round * std::max(r.chain, r.work / 640.0);
     const double passes = 40.0 + (M.m3 > 0 ? 3.3e-4 : 1.7e-4) * cells;
     return passes < phases;
 }
@@ -919,6 +951,10 @@ int ctx3_step_fused(const Fused3IO& io, double dx, double dy, double dz, double 
 }
 void ctx3_plan_tiles(const std::vector<Patch3>& patches, const LevelFaces3& faces, Tile3Plan& plan) {
     plan_tiles3(patches, g3.cfg.nvar, &faces, plan);
+}
+bool ctx3_fused_pays(const std::vector<Patch3>& patches, const std::vector<Block3>* blocks,
+                     const Tile3Plan& plan) {
+    return fused_pays(patches, blocks, plan);
 }
 void ctx3_plan_blocks(const std::vector<Patch3>& patches, int plane_block,
                       std::vector<Block3> out[4]) {

@@ -269,13 +269,14 @@ LevelFaces3 register_faces(const Lev3& L, bool fine) {
 }
 
 // The fused step of a level; where a tile's marks or the card have no room for
-// it, the level takes the phase kernels.
+// it, or it does not pay, the level takes the phase kernels.
 int plan_fused(int level) {
     Lev3& L = A.lev[level];
     L.fused = false;
     if (ctx3_esize() != 4 || L.patches.empty()) return AMRGPU_OK;
     ctx3_plan_tiles(L.patches, register_faces(L, level >= 2), L.tiles);
     if (L.tiles.lds > 160 * 1024) return AMRGPU_OK;   // too many marks in a tile
+    if (!ctx3_fused_pays(L.patches, L.blocks, L.tiles)) return AMRGPU_OK;
     dfree(L.d_tiles);
     dfree(L.d_marks);
     auto up = [](auto*& d, const auto& h) {

@@ -93,6 +93,9 @@ int ctx3_step(const Step3IO& io, double dx, double dy, double dz, double dt, int
 bool ctx3_fused();
 int ctx3_step_fused(const Fused3IO& io, double dx, double dy, double dz, double dt);
 void ctx3_plan_tiles(const std::vector<Patch3>& patches, const LevelFaces3& faces, Tile3Plan& plan);
+// whether a level's step is better off fused than by its blocks' phase kernels
+bool ctx3_fused_pays(const std::vector<Patch3>& patches, const std::vector<Block3>* blocks,
+                     const Tile3Plan& plan);
 // the work lists of a batch: per sweep (grid, plane block), largest first;
 // update and totals (grid, 256 cells)
 void ctx3_plan_blocks(const std::vector<Patch3>& patches, int plane_block,

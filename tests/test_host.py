@@ -313,3 +313,28 @@ def child_advection_route(fake, sizes, transverse, passes):
         assert bool(fake.launches("pass3_solve")) == want, solver
         assert bool(fake.launches("sweep3_phase")) == (not want), solver
         capi3.finalize3()
+
+
+@pytest.mark.parametrize("n,transverse,fused", [(8, 22, True), (12, 22, False), (14, 11, False),
+                                                (16, 22, True), (46, 22, True), (12, 0, False),
+                                                (8, 0, True), (46, 0, True)])
+def test_route_of_fp32_advection_levels(n, transverse, fused):
+    """A level's fused step where it is the faster one: not for the advection
+    solver on few grids that make one large tile each."""
+    run("child_advection_levels", n, transverse, fused)
+
+
+def child_advection_levels(fake, n, transverse, fused):
+    from amrclaw_amd import capi, capi3
+    from amrclaw_amd.hierarchy import Hier3
+    for solver, nvar, want in ((capi.ADVECTION, 1, fused), (capi.EULER, 5, True)):
+        H = Hier3(nvar)
+        H.add_level([(0, n - 1) * 3], (1 / n,) * 3, 0.1 / n, 0.0, (n, n, n))
+        H.add_level([(4, 11) * 3], (0.5 / n,) * 3, 0.05 / n, 0.0, (2 * n, 2 * n, 2 * n))
+        capi3.init3(capi3.make_config3(solver, precision=capi.FP32, transverse=transverse))
+        capi3.load_hierarchy3(H)
+        fake.clear()
+        capi3.advance_level3(1)
+        assert bool(fake.launches("sweep3_tile")) == want, solver
+        assert bool(fake.launches("sweep3_phase")) == (not want), solver
+        capi3.finalize3()
