@@ -130,30 +130,104 @@ def test_level_update3_ratio_mix_fp64_bit_exact(gpu):
         capi3.finalize3()
 
 
-@pytest.mark.parametrize("case", BCS[:1] + BCS[3:])
-def test_level_update3_fp32(gpu, case):
-    print("amr3 fp32", case, flush=True)
-    H = _hier(orc.EULER, case, 0)
+class AlternatingAMR3(capi3.DeviceAMR3):
+    """The device's level update, its level steps by the phase kernels and the
+    fused kernel in turn."""
+    steps = 0
+
+    def advanc(self, level):
+        capi3.set_step_mode3((capi3.STEP_PHASES, capi3.STEP_FUSED)[self.steps % 2])
+        self.steps += 1
+        return super().advanc(level)
+
+
+def _hier32(case, seed):
+    H = _hier(orc.EULER, case, seed)
     for L in H.levels:
         L["qnew"][:] = L["qnew"].astype(np.float32)
         L["qold"][:] = L["qold"].astype(np.float32)
+    return H
+
+
+@pytest.mark.parametrize("mode", [capi3.STEP_FUSED, capi3.STEP_PHASES, None])
+@pytest.mark.parametrize("case", BCS[:1] + BCS[3:])
+def test_level_update3_fp32(gpu, case, mode):
+    """Either step mode, and the two in turn (None; the fused step swaps the
+    buffers that the phase kernels copy and update in place): new values with
+    their ghost cells and the old time of every level that keeps it."""
+    print("amr3 fp32", case, mode, flush=True)
+    H = _hier32(case, 0)
     p = orc.make_params3(orc.EULER)
     O = orc.OracleAMR3(p, H.copy())
     _init(orc.EULER, capi3.FP32)
     try:
-        D = capi3.DeviceAMR3(H)
+        D = AlternatingAMR3(H) if mode is None else capi3.DeviceAMR3(H)
+        if mode is not None:
+            capi3.set_step_mode3(mode)
         lo, ld = [], []
         for _ in range(2):
             berger_oliger3(O, O.H, 1, lo)
             berger_oliger3(D, H, 1, ld)
         for l in range(1, H.nlev + 1):
-            got = capi3.read_level3(H, l, 0)
-            want = O.H.levels[l - 1]["qnew"]
-            assert rel_l1(got, want) <= 1e-5, (l, rel_l1(got, want))
+            for which, name in ((0, "qnew"), (1, "qold"))[:2 if l < H.nlev else 1]:
+                got = capi3.read_level3(H, l, which)
+                want = O.H.levels[l - 1][name]
+                assert rel_l1(got, want) <= 1e-5, (l, name, rel_l1(got, want))
         for (la, (_, ca)), (lb, (_, cb)) in zip(lo, ld):
             assert la == lb and abs(ca - cb) <= 1e-5 * max(ca, 1e-30)
     finally:
         capi3.finalize3()
+
+
+@pytest.mark.parametrize("case", BCS[:1] + BCS[3:])
+def test_fused_level_step_registers(gpu, case):
+    """What a fused level step leaves in the registers, from the faces marked in
+    its tiles, against the phase kernels' flux arrays.  A face sums 13 increments
+    (its own and six of either other sweep), each formed by some 30 FP32
+    operations, in another order in either kernel: 43 roundings of 2^-24 of the
+    sum of their sizes, here taken as four times the largest flux; a slot holds up
+    to 1 + 2 x 4 faces' (fluxsv, then fluxad of two fine steps)."""
+    print("amr3 fused registers", case, flush=True)
+    H = _hier32(case, 3)
+    got = {}
+    for mode in (capi3.STEP_PHASES, capi3.STEP_FUSED):
+        _init(orc.EULER, capi3.FP32)
+        try:
+            capi3.set_step_mode3(mode)
+            D = capi3.DeviceAMR3(H)
+            regs = []
+            for steps in ((1,), (2, 2)):      # fluxsv alone, then with fluxad's sums
+                for l in steps:
+                    D.advanc(l)
+                regs.append([capi3.get_registers3(2, k, 5)[0]
+                             for k in range(len(H.levels[1]["boxes"]))])
+            got[mode] = regs
+        finally:
+            capi3.finalize3()
+    scale = max(np.abs(r).max() for r in got[capi3.STEP_PHASES][0])
+    assert scale > 0
+    for part, faces in ((0, 1), (1, 9)):
+        for a, b in zip(got[capi3.STEP_PHASES][part], got[capi3.STEP_FUSED][part]):
+            assert np.abs(a - b).max() <= faces * 43 * 2.0 ** -24 * 4 * scale, part
+
+
+def test_fused_level_steps_are_deterministic(gpu):
+    """Level steps with marked faces, all levels, twice from the same state:
+    solutions and registers bit for bit."""
+    H = _hier32(BCS[3], 4)
+    out = []
+    for _ in range(2):
+        _init(orc.EULER, capi3.FP32)
+        try:
+            D = capi3.DeviceAMR3(H)
+            berger_oliger3(D, H, 1)
+            out.append([capi3.read_level3(H, l) for l in range(1, H.nlev + 1)] +
+                       [capi3.get_registers3(l, k, 5)[0] for l in range(2, H.nlev + 1)
+                        for k in range(len(H.levels[l - 1]["boxes"]))])
+        finally:
+            capi3.finalize3()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
 
 
 @pytest.mark.parametrize("solver", [orc.EULER, orc.ADVECTION])

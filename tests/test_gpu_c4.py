@@ -71,8 +71,11 @@ def _mass(H, q, l):
     return tot * L["hx"] * L["hy"]
 
 
-@pytest.mark.parametrize("launch", [None, capi.LAUNCH_PER_PATCH, capi.LAUNCH_MARCH])
+@pytest.mark.parametrize("launch", [None, capi.LAUNCH_PER_PATCH, capi.LAUNCH_PERSISTENT,
+                                    capi.LAUNCH_MARCH])
 def test_c4_fp64_bit_exact(c4, launch):
+    """The default launch marches here; the persistent one runs the tile sweep
+    with its registers."""
     H, O, olog = c4
     print("c4 fp64", launch, flush=True)
     try:
@@ -80,7 +83,7 @@ def test_c4_fp64_bit_exact(c4, launch):
         assert dlog == olog, (dlog, olog)
         for l in (1, 2):
             assert np.array_equal(capi.read_level(H, l, 0), O.H.levels[l - 1]["qnew"]), l
-        if launch is None:
+        if launch in (None, capi.LAUNCH_PERSISTENT):
             for k in range(0, NPATCH, 97):
                 sv, qc = capi.get_registers(2, k, 4, 4096)
                 ref = O.reg(2, k).reshape(2, -1, 4)

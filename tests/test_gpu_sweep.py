@@ -236,16 +236,20 @@ def test_mixed_occupancy_bounds_agree(gpu):
         capi.finalize()
 
 
+SMALL_TILE_SIZES = [(12, 12), (13, 13), (28, 12), (29, 25), (1, 40), (40, 1), (11, 30), (61, 37),
+                    (16, 12)]
+
+
 @pytest.mark.parametrize("solver", ["acoustics", "euler"])
-@pytest.mark.parametrize("ngrids", [9, 120])
+@pytest.mark.parametrize("ngrids", [9, 135])
 def test_small_tiles_bit_exact(gpu, solver, ngrids):
     """Levels of few grids are cut into smaller tiles in the batched launch (9
-    grids) and as the caps say beyond that (120); the persistent launch always
-    takes the caps: the same FP64 bits and Courant number."""
+    grids) and as the caps say beyond that (135; which grids are cut how is
+    checked in test_host.py); the persistent launch always takes the caps: the
+    same FP64 bits and Courant number."""
     sid = SOLVERS[solver]
     rng = np.random.default_rng(ngrids)
-    sizes = [(12, 12), (13, 13), (28, 12), (29, 25), (1, 40), (40, 1), (11, 30), (61, 37), (16, 12)]
-    sizes = [sizes[k % len(sizes)] for k in range(ngrids)]
+    sizes = [SMALL_TILE_SIZES[k % len(SMALL_TILE_SIZES)] for k in range(ngrids)]
     boxes, x = [], 0
     for mx, my in sizes:
         boxes.append((x, x + mx - 1, 0, my - 1))

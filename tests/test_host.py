@@ -338,3 +338,61 @@ def child_advection_levels(fake, n, transverse, fused):
         assert bool(fake.launches("sweep3_tile")) == want, solver
         assert bool(fake.launches("sweep3_phase")) == (not want), solver
         capi3.finalize3()
+
+
+@pytest.mark.parametrize("solver", ["acoustics", "euler"])
+@pytest.mark.parametrize("ngrids,small", [(9, True), (135, False)])
+def test_cut_of_few_grids(solver, ngrids, small):
+    """The levels of test_gpu_sweep.py::test_small_tiles_bit_exact: cut into 12x12
+    tiles at most, or by the library's caps, and swept by tiles either way."""
+    run("child_cut", solver, ngrids, small)
+
+
+def child_cut(fake, solver, ngrids, small):
+    from amrclaw_amd import capi
+    from tests.common import SOLVERS
+    from tests.test_gpu_sweep import SMALL_TILE_SIZES
+    sizes = [SMALL_TILE_SIZES[k % len(SMALL_TILE_SIZES)] for k in range(ngrids)]
+    boxes, x = [], 0
+    for mx, my in sizes:
+        boxes.append((x, x + mx - 1, 0, my - 1))
+        x += mx
+    n = {}
+    for mode in (capi.LAUNCH_BATCHED, capi.LAUNCH_PERSISTENT):
+        capi.init(capi.make_config(SOLVERS[solver]))
+        capi.set_launch_mode(mode)
+        capi.set_level(1, boxes, 1 / 64, 1 / 48)
+        fake.clear()
+        capi.sweep_level(1, 0.002)
+        assert not fake.launches("sweep_march")
+        (launch,) = fake.launches("sweep_kernel") or fake.launches("sweep_persist")
+        n[mode] = launch[1]
+        capi.finalize()
+    cut = lambda size, cap: -(-size // cap)
+    twelve = sum(cut(mx, 12) * cut(my, 12) for mx, my in sizes)
+    caps = sum(cut(mx, 28) * cut(my, 12) for mx, my in sizes)
+    assert caps < twelve and n[capi.LAUNCH_BATCHED] == (twelve if small else caps)
+
+
+@pytest.mark.parametrize("solver,precision,grids,marches", [
+    ("euler", "FP64", [(100, 100)] * 60, True), ("euler", "FP64", [(30, 30)] * 20, False),
+    ("euler", "MIXED", [(100, 100)] * 60, False), ("euler", "FP32", [(100, 100)] * 60, False),
+    ("acoustics", "FP64", [(100, 100)] * 60, False)])
+def test_sweep_of_the_default_launch(solver, precision, grids, marches):
+    run("child_default_sweep", solver, precision, grids, marches)
+
+
+def child_default_sweep(fake, solver, precision, grids, marches):
+    from amrclaw_amd import capi
+    from tests.common import SOLVERS
+    boxes, x = [], 0
+    for mx, my in grids:
+        boxes.append((x, x + mx - 1, 0, my - 1))
+        x += mx
+    capi.init(capi.make_config(SOLVERS[solver], precision=getattr(capi, precision)))
+    capi.set_level(1, boxes, 0.01, 0.01)
+    fake.clear()
+    capi.sweep_level(1, 1e-3)
+    assert bool(fake.launches("sweep_march")) == marches
+    assert bool(fake.launches("sweep_kernel")) == (not marches)
+    capi.finalize()
