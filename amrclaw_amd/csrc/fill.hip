@@ -147,30 +147,31 @@ __device__ __forceinline__ void interp_cell(const BufRef<S>& crs, const BufRef<S
     }
 }
 
-// one side of bc2amr: the cells [i0, i0 + ni) x [j0, j0 + nj) from the cells
-// `from` maps them to (none of them on this side), component `flip` negated;
-// components m0 .. m0 + C - 1 of B cells a thread in flight.  By cells, so that
+// One side of bc2amr: the cells [i0, i0 + ni) x [j0, j0 + nj), none of which is
+// read, from the cells (ai i + bi, aj j + bj), component `flip` negated.
+struct BcSide { int ni, nj, i0, j0, ai, bi, aj, bj, flip; };
+
+// Components m0 .. m0 + C - 1 of B cells a thread in flight.  By cells, so that
 // the digits are stepped once a cell: the four sides of a 1024^2 grid of four
 // components take a ghost fill of 32 us, element by element 52.
-template <int NT, int C, int B, typename S, class From>
-__device__ __forceinline__ void bc_cells(const BufRef<S>& b, int tid, int m0, int ni, int nj, int i0,
-                                         int j0, int flip, const From& from) {
-    const int n = ni * nj;
-    Digits2<NT> u(tid, ni, 1 << 30);   // (i, j) of a cell; j does not wrap
+template <int NT, int C, int B, typename S>
+__device__ __forceinline__ void bc_cells(const BufRef<S>& b, const BcSide& sd, int tid, int m0) {
+    const int n = sd.ni * sd.nj;
+    Digits2<NT> u(tid, sd.ni, 1 << 30);   // (i, j) of a cell; j does not wrap
     for (int t = tid; t < n; t += B * NT) {
         double v[B][C];
         int64_t d[B];
 #pragma unroll
         for (int k = 0; k < B; k++, u.step()) {
-            int i = i0 + u.i, j = j0 + u.j;
+            const int i = sd.i0 + u.i, j = sd.j0 + u.j;
             d[k] = t + NT * k < n ? (int64_t)m0 * b.plane + (int64_t)j * b.nrow + i : -1;
             if (d[k] >= 0) {
-                from(i, j);
-                const int64_t s = (int64_t)m0 * b.plane + (int64_t)j * b.nrow + i;
+                const int64_t s = (int64_t)m0 * b.plane + (int64_t)(sd.aj * j + sd.bj) * b.nrow +
+                                  (sd.ai * i + sd.bi);
 #pragma unroll
                 for (int m = 0; m < C; m++) {
                     v[k][m] = b.at(s + (int64_t)m * b.plane);
-                    if (m0 + m == flip) v[k][m] = -v[k][m];
+                    if (m0 + m == sd.flip) v[k][m] = -v[k][m];
                 }
             }
         }
@@ -182,14 +183,13 @@ __device__ __forceinline__ void bc_cells(const BufRef<S>& b, int tid, int m0, in
             }
     }
 }
-template <int NT, typename S, class From>
-__device__ __forceinline__ void bc_side(const BufRef<S>& b, int tid, int nv, int ni, int nj, int i0,
-                                        int j0, int flip, const From& from) {
+template <int NT, typename S>
+__device__ __forceinline__ void bc_side(const BufRef<S>& b, const BcSide& sd, int tid, int nv) {
     int m = 0;
-    for (; m + 4 <= nv; m += 4) bc_cells<NT, 4, 2>(b, tid, m, ni, nj, i0, j0, flip, from);
-    if (nv - m == 3) bc_cells<NT, 3, 3>(b, tid, m, ni, nj, i0, j0, flip, from);
-    else if (nv - m == 2) bc_cells<NT, 2, 4>(b, tid, m, ni, nj, i0, j0, flip, from);
-    else if (nv - m == 1) bc_cells<NT, 1, 8>(b, tid, m, ni, nj, i0, j0, flip, from);
+    for (; m + 4 <= nv; m += 4) bc_cells<NT, 4, 2>(b, sd, tid, m);
+    if (nv - m == 3) bc_cells<NT, 3, 3>(b, sd, tid, m);
+    else if (nv - m == 2) bc_cells<NT, 2, 4>(b, sd, tid, m);
+    else if (nv - m == 1) bc_cells<NT, 1, 8>(b, sd, tid, m);
 }
 
 constexpr int FILL_CHUNK = 8;   // items read at a time
@@ -306,32 +306,24 @@ __device__ __forceinline__ void fill_op(const FillArgs& a, const FillProg& pr, c
         }
     } else if (op.type == FOP_BC) {
         // sides in the reference's order, each complete before the next:
-        // extrapolation (1) or mirrored (wall, 3)
+        // extrapolation (1) or mirrored (wall, 3).  One loop over the sides, not
+        // four copies of its body: the FP32 kernel would keep its arguments in
+        // scratch (1.2 KB a lane, six times the time).
         const int nrow = op.ni, ncol = op.nj;
-        const int nxl = op.bc[0], nyb = op.bc[2];
-        const int ibeg = op.bc[1], jbeg = op.bc[3];   // 1-based first column / row set
-        if (nxl > 0 && (a.mthbc[0] == 1 || a.mthbc[0] == 3)) {
-            const bool wall = a.mthbc[0] == 3;
-            bc_side<NT>(dst, tid, nv, nxl, ncol, 0, 0, wall ? 1 : -1,
-                        [=](int& i, int&) { i = wall ? 2 * nxl - 1 - i : nxl; });
-        }
-        __syncthreads();
-        if (ibeg > 0 && (a.mthbc[1] == 1 || a.mthbc[1] == 3)) {
-            const bool wall = a.mthbc[1] == 3;
-            bc_side<NT>(dst, tid, nv, nrow - ibeg + 1, ncol, ibeg - 1, 0, wall ? 1 : -1,
-                        [=](int& i, int&) { i = wall ? 2 * ibeg - 3 - i : ibeg - 2; });
-        }
-        __syncthreads();
-        if (nyb > 0 && (a.mthbc[2] == 1 || a.mthbc[2] == 3)) {
-            const bool wall = a.mthbc[2] == 3;
-            bc_side<NT>(dst, tid, nv, nrow, nyb, 0, 0, wall ? 2 : -1,
-                        [=](int&, int& j) { j = wall ? 2 * nyb - 1 - j : nyb; });
-        }
-        __syncthreads();
-        if (jbeg > 0 && (a.mthbc[3] == 1 || a.mthbc[3] == 3)) {
-            const bool wall = a.mthbc[3] == 3;
-            bc_side<NT>(dst, tid, nv, nrow, ncol - jbeg + 1, 0, jbeg - 1, wall ? 2 : -1,
-                        [=](int&, int& j) { j = wall ? 2 * jbeg - 3 - j : jbeg - 2; });
+#pragma unroll 1
+        for (int side = 0; side < 4; side++) {
+            if (side > 0) __syncthreads();
+            // cells on a low side, the 1-based first column / row of a high one
+            const int w = side == 0 ? op.bc[0] : (side == 1 ? op.bc[1] : (side == 2 ? op.bc[2] : op.bc[3]));
+            const int kind = a.mthbc[side];
+            if (w <= 0 || (kind != 1 && kind != 3)) continue;
+            const bool high = side & 1, y = side >= 2, wall = kind == 3;
+            const int n = high ? (y ? ncol : nrow) - w + 1 : w, from = high ? w - 1 : 0;
+            const int mul = wall ? -1 : 0;
+            const int add = wall ? (high ? 2 * w - 3 : 2 * w - 1) : (high ? w - 2 : w);
+            BcSide sd{n, ncol, from, 0, mul, add, 1, 0, wall ? 1 : -1};
+            if (y) sd = BcSide{nrow, n, 0, from, 1, 0, mul, add, wall ? 2 : -1};
+            bc_side<NT>(dst, sd, tid, nv);
         }
     }
 }

@@ -21,16 +21,17 @@
 //     (3-D):150-173 with fm = fp = F for the transverse increments of
 //     step3.f:221-250, 279-310), the normal fluxes as
 //     q(c) -= dt/h (faddm(c+1) - faddp(c));
-//   * four waves solve at once, any lines, and add in two phases whose waves
-//     touch no cell of each other, the lanes of a wave in ordered steps
-//     (tile3_rounds, tile3_sweep): no atomics on dq, the sums are formed in a
-//     fixed order and the result is deterministic.
+//   * four waves solve at once, any lines, and those that add at the same time
+//     touch no cell of each other (all four, or in small tiles two after the
+//     other two), the lanes of a wave in ordered steps (tile3_rounds,
+//     tile3_sweep): no atomics on dq, the sums are formed in a fixed order and
+//     the result is deterministic.
 // The per-interface arithmetic (rpn3, limiter, cqxx, the rpt3 / rptt3
 // splits and their 1/2, 1/6 weights, flux3.f:220-628) is that of the phase
 // kernel; only the order in which each cell's increments are summed differs
 // from the reference, so the result agrees with it to FP32 rounding.  The
-// grid's ghost cells are read, never written: the step reads q from one
-// buffer and writes the updated interiors into another.
+// step reads q from one buffer and writes the updated interiors into another,
+// whose ghost cells a batch keeps equal to the first's and a level's step copies.
 //
 // Bound by vector issue (the SIMDs issue vector instructions in about 80 % of
 // their cycles at 4 cycles each), so what counts is instructions per
@@ -72,7 +73,7 @@ struct Mark3 {
 
 struct Tile3Args {
     const void* qin;                // solutions at time t (grid layout of Patch3)
-    void* qout;                     // interiors at t + dt (ghost cells untouched)
+    void* qout;                     // interiors at t + dt (ghost cells: see marks)
     const Patch3* patches;
     const Tile3* tiles;
     int32_t ntiles;
@@ -83,9 +84,10 @@ struct Tile3Args {
     double dtd[3];                  // dt/dx, dt/dy, dt/dz
     Method3 meth;
     unsigned long long* cfl_patch;  // per-patch max Courant number (double bits)
-    // a level's step (null for a batch): the marked faces and the level's flux
-    // blocks, of which only those faces are written (merged form, as the phase
-    // kernels leave them); the ghost cells of qout receive qin's
+    // a level's step (face null for a batch): the marked faces and the level's
+    // flux blocks, of which only those faces are written (merged form, as the
+    // phase kernels leave them); the ghost cells of qout receive qin's (a batch's
+    // stay as they are)
     const Mark3* marks;
     float* face;
 };

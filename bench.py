@@ -134,7 +134,7 @@ def parse():
     ap.add_argument("--step3", choices=["fused", "phases"], default="fused",
                     help="3-D FP32 step: fused (one kernel per tile, faces on chip; the "
                          "library's FP32 default) or phases (x, y, z sweep kernels with the "
-                         "flux arrays in HBM, then the update); FP64 always runs phases")
+                         "flux arrays in HBM, then the update); FP64 has its own two passes")
     ap.add_argument("--copy-calibration", type=int, default=0, metavar="MIB",
                     help="only run a plain device-to-device copy of MIB MiB "
                          "(reference kernel for scaling FETCH_SIZE/WRITE_SIZE)")

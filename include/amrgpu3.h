@@ -78,8 +78,11 @@ int amrgpu3_step_patches(double dx, double dy, double dz, double dt, double* cfl
  * direction, every face kept on chip and each face value added straight to
  * the two cells it separates; the same interface arithmetic, summed in
  * another order (agrees with mode 0 to FP32 rounding); no flux arrays (a
- * level's step keeps the faces its registers read).  FP64
- * runs mode 0 only (bit for bit the reference). No reference counterpart. */
+ * level's step keeps the faces its registers read; a level whose phase kernels
+ * are faster, or for which the card has no room, takes them in this mode too).
+ * FP64 runs mode 0 only, in the reference's order bit for bit: by the phase
+ * kernels, or in two passes over a work space of at most 4 GB, which is kept
+ * until amrgpu3_finalize. No reference counterpart. */
 int amrgpu3_set_step_mode(int mode);
 
 /* The six flux arrays of the last step of one grid, in stepgrid's shape
