@@ -550,18 +550,17 @@ std::vector<MarchWave> march_waves(const Level& L, int cap) {
 // (the halo re-solved).  With the chip full the level's rows are bound by
 // vector issue instead.
 //   FP32 arithmetic, two waves per SIMD: 3.05 us a row alone, 1.37 times the
-//   lone wave's rate per resident wave when full; the two bounds blended by
-//   their cubes follow the measured times of 24 .. 4096 uneven grids within
-//   15 % and pick a cap within 12 % of the best.  Mixed Euler level, mx, my
-//   even U[8,128], sweep uncut / cut: 24 grids 404 / 29 us (4 rows), 256 430
-//   / 85 us (12 .. 16 rows), 1024 445 / 260 us (32 rows), 4096 843 / 849 us
-//   (96 rows).
+//   lone wave's rate per resident wave when full, the two bounds blended by
+//   their cubes.
 //   FP64, one wave per SIMD: 4.9 us a row, and waves beyond the SIMDs wait
-//   for a whole march: the rows of a full chip plus half a march (24 .. 2048
-//   grids within 20 %): 256 grids 811 us uncut, 215 cut, 2048 1316 / 1238.
-// (These were measured at one build; with the cells' shared quantities and the
-// sums by strength the cut marches take: mixed 24 grids 26 us, 256 81, 1024
-// 232, 4096 755; FP64 256 grids 207 us, 2048 1071.)
+//   for a whole march: the rows of a full chip plus half a march.
+// The absolute times are those of an earlier form of the solvers (today's are
+// 10 to 15 % shorter throughout); what they are for is the choice, and that
+// was measured against every cap.  A step of mx, my even U[8,128], the cap
+// chosen / the best cap, us: mixed 24 grids 38.7 / 38.7 (4 rows), 256 100 / 89,
+// 1024 264 / 253, 4096 834 / 833; FP64 24 grids 54.9 / 54.7, 100 104 / 104, 256
+// 217 / 204, 512 330 / 328, 2048 1214 / 1169: within 13 % (mixed) and 6 %
+// (FP64) of the best.
 std::vector<MarchWave> plan_march(const Level& L, double* cost_out = nullptr) {
     const bool f64 = run_precision() == 0;
     constexpr double SIMDS = 1024;   // 256 CUs x 4

@@ -22,7 +22,8 @@
 // 1.75 TB/s (a large copy on this card writes 2.4 TB/s) and read it back at 2.8
 // TB/s.  Measured against the phase kernels, FP64 Euler, method(3) = 22, a step:
 // one grid of 21x18x13 1,140 -> 88 us, 32 grids 2,147 -> 649 us, 128 3,443 ->
-// 2,084 us, 512 12.35 -> 7.65 ms.
+// 2,084 us, 512 12.35 -> 7.65 ms; with one Courant atomic a workgroup and grid
+// instead of one a wave, 512 6.9 ms, 8 grids of 40^3 1,050 -> 900 us.
 #pragma once
 #include "lanes.hpp"
 #include "sweep3.hpp"

@@ -42,7 +42,9 @@
 // (2,023,768 cells) from 984 to 700 us a step.  Full chunks from any rows, added
 // in two phases, instead of waves of one row each in three classes of rows: 700
 // -> 680 us, 6 grids 141 -> 134, the levels of a 64^3 run (tiles of 8 .. 11
-// cells) 11.7 -> 10.2 ms.
+// cells) 11.7 -> 10.2 ms.  One phase instead of two in the sweeps whose waves lie
+// far enough apart: 512 grids of 16 .. 32 cells 1.31 -> 1.18 ms, 8 grids of 40^3
+// 260 -> 234 us.
 #pragma once
 #include <cstdint>
 #include "lanes.hpp"

@@ -55,7 +55,7 @@ MEASURED_TRAFFIC = {
                                            "profiles/level_update_euler_fp32_4096.md"),
     ("euler2d", "mixed", 4096, "march"): (413374 * 2048 + 782991 * 1024,
                                           "profiles/level_update_euler_mixed_4096_march.md"),
-    ("euler3d", "fp32", 512, "fused"): (69493 * 2048 + 96823 * 1024,
+    ("euler3d", "fp32", 512, "fused"): (69501 * 2048 + 96812 * 1024,
                                         "profiles/step3_euler_fp32_512_fused.md"),
     ("euler3d", "fp32", 512, "phases"): (
         (271400 + 875200 + 1415000 + 330700) * 2048 + (801800 + 1136000 + 1143000 + 98580) * 1024,
@@ -68,7 +68,7 @@ MEASURED_VALU = {
                                           "profiles/level_update_euler_mixed_4096_march.md"),
     ("euler2d", "mixed", 4096, "batched"): (684756659,
                                             "profiles/level_update_euler_mixed_4096.md"),
-    ("euler3d", "fp32", 512, "fused"): (575255843, "profiles/step3_euler_fp32_512_fused.md"),
+    ("euler3d", "fp32", 512, "fused"): (575447124, "profiles/step3_euler_fp32_512_fused.md"),
 }
 SIMD_COUNT = 1024                 # 256 CUs x 4 SIMDs
 CLOCK_HZ = 2.4e9                  # peak engine clock

@@ -408,7 +408,9 @@ int amrgpu_get_gauge_records(int maxrec, int* nrec, int* gauge, int* level, doub
  * arithmetic bit for bit, as the library's own FP64 units do.
  *
  * The function pointers take the library's launch-argument blocks as
- * opaque pointers and return a hipError_t value (0 = success).  The table
+ * opaque pointers and return a hipError_t value (0 = success).  `qad` owes the
+ * register sums only: the copy of the Courant maxima that the library's own qad
+ * kernel makes on the way is made apart for a plug-in's levels.  The table
  * records the sizes of those blocks as its translation unit saw them; the
  * library refuses a table built against other headers. */
 #define AMRGPU_SOLVER_ABI 2
