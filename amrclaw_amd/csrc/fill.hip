@@ -7,28 +7,37 @@
 
 namespace amrgpu {
 
-template <typename S>
-struct BufRef {
-    S* lvl;          // a level's storage
-    double* scr;     // FP64 scratch or arena
+// the values of a buffer: a level's storage, or FP64 scratch or arena
+template <typename E>
+struct Cells {
+    E* p;
     int32_t nrow, plane;
     __device__ double load(int m, int i, int j) const { return at((int64_t)m * plane + (int64_t)j * nrow + i); }
-    __device__ double at(int64_t k) const { return lvl ? (double)lvl[k] : scr[k]; }
+    __device__ double at(int64_t k) const { return (double)p[k]; }
     __device__ void store(int m, int i, int j, double v) const { put((int64_t)m * plane + (int64_t)j * nrow + i, v); }
-    __device__ void put(int64_t k, double v) const {
-        if (lvl) lvl[k] = (S)v; else scr[k] = v;
-    }
+    __device__ void put(int64_t k, double v) const { p[k] = (E)v; }
 };
 
-template <typename S>
-__device__ BufRef<S> bufref(const FillArgs& a, const FillProg& pr, int space, int64_t off, int nrow,
-                            int plane) {
-    BufRef<S> r;
-    r.lvl = space >= 0 ? static_cast<S*>(a.lvl_new[space]) + off : nullptr;
-    r.scr = space >= 0 ? nullptr : (space == FSP_SCRATCH ? pr.scratch : a.arena) + off;
-    r.nrow = nrow;
-    r.plane = plane;
-    return r;
+// what an operation other than FOP_COPY reads: always scratch or arena
+__device__ __forceinline__ Cells<const double> src_cells(const FillArgs& a, const FillProg& pr, const FillItem& op) {
+    return {(op.src_space == FSP_SCRATCH ? pr.scratch : a.arena) + op.src_off, op.src_nrow, op.src_plane};
+}
+
+// f(the operation's destination).  The kind is told apart here, once: asked for
+// at every element, it doubled the loads, stores and addresses in flight of the
+// FP32 kernels (151 registers, now 117 and 127; a ghost fill of a 1024^2 level 43.7
+// -> 31.4 us, of 64 grids of 32^2 22.3 -> 20.7, of 1,600 of 24^2 75.6 -> 70.6).
+template <typename S, class F>
+__device__ __forceinline__ void with_dst(const FillArgs& a, const FillProg& pr, const FillItem& op, const F& f) {
+    double* w = (op.dst_space == FSP_SCRATCH ? pr.scratch : a.arena) + op.dst_off;
+    if constexpr (sizeof(S) == sizeof(double)) {
+        if (op.dst_space >= 0) w = static_cast<double*>(a.lvl_new[op.dst_space]) + op.dst_off;
+        f(Cells<double>{w, op.dst_nrow, op.dst_plane});
+    } else if (op.dst_space >= 0) {
+        f(Cells<S>{static_cast<S*>(a.lvl_new[op.dst_space]) + op.dst_off, op.dst_nrow, op.dst_plane});
+    } else {
+        f(Cells<double>{w, op.dst_nrow, op.dst_plane});
+    }
 }
 
 // cell idx of the ring cstore.f walks: sides 1 (left column), 2 (top row), 3
@@ -96,8 +105,8 @@ struct Digits2 {
 
 // every element (cell x component) of a rectangle from `load` into `dst`,
 // four elements a thread in flight
-template <int NT, typename S, class Load>
-__device__ __forceinline__ void copy_rect(const FillItem& op, const BufRef<S>& dst, int tid, int nv,
+template <int NT, typename E, class Load>
+__device__ __forceinline__ void copy_rect(const FillItem& op, const Cells<E>& dst, int tid, int nv,
                                           const Load& load) {
     const int n = op.ni * op.nj * nv;
     Digits2<NT> u(tid, op.ni, op.nj);
@@ -118,9 +127,9 @@ __device__ __forceinline__ void copy_rect(const FillItem& op, const BufRef<S>& d
 // components n .. n + C - 1 of the interpolation at one fine cell: all the
 // coarse values are loaded before the first store (to an array the compiler
 // cannot tell apart from theirs)
-template <int C, typename S>
-__device__ __forceinline__ void interp_cell(const BufRef<S>& crs, const BufRef<S>& dst, int n, int64_t s,
-                                            int64_t d, double eta1, double eta2) {
+template <int C, typename E>
+__device__ __forceinline__ void interp_cell(const Cells<const double>& crs, const Cells<E>& dst, int n,
+                                            int64_t s, int64_t d, double eta1, double eta2) {
     double p10[C], m10[C], c0[C], p01[C], m01[C];
 #pragma unroll
     for (int k = 0; k < C; k++) {
@@ -154,8 +163,8 @@ struct BcSide { int ni, nj, i0, j0, ai, bi, aj, bj, flip; };
 // Components m0 .. m0 + C - 1 of B cells a thread in flight.  By cells, so that
 // the digits are stepped once a cell: the four sides of a 1024^2 grid of four
 // components take a ghost fill of 32 us, element by element 52.
-template <int NT, int C, int B, typename S>
-__device__ __forceinline__ void bc_cells(const BufRef<S>& b, const BcSide& sd, int tid, int m0) {
+template <int NT, int C, int B, typename E>
+__device__ __forceinline__ void bc_cells(const Cells<E>& b, const BcSide& sd, int tid, int m0) {
     const int n = sd.ni * sd.nj;
     Digits2<NT> u(tid, sd.ni, 1 << 30);   // (i, j) of a cell; j does not wrap
     for (int t = tid; t < n; t += B * NT) {
@@ -183,8 +192,8 @@ __device__ __forceinline__ void bc_cells(const BufRef<S>& b, const BcSide& sd, i
             }
     }
 }
-template <int NT, typename S>
-__device__ __forceinline__ void bc_side(const BufRef<S>& b, const BcSide& sd, int tid, int nv) {
+template <int NT, typename E>
+__device__ __forceinline__ void bc_side(const Cells<E>& b, const BcSide& sd, int tid, int nv) {
     int m = 0;
     for (; m + 4 <= nv; m += 4) bc_cells<NT, 4, 2>(b, sd, tid, m);
     if (nv - m == 3) bc_cells<NT, 3, 3>(b, sd, tid, m);
@@ -207,7 +216,6 @@ __device__ __forceinline__ FillItem uniform_item(const int32_t* sh) {
 template <typename S, int NT>
 __device__ __forceinline__ void fill_op(const FillArgs& a, const FillProg& pr, const FillItem& op, int tid) {
     const int nv = a.nv;
-    const BufRef<S> dst = bufref<S>(a, pr, op.dst_space, op.dst_off, op.dst_nrow, op.dst_plane);
     const int ncell = op.ni * op.nj;
 
     if (op.type == FOP_COPY) {
@@ -219,75 +227,83 @@ __device__ __forceinline__ void fill_op(const FillArgs& a, const FillProg& pr, c
         else if (op.flags & FOPF_BIG) mode = a.big_old ? TIME_OLD : TIME_NEW;
         const double ai = a.alphai[op.src_space], ac = a.alphac[op.src_space];
         const S* q1 = mode == TIME_OLD ? qo : qn;
-        if (mode != TIME_BLEND)
-            copy_rect<NT, S>(op, dst, tid, nv, [&](int64_t k) { return (double)q1[k]; });
-        else
-            copy_rect<NT, S>(op, dst, tid, nv, [&](int64_t k) { return (double)qn[k] * ai + (double)qo[k] * ac; });
+        with_dst<S>(a, pr, op, [&](const auto& dst) {
+            if (mode != TIME_BLEND)
+                copy_rect<NT>(op, dst, tid, nv, [&](int64_t k) { return (double)q1[k]; });
+            else
+                copy_rect<NT>(op, dst, tid, nv, [&](int64_t k) { return (double)qn[k] * ai + (double)qo[k] * ac; });
+        });
     } else if (op.type == FOP_INTERP) {
-        const BufRef<S> crs = bufref<S>(a, pr, op.src_space, op.src_off, op.src_nrow, op.src_plane);
+        const Cells<const double> crs = src_cells(a, pr, op);
         const double dxf = a.hx[op.level], dyf = a.hy[op.level];
         const double dxc = a.hx[op.level - 1], dyc = a.hy[op.level - 1];
         const double xlow_coarse = a.xlower + op.iplo * dxc;
         const double ylow_coarse = a.ylower + op.jplo * dyc;
         const double ratiox = (double)op.ratx, ratioy = (double)op.raty;
         const unsigned char* mask = pr.masks + op.mask_off;
-        Digits2<NT> u(tid, op.ni, 1 << 30);   // (i, j) of cell c; j does not wrap
-        for (int c = tid; c < ncell; c += NT, u.step()) {
-            if (mask[c]) continue;
-            const int jf = u.j + 1, if_ = u.i + 1;   // 1-based
-            const int j_coarse = (int)floor((double)(jf + op.jlo - 1) / ratioy) - op.jplo + 1;
-            const double ycent_coarse = ylow_coarse + ((double)j_coarse - .5) * dyc;
-            const double ycent_fine = a.ylower + ((double)(jf - 1 + op.jlo) + .5) * dyf;
-            const double eta2 = (ycent_fine - ycent_coarse) / dyc;
-            const int i_coarse = (int)floor((double)(if_ + op.ilo - 1) / ratiox) - op.iplo + 1;
-            const double xcent_coarse = xlow_coarse + ((double)i_coarse - .5) * dxc;
-            const double xcent_fine = a.xlower + ((double)(if_ - 1 + op.ilo) + .5) * dxf;
-            const double eta1 = (xcent_fine - xcent_coarse) / dxc;
-            const int64_t s = (int64_t)(j_coarse - 1) * crs.nrow + i_coarse - 1;
-            const int64_t d = op.dst_shift + (int64_t)u.j * dst.nrow + u.i;
-            int n = 0;
-            for (; n + 4 <= nv; n += 4) interp_cell<4, S>(crs, dst, n, s, d, eta1, eta2);
-            if (nv - n == 3) interp_cell<3, S>(crs, dst, n, s, d, eta1, eta2);
-            else if (nv - n == 2) interp_cell<2, S>(crs, dst, n, s, d, eta1, eta2);
-            else if (nv - n == 1) interp_cell<1, S>(crs, dst, n, s, d, eta1, eta2);
-        }
+        with_dst<S>(a, pr, op, [&](const auto& dst) {
+            Digits2<NT> u(tid, op.ni, 1 << 30);   // (i, j) of cell c; j does not wrap
+            for (int c = tid; c < ncell; c += NT, u.step()) {
+                if (mask[c]) continue;
+                const int jf = u.j + 1, if_ = u.i + 1;   // 1-based
+                const int j_coarse = (int)floor((double)(jf + op.jlo - 1) / ratioy) - op.jplo + 1;
+                const double ycent_coarse = ylow_coarse + ((double)j_coarse - .5) * dyc;
+                const double ycent_fine = a.ylower + ((double)(jf - 1 + op.jlo) + .5) * dyf;
+                const double eta2 = (ycent_fine - ycent_coarse) / dyc;
+                const int i_coarse = (int)floor((double)(if_ + op.ilo - 1) / ratiox) - op.iplo + 1;
+                const double xcent_coarse = xlow_coarse + ((double)i_coarse - .5) * dxc;
+                const double xcent_fine = a.xlower + ((double)(if_ - 1 + op.ilo) + .5) * dxf;
+                const double eta1 = (xcent_fine - xcent_coarse) / dxc;
+                const int64_t s = (int64_t)(j_coarse - 1) * crs.nrow + i_coarse - 1;
+                const int64_t d = op.dst_shift + (int64_t)u.j * dst.nrow + u.i;
+                int n = 0;
+                for (; n + 4 <= nv; n += 4) interp_cell<4>(crs, dst, n, s, d, eta1, eta2);
+                if (nv - n == 3) interp_cell<3>(crs, dst, n, s, d, eta1, eta2);
+                else if (nv - n == 2) interp_cell<2>(crs, dst, n, s, d, eta1, eta2);
+                else if (nv - n == 1) interp_cell<1>(crs, dst, n, s, d, eta1, eta2);
+            }
+        });
     } else if (op.type == FOP_FILVAL) {
         // src: the coarse patch grown by one coarse cell (ni x nj); dst: the
         // new grid; mask: its interior cells, row by row, 1 where an old
         // grid supplied the value (the reference's setflags test)
-        const BufRef<S> crs = bufref<S>(a, pr, op.src_space, op.src_off, op.src_nrow, op.src_plane);
+        const Cells<const double> crs = src_cells(a, pr, op);
         const int rx = op.ratx, ry = op.raty, mic = op.ni, mjc = op.nj;
         const int ncx = mic - 2, ncc = ncx * (mjc - 2), nx = ncx * rx;
         const unsigned char* mask = pr.masks + op.mask_off;
-        for (int t = tid; t < ncc * nv; t += NT) {
-            const int m = t / ncc, c = t - m * ncc;
-            const int jc = c / ncx + 1, ic = c - (jc - 1) * ncx + 1;   // 0-based, 1..mic-2
-            const double vc = crs.load(m, ic, jc);
-            const double vxp = crs.load(m, ic + 1, jc), vxm = crs.load(m, ic - 1, jc);
-            const double vyp = crs.load(m, ic, jc + 1), vym = crs.load(m, ic, jc - 1);
-            double s1p = vxp - vc, s1m = vc - vxm;
-            double slopex = fmin(fabs(s1p), fabs(s1m)) * copysign(1.0, vxp - vxm);
-            if (s1m * s1p <= 0.0) slopex = 0.0;
-            s1p = vyp - vc;
-            s1m = vc - vym;
-            double slopey = fmin(fabs(s1p), fabs(s1m)) * copysign(1.0, vyp - vym);
-            if (s1m * s1p <= 0.0) slopey = 0.0;
-            for (int jco = 1; jco <= ry; jco++) {
-                const double yoff = ((double)jco - 0.5) / (double)ry - 0.5;
-                const int jf = (jc - 1) * ry + jco - 1;                    // interior, 0-based
-                for (int ico = 1; ico <= rx; ico++) {
-                    const double xoff = ((double)ico - 0.5) / (double)rx - 0.5;
-                    const int if_ = (ic - 1) * rx + ico - 1;
-                    if (!mask[(int64_t)jf * nx + if_])
-                        dst.store(m, NGHOST + if_, NGHOST + jf, vc + xoff * slopex + yoff * slopey);
+        with_dst<S>(a, pr, op, [&](const auto& dst) {
+            for (int t = tid; t < ncc * nv; t += NT) {
+                const int m = t / ncc, c = t - m * ncc;
+                const int jc = c / ncx + 1, ic = c - (jc - 1) * ncx + 1;   // 0-based, 1..mic-2
+                const double vc = crs.load(m, ic, jc);
+                const double vxp = crs.load(m, ic + 1, jc), vxm = crs.load(m, ic - 1, jc);
+                const double vyp = crs.load(m, ic, jc + 1), vym = crs.load(m, ic, jc - 1);
+                double s1p = vxp - vc, s1m = vc - vxm;
+                double slopex = fmin(fabs(s1p), fabs(s1m)) * copysign(1.0, vxp - vxm);
+                if (s1m * s1p <= 0.0) slopex = 0.0;
+                s1p = vyp - vc;
+                s1m = vc - vym;
+                double slopey = fmin(fabs(s1p), fabs(s1m)) * copysign(1.0, vyp - vym);
+                if (s1m * s1p <= 0.0) slopey = 0.0;
+                for (int jco = 1; jco <= ry; jco++) {
+                    const double yoff = ((double)jco - 0.5) / (double)ry - 0.5;
+                    const int jf = (jc - 1) * ry + jco - 1;                    // interior, 0-based
+                    for (int ico = 1; ico <= rx; ico++) {
+                        const double xoff = ((double)ico - 0.5) / (double)rx - 0.5;
+                        const int if_ = (ic - 1) * rx + ico - 1;
+                        if (!mask[(int64_t)jf * nx + if_])
+                            dst.store(m, NGHOST + if_, NGHOST + jf, vc + xoff * slopex + yoff * slopey);
+                    }
                 }
             }
-        }
+        });
     } else if (op.type == FOP_COPYBACK) {
-        const BufRef<S> src = bufref<S>(a, pr, op.src_space, op.src_off, op.src_nrow, op.src_plane);
-        copy_rect<NT, S>(op, dst, tid, nv, [&](int64_t k) { return src.at(k); });
+        const Cells<const double> src = src_cells(a, pr, op);
+        with_dst<S>(a, pr, op, [&](const auto& dst) {
+            copy_rect<NT>(op, dst, tid, nv, [&](int64_t k) { return src.at(k); });
+        });
     } else if (op.type == FOP_RING) {
-        const BufRef<S> src = bufref<S>(a, pr, op.src_space, op.src_off, op.src_nrow, op.src_plane);
+        const Cells<const double> src = src_cells(a, pr, op);
         double* qc1d = a.lvl_reg[op.level] + op.dst_off;
         const int len = 2 * (op.ni - 2 + op.nj - 2);
         for (int t = tid; t < len * nv; t += NT) {
@@ -296,7 +312,8 @@ __device__ __forceinline__ void fill_op(const FillArgs& a, const FillProg& pr, c
         }
     } else if (op.type == FOP_COARSEN) {
         // coarsen.f:15-30: dst(i, j) = mean of src(2i..2i+1, 2j..2j+1)
-        const BufRef<S> src = bufref<S>(a, pr, op.src_space, op.src_off, op.src_nrow, op.src_plane);
+        const Cells<const double> src = src_cells(a, pr, op);
+        const Cells<double> dst{a.arena + op.dst_off, op.dst_nrow, op.dst_plane};
         for (int t = tid; t < ncell * nv; t += NT) {
             const int m = t / ncell, c = t - m * ncell;
             const int j = c / op.ni, i = c - j * op.ni;
@@ -309,22 +326,24 @@ __device__ __forceinline__ void fill_op(const FillArgs& a, const FillProg& pr, c
         // extrapolation (1) or mirrored (wall, 3).  One loop over the sides, not
         // four copies of its body: the FP32 kernel would keep its arguments in
         // scratch (1.2 KB a lane, six times the time).
-        const int nrow = op.ni, ncol = op.nj;
+        with_dst<S>(a, pr, op, [&](const auto& dst) {
+            const int nrow = op.ni, ncol = op.nj;
 #pragma unroll 1
-        for (int side = 0; side < 4; side++) {
-            if (side > 0) __syncthreads();
-            // cells on a low side, the 1-based first column / row of a high one
-            const int w = side == 0 ? op.bc[0] : (side == 1 ? op.bc[1] : (side == 2 ? op.bc[2] : op.bc[3]));
-            const int kind = a.mthbc[side];
-            if (w <= 0 || (kind != 1 && kind != 3)) continue;
-            const bool high = side & 1, y = side >= 2, wall = kind == 3;
-            const int n = high ? (y ? ncol : nrow) - w + 1 : w, from = high ? w - 1 : 0;
-            const int mul = wall ? -1 : 0;
-            const int add = wall ? (high ? 2 * w - 3 : 2 * w - 1) : (high ? w - 2 : w);
-            BcSide sd{n, ncol, from, 0, mul, add, 1, 0, wall ? 1 : -1};
-            if (y) sd = BcSide{nrow, n, 0, from, 1, 0, mul, add, wall ? 2 : -1};
-            bc_side<NT>(dst, sd, tid, nv);
-        }
+            for (int side = 0; side < 4; side++) {
+                if (side > 0) __syncthreads();
+                // cells on a low side, the 1-based first column / row of a high one
+                const int w = side == 0 ? op.bc[0] : (side == 1 ? op.bc[1] : (side == 2 ? op.bc[2] : op.bc[3]));
+                const int kind = a.mthbc[side];
+                if (w <= 0 || (kind != 1 && kind != 3)) continue;
+                const bool high = side & 1, y = side >= 2, wall = kind == 3;
+                const int n = high ? (y ? ncol : nrow) - w + 1 : w, from = high ? w - 1 : 0;
+                const int mul = wall ? -1 : 0;
+                const int add = wall ? (high ? 2 * w - 3 : 2 * w - 1) : (high ? w - 2 : w);
+                BcSide sd{n, ncol, from, 0, mul, add, 1, 0, wall ? 1 : -1};
+                if (y) sd = BcSide{nrow, n, 0, from, 1, 0, mul, add, wall ? 2 : -1};
+                bc_side<NT>(dst, sd, tid, nv);
+            }
+        });
     }
 }
 

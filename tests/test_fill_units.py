@@ -81,6 +81,9 @@ static bool check(const FillPlan& P, const HierGeom& H, const char* what) {
         if (P.units[u].item0 != at || P.units[u].n < 1) return std::printf("%s: units\n", what), false;
         for (int k = 0; k < P.units[u].n; k++, at++) {
             const int o = P.order[at];
+            // what an operation other than a copy reads is FP64 scratch or arena
+            if (P.ops[o].type != FOP_COPY && P.ops[o].type != FOP_BC && P.bufs[P.ops[o].src].kind == 0)
+                return std::printf("%s: operation %d (type %d) reads a level\n", what, o, P.ops[o].type), false;
             if (unit[o] >= 0) return std::printf("%s: twice\n", what), false;
             unit[o] = u;
             if (k > 0 && P.ops[P.order[at - 1]].stage > P.ops[o].stage)

@@ -1,7 +1,7 @@
-"""CPU check of what the built kernels keep in scratch (private memory in HBM), read
-from the metadata of the library's own gfx950 code objects: a kernel that the
-compiler gave room for its arguments there runs several times slower, with the
-same results."""
+"""CPU check of the scratch (private memory in HBM) and the registers of the built
+kernels, read from the metadata of the library's own gfx950 code objects: a kernel
+that the compiler gave room for its arguments in scratch, or many more registers
+than it needs, runs slower, with the same results."""
 import os
 import re
 import struct
@@ -33,7 +33,7 @@ def code_objects(blob):
 
 @pytest.mark.skipif(not os.path.exists(READELF), reason="no llvm-readelf")
 def test_scratch_of_the_kernels():
-    scratch = {}
+    scratch, vgprs = {}, {}
     blob = open(capi.LIBPATH, "rb").read()
     with tempfile.TemporaryDirectory() as d:
         for k, co in enumerate(code_objects(blob)):
@@ -42,12 +42,14 @@ def test_scratch_of_the_kernels():
             notes = subprocess.run([READELF, "--notes", f], capture_output=True, text=True,
                                    check=True).stdout
             # (a kernel's keys stand in alphabetical order: its name before its
-            # private_segment_fixed_size)
+            # private_segment_fixed_size and vgpr_count)
             name = None
-            for key, value in re.findall(r"\.(name|private_segment_fixed_size):\s+(\S+)", notes):
-                if key == "private_segment_fixed_size" and name:
-                    scratch[name] = int(value)
-                name = value if key == "name" and value.startswith("_Z") else name
+            for key, value in re.findall(r"\.(name|private_segment_fixed_size|vgpr_count):\s+(\S+)",
+                                         notes):
+                if key == "name":
+                    name = value if value.startswith("_Z") else name
+                elif name:
+                    (vgprs if key == "vgpr_count" else scratch)[name] = int(value)
     fill = {n: v for n, v in scratch.items() if "fill_kernel" in n}
     assert len(fill) == 4 and len(scratch) > 100, (len(fill), len(scratch))
     # the kernels of every step; a few spilled scalar registers are no loss
@@ -56,3 +58,5 @@ def test_scratch_of_the_kernels():
         sizes = {n: v for n, v in scratch.items() if part in n}
         assert sizes and max(sizes.values()) <= 256, sizes
     assert max(fill.values()) <= 64, fill
+    # four waves a SIMD: the fill waits for its loads
+    assert max(vgprs[n] for n in fill) <= 128, {n: vgprs[n] for n in fill}
